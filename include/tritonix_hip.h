@@ -231,6 +231,8 @@ typedef struct tnx_conv2d_args {
   int32_t out_f32;     /* non-zero: `output` is binary32, the fp32 sums (+ bias) unrounded -- what makes a float32
                           convolution a three-term bf16 one: split the input along its channels with
                           tnx_split_f32(side 0) and the weight with side 2, tripling c_in                    */
+  void* workspace;     /* device scratch for the packed route, 256-byte aligned; NULL = do not take it       */
+  size_t workspace_bytes;
 } tnx_conv2d_args;
 
 /* How the slabs reach LDS.  Two kernels exist: one stages both operands through registers (any stride, padding,
@@ -254,6 +256,14 @@ enum tnx_conv_loader {
 
 /* Launch one conv2d forward.  Returns a tnx_status.  Asynchronous, allocates nothing. */
 int tnx_conv2d_forward(const tnx_conv2d_args* args);
+
+/* Scratch bytes of the packed route for these args (TNX_CONV_LOADER_AUTO and no tile given), or 0 where the library
+ * does not take it: input and weight are copied into a channels-last layout with the zero padding written out, and
+ * the convolution is one GEMM launch over that -- any stride, padding, dilation and channel count.  Give a workspace
+ * of at least this size (no initialisation needed) in args->workspace and tnx_conv2d_forward takes the route; without one it
+ * runs the kernels above.  With a workspace, dtype may be TNX_F32 (input, weight and output binary32, out_f32 set):
+ * the copy then cuts the operands into their bf16 terms.  Calls that share a workspace must be ordered. */
+size_t tnx_conv2d_workspace_bytes(const tnx_conv2d_args* args);
 
 /* TNX_OK if tnx_conv2d_forward would accept these args (pointers are not inspected, apart from their
  * alignment), otherwise the status it would return.  Pure host arithmetic. */

@@ -30,7 +30,8 @@ CONV_LOADER_AUTO, CONV_LOADER_REGISTERS, CONV_LOADER_DMA, CONV_LOADER_GEMM = 0, 
 
 EXPORTS = ("tnx_gemm", "tnx_gemm_static_workspace", "tnx_gemm_workspace_bytes", "tnx_gemm_lds_bytes", "tnx_gemm_supported",
            "tnx_gemm_default_config", "tnx_tile_coords", "tnx_split_f32", "tnx_kernel_count", "tnx_kernel_name", "tnx_strerror",
-           "tnx_last_hip_error", "tnx_version", "tnx_conv2d_forward", "tnx_conv2d_supported", "tnx_conv2d_output_size",
+           "tnx_last_hip_error", "tnx_version", "tnx_conv2d_forward", "tnx_conv2d_workspace_bytes", "tnx_conv2d_supported",
+           "tnx_conv2d_output_size",
            "tnx_conv2d_default_config", "tnx_conv2d_kernel_count", "tnx_conv2d_kernel_name")
 
 
@@ -64,6 +65,7 @@ class Conv2dArgs(ctypes.Structure):
         ("block_pixels", ctypes.c_int32), ("block_cout", ctypes.c_int32), ("block_k", ctypes.c_int32),
         ("group_pixels", ctypes.c_int32), ("loader", ctypes.c_int32),
         ("stream", ctypes.c_void_p), ("out_f32", ctypes.c_int32),
+        ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_size_t),
     ]
 
 
@@ -111,6 +113,8 @@ def load() -> ctypes.CDLL:
     for name in ("tnx_conv2d_forward", "tnx_conv2d_supported", "tnx_conv2d_default_config"):
         getattr(lib, name).argtypes = [cp]
         getattr(lib, name).restype = ctypes.c_int
+    lib.tnx_conv2d_workspace_bytes.argtypes = [cp]
+    lib.tnx_conv2d_workspace_bytes.restype = ctypes.c_size_t
     lib.tnx_conv2d_output_size.argtypes = [cp, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
     lib.tnx_conv2d_output_size.restype = None
     lib.tnx_conv2d_kernel_count.argtypes = []

@@ -144,6 +144,37 @@ def conv_instance_list(quick=False):
     return out
 
 
+# (block_cout, block_pixels, waves, ring slots) of the packed conv2d kernels, block_k = 64.  Widths between 128 and 256
+# pixels: what divides a layer into whole rounds of the 256 CUs (256 channels, batch 32, 56x56: 392 tiles of 256 pixels,
+# 448 of 224: two rounds each, the second shorter).
+GATHER_TILES = ((256, 256, 8, 2), (256, 224, 8, 2), (256, 192, 8, 2), (256, 128, 8, 3), (128, 256, 8, 3), (128, 128, 8, 3), (128, 128, 8, 2),
+                (64, 256, 8, 3), (64, 128, 8, 3), (64, 128, 4, 3), (64, 64, 4, 4))
+
+
+def generate_gather(tiles, gen):
+    """Instance files of the packed conv2d kernels (one per dtype and tile) and their table."""
+    files, names = [], []
+    for dt in ("bf16", "f16"):
+        for bm, bn, nw, st in tiles:
+            name = f"gather_{dt}_c{bm}_p{bn}_w{nw}_s{st}"
+            text = (f'// generated by tritonix_amd/build.py -- do not edit\n#include "{CSRC}/registry.h"\n'
+                    f"namespace tnx {{\nstatic GatherEntry k_{name}[] = {{\n    TNX_GATHER_ENTRY({TAGS[dt][0]}, {bm}, {bn}, {nw}, {st})\n}};\n"
+                    f"GatherGroup g_{name} = {{k_{name}, 1}};\n}}\n")
+            path = os.path.join(gen, name + ".hip")
+            write_if_changed(path, text)
+            files.append(path)
+            names.append(name)
+    decl = "\n".join(f"extern GatherGroup g_{n};" for n in names)
+    ptrs = ", ".join(f"&g_{n}" for n in names) or "nullptr"
+    text = (f'// generated by tritonix_amd/build.py -- do not edit\n#include "{CSRC}/registry.h"\nnamespace tnx {{\n{decl}\n}}\n'
+            f"using namespace tnx;\n"
+            f'extern "C" const GatherGroup* const* tnx_gather_groups(int* n) {{\n'
+            f"  static const GatherGroup* const all[] = {{{ptrs}}};\n  *n = {len(names)};\n  return all;\n}}\n")
+    path = os.path.join(gen, "gather_groups.hip")
+    write_if_changed(path, text)
+    return files + [path]
+
+
 def parse_only_conv(spec):
     """'bf16:128:128:64,...' (dtype:block_cout:block_pixels:block_k) for development builds."""
     out = []
@@ -279,7 +310,7 @@ _resources = {}
 
 def _compile(src, obj, verbose, force=True):
     deps = [src, os.path.join(CSRC, "gemm_tile.h"), os.path.join(CSRC, "gemm_skinny.h"), os.path.join(CSRC, "registry.h"),
-            os.path.join(CSRC, "conv_tile.h"),
+            os.path.join(CSRC, "conv_tile.h"), os.path.join(CSRC, "conv_pack.h"),
             os.path.join(ROOT, "include", "tritonix_hip.h"), os.path.abspath(__file__)]
     if not force and os.path.exists(obj) and os.path.getmtime(obj) > max(os.path.getmtime(d) for d in deps):
         return obj
@@ -304,11 +335,11 @@ def _compile(src, obj, verbose, force=True):
 
 def demangled_tile(name):
     """'bf16 256x256x64 w4 s2 fast' from a mangled gemm_tile_kernel instantiation (None for other kernels)."""
-    m = re.search(r"gemm_tile_kernelINS_(\d)Tag(\w+?)ENS_7TileCfgIS1_Li(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)EEELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
+    m = re.search(r"gemm_tile_kernelINS_(\d)Tag(\w+?)ENS_7TileCfgIS1_Li(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)EEELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
     if not m:
         return None
-    _, tag, bm, bn, bk, nw, st, fast, persist, bt, conv = m.groups()
-    kind = "conv" if conv == "1" else "bt" if bt == "1" else "persistent" if persist == "1" else "fast" if fast == "1" else "generic"
+    _, tag, bm, bn, bk, nw, st, fast, persist, bt, conv, gather = m.groups()
+    kind = "packed conv" if gather == "1" else "conv" if conv == "1" else "bt" if bt == "1" else "persistent" if persist == "1" else "fast" if fast == "1" else "generic"
     return f"{tag.lower()} {bm}x{bn}x{bk} w{nw} s{st} {kind}"
 
 
@@ -319,13 +350,14 @@ def build(jobs=None, quick=False, verbose=True, force=True, only=None, out=None,
     ``-D`` macros; they use their own object directory so the full build's objects stay valid."""
     global BUILD
     jobs = jobs or min(8, os.cpu_count() or 1)
-    instances = parse_only(only) if only else ([] if only_conv else instance_list(quick=quick))
+    instances = [] if only == "gather" else parse_only(only) if only else ([] if only_conv else instance_list(quick=quick))
     conv_instances = parse_only_conv(only_conv) if only_conv else ([] if only else conv_instance_list(quick=quick))
     lib = out or LIB
     if only or only_conv or out or defines:
         BUILD = os.path.join(ROOT, "build", "dev_" + os.path.basename(lib).replace(".", "_"))
     DEVICE_FLAGS.extend(f"-D{d}" for d in defines)
-    srcs = generate(instances) + generate_conv(conv_instances, os.path.join(BUILD, "gen")) + [
+    srcs = generate(instances) + generate_conv(conv_instances, os.path.join(BUILD, "gen")) + generate_gather(
+        GATHER_TILES if not (only or only_conv) or only == "gather" else (), os.path.join(BUILD, "gen")) + [
         os.path.join(CSRC, "capi.hip"), os.path.join(CSRC, "skinny.hip"),
         os.path.join(CSRC, "conv.hip")]
     objdir = os.path.join(BUILD, "obj")

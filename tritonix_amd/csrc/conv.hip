@@ -5,6 +5,7 @@
 #include <string.h>
 
 #include "../../include/tritonix_hip.h"
+#include "conv_pack.h"
 #include "conv_tile.h"
 #include "registry.h"
 
@@ -12,6 +13,7 @@ using namespace tnx;
 
 extern "C" const ConvGroup* tnx_conv_groups(int* ngroups);      // generated
 extern "C" const KernelGroup* tnx_kernel_groups(int* ngroups);  // generated
+extern "C" const GatherGroup* const* tnx_gather_groups(int* ngroups);  // generated
 
 // The GEMM kernel's conv2d variant for this tile (three ring slots), or null.  Eight waves are preferred (and the
 // only ones built): the loader's address arithmetic and the fix-up are vector instructions in the MFMA stream, and
@@ -347,6 +349,203 @@ static void fill_dma(const tnx_conv2d_args* a, const Resolved& r, GemmParams* p,
   *grid = (unsigned)((int64_t)p->tiles_m * p->tiles_n);
 }
 
+// ---------------------------------------------------------------------------
+// packed route: one pass lays input and weight out (conv_pack.h), one GEMM launch over them.  Bound by the GEMM (MFMA and
+// the start and end of its tiles) on wide layers, by the two launches on small ones.  Measured against the kernels that
+// gather taps themselves, whole call, bf16/f16, 3x3: 256 channels of 56x56, batch 32: 155 -> 114 us (pass 18, GEMM 96:
+// 1230 TFLOP/s); 128 channels of 56x56, stride 2: 42.8 -> 22.8; 512 of 7x7, batch 8: 137 -> 23; float32, 256 of 14x14: 242 -> 23.
+// ---------------------------------------------------------------------------
+struct PackedPlan {
+  const GatherEntry* e;
+  int split;                       // K slices per tile
+  int h_out, w_out;
+  int rows, cols, step_h, step_w;  // packed image; input rows / columns per packed row / column
+  int terms, cp8, chunks, kt;      // bf16 terms per element; channel groups of 8 per term; k chunks; K slabs
+  int hwp;
+  int64_t n_total;
+  int64_t slices_bytes, w_bytes, x_bytes;     // workspace: counters and K slices, weight, input
+  int64_t total_bytes;
+};
+
+// microseconds per round of workgroups and per K slab of one, and workgroups that share a CU, per packed tile
+struct GatherCost {
+  int bm, bn, nw, stages;
+  double fixed, slab;
+  int per_cu;
+};
+static const GatherCost GATHER_COST[] = {
+    {256, 256, 8, 2, 9.5, 1.12, 1}, {256, 224, 8, 2, 8.2, 1.03, 1}, {256, 192, 8, 2, 5.8, 0.92, 1}, {256, 128, 8, 3, 5.2, 0.555, 1},
+    {128, 256, 8, 3, 5.1, 0.584, 1}, {128, 128, 8, 3, 3.1, 0.341, 1}, {128, 128, 8, 2, 2.9, 0.935, 2}, {64, 256, 8, 3, 2.8, 0.422, 1},
+    {64, 128, 8, 3, 1.8, 0.483, 2}, {64, 128, 4, 3, 2.6, 0.481, 2}, {64, 64, 4, 4, 1.3, 0.272, 2}};
+static const GatherCost* gather_cost(const GatherEntry& e) {
+  for (const GatherCost& c : GATHER_COST)
+    if (c.bm == e.bm && c.bn == e.bn && c.nw == e.nw && c.stages == e.stages) return &c;
+  return nullptr;
+}
+
+static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
+
+static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p) {
+  if (!a || a->loader != TNX_CONV_LOADER_AUTO || a->block_cout || a->block_pixels || a->block_k) return false;
+  tnx_conv2d_args t = *a;
+  const bool f32 = a->dtype == TNX_F32;
+  if (f32) t.dtype = TNX_BF16;
+  int32_t h_out = 0, w_out = 0;
+  if (check_problem(&t, &h_out, &w_out) != TNX_OK) return false;
+  if (f32 ? a->out_f32 == 0 : gemm_problem_ok(a)) return false;
+  // The pass over the operands costs about 4 us of its own, which a short K loop does not pay back: measured on 120 layers,
+  // the kernels that gather for themselves win below 145 multiply-adds per output (3 channels 3x3: 6.4-8.7 against
+  // 10.2-11.7 us; 16 channels 3x3: 8.8 / 11.7), the packed route above (17 channels: 15.5 / 11.9, 24: 13.0 / 11.9, 64 at
+  // 56x56: 38 / 31).  A 1x1 filter (here with a stride) reads every input element once either way, so its line lies higher
+  // (256 channels, 56x56: 20.0 / 24.0; 512, 28x28: 23.6 / 19.1).  float32 has three terms per element and its alternative
+  // an extra pass over both operands.
+  const int64_t macs = (int64_t)a->c_in * a->filter_h * a->filter_w;
+  if (f32 ? macs <= 48 : macs <= (a->filter_h * a->filter_w == 1 ? 256 : 144)) return false;
+  *p = PackedPlan{};
+  p->h_out = h_out; p->w_out = w_out;
+  // a filter one row high reads only every stride_h-th input row: only those are packed (likewise for columns)
+  p->step_h = a->filter_h == 1 ? a->stride_h : 1;
+  p->step_w = a->filter_w == 1 ? a->stride_w : 1;
+  const int sh = a->filter_h == 1 ? 1 : a->stride_h, sw = a->filter_w == 1 ? 1 : a->stride_w;
+  p->rows = (h_out - 1) * sh + (a->filter_h - 1) * a->dil_h + 1;
+  p->cols = (w_out - 1) * sw + (a->filter_w - 1) * a->dil_w + 1;
+  p->terms = f32 ? 3 : 1;
+  p->cp8 = (a->c_in + 7) / 8;
+  const int64_t taps = (int64_t)a->filter_h * a->filter_w * p->terms;
+  // the kernel's offset table has one entry per k chunk (it reads one slab past the end), or one per slab where a filter
+  // tap's channels are whole slabs: a long k is padded to that
+  if (p->cp8 * p->terms % 8 && ((taps * p->cp8 + 7) / 8 + 1) * 32 > GATHER_TABLE_BYTES) p->cp8 = (p->cp8 + 7) / 8 * 8;
+  const int64_t chunks = taps * p->cp8, kt = (chunks + 7) / 8;
+  if ((p->cp8 * p->terms % 8 ? (kt + 1) * 8 : kt + 1) * 4 > GATHER_TABLE_BYTES) return false;
+  p->chunks = (int)chunks; p->kt = (int)kt;
+  p->hwp = (h_out * w_out + 7) / 8 * 8;
+  p->n_total = (int64_t)a->batch * p->hwp;
+  p->x_bytes = (int64_t)a->batch * p->rows * p->cols * p->terms * p->cp8 * 16;
+  p->w_bytes = (int64_t)a->c_out * kt * 128;
+  const int64_t lim = (1ll << 31) - 4096;
+  if (p->n_total >= lim || p->x_bytes >= lim || p->w_bytes >= lim || (int64_t)a->c_out * kt * 8 >= lim) return false;
+
+  // Tile and K cut with the smallest modelled time: rounds of workgroups x (fixed + per K slab), with the constants of
+  // GATHER_COST; a round is one workgroup per CU, two where two fit its LDS, and a last, partial one costs 0.9 of a
+  // full one.  A K cut adds its hand-over.  Constants and form are a least-squares fit to 1,500 measured (layer, tile, cut)
+  // triples on 120 layers; choosing by it costs 1.5 % against the best measured tile in the mean, 12 % at worst on
+  // all but one.
+  double best = 1e300;
+  int ng = 0;
+  const GatherGroup* const* g = tnx_gather_groups(&ng);
+  for (int i = 0; i < ng; ++i)
+    for (int j = 0; j < g[i]->count; ++j) {
+      const GatherEntry& e = g[i]->entries[j];
+      if (e.dtype != t.dtype) continue;
+      const GatherCost* cost = gather_cost(e);
+      if (!cost) continue;
+      const int64_t tiles = ((a->c_out + e.bm - 1) / e.bm) * ((p->n_total + e.bn - 1) / e.bn);
+      const double area = e.bm * e.bn / 65536.0;
+      for (int s = 1; s <= 16; s *= 2) {
+        if (s > 1 && (kt / s < 4 || tiles * s > 512)) break;
+        const int64_t slots = 256 * cost->per_cu, full = tiles * s / slots, rem = tiles * s % slots;
+        double rounds = (double)full;
+        if (rem) rounds += rem > 256 * (cost->per_cu - 1) ? 0.9 : 0.9 * (0.5 + 0.5 * (double)rem / (double)slots);
+        double c = rounds * (cost->fixed + cost->slab * (double)((kt + s - 1) / s));
+        if (s > 1) c += 2.2 + 3.0 * s * area + 1.8 * area;
+        if (c < best) { best = c; p->e = &e; p->split = s; }
+      }
+    }
+  if (!p->e) return false;
+  const int64_t tiles = ((a->c_out + p->e->bm - 1) / p->e->bm) * ((p->n_total + p->e->bn - 1) / p->e->bn);
+  if (tiles * p->split >= lim || (p->split > 1 && tiles > WS_MAX_TILES)) return false;
+  p->slices_bytes = p->split > 1 ? WS_COUNTER_BYTES + (int64_t)p->split * tiles * p->e->bm * p->e->bn * 4 : 0;
+  if (p->slices_bytes >= (1ll << 32)) return false;
+  p->total_bytes = up256(p->slices_bytes) + up256(p->w_bytes) + up256(p->x_bytes);
+  return true;
+}
+
+extern "C" size_t tnx_conv2d_workspace_bytes(const tnx_conv2d_args* a) {
+  PackedPlan p;
+  return packed_plan(a, &p) ? (size_t)p.total_bytes : 0;
+}
+
+static int packed_forward(const tnx_conv2d_args* a, const PackedPlan& pl) {
+  uint8_t* ws = (uint8_t*)a->workspace;
+  uint8_t* wp = ws + up256(pl.slices_bytes);
+  uint8_t* xp = wp + up256(pl.w_bytes);
+  const int cpt = pl.cp8 * pl.terms;
+  const bool f32 = a->dtype == TNX_F32;
+  const GatherEntry& e = *pl.e;
+  const int64_t tiles_m = (a->c_out + e.bm - 1) / e.bm, tiles_n = (pl.n_total + e.bn - 1) / e.bn;
+
+  PackParams k;
+  memset(&k, 0, sizeof k);
+  k.x = (const uint8_t*)a->input; k.w = (const uint8_t*)a->weight; k.xp = xp; k.wp = wp;
+  if (pl.split > 1) { k.counters = (int*)ws; k.ncounters = (int)(tiles_m * tiles_n); }
+  k.c_in = a->c_in; k.h_in = a->h_in; k.w_in = a->w_in; k.taps = a->filter_h * a->filter_w;
+  k.rows = pl.rows; k.cols = pl.cols; k.step_h = pl.step_h; k.step_w = pl.step_w;
+  k.pad_h = a->pad_h; k.pad_w = a->pad_w;
+  k.cp8 = pl.cp8; k.chunks = pl.chunks; k.chunks_pad = pl.kt * 8;
+  // columns that can hold input: the chunks cover those, `lead` padding columns before them
+  k.lead = pl.step_w == 1 && a->pad_w < pl.cols ? a->pad_w : 0;
+  const int inside = pl.step_w == 1 && a->pad_w < pl.cols ? (a->w_in < pl.cols - k.lead ? a->w_in : pl.cols - k.lead) : pl.cols;
+  k.wchunks = (inside + 7) / 8;
+  k.whole = cpt % 8 == 0;
+  k.div_taps = make_fastdiv((uint32_t)(a->filter_h * a->filter_w));
+  k.cgb = (pl.cp8 + 7) / 8;
+  const int64_t x_items = (int64_t)a->batch * pl.rows * k.wchunks, waves = (x_items + 7) / 8 * k.cgb;
+  const int64_t w_items = (int64_t)a->c_out * k.chunks_pad;
+  if (x_items >= (1ll << 31) || waves >= (1ll << 31)) return TNX_E_UNSUPPORTED;
+  k.x_items = (int)x_items;
+  k.w_items = (int)w_items;
+  k.x_elems = (int)((int64_t)a->batch * a->c_in * a->h_in * a->w_in);
+  const int64_t w_threads = w_items > k.ncounters ? w_items : k.ncounters;
+  k.w_blocks = (unsigned)((w_threads + 255) / 256);
+  k.div_cgb = make_fastdiv((uint32_t)k.cgb);
+  k.div_row = make_fastdiv((uint32_t)pl.rows);
+  k.div_wchunks = make_fastdiv((uint32_t)k.wchunks);
+  k.div_cpt = make_fastdiv((uint32_t)cpt);
+  k.div_cp8 = make_fastdiv((uint32_t)pl.cp8);
+  k.div_chunks = make_fastdiv((uint32_t)k.chunks_pad);
+  const unsigned blocks = k.w_blocks + (unsigned)((waves + 3) / 4);
+  hipStream_t stream = (hipStream_t)a->stream;
+  if (f32) hipLaunchKernelGGL((conv_pack_kernel<float>), dim3(blocks), dim3(256), 0, stream, k);
+  else hipLaunchKernelGGL((conv_pack_kernel<uint16_t>), dim3(blocks), dim3(256), 0, stream, k);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) { note_hip_error((int)err); return TNX_E_HIP; }
+
+  GemmParams p;
+  memset(&p, 0, sizeof p);
+  p.a = wp; p.b = xp; p.c = (uint8_t*)a->output; p.ws = ws;
+  p.m = a->c_out; p.n = pl.n_total; p.k = (int64_t)pl.kt * 64;
+  p.sam = p.k; p.sak = 1; p.sbk = 1; p.sbn = 0;
+  p.tiles_m = (int)tiles_m; p.tiles_n = (int)tiles_n;
+  p.group_m = 8;
+  p.split_k = pl.split;
+  p.ktiles_per_split = (pl.kt + pl.split - 1) / pl.split;
+  p.out_dtype = f32 || a->out_f32 ? TNX_F32 : a->dtype;
+  const int hw_out = pl.h_out * pl.w_out;
+  // the output side is conv2d's epilogue on planes of one row of hwp pixels
+  ConvGeom& g = p.cv;
+  g.c_out = a->c_out; g.h_out = 1; g.w_out = hw_out; g.wp = pl.hwp;
+  g.n_total = (int)pl.n_total;
+  g.div_hwp = g.div_wp = make_fastdiv((uint32_t)pl.hwp);
+  g.bias = (const uint8_t*)a->bias;
+  g.bias_dtype = a->bias_dtype;
+  PackGeom& q = p.pk;
+  q.hw_out = hw_out; q.hwp = pl.hwp; q.w_out = pl.w_out;
+  q.div_hwp = g.div_hwp; q.div_w = make_fastdiv((uint32_t)pl.w_out);
+  const uint32_t px = (uint32_t)cpt * 16u;             // bytes of one packed pixel
+  q.img_bytes = (uint32_t)pl.rows * (uint32_t)pl.cols * px;
+  q.row_bytes = (uint32_t)(a->filter_h == 1 ? 1 : a->stride_h) * (uint32_t)pl.cols * px;
+  q.col_bytes = (uint32_t)(a->filter_w == 1 ? 1 : a->stride_w) * px;
+  q.chunks = pl.chunks; q.cpt = cpt; q.fw = a->filter_w; q.taps = a->filter_h * a->filter_w;
+  q.div_taps = k.div_taps;
+  q.div_cpt = k.div_cpt; q.div_fw = make_fastdiv((uint32_t)a->filter_w);
+  q.tap_row_bytes = (uint32_t)a->dil_h * (uint32_t)pl.cols * px;
+  q.tap_col_bytes = (uint32_t)a->dil_w * px;
+  q.x_bytes = (uint32_t)pl.x_bytes;
+  err = e.launch(p, (unsigned)(tiles_m * tiles_n * pl.split), stream);
+  if (err != hipSuccess) { note_hip_error((int)err); return TNX_E_HIP; }
+  return TNX_OK;
+}
+
 extern "C" int tnx_conv2d_supported(const tnx_conv2d_args* a) {
   Resolved r;
   return resolve(a, &r, false);
@@ -368,6 +567,17 @@ extern "C" int tnx_conv2d_default_config(tnx_conv2d_args* a) {
 }
 
 extern "C" int tnx_conv2d_forward(const tnx_conv2d_args* a) {
+  if (a && a->workspace) {
+    PackedPlan pl;
+    if (packed_plan(a, &pl)) {
+      if (a->workspace_bytes < (size_t)pl.total_bytes || ((uintptr_t)a->workspace & 255)) return TNX_E_WORKSPACE;
+      const unsigned in_align = a->dtype == TNX_F32 ? 3 : 1, out_align = a->out_f32 ? 3 : 1;
+      if (!a->input || !a->weight || !a->output || ((uintptr_t)a->input & in_align) || ((uintptr_t)a->weight & in_align) ||
+          ((uintptr_t)a->output & out_align) || (a->bias && ((uintptr_t)a->bias & (a->bias_dtype == TNX_F32 ? 3 : 1))))
+        return TNX_E_INVALID;
+      return packed_forward(a, pl);
+    }
+  }
   Resolved r;
   const int st = resolve(a, &r, true);
   if (st != TNX_OK) return st;

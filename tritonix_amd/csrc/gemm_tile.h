@@ -96,6 +96,22 @@ struct ConvGeom {
   int bias_dtype;
 };
 
+// Geometry of a conv2d forward over a packed input (gemm_tile_kernel<..., GATHER>): the input has been copied to
+// [image][row][column][channel], channels in groups of eight, with its zero padding written out, and the weight to
+// [c_out][filter tap][channel].  The B operand is then k-contiguous: row n of a slab is 128 bytes of pixel n's window,
+// found at (offset of the pixel) + (offset of the slab's filter tap and channels), and nothing in the loader depends
+// on the stride, the dilation or where the image ends.
+struct PackGeom {
+  int hw_out, hwp, w_out;          // pixels of an output plane, the same rounded up to 8, width of an output row
+  FastDiv div_hwp, div_w;
+  uint32_t img_bytes, row_bytes, col_bytes;   // packed input: one image, one output row, one output column further
+  int chunks, cpt, fw;             // 16-byte chunks of k that exist, chunks per filter tap, filter width
+  int taps;                        // filter height * width
+  FastDiv div_cpt, div_fw, div_taps;
+  uint32_t tap_row_bytes, tap_col_bytes;      // one filter row, one filter column further
+  uint32_t x_bytes;                // size of the packed input (< 2^31)
+};
+
 struct GemmParams {
   const uint8_t* a;
   const uint8_t* b;
@@ -121,6 +137,7 @@ struct GemmParams {
   int batch;              // uncut, non-persistent launches of tiles up to 128x128: the grid holds `batch` problems that share A (0 or 1: one problem);
   int64_t b_batch_bytes, c_batch_bytes;   // problem i reads B + i * b_batch_bytes and writes C + i * c_batch_bytes
   ConvGeom cv;            // read by the CONV kernels; cv.bias / cv.bias_dtype also by the plain epilogue (a bias per row of C)
+  PackGeom pk;            // read by the GATHER kernels (with cv's output side)
 };
 
 // ---------------------------------------------------------------------------
@@ -359,7 +376,8 @@ struct TileCfg {
   static constexpr int ES = T::ES;
   static constexpr int BM = BM_, BN = BN_, BK = BK_, NW = NW_, STAGES = STAGES_;
   static constexpr int THREADS = NW * 64;
-  static constexpr int WGM = (NW == 4) ? 2 : (BM > BN ? 4 : 2);  // wave grid
+  // wave grid: 2 x 2 / 4 x 2 / 2 x 4; widths that no 16-column MFMA tile halves keep every wave on all columns
+  static constexpr int WGM = (NW == 4) ? ((BN / 2) % 16 ? 4 : 2) : (BM > BN ? 4 : 2);
   static constexpr int WGN = NW / WGM;
   static constexpr int WTM = BM / WGM, WTN = BN / WGN;            // wave tile
   // MFMA shape: 16x16 (x32 for 16-bit, x64 for int8).  With operands that toggle like real data the part runs
@@ -382,10 +400,13 @@ struct TileCfg {
   static constexpr int A_LPW = (A_LOADS + NW - 1) / NW, B_LPW = (B_LOADS + NW - 1) / NW;
   static constexpr int LPW = A_LPW + B_LPW;                       // DMA ops one wave issues per slab
   static constexpr int ACC_N = (MI == 32) ? 16 : 4;
-  static constexpr bool VALID =
-      (WTM % 16 == 0) && (WTN % 16 == 0) && (BK * ES) % KB == 0 && KSTEPS >= 1 && CPR_A >= 4 &&
-      CPR_B >= 8 && CPR_B % (ES == 1 ? 4 : 8) == 0 && A_BYTES % 1024 == 0 && B_BYTES % 1024 == 0 &&
-      A_LOADS % NW == 0 && B_LOADS % NW == 0 && LDS_BYTES <= 163840 && TM * TN * ACC_N <= 256 && (STAGES - 2) * LPW <= 63 && STAGES >= 2;
+  static constexpr bool VALID_ANY =
+      (WTM % 16 == 0) && (WTN % 16 == 0) && (BK * ES) % KB == 0 && KSTEPS >= 1 && CPR_A >= 4 && A_BYTES % 1024 == 0 &&
+      B_BYTES % 1024 == 0 && A_LOADS % NW == 0 && LDS_BYTES <= 163840 && TM * TN * ACC_N <= 256 && (STAGES - 2) * LPW <= 63 && STAGES >= 2;
+  static constexpr bool VALID = VALID_ANY && CPR_B >= 8 && CPR_B % (ES == 1 ? 4 : 8) == 0 && B_LOADS % NW == 0;
+  // GATHER: the B slab has the layout of the A slab, so its width only has to be whole DMA ops (8 rows); ops that do
+  // not divide over the waves are issued twice (the same bytes to the same place)
+  static constexpr bool VALID_GATHER = VALID_ANY && ES == 2 && BK * ES == 128 && BN % 16 == 0;
 
   // chunk-index XOR applied to row `row` of the A slab.  A fragment read is one ds_read_b128 with lane = 16 * kg +
   // row: the LDS serves it in four cycles of 16 lanes, and the 16 are not consecutive lanes -- measured with a
@@ -858,9 +879,10 @@ struct __attribute__((packed, aligned(2))) Loose16 {
 // Epilogue of the CONV kernels: rows are output channels, columns are pixels of the padded pixel index space.  Same
 // pass through the wave's LDS strip as epilogue_store; a 16-byte chunk is 8 pixels of one output row, so it is one
 // run of the NCHW output (cut at w_out: the pixels past it exist only in the index space).  Bias is added in fp32.
-template <class T, class C, class O, class ACC>
+// FROM_WS: the values are the sum of the split-K slices in the workspace, as in epilogue_store.
+template <class T, class C, class O, bool FROM_WS = false, class ACC>
 __device__ __forceinline__ void epilogue_store_conv(ACC (&acc)[C::TM][C::TN], uint8_t* ybase, uint32_t lds_strip, int lane,
-                                                    int gm0, int gn0, const ConvGeom& g) {
+                                                    int gm0, int gn0, const ConvGeom& g, const SliceSrc& src = SliceSrc{nullptr, 0, 0, false}) {
   typedef typename O::raw raw;                          // 16-bit outputs, or binary32 (the fp32 sums + bias as they are)
   typedef float acc4 __attribute__((ext_vector_type(4)));
   constexpr int MI = C::MI;
@@ -869,19 +891,28 @@ __device__ __forceinline__ void epilogue_store_conv(ACC (&acc)[C::TM][C::TN], ui
   constexpr int ROWS = EpiStage<C>::ROWS;
   constexpr int CPRW = C::WTN / 8;                       // a lane handles 8 pixels: one 16-byte chunk of the im2col slab
   constexpr int ITERS = (ROWS * CPRW + 63) / 64;
-  constexpr int UNR = ITERS % 4 == 0 ? 4 : (ITERS % 2 == 0 ? 2 : 1);
+  constexpr int UNR = ITERS % 4 == 0 ? 4 : ITERS <= 7 ? ITERS : (ITERS % 2 == 0 ? 2 : 1);
   static_assert(EpiStage<C>::RB == 1 && C::WTN % 8 == 0, "one row-block per pass, 8 outputs per chunk");
   raw* yp = (raw*)ybase;
   const uint32_t wbase = lds_strip + (lane % MI) * PITCH + (lane / MI) * 16;
 #pragma unroll
   for (int i = 0; i < C::TM; ++i) {
     if (gm0 + i * MI >= g.c_out) break;
+    if constexpr (!FROM_WS) {
 #pragma unroll
-    for (int j = 0; j < C::TN; ++j)
+      for (int j = 0; j < C::TN; ++j)
 #pragma unroll
-      for (int q = 0; q < NGRP; ++q)
-        *TNX_LDS(acc4, wbase + (j * MI + q * 8) * 4) =
-            acc4{acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        for (int q = 0; q < NGRP; ++q)
+          *TNX_LDS(acc4, wbase + (j * MI + q * 8) * 4) =
+              acc4{acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+    } else {
+      const __amdgpu_buffer_rsrc_t win = agent_window(src.base);
+      const uint32_t q0 = (uint32_t)i * (C::TN * NGRP) * 1024u + lane * 16u;
+      const bool row_ok = gm0 + i * MI + lane % MI < g.c_out;
+      if (src.nslices <= 2) sum_slices<acc4, 2, C::TN * NGRP, MI, NGRP>(win, q0, src, wbase, row_ok);
+      else if (src.nslices <= 4) sum_slices<acc4, 4, C::TN * NGRP, MI, NGRP>(win, q0, src, wbase, row_ok);
+      else sum_slices<acc4, 8, C::TN * NGRP, MI, NGRP>(win, q0, src, wbase, row_ok);
+    }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
 #pragma unroll 1
     for (int it0 = 0; it0 < ITERS; it0 += UNR) {
@@ -920,8 +951,13 @@ __device__ __forceinline__ void epilogue_store_conv(ACC (&acc)[C::TM][C::TN], ui
           i32x4 v[sizeof(raw) / 2];
           __builtin_memcpy(v, out, 8 * sizeof(raw));
 #pragma unroll
-          for (int h = 0; h < (int)sizeof(raw) / 2; ++h)
-            store16_stream_loose((uint8_t*)dst + 16 * h, v[h]);    // element-aligned: w_out need not be a multiple of 8
+          for (int h = 0; h < (int)sizeof(raw) / 2; ++h) {         // element-aligned: w_out need not be a multiple of 8
+            // binary32: the two stores of a lane interleave with its neighbours', so each fills half of every cache line;
+            // kept in the L2 the halves meet there, hinted they go out one by one (1984 channels of 17x17, batch 64:
+            // 116 -> 64 us)
+            if constexpr (sizeof(raw) == 4) *(i32x4_loose*)((uint8_t*)dst + 16 * h) = v[h];
+            else store16_stream_loose((uint8_t*)dst + 16 * h, v[h]);
+          }
         } else {
 #pragma unroll 1
           for (int x = 0; x < valid; ++x) dst[x] = out[x];
@@ -931,6 +967,9 @@ __device__ __forceinline__ void epilogue_store_conv(ACC (&acc)[C::TM][C::TN], ui
     __builtin_amdgcn_s_waitcnt(0xC07F);
   }
 }
+
+// GATHER: the table of k-chunk offsets behind the ring
+constexpr int GATHER_TABLE_BYTES = 8192;
 
 template <class X> struct TypeTag { typedef X type; };
 template <bool B> struct BoolTag { static constexpr bool value = B; };
@@ -952,13 +991,18 @@ template <int V> struct IntTag { static constexpr int value = V; };
 // the middle of period t+1 (by then only that period's own loads may still be outstanding), fixed in the second
 // half of period t+1 -- one read-modify-write of the chunk per op, slotted behind MFMAs -- and published by barrier
 // t+2, before whose period nothing reads it.  16-bit types, stride_w == 1, k % BK == 0.
-template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false>
+// GATHER (with BT): conv2d forward over a packed input (PackGeom): the rows of the k-contiguous B slab are the windows of
+// BN output pixels.  A lane's DMA ops fetch the same 16-byte k chunk of different pixels, so an op's offset is the
+// pixel's, kept in a register, plus the chunk's (filter tap, channels), read once per slab from a table in LDS.  Chunks
+// past the end of k get an offset outside the buffer and arrive as zeros.
+template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false>
 __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   constexpr int ES = C::ES, BM = C::BM, BN = C::BN, BK = C::BK, NW = C::NW, STAGES = C::STAGES;
   constexpr int MI = C::MI, TM = C::TM, TN = C::TN;
-  static_assert(C::VALID, "tile configuration not supported by this kernel");
+  static_assert(GATHER ? C::VALID_GATHER : C::VALID, "tile configuration not supported by this kernel");
+  static_assert(!GATHER || (FAST && BT && !PERSIST && !CONV), "the packed conv2d variant is a k-contiguous-B kernel");
   static_assert(!PERSIST || FAST, "the persistent kernel is built with the DMA loader only");
-  static_assert(!BT || (FAST && C::B_LOADS % NW == 0), "the k-contiguous B variant is built with the DMA loader only");
+  static_assert(!BT || (FAST && (GATHER || C::B_LOADS % NW == 0)), "the k-contiguous B variant is built with the DMA loader only");
   static_assert(!CONV || (FAST && !PERSIST && !BT && ES == 2 && STAGES == 3 && MI == 16 && (NW * 64) % C::CPR_B == 0),
                 "the conv2d variant: DMA loader, 16-bit types, three ring slots");
   typedef Mma<T, MI> MMA;
@@ -966,7 +1010,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   typedef typename T::acc_s acc_s;
   // Several problems in one grid and a bias per row (GemmParams::batch, cv.bias) exist in the tiles up to 128x128:
   // the 256-wide tiles have no register to spare for the extra state (measured: 20 more spilled registers, -0.4 %).
-  constexpr bool MULTI = !PERSIST && !CONV && multi_problem_tile<C>();
+  constexpr bool MULTI = !PERSIST && !CONV && !GATHER && multi_problem_tile<C>();
 
   // one workgroup per tile: the epilogue strips are laid over the ring once the K loop is done.
   // persistent: the ring is refilled for the next tile during the epilogue, so the strips follow it.
@@ -974,7 +1018,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   // CONV: behind the ring, a table of the 81 16-byte masks that keep elements [lo, hi) of a chunk (0 <= lo, hi <= 8),
   // and two tables of the filter taps of one K slab (BK entries of 8 bytes: element offset, dh | dw << 16)
   constexpr int CV_TABLE_BYTES = CONV ? 81 * 16 + 2 * BK * 8 : 0;
-  constexpr int SMEM_BYTES = (PERSIST ? C::LDS_BYTES + PairStrip<C>::BYTES : RING_OR_STRIPS) + CV_TABLE_BYTES;
+  constexpr int SMEM_BYTES = (PERSIST ? C::LDS_BYTES + PairStrip<C>::BYTES : RING_OR_STRIPS) + CV_TABLE_BYTES +
+                             (GATHER ? GATHER_TABLE_BYTES : 0);
   static_assert(SMEM_BYTES <= 163840, "LDS budget of one CU exceeded");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[SMEM_BYTES];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(uint8_t __attribute__((address_space(3)))*)smem;
@@ -1035,7 +1080,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   // no multiple of BK, rows that are not 16-byte aligned or an N that ends inside a chunk, the host sets tail_slab
   // and the last slab of the K range (the only one whose chunks can cross the end of a row of A, or the end of the
   // last row of B) is left out of the ring and loaded element by element, zero-filled, after the K loop.
-  const bool tail_here = FAST && !PERSIST && !CONV && p.tail_slab != 0 && kt1 == kt_total && kt1 > kt0;
+  const bool tail_here = FAST && !PERSIST && !CONV && !GATHER && p.tail_slab != 0 && kt1 == kt_total && kt1 > kt0;
   const int KT = kt1 > kt0 ? kt1 - kt0 - (tail_here ? 1 : 0) : 0;          // slabs of this workgroup in the ring (per tile)
 
   // ---- the tile the loader works on: origin, DMA bases and per-lane byte offsets.
@@ -1080,8 +1125,44 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     cv_rsrc = i32x4{(int)__builtin_amdgcn_readfirstlane((uint32_t)xa), (int)(__builtin_amdgcn_readfirstlane((uint32_t)(xa >> 32)) & 0xffff),
                     (int)__builtin_amdgcn_readfirstlane(p.cv.x_bytes), 0x00020000};
   }
+  // GATHER: chunk offsets of this workgroup's K range: one entry per chunk, or per slab when a filter tap's channels are
+  // whole slabs (the chunk's place in the slab is then part of the pixel offset).  All chunks a lane fetches have the
+  // same place in their slab: the swizzle of a row depends on the row modulo 8, which is lane / 8.
+  const uint32_t g_table = lds0 + RING_OR_STRIPS;
+  const int g_chunk = (lane & 7) ^ C::swzA(lane >> 3);
+  const bool g_whole = GATHER && p.pk.cpt % 8 == 0;
+  uint32_t g_at = g_table + (g_whole ? 0 : g_chunk * 4);     // entry of the next slab to issue
+  uint32_t g_tap = 0;                                        // offset of the slab being issued
+  i32x4 g_rsrc = {0, 0, 0, 0};
+  if constexpr (GATHER) {
+    const PackGeom& g = p.pk;
+    const int ents = g_whole ? kt1 - kt0 : (kt1 - kt0) * 8;
+    for (int e = tid; e < ents; e += C::THREADS) {
+      const int k8 = kt0 * 8 + (g_whole ? e * 8 : e);
+      int tap, c8;
+      if (g_whole) {        // slabs of 64 channels, the filter taps of one slab after another
+        const int cs = (int)fd_div((uint32_t)(kt0 + e), g.div_taps);
+        tap = kt0 + e - cs * g.taps;
+        c8 = cs * 8;
+      } else {
+        tap = (int)fd_div((uint32_t)k8, g.div_cpt);
+        c8 = k8 - tap * g.cpt;
+      }
+      const int r = (int)fd_div((uint32_t)tap, g.div_fw), s = tap - r * g.fw;
+      const uint32_t off = (uint32_t)r * g.tap_row_bytes + (uint32_t)s * g.tap_col_bytes + (uint32_t)c8 * 16u;
+      *TNX_LDS(uint32_t, g_table + e * 4) = k8 < g.chunks ? off : 0x80000000u;
+    }
+    const uint64_t xa = (uint64_t)(uintptr_t)p.b;
+    g_rsrc = i32x4{(int)__builtin_amdgcn_readfirstlane((uint32_t)xa), (int)(__builtin_amdgcn_readfirstlane((uint32_t)(xa >> 32)) & 0xffff),
+                   (int)__builtin_amdgcn_readfirstlane(g.x_bytes), 0x00020000};
+  }
   const uint8_t* a_sbase = p.a;
   const uint8_t* b_sbase = p.b;
+  // DMA op q of this wave moves 1 KiB number b_op(q) of the B slab
+  auto b_op = [&](int q) __attribute__((always_inline)) {
+    const int op = q * NW + wave;
+    return C::B_LOADS % NW != 0 && op >= C::B_LOADS ? C::B_LOADS - 1 : op;
+  };
   auto place_tile = [&](int tile_m, int tile_n) __attribute__((always_inline)) {
     m0 = (int64_t)tile_m * BM;
     n0 = (int64_t)tile_n * BN;
@@ -1133,7 +1214,17 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
 #pragma unroll
       for (int q = 0; q < (CONV ? 0 : C::B_LPW); ++q) {
         int P = (q * NW + wave) * 64 + lane;
-        if (BT) {
+        if constexpr (GATHER) {
+          const PackGeom& g = p.pk;
+          int n = (int)n0 + b_op(q) * 8 + (lane >> 3);
+          n = n < p.cv.n_total ? n : p.cv.n_total - 1;          // pixels past the end are computed and dropped
+          const int img = (int)fd_div((uint32_t)n, g.div_hwp);
+          int r = n - img * g.hwp;
+          r = r < g.hw_out ? r : g.hw_out - 1;
+          const int ho = (int)fd_div((uint32_t)r, g.div_w), wo = r - ho * g.w_out;
+          b_voff[q] = (uint32_t)img * g.img_bytes + (uint32_t)ho * g.row_bytes + (uint32_t)wo * g.col_bytes +
+                      (g_whole ? (uint32_t)g_chunk * 16u : 0u);
+        } else if (BT) {
           // rows of the slab are columns of B: same chunk layout and swizzle as the A slab
           int row = P / C::CPR_A, cs = P % C::CPR_A;
           int c = cs ^ C::swzA(row);
@@ -1407,6 +1498,16 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     }
   };
 
+  auto gather_go = [&](int qb) __attribute__((always_inline)) {
+    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(b_voff[qb] + g_tap), "s"(g_rsrc) : "memory");
+  };
+  auto gather_next = [&]() __attribute__((always_inline)) {
+    if constexpr (GATHER) {
+      g_tap = *TNX_LDS(uint32_t, g_at);
+      g_at += g_whole ? 4 : 32;
+    }
+  };
+
   // one DMA op (q-th of this wave) of local slab t, into ring slot t % STAGES
   auto dma_op = [&](int q, uint32_t stage_base) __attribute__((always_inline)) {
     if (CONV && q >= C::A_LPW) {
@@ -1416,6 +1517,10 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
       conv_go();
     } else if (q < C::A_LPW) {
       dma16(a_sbase, a_voff[q], stage_base + (q * NW + wave) * 1024);
+    } else if (GATHER) {
+      dma16_set_m0(stage_base + C::A_BYTES + b_op(q - C::A_LPW) * 1024);
+      asm volatile("s_nop 0" ::: "memory");
+      gather_go(q - C::A_LPW);
     } else {
       // short tiles are the ones used on skinny problems, where B is the HBM stream
       if (BM <= 64 && p.b_once)
@@ -1428,10 +1533,11 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   auto dma_target = [&](int q, uint32_t stage_base) __attribute__((always_inline)) {
     if (CONV && q >= C::A_LPW) conv_prepare(q - C::A_LPW, stage_base);
     if (q < C::A_LPW) dma16_set_m0(stage_base + (q * NW + wave) * 1024);
-    else dma16_set_m0(stage_base + C::A_BYTES + ((q - C::A_LPW) * NW + wave) * 1024);
+    else dma16_set_m0(stage_base + C::A_BYTES + b_op(q - C::A_LPW) * 1024);
   };
   auto dma_go = [&](int q) __attribute__((always_inline)) {
     if (CONV && q >= C::A_LPW) conv_go();
+    else if (GATHER && q >= C::A_LPW) gather_go(q - C::A_LPW);
     else if (q < C::A_LPW) dma16_go<false>(a_sbase, a_voff[q]);
     else if (BM <= 64 && p.b_once) dma16_go<true>(b_sbase, b_voff[q - C::A_LPW]);
     else dma16_go<false>(b_sbase, b_voff[q - C::A_LPW]);
@@ -1439,7 +1545,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   auto dma_advance = [&]() __attribute__((always_inline)) {
     if (TNX_LADDER == 3) return;        // + DMA ops, always of the tile's first slabs (served by the L2)
     a_sbase += BK * ES;
-    if (!CONV) b_sbase += BT ? (int64_t)BK * ES : (int64_t)BK * p.sbk * ES;
+    if (GATHER) gather_next();
+    else if (!CONV) b_sbase += BT ? (int64_t)BK * ES : (int64_t)BK * p.sbk * ES;
   };
   auto stage_of = [&](int t) __attribute__((always_inline)) { return lds0 + (uint32_t)(t % STAGES) * C::STAGE_BYTES; };
 
@@ -1640,6 +1747,10 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
       conv_tab_write();                       // slab 3 -> table 1
       __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the fix-up writes are done before the barrier that follows
       return;
+    }
+    if constexpr (GATHER) {
+      __syncthreads();                                  // the offset table is complete
+      gather_next();
     }
 #pragma unroll
     for (int s = 0; s < STAGES; ++s) {
@@ -1844,7 +1955,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     }
     if (PINGPONG_TILE && KT >= 2 && (KT & 1) == 0) pingpong_loop();
     else k_loop();
-    if constexpr (FAST && !CONV) {
+    if constexpr (FAST && !CONV && !GATHER) {
       if (tail_here) {
         // the left-out slab: every wave is done with the ring, slot 0 takes it, one slab of MFMAs follows
         __syncthreads();
@@ -1870,6 +1981,26 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     if constexpr (CONV) {
       if (p.out_dtype == DT_F32) epilogue_store_conv<T, C, OutF32>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
       else epilogue_store_conv<T, C, O>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
+      return;
+    }
+    if constexpr (GATHER) {
+      auto finish_conv = [&](auto otag) __attribute__((always_inline)) {
+        typedef typename decltype(otag)::type OT;
+        if (cut) {
+          const int ncut = ntiles - p.split_tile0, ctile = logical - p.split_tile0;
+          const int64_t slice_stride = (int64_t)ncut * BM * BN * 4;
+          uint8_t* wave0 = p.ws + WS_COUNTER_BYTES + ((int64_t)ctile * NW + wave) * (C::WTM * C::WTN * 4);
+          if (!splitk_arrive<T, C>(acc, wave0 + split * slice_stride, strip, lane, gm0, p.m, (int*)p.ws + ctile, (int*)smem,
+                                   p.split_k, false))
+            return;
+          epilogue_store_conv<T, C, OT, true>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv,
+                                              SliceSrc{wave0, (uint32_t)slice_stride, p.split_k, false});
+        } else {
+          epilogue_store_conv<T, C, OT>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
+        }
+      };
+      if (p.out_dtype == DT_F32) finish_conv(TypeTag<OutF32>{});
+      else finish_conv(TypeTag<O>{});
       return;
     }
     // the output type: the input's own 16-bit type (int32 for int8), or binary32 where that epilogue is built

@@ -38,15 +38,25 @@ int gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra);
 // two ring slots first); false: none built
 bool gemm_tile_for(int dtype, int bm, int bn, int bk, int* num_warps, int* num_stages);
 
+// conv2d over a packed input (gemm_tile_kernel<..., GATHER>), block_k = 64: tiles of channels x pixels
+struct GatherEntry {
+  int dtype, bm, bn, nw, stages;
+  launch_fn launch;
+};
+struct GatherGroup {
+  GatherEntry* entries;
+  int count;
+};
+
 struct KernelGroup {
   KernelEntry* entries;
   int count;
 };
 
-template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false>
+template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false>
 hipError_t launch_tile(const GemmParams& p, unsigned grid, hipStream_t stream) {
-  static_assert(C::VALID, "tile configuration is not buildable");
-  hipLaunchKernelGGL((gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV>), dim3(grid), dim3(C::THREADS), 0, stream, p);
+  static_assert(GATHER ? C::VALID_GATHER : C::VALID, "tile configuration is not buildable");
+  hipLaunchKernelGGL((gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV, GATHER>), dim3(grid), dim3(C::THREADS), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -105,6 +115,9 @@ template <class T, class C, bool WANTED> struct GenericLaunch {
 template <class T, class C> struct GenericLaunch<T, C, true> {
   static constexpr launch_fn fn = &launch_tile<T, C, false>;
 };
+
+#define TNX_GATHER_ENTRY(TAG, BM, BN, NW, ST) \
+  {TAG::ID, BM, BN, NW, ST, &launch_tile<TAG, TileCfg<TAG, BM, BN, 64, NW, ST>, true, false, true, false, true>}
 
 #define TNX_ENTRY(TAG, BM, BN, BK, NW, ST, GENERIC)                                                          \
   {TAG::ID, BM, BN, BK, NW, ST, TileCfg<TAG, BM, BN, BK, NW, ST>::LDS_BYTES,                                 \

@@ -7,7 +7,9 @@ GROUP_SIZE_M=, OUT_DTYPE=, USE_TF32=)`` keep the argument order and meaning of
 tritonix/ops/conv2d/forward.py:19-48 and :202-311; both end in one ``tnx_conv2d_forward`` through the C ABI on
 torch's current stream.  Float16 and bfloat16 are built; float32 tensors (the reference convolves them in TF32,
 which gfx950 has no matrix instruction for) run as a three-term bf16 convolution over 3 c_in channels with an fp32
-result (``_split_f32``), on the register-staged kernels and the 1x1 GEMM route.
+result.  Where no tile is named the library may copy the operands into a channels-last layout first and run the
+k-contiguous GEMM kernel over that (``tnx_conv2d_workspace_bytes``; the scratch is allocated here, per call); float32
+operands are cut into their terms by that copy, or by ``_split_f32`` for the kernels that do not take it.
 """
 from __future__ import annotations
 
@@ -89,7 +91,16 @@ def _raise_for_status(status: int, a: _C.Conv2dArgs) -> None:
 def _args(out, input, weight, bias, batch, c_in, h_in, w_in, c_out, filter_h, filter_w, stride, padding, dilation,
           block_m: int, block_n: int, block_k: int, group_m: int, loader: int = 0) -> _C.Conv2dArgs:
     a = _C.Conv2dArgs()
-    if input.dtype == torch.float32:
+    if not (block_m or block_n or block_k or loader) and input.is_cuda and input.dtype in _DTYPES:
+        # the library's own choice: with scratch it may lay the operands out for the packed kernels
+        a.batch, a.c_in, a.h_in, a.w_in, a.c_out, a.filter_h, a.filter_w = batch, c_in, h_in, w_in, c_out, filter_h, filter_w
+        a.stride_h, a.stride_w, a.pad_h, a.pad_w, a.dil_h, a.dil_w = *stride, *padding, *dilation
+        a.dtype, a.out_f32 = _DTYPES[input.dtype], input.dtype == torch.float32
+        need = _C.load().tnx_conv2d_workspace_bytes(ctypes.byref(a))
+        if need:
+            ws = torch.empty(need, dtype=torch.uint8, device=input.device)
+            a.workspace, a.workspace_bytes, a._keep = ws.data_ptr(), need, (ws,)
+    if input.dtype == torch.float32 and not a.workspace:
         if not (input.is_cuda and weight.is_cuda and out.is_cuda):
             raise ValueError("conv2d_forward: input, weight and output must be tensors on a HIP device (there is no CPU path)")
         input, weight, c_in = _split_f32(input, weight, batch, c_in, h_in, w_in, c_out, filter_h, filter_w)
@@ -238,6 +249,60 @@ def _time_kernel(fn, iters=10, warmup=5, regions=3):
     return best
 
 
+# bound arguments of problems met before, without their pointers: (struct, output shape, scratch bytes) by sizes and types
+_PLANS: Dict[tuple, tuple] = {}
+_MAX_PLANS = 1024
+
+
+def _launch_planned(input, weight, bias, stride, padding, dilation) -> Optional[torch.Tensor]:
+    """The library's own choice for a problem, launched from its remembered argument struct: a call then only fills in
+    pointers (binding every argument by name anew costs 10 us of host time, twice what a small layer takes on the
+    GPU).  None: the ordinary path has to bind it (float32 without the packed kernels, arguments it has to refuse)."""
+    if bias is not None and not (bias.is_cuda and bias.is_contiguous()):
+        return None
+    dev = input.get_device()
+    key = (input.shape, weight.shape, stride, padding, dilation, input.dtype, weight.dtype, weight.get_device(), dev,
+           None if bias is None else (bias.dtype, bias.numel()))
+    plan = _PLANS.get(key)
+    lib = _C.load()
+    if plan is None:
+        n, c_in, h_in, w_in = input.shape
+        c_out, _, r, s = weight.shape
+        h_out, w_out = output_size(h_in, w_in, r, s, stride, padding, dilation)
+        if (weight.dtype != input.dtype or input.dtype not in _DTYPES or weight.get_device() != dev or h_out <= 0 or w_out <= 0
+                or (bias is not None and (bias.dtype not in _DTYPES or bias.numel() != c_out))):
+            return None
+        a = _C.Conv2dArgs()
+        a.batch, a.c_in, a.h_in, a.w_in, a.c_out, a.filter_h, a.filter_w = n, c_in, h_in, w_in, c_out, r, s
+        a.stride_h, a.stride_w, a.pad_h, a.pad_w, a.dil_h, a.dil_w = *stride, *padding, *dilation
+        a.dtype, a.out_f32, a.group_pixels = _DTYPES[input.dtype], input.dtype == torch.float32, 8
+        a.bias_dtype = 0 if bias is None else _DTYPES[bias.dtype]
+        need = lib.tnx_conv2d_workspace_bytes(ctypes.byref(a))
+        if input.dtype == torch.float32 and not need:
+            return None
+        if len(_PLANS) >= _MAX_PLANS:
+            _PLANS.clear()
+        plan = _PLANS[key] = (a, (n, c_out, h_out, w_out), need)
+    template, shape, need = plan
+    a = _C.Conv2dArgs.from_buffer_copy(template)          # its own copy: calls from several threads share the template
+    out = input.new_empty(shape)
+    a.input, a.weight, a.output = input.data_ptr(), weight.data_ptr(), out.data_ptr()
+    if bias is not None:
+        a.bias = bias.data_ptr()
+    if need:
+        ws = torch.empty(need, dtype=torch.uint8, device=input.device)
+        a.workspace, a.workspace_bytes = ws.data_ptr(), need
+    a.stream = torch.cuda.current_stream(dev).cuda_stream
+    if dev != torch.cuda.current_device():
+        with torch.cuda.device(dev):
+            status = lib.tnx_conv2d_forward(ctypes.byref(a))
+    else:
+        status = lib.tnx_conv2d_forward(ctypes.byref(a))
+    if status != _C.OK:
+        _raise_for_status(status, a)
+    return out
+
+
 def conv2d_forward(
     input: torch.Tensor,
     weight: torch.Tensor,
@@ -260,6 +325,12 @@ def conv2d_forward(
     c_out, c_in_w, r, s = weight.shape
     assert c_in == c_in_w
     stride, padding, dilation = tuple(stride), tuple(padding), tuple(dilation)
+    if config is None and os.environ.get("TRITONIX_AUTOTUNE", "1") in ("0", "false", "False"):
+        config = dict(BLOCK_SIZE_M=0, BLOCK_SIZE_N=0, BLOCK_SIZE_K=0)      # no timing runs: the library's own choice
+        if input.is_cuda and weight.is_cuda:
+            out = _launch_planned(input, weight, bias, stride, padding, dilation)
+            if out is not None:
+                return out
     h_out, w_out = output_size(h_in, w_in, r, s, stride, padding, dilation)
     gemm_m, gemm_n, gemm_k = n * h_out * w_out, c_out, c_in * r * s
     out = input.new_empty((n, c_out, h_out, w_out))
@@ -270,8 +341,6 @@ def conv2d_forward(
             stride[0], stride[1], padding[0], padding[1], dilation[0], dilation[1], gemm_m, gemm_n, gemm_k,
             BLOCK_SIZE_M=bm, BLOCK_SIZE_N=bn, BLOCK_SIZE_K=bk, GROUP_SIZE_M=g, USE_TF32=use_tf32, LOADER=loader)
 
-    if config is None and os.environ.get("TRITONIX_AUTOTUNE", "1") in ("0", "false", "False"):
-        config = dict(BLOCK_SIZE_M=0, BLOCK_SIZE_N=0, BLOCK_SIZE_K=0)      # no timing runs: the library's own choice
     if config is None:
         key = (n, c_in, h_in, w_in, c_out, r, s, stride, padding, dilation, input.dtype)
         cfg = _CONV_FWD_CONFIG_CACHE.get(key)
@@ -284,6 +353,10 @@ def conv2d_forward(
                     continue
                 if t < best_time:
                     best_time, best = t, dict(BLOCK_SIZE_M=bm, BLOCK_SIZE_N=bn, BLOCK_SIZE_K=bk, GROUP_SIZE_M=g)
+            # the library's own choice is one more candidate: with scratch it may be the packed kernels, which no tile names
+            t = _time_kernel(lambda: launch(0, 0, 0, 8))
+            if t < best_time:
+                best_time, best = t, dict(BLOCK_SIZE_M=0, BLOCK_SIZE_N=0, BLOCK_SIZE_K=0, GROUP_SIZE_M=8)
             if (r, s) == (1, 1) and stride == (1, 1) and padding == (0, 0):
                 # a 1x1 layer is a plain GEMM per image: the library's GEMM route with its own tile is one more candidate
                 try:
