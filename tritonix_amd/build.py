@@ -335,11 +335,11 @@ def _compile(src, obj, verbose, force=True):
 
 def demangled_tile(name):
     """'bf16 256x256x64 w4 s2 fast' from a mangled gemm_tile_kernel instantiation (None for other kernels)."""
-    m = re.search(r"gemm_tile_kernelINS_(\d)Tag(\w+?)ENS_7TileCfgIS1_Li(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)EEELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
+    m = re.search(r"gemm_tile_kernelINS_(\d)Tag(\w+?)ENS_7TileCfgIS1_Li(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)EEELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
     if not m:
         return None
-    _, tag, bm, bn, bk, nw, st, fast, persist, bt, conv, gather = m.groups()
-    kind = "packed conv" if gather == "1" else "conv" if conv == "1" else "bt" if bt == "1" else "persistent" if persist == "1" else "fast" if fast == "1" else "generic"
+    _, tag, bm, bn, bk, nw, st, fast, persist, bt, conv, gather, at = m.groups()
+    kind = "at" if at == "1" else "packed conv" if gather == "1" else "conv" if conv == "1" else "bt" if bt == "1" else "persistent" if persist == "1" else "fast" if fast == "1" else "generic"
     return f"{tag.lower()} {bm}x{bn}x{bk} w{nw} s{st} {kind}"
 
 

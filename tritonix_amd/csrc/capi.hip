@@ -84,7 +84,8 @@ static int check_common(const tnx_gemm_args* a) {
 // Which DMA loader the operands can take: 0 = none (element-wise loader only), 1 = row-major B
 // (stride_bn == 1), 2 = k-contiguous B (stride_bk == 1, the layout of x @ w.t()).  Both need row-major A,
 // 16-byte aligned rows and base pointers and k % block_k == 0.
-// 0: element-wise loader; 1: DMA loader, A and B row-major; 2: DMA loader, B k-contiguous.
+// 0: element-wise loader; 1: DMA loader, A and B row-major; 2: DMA loader, B k-contiguous; 3: DMA loader, A m-contiguous,
+// B row-major (only in the tiles built for it).
 // *tail (layout 1 only): the operands are row-major but not as the DMA loader likes them best -- K no multiple of
 // block_k, rows or base pointers not 16-byte aligned (the loads take any byte address: probed on the hardware),
 // N ending inside a 16-byte chunk -- so the last K slab, the only one whose chunks can cross the end of a row of A
@@ -93,6 +94,16 @@ static int dma_layout(const tnx_gemm_args* a, bool* tail = nullptr) {
   const int es = elem_size(a->in_dtype);
   const int vec = 16 / es;
   if (tail) *tail = false;
+  if (a->stride_am == 1 && a->stride_ak != 1 && a->stride_bn == 1 && a->k > 0 && a->stride_ak >= a->m && a->stride_bk >= a->n &&
+      (int64_t)a->block_k * a->stride_ak * es + (int64_t)a->block_m * es < (1ll << 32) &&
+      (int64_t)a->block_k * a->stride_bk * es + (int64_t)a->block_n * es < (1ll << 32)) {
+    const bool aligned = (a->stride_ak * es) % 16 == 0 && (a->stride_bk * es) % 16 == 0 && !((uintptr_t)a->a & 15) && !((uintptr_t)a->b & 15);
+    if (aligned && a->k % a->block_k == 0 && a->m % vec == 0 && a->n % vec == 0) return 3;
+    if (tail) {
+      *tail = true;
+      return 3;
+    }
+  }
   if (a->stride_ak != 1 || a->k == 0 || a->stride_am < 0) return 0;
   // per-lane DMA offsets are 32-bit
   if ((int64_t)a->block_m * a->stride_am * es >= (1ll << 32)) return 0;
@@ -138,8 +149,9 @@ extern "C" size_t tnx_gemm_workspace_bytes(const tnx_gemm_args* a) {
 }
 
 static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool* fast, bool inspect_ptrs, bool* bt = nullptr,
-                          bool* tail = nullptr) {
+                          bool* tail = nullptr, bool* at = nullptr) {
   if (bt) *bt = false;
+  if (at) *at = false;
   if (tail) *tail = false;
   int st = check_common(a);
   if (st != TNX_OK) return st;
@@ -168,13 +180,14 @@ static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool*
   bool tail_slab = false;
   // the persistent kernel keeps the strict layout
   const int layout = dma_layout(&tmp, (a->schedule & TNX_SCHED_PERSISTENT) ? nullptr : &tail_slab);
-  if (tail) *tail = tail_slab;
-  bool f = layout == 1 || (layout == 2 && e->fast_bt);
+  bool f = layout == 1 || (layout == 2 && e->fast_bt) || (layout == 3 && e->fast_at);
+  if (tail) *tail = f && tail_slab;
   if (!f && !e->generic) return TNX_E_UNSUPPORTED;
   if (a->schedule & TNX_SCHED_PERSISTENT) {
     if (!e->persist || layout != 1 || a->split_k != 1 || a->k < (int64_t)a->num_stages * a->block_k) return TNX_E_UNSUPPORTED;
   }
   if (bt) *bt = f && layout == 2;
+  if (at) *at = f && layout == 3;
   int64_t tiles = ((a->m + a->block_m - 1) / a->block_m) * ((a->n + a->block_n - 1) / a->block_n);
   if (tiles * a->split_k > 0x7fffffffll) return TNX_E_UNSUPPORTED;
   if (cut_tiles(a) > WS_MAX_TILES) return TNX_E_UNSUPPORTED;  // one arrival counter per cut tile
@@ -233,8 +246,8 @@ bool tnx::gemm_tile_for(int dtype, int bm, int bn, int bk, int* num_warps, int* 
 
 int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra) {
   const KernelEntry* e = nullptr;
-  bool fast = false, bt = false, tail_slab = false;
-  int st = supported_impl(a, &e, &fast, true, &bt, &tail_slab);
+  bool fast = false, bt = false, at = false, tail_slab = false;
+  int st = supported_impl(a, &e, &fast, true, &bt, &tail_slab, &at);
   if (st != TNX_OK) return st;
   if (extra && (e->bm * e->bn > 128 * 128 || a->split_k != 1 || (a->schedule & TNX_SCHED_PERSISTENT) || is_skinny_cfg(a) || extra->batch < 1 ||
                 a->epilogue != TNX_EPI_NONE || (extra->bias && a->in_dtype == TNX_I8)))
@@ -298,7 +311,7 @@ int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra) {
     err = e->persist(p, (unsigned)(tiles < cus ? tiles : cus), stream);
   } else {
     unsigned grid = a->split_k > 1 ? (unsigned)(p.split_tile0 + ncut * a->split_k) : (unsigned)((int64_t)p.tiles_m * p.tiles_n * problems);
-    err = (bt ? e->fast_bt : fast ? e->fast : e->generic)(p, grid, stream);
+    err = (at ? e->fast_at : bt ? e->fast_bt : fast ? e->fast : e->generic)(p, grid, stream);
   }
   if (err != hipSuccess) { g_last_hip_error = (int)err; return TNX_E_HIP; }
 
@@ -391,15 +404,17 @@ extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
   a->tail_tiles = 0;
   a->schedule = TNX_SCHED_DEFAULT;
   a->block_k = bk;
-  bool dma_ok;
+  bool dma_ok, at = false;
   {
     tnx_gemm_args t = *a;   // a and b, when given, count with their base alignment (null = aligned)
     if (t.stride_ak == 0 && t.stride_bn == 0) { t.stride_am = t.k; t.stride_ak = 1; t.stride_bk = t.n; t.stride_bn = 1; }
     t.block_m = 128; t.block_n = 128; t.block_k = bk;
     bool tail_slab = false;
-    dma_ok = dma_layout(&t, &tail_slab) != 0;     // every tile the choice below proposes is built for both DMA layouts
+    const int layout = dma_layout(&t, &tail_slab);
+    dma_ok = layout != 0;     // every tile the choice below proposes is built for the DMA layouts ...
+    at = layout == 3;         // ... except the 64-row int8 tiles, whose rows are too short to read an m-contiguous A from
   }
-  if (a->m <= 64 && dma_ok) {
+  if (a->m <= 64 && dma_ok && !(at && es == 1)) {
     // skinny: B is streamed once; K is split until every CU owns one workgroup (measured on the
     // M=16, N=4096, K=14336 shape: 8 waves, 3 stages, 256 workgroups stream at the HBM read limit)
     a->block_m = 64; a->block_n = 128; a->num_stages = 3; a->num_warps = 8;
@@ -436,12 +451,12 @@ extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
   // int8: rows of a 64-wide B tile are too short for the transposing read; the 192-wide tiles exist for it too
   // (3072 x 4096 x 4096: 53.6 -> 45.7 us with 192x256, 4096 x 3072 x 4096: 52.8 -> 47.3 us with 256x192)
   // (a binary32 result exists on the tiles up to 128x128 only)
-  auto usable = [&](int i) { return (es == 2 || i != 4) && (a->out_dtype != TNX_F32 || (i >= 2 && i <= 4)); };
+  auto usable = [&](int i) { return (es == 2 || i != 4) && !(at && es == 1 && i == 3) && (a->out_dtype != TNX_F32 || (i >= 2 && i <= 4)); };
   const double cu_flops = 5.5e12 * (es == 1 ? 1.7 : 1.0);          // per CU with the largest tile
   const double launch = 3e-6, handover = 9e-6, readback = 60e9;
   const int64_t kt = (a->k + bk - 1) / bk;
   double best = 1e300;
-  int bi = es == 1 ? 3 : 4, bs = 1, btail = 0;
+  int bi = es == 1 ? (at ? 2 : 3) : 4, bs = 1, btail = 0;
   auto offer = [&](double t, int i, int s, int tail) {
     if (t < best * 0.97) { best = t; bi = i; bs = s; btail = tail; }   // ties go to the earlier (larger, less cut) choice
   };
@@ -478,6 +493,7 @@ extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
   // price of half again as many LDS reads, which is what loses on the long, power-limited 8192^3 loops.
   // (cut tiles too: 4096 x 5120 x 4096 with its last 64 tiles cut, 155 -> 140 us)
   if (es == 2 && bi == 0 && kt <= 64) a->num_warps = 8;
+  if (at && bi == 0) a->num_warps = 8;                               // the only 256x256 kernels built for an m-contiguous A
   a->split_k = bs;
   a->tail_tiles = btail;
   // Grids of several rounds of 256 tiles in both directions: the super-block order keeps what one round reads
@@ -566,6 +582,7 @@ extern "C" const char* tnx_kernel_name(int idx) {
       snprintf(buf, sizeof(buf), "%s %d %d %d %d %d%s%s", dn, e.bm, e.bn, e.bk, e.nw, e.stages, e.generic ? " generic" : "",
                e.persist ? " persistent" : "");
       if (e.fast_bt) strncat(buf, " bt", sizeof(buf) - strlen(buf) - 1);
+      if (e.fast_at) strncat(buf, " at", sizeof(buf) - strlen(buf) - 1);
       return buf;
     }
     idx -= g[i].count;

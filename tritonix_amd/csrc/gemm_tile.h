@@ -406,6 +406,8 @@ struct TileCfg {
   static constexpr bool VALID = VALID_ANY && CPR_B >= 8 && CPR_B % (ES == 1 ? 4 : 8) == 0 && B_LOADS % NW == 0;
   // GATHER: the B slab has the layout of the A slab, so its width only has to be whole DMA ops (8 rows); ops that do
   // not divide over the waves are issued twice (the same bytes to the same place)
+  // AT: the A slab is BK rows of BM elements, read like a row-major B slab
+  static constexpr bool VALID_AT = VALID && BM * ES / 16 >= 8 && (BM * ES / 16) % (ES == 1 ? 4 : 8) == 0 && KSTEPS % 2 == 0;
   static constexpr bool VALID_GATHER = VALID_ANY && ES == 2 && BK * ES == 128 && BN % 16 == 0;
 
   // chunk-index XOR applied to row `row` of the A slab.  A fragment read is one ds_read_b128 with lane = 16 * kg +
@@ -423,15 +425,17 @@ struct TileCfg {
   // (A transposing read serves the four 16-lane groups of a wave in two passes; with 16x16 MFMA tiles the two
   // groups of a pass read the same columns 8 k rows apart (16 for int8), so one more row bit enters the XOR to
   // keep them on different banks: it moves the second group onto exactly the chunk slots the first leaves free.)
-  static __host__ __device__ constexpr int swzB(int row) {
+  static __host__ __device__ constexpr int swzB(int row) { return swzT<CPR_B>(row); }
+  // the same for any slab of k rows that transposing reads serve, CPR chunks per row
+  template <int CPR> static __host__ __device__ constexpr int swzT(int row) {
     if (ES == 2) {
       const int pass = MI == 16 ? (((row >> 3) ^ (row >> 4)) & 1) << 1 : 0;
-      if (CPR_B % 16 == 0) { int k = row & 3; return ((2 * k + (k >> 1)) << 1) ^ pass; }
+      if (CPR % 16 == 0) { int k = row & 3; return ((2 * k + (k >> 1)) << 1) ^ pass; }
       return ((row & 3) << 1) ^ pass;       // stays inside a group of 8 chunks: also for rows of 24 chunks (BN = 192)
     } else {
       const int pass = MI == 16 ? ((row >> 4) ^ (row >> 5)) & 1 : 0;
-      if (CPR_B % 16 == 0) { int k = row & 7; return (2 * k + (k >> 2)) ^ pass; }
-      if (CPR_B % 8 == 0) return (row & 7) ^ pass;
+      if (CPR % 16 == 0) { int k = row & 7; return (2 * k + (k >> 2)) ^ pass; }
+      if (CPR % 8 == 0) return (row & 7) ^ pass;
       // Rows of 12 chunks (BN = 192), 192 bytes: consecutive rows already start 48 banks apart, so the 8 rows of a
       // 16-lane group only collide with the row 4 below, and the two groups of a pass (rows r and r + 16) with each
       // other: one XOR bit for each, inside a group of 4 chunks.
@@ -991,16 +995,19 @@ template <int V> struct IntTag { static constexpr int value = V; };
 // the middle of period t+1 (by then only that period's own loads may still be outstanding), fixed in the second
 // half of period t+1 -- one read-modify-write of the chunk per op, slotted behind MFMAs -- and published by barrier
 // t+2, before whose period nothing reads it.  16-bit types, stride_w == 1, k % BK == 0.
+// AT: A is m-contiguous (element (m, k) at a + k * stride_ak + m, the layout of `x.t() @ dy`): its slab sits in LDS as
+// BK rows of BM elements exactly like a row-major B slab, and its fragments are read with the transposing reads.
 // GATHER (with BT): conv2d forward over a packed input (PackGeom): the rows of the k-contiguous B slab are the windows of
 // BN output pixels.  A lane's DMA ops fetch the same 16-byte k chunk of different pixels, so an op's offset is the
 // pixel's, kept in a register, plus the chunk's (filter tap, channels), read once per slab from a table in LDS.  Chunks
 // past the end of k get an offset outside the buffer and arrive as zeros.
-template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false>
+template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false, bool AT = false>
 __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   constexpr int ES = C::ES, BM = C::BM, BN = C::BN, BK = C::BK, NW = C::NW, STAGES = C::STAGES;
   constexpr int MI = C::MI, TM = C::TM, TN = C::TN;
   static_assert(GATHER ? C::VALID_GATHER : C::VALID, "tile configuration not supported by this kernel");
   static_assert(!GATHER || (FAST && BT && !PERSIST && !CONV), "the packed conv2d variant is a k-contiguous-B kernel");
+  static_assert(!AT || (FAST && !PERSIST && !BT && !CONV && C::VALID_AT), "the m-contiguous A variant is built with the DMA loader, row-major B");
   static_assert(!PERSIST || FAST, "the persistent kernel is built with the DMA loader only");
   static_assert(!BT || (FAST && (GATHER || C::B_LOADS % NW == 0)), "the k-contiguous B variant is built with the DMA loader only");
   static_assert(!CONV || (FAST && !PERSIST && !BT && ES == 2 && STAGES == 3 && MI == 16 && (NW * 64) % C::CPR_B == 0),
@@ -1011,6 +1018,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   // Several problems in one grid and a bias per row (GemmParams::batch, cv.bias) exist in the tiles up to 128x128:
   // the 256-wide tiles have no register to spare for the extra state (measured: 20 more spilled registers, -0.4 %).
   constexpr bool MULTI = !PERSIST && !CONV && !GATHER && multi_problem_tile<C>();
+
+  constexpr int AT_CPR = BM * ES / 16, AT_ROWB = BM * ES;    // AT: chunks and bytes of an A slab row
 
   // one workgroup per tile: the epilogue strips are laid over the ring once the K loop is done.
   // persistent: the ring is refilled for the next tile during the epilogue, so the strips follow it.
@@ -1169,12 +1178,20 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     if (FAST) {
       const int64_t lda = p.sam, ldb = BT ? p.sbn : p.sbk;
       // wave-uniform by construction; say so, so both stay in SGPRs for the DMA's scalar base operand
-      a_sbase = uniform_ptr(p.a + (m0 * lda + (int64_t)kt0 * BK) * ES);
+      a_sbase = uniform_ptr(AT ? p.a + ((int64_t)kt0 * BK * p.sak + m0) * ES : p.a + (m0 * lda + (int64_t)kt0 * BK) * ES);
       b_sbase = uniform_ptr(BT ? p.b + (n0 * ldb + (int64_t)kt0 * BK) * ES : p.b + ((int64_t)kt0 * BK * ldb + n0) * ES);
       const int64_t mrem = p.m - 1 - m0;  // last valid row inside this tile
 #pragma unroll
       for (int q = 0; q < C::A_LPW; ++q) {
         int P = (q * NW + wave) * 64 + lane;
+        if constexpr (AT) {
+          // rows of the slab are k, as in a row-major B slab: chunks past M as chunks past N there
+          int row = P / AT_CPR, cs = P % AT_CPR;
+          int c = cs ^ C::template swzT<AT_CPR>(row);
+          if (m0 + (int64_t)c * (16 / ES) >= p.m || (!p.tail_slab && m0 + (int64_t)(c + 1) * (16 / ES) > p.m)) c = 0;
+          a_voff[q] = (uint32_t)((int64_t)row * p.sak * ES + c * 16);
+          continue;
+        }
         int row = P / C::CPR_A, cs = P % C::CPR_A;
         int c = cs ^ C::swzA(row);
         int64_t r = row < mrem ? row : mrem;
@@ -1261,9 +1278,23 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   // chunk idx of the A part of slab kt_global: row idx / CPR_A, k chunk idx % CPR_A
   auto gen_fetch_a = [&](int kt_global, int idx) __attribute__((always_inline)) -> i32x4 {
     const gen_elem_t* ap = (const gen_elem_t*)p.a;
+    i32x4 v = {0, 0, 0, 0};
+    if constexpr (AT) {
+      const int64_t gk = (int64_t)kt_global * BK + idx / AT_CPR, gm = m0 + (int64_t)(idx % AT_CPR) * EPC;
+      if (idx < BK * AT_CPR && gk < p.k && gm < p.m) {
+        if (p.sam == 1 && gm + EPC <= p.m) {
+          v = *(const gen_chunk_t*)(ap + gk * p.sak + gm);
+        } else {
+          gen_elem_t e[EPC];
+#pragma unroll
+          for (int x = 0; x < EPC; ++x) e[x] = gm + x < p.m ? ap[gk * p.sak + (gm + x) * p.sam] : (gen_elem_t)0;
+          __builtin_memcpy(&v, e, 16);
+        }
+      }
+      return v;
+    }
     const int row = idx / C::CPR_A, cs = idx % C::CPR_A;
     const int64_t gm = m0 + row, gk = (int64_t)kt_global * BK + cs * EPC;
-    i32x4 v = {0, 0, 0, 0};
     if (idx < BM * C::CPR_A && gm < p.m && gk < p.k) {
       if (p.sak == 1 && gk + EPC <= p.k) {
         v = *(const gen_chunk_t*)(ap + gm * p.sam + gk);
@@ -1311,6 +1342,11 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     return v;
   };
   auto gen_store_a = [&](uint32_t stage_base, int idx, i32x4 v) __attribute__((always_inline)) {
+    if constexpr (AT) {
+      const int row = idx / AT_CPR, cs = idx % AT_CPR;
+      if (idx < BK * AT_CPR) *TNX_LDS(i32x4, stage_base + row * AT_ROWB + ((cs ^ C::template swzT<AT_CPR>(row)) << 4)) = v;
+      return;
+    }
     const int row = idx / C::CPR_A, cs = idx % C::CPR_A;
     if (idx < BM * C::CPR_A) *TNX_LDS(i32x4, stage_base + row * C::ROWB_A + ((cs ^ C::swzA(row)) << 4)) = v;
   };
@@ -1544,7 +1580,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   };
   auto dma_advance = [&]() __attribute__((always_inline)) {
     if (TNX_LADDER == 3) return;        // + DMA ops, always of the tile's first slabs (served by the L2)
-    a_sbase += BK * ES;
+    a_sbase += AT ? (int64_t)BK * p.sak * ES : (int64_t)BK * ES;
     if (GATHER) gather_next();
     else if (!CONV) b_sbase += BT ? (int64_t)BK * ES : (int64_t)BK * p.sbk * ES;
   };
@@ -1573,6 +1609,16 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     b_joff[j] = (uint32_t)(((16 / ES) * b_kg + b_sub) * C::ROWB_B) + (((colb >> 4) ^ b_sw) << 4) + (colb & 15);
   }
 
+  // m-contiguous A: as a row-major B slab
+  const int at_colb0 = (wy * C::WTM) * ES + ((ES == 2) ? 8 * (li & 3) : 8 * (li & 1));
+  const int at_sw = C::template swzT<AT_CPR>((16 / ES) * b_kg + b_sub);
+  uint32_t at_off[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    int colb = at_colb0 + i * MI * ES;
+    at_off[i] = (uint32_t)(((16 / ES) * b_kg + b_sub) * AT_ROWB) + (((colb >> 4) ^ at_sw) << 4) + (colb & 15);
+  }
+
   // k-contiguous B: fragment j of k step ks sits at bt_koff[ks] + j * MI rows, read like an A fragment
   const int bt_row = wx * C::WTN + (lane % MI);
   uint32_t bt_koff[C::KSTEPS];
@@ -1589,18 +1635,44 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   // two register sets of fragments: one being multiplied, one being filled
   i32x4 fa[2][TM];
   i32x2 fb[2][TN][2];
+  i32x2 fat[2][TM][2];          // m-contiguous A: two transposing reads per fragment
   i32x4 fbq[2][TN];             // k-contiguous B: one 16-byte read per fragment
   constexpr int NBREAD = BT ? TN : 2 * TN;
-  constexpr int NREAD = NBREAD + TM, NMMA = TM * TN;
+  constexpr int NREAD = NBREAD + (AT ? 2 * TM : TM), NMMA = TM * TN;
   constexpr int RPM = (NREAD + NMMA - 1) / NMMA;        // LDS reads slotted behind each MFMA
   constexpr int DPM = (C::LPW + NMMA - 1) / NMMA;       // DMA ops slotted behind each MFMA
 
+  // The swizzle XORs chunk-index bits that hold nothing but the fragment's number, so the offset of fragment j of an A^T
+  // or B slab is that of fragment 0 with j * MI * ES XOR-ed in.  The 256-wide AT tiles form it that way, one vector
+  // instruction per fragment: kept in registers, 12 offsets for each of two slots (which lie further apart than an LDS
+  // instruction's immediate reaches) spill inside the K loop (4096 x 4096 x 2048: 184 us, with the XOR 55).  The asm
+  // keeps the compiler from computing them ahead of the loop all the same.
+  constexpr bool XOR_OFFS = AT && C::STAGE_BYTES >= 65536;
+  uint32_t xo_at = 0, xo_b = 0;
+  auto xor_off = [&](uint32_t base, int bits) __attribute__((always_inline)) {
+    uint32_t r;
+    asm volatile("v_xor_b32 %0, %1, %2" : "=v"(r) : "i"(bits), "v"(base));
+    return r;
+  };
   auto read_one = [&](int set, int idx, uint32_t sa, uint32_t sb, int ks) __attribute__((always_inline)) {
     if (BT && idx < NBREAD) {
       fbq[set][idx] = *TNX_LDS(i32x4, sb + bt_koff[ks] + idx * MI * C::ROWB_A);
     } else if (idx < NBREAD) {
       int j = idx >> 1, h = idx & 1;
-      fb[set][j][h] = lds_read_tr<ES>(sb + b_joff[j] + ks * C::MMA_K * C::ROWB_B + h * RPR * C::ROWB_B);
+      if constexpr (XOR_OFFS) {
+        if (h == 0) xo_b = xor_off(sb + b_joff[0], j * MI * ES);
+        fb[set][j][h] = lds_read_tr<ES>(xo_b + ks * C::MMA_K * C::ROWB_B + h * RPR * C::ROWB_B);
+      } else {
+        fb[set][j][h] = lds_read_tr<ES>(sb + b_joff[j] + ks * C::MMA_K * C::ROWB_B + h * RPR * C::ROWB_B);
+      }
+    } else if (AT) {
+      int i = (idx - NBREAD) >> 1, h = (idx - NBREAD) & 1;
+      if constexpr (XOR_OFFS) {
+        if (h == 0) xo_at = xor_off(sa + at_off[0], i * MI * ES);
+        fat[set][i][h] = lds_read_tr<ES>(xo_at + ks * C::MMA_K * AT_ROWB + h * RPR * AT_ROWB);
+      } else {
+        fat[set][i][h] = lds_read_tr<ES>(sa + at_off[i] + ks * C::MMA_K * AT_ROWB + h * RPR * AT_ROWB);
+      }
     } else {
       int i = idx - NBREAD;
       fa[set][i] = *TNX_LDS(i32x4, sa + a_koff[ks] + i * MI * C::ROWB_A);
@@ -1610,7 +1682,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     int i = idx / TN, j = idx % TN;
     if (i & 1) j = TN - 1 - j;   // serpentine walk of the wave's MFMA tiles: one operand changes per instruction, never both
     i32x4 b4 = BT ? fbq[set][j] : i32x4{fb[set][j][0].x, fb[set][j][0].y, fb[set][j][1].x, fb[set][j][1].y};
-    acc[i][j] = MMA::run(b4, fa[set][i], acc[i][j]);   // rows = n, cols = m: the tile comes out transposed
+    i32x4 a4 = AT ? i32x4{fat[set][i][0].x, fat[set][i][0].y, fat[set][i][1].x, fat[set][i][1].y} : fa[set][i];
+    acc[i][j] = MMA::run(b4, a4, acc[i][j]);   // rows = n, cols = m: the tile comes out transposed
   };
 
   // ---- pipeline ----------------------------------------------------------

@@ -19,6 +19,7 @@ struct KernelEntry {
   launch_fn persist;  // DMA loader, one workgroup per CU walking its tiles; may be null
   launch_fn fast_bt;  // DMA loader for k-contiguous B (stride_bk == 1, the `x @ w.t()` layout); may be null
   launch_fn conv;     // conv2d forward on the DMA loader (GemmParams::cv); may be null
+  launch_fn fast_at;  // DMA loader for m-contiguous A (stride_am == 1, the `x.t() @ dy` layout), row-major B; may be null
 };
 
 // records the hipError_t behind a TNX_E_HIP for tnx_last_hip_error() (per thread)
@@ -53,10 +54,11 @@ struct KernelGroup {
   int count;
 };
 
-template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false>
+template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false,
+          bool AT = false>
 hipError_t launch_tile(const GemmParams& p, unsigned grid, hipStream_t stream) {
   static_assert(GATHER ? C::VALID_GATHER : C::VALID, "tile configuration is not buildable");
-  hipLaunchKernelGGL((gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV, GATHER>), dim3(grid), dim3(C::THREADS), 0, stream, p);
+  hipLaunchKernelGGL((gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV, GATHER, AT>), dim3(grid), dim3(C::THREADS), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -107,6 +109,23 @@ template <class T, class C> struct ConvLaunch<T, C, true> {
   static constexpr launch_fn fn = &launch_tile<T, C, true, false, false, true>;
 };
 
+// The m-contiguous-A variant exists for the tiles the built-in choice proposes, with the waves and slots it gives them.
+// (64 rows of int8 are too short for the transposing read; the 256x256 tile takes eight waves for every K: with four it
+// spills.)
+template <class C> constexpr bool at_ok() {
+  return C::BK * C::ES == 128 && C::VALID_AT &&
+         ((C::BM == 256 && C::BN == 256 && C::NW == 8 && C::STAGES == 2) || (C::BM == 256 && C::BN == 128 && C::NW == 4 && C::STAGES == 3) ||
+          (C::BM == 128 && C::BN == 128 && C::NW == 8 && C::STAGES == 3) || (C::BM == 64 && C::BN == 128 && C::NW == 8 && C::STAGES == 3) ||
+          (C::BM == 64 && C::BN == 64 && C::NW == 4 && C::STAGES == 4) || (C::BM == 192 && C::BN == 192 && C::NW == 8 && C::STAGES == 3) ||
+          ((C::BM == 192 || C::BN == 192) && C::BM != C::BN && C::NW == 8 && C::STAGES == 2));
+}
+template <class T, class C, bool OK = at_ok<C>()> struct AtLaunch {
+  static constexpr launch_fn fn = nullptr;
+};
+template <class T, class C> struct AtLaunch<T, C, true> {
+  static constexpr launch_fn fn = &launch_tile<T, C, true, false, false, false, false, true>;
+};
+
 // The element-wise loader is built only for the tiles that ask for it (a conditional expression would instantiate
 // the kernel for every tile and merely not point at it).
 template <class T, class C, bool WANTED> struct GenericLaunch {
@@ -124,6 +143,6 @@ template <class T, class C> struct GenericLaunch<T, C, true> {
    &launch_tile<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>, true>,                                                \
    GenericLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>, GENERIC>::fn,                                        \
    PersistLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::fn, BtLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::fn,     \
-   ConvLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::fn}
+   ConvLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::fn, AtLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::fn}
 
 }  // namespace tnx

@@ -173,10 +173,10 @@ def glu(x: torch.Tensor, w12: torch.Tensor, activation: str = "silu") -> torch.T
         raise ValueError("the interleaved weight must have an even number of columns")
     if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
         raise ValueError(f"glu is built for float16, bfloat16 and float32, got {x.dtype}")
-    x, w12 = _mm.dma_operands(x, w12)
+    x, w12, layout = _mm.engine_operands(x, w12)
     m, k = x.shape
     n = w12.shape[1]
-    key = (m, n, k, x.dtype, _mm.dma_layout(x, w12))
+    key = (m, n, k, x.dtype, layout)
     return _mm.run_memoised(_glu_cfg, "glu", key, glu_kernel, lambda cfg: _launch_glu(x, w12, cfg, activation),
                             lambda: _mm.default_config(x, w12))
 
