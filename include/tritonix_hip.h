@@ -200,6 +200,14 @@ int tnx_tile_coords(int schedule, int id, int tiles_m, int tiles_n, int group_m,
 int tnx_split_f32(const float* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c, void* dst, int side,
                   void* stream);
 
+/* A float32 product in two launches: both operands of `args` (in_dtype = out_dtype = TNX_F32; any strides) are cut into
+ * those terms in one pass, then multiplied as the bf16 problem.  Tile, K cut and workspace are those of the bf16
+ * problem (tnx_gemm_default_config fills them for in_dtype = TNX_F32); GLU epilogues apply as in tnx_gemm.  scratch: at
+ * least tnx_gemm_f32_scratch_bytes(args) bytes, 256-byte aligned, no initialisation needed; calls that share it must be
+ * ordered.  Asynchronous, allocates nothing. */
+size_t tnx_gemm_f32_scratch_bytes(const tnx_gemm_args* args);
+int tnx_gemm_f32(const tnx_gemm_args* args, void* scratch, size_t scratch_bytes);
+
 /* Number of compiled tile kernels, and a description of the i-th one:
  * "dtype bm bn bk warps stages [generic] [persistent]" as a NUL-terminated string (static storage);
  * "generic": also built with the element-wise loader; "persistent": also built for TNX_SCHED_PERSISTENT. */

@@ -335,12 +335,12 @@ def _compile(src, obj, verbose, force=True):
 
 def demangled_tile(name):
     """'bf16 256x256x64 w4 s2 fast' from a mangled gemm_tile_kernel instantiation (None for other kernels)."""
-    m = re.search(r"gemm_tile_kernelINS_(\d)Tag(\w+?)ENS_7TileCfgIS1_Li(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)EEELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
+    m = re.search(r"gemm_tile_kernelINS_(\d)Tag(\w+?)ENS_7TileCfgIS1_Li(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)EEELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
     if not m:
         return None
-    _, tag, bm, bn, bk, nw, st, fast, persist, bt, conv, gather, at = m.groups()
+    _, tag, bm, bn, bk, nw, st, fast, persist, bt, conv, gather, at, out32 = m.groups()
     kind = "at" if at == "1" else "packed conv" if gather == "1" else "conv" if conv == "1" else "bt" if bt == "1" else "persistent" if persist == "1" else "fast" if fast == "1" else "generic"
-    return f"{tag.lower()} {bm}x{bn}x{bk} w{nw} s{st} {kind}"
+    return f"{tag.lower()} {bm}x{bn}x{bk} w{nw} s{st} {kind}{' f32 out' if out32 == '1' else ''}"
 
 
 def build(jobs=None, quick=False, verbose=True, force=True, only=None, out=None, defines=(), only_conv=None):
@@ -359,7 +359,7 @@ def build(jobs=None, quick=False, verbose=True, force=True, only=None, out=None,
     srcs = generate(instances) + generate_conv(conv_instances, os.path.join(BUILD, "gen")) + generate_gather(
         GATHER_TILES if not (only or only_conv) or only == "gather" else (), os.path.join(BUILD, "gen")) + [
         os.path.join(CSRC, "capi.hip"), os.path.join(CSRC, "skinny.hip"),
-        os.path.join(CSRC, "conv.hip")]
+        os.path.join(CSRC, "conv.hip"), os.path.join(CSRC, "f32.hip")]
     objdir = os.path.join(BUILD, "obj")
     os.makedirs(objdir, exist_ok=True)
     objs = [os.path.join(objdir, os.path.basename(s)[:-4] + ".o") for s in srcs]

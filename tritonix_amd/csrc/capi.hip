@@ -72,7 +72,8 @@ static int check_common(const tnx_gemm_args* a) {
   // ... or binary32 for the 16-bit float types, on the tiles that carry that epilogue (f32_out_tile in gemm_tile.h)
   int want_out = a->in_dtype == TNX_I8 ? TNX_I32 : a->in_dtype;
   if (a->out_dtype != want_out) {
-    const bool f32_out = a->out_dtype == TNX_F32 && a->in_dtype != TNX_I8 && (int64_t)a->block_m * a->block_n <= 128 * 128 &&
+    const bool f32_out = a->out_dtype == TNX_F32 && a->in_dtype != TNX_I8 &&
+                         ((int64_t)a->block_m * a->block_n <= 128 * 128 || (find_entry(a) && find_entry(a)->out32[0])) &&
                          !(a->schedule & TNX_SCHED_PERSISTENT) && !is_skinny_cfg(a);
     if (!f32_out) return TNX_E_UNSUPPORTED;
   }
@@ -149,7 +150,7 @@ extern "C" size_t tnx_gemm_workspace_bytes(const tnx_gemm_args* a) {
 }
 
 static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool* fast, bool inspect_ptrs, bool* bt = nullptr,
-                          bool* tail = nullptr, bool* at = nullptr) {
+                          bool* tail = nullptr, bool* at = nullptr, bool padded = false) {
   if (bt) *bt = false;
   if (at) *at = false;
   if (tail) *tail = false;
@@ -177,9 +178,11 @@ static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool*
   if (!e) return TNX_E_UNSUPPORTED;
   tnx_gemm_args tmp = *a;
   if (!inspect_ptrs) { tmp.a = nullptr; tmp.b = nullptr; }
+  if (padded) { tmp.m = (tmp.m + 7) / 8 * 8; tmp.n = (tmp.n + 7) / 8 * 8; }    // 16-bit operands: chunks of 8 elements
   bool tail_slab = false;
   // the persistent kernel keeps the strict layout
   const int layout = dma_layout(&tmp, (a->schedule & TNX_SCHED_PERSISTENT) ? nullptr : &tail_slab);
+  if (a->out_dtype == TNX_F32 && e->out32[0] && layout == 0) return TNX_E_UNSUPPORTED;   // DMA loaders only
   bool f = layout == 1 || (layout == 2 && e->fast_bt) || (layout == 3 && e->fast_at);
   if (tail) *tail = f && tail_slab;
   if (!f && !e->generic) return TNX_E_UNSUPPORTED;
@@ -244,10 +247,23 @@ bool tnx::gemm_tile_for(int dtype, int bm, int bn, int bk, int* num_warps, int* 
   return true;
 }
 
-int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra) {
+void tnx::gemm_tile_layouts(const tnx_gemm_args* a, bool* bt, bool* at) {
+  const KernelEntry* e = find_entry(a);
+  *bt = e && e->fast_bt;
+  *at = e && e->fast_at;
+}
+
+int tnx::gemm_check(const tnx_gemm_args* a, bool padded) {
+  const int st = supported_impl(a, nullptr, nullptr, true, nullptr, nullptr, nullptr, padded);
+  if (st != TNX_OK) return st;
+  const size_t need = tnx_gemm_workspace_bytes(a);
+  return need > 0 && (!a->workspace || a->workspace_bytes < need || ((uintptr_t)a->workspace & 255)) ? TNX_E_WORKSPACE : TNX_OK;
+}
+
+int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, bool padded) {
   const KernelEntry* e = nullptr;
   bool fast = false, bt = false, at = false, tail_slab = false;
-  int st = supported_impl(a, &e, &fast, true, &bt, &tail_slab, &at);
+  int st = supported_impl(a, &e, &fast, true, &bt, &tail_slab, &at, padded);
   if (st != TNX_OK) return st;
   if (extra && (e->bm * e->bn > 128 * 128 || a->split_k != 1 || (a->schedule & TNX_SCHED_PERSISTENT) || is_skinny_cfg(a) || extra->batch < 1 ||
                 a->epilogue != TNX_EPI_NONE || (extra->bias && a->in_dtype == TNX_I8)))
@@ -288,6 +304,8 @@ int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra) {
   p.c_vec_ok = a->stride_cn == 1 && ((a->stride_cm * es_out) % 16) == 0 && (((uintptr_t)a->c) % 16) == 0;
   p.c_row_ok = a->stride_cn == 1;
   p.tail_slab = tail_slab ? 1 : 0;
+  p.m_load = padded ? (a->m + 7) / 8 * 8 : a->m;
+  p.n_load = padded ? (a->n + 7) / 8 * 8 : a->n;
   int64_t problems = 1;
   if (extra) {
     p.batch = extra->batch;
@@ -311,7 +329,10 @@ int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra) {
     err = e->persist(p, (unsigned)(tiles < cus ? tiles : cus), stream);
   } else {
     unsigned grid = a->split_k > 1 ? (unsigned)(p.split_tile0 + ncut * a->split_k) : (unsigned)((int64_t)p.tiles_m * p.tiles_n * problems);
-    err = (at ? e->fast_at : bt ? e->fast_bt : fast ? e->fast : e->generic)(p, grid, stream);
+    if (a->out_dtype == TNX_F32 && e->out32[0])
+      err = e->out32[at ? 2 : bt ? 1 : 0](p, grid, stream);
+    else
+      err = (at ? e->fast_at : bt ? e->fast_bt : fast ? e->fast : e->generic)(p, grid, stream);
   }
   if (err != hipSuccess) { g_last_hip_error = (int)err; return TNX_E_HIP; }
 
@@ -390,6 +411,23 @@ extern "C" int tnx_gemm_static_workspace(const tnx_gemm_args* a) {
 
 extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
   if (!a) return TNX_E_INVALID;
+  if (a->in_dtype == TNX_F32) {
+    // the bf16 problem tnx_gemm_f32 makes of it: three terms along k, aligned operands, k or the other dimension
+    // contiguous as in the float32 operand
+    tnx_gemm_args t = *a;
+    t.in_dtype = TNX_BF16; t.out_dtype = TNX_F32;
+    t.a = t.b = nullptr;
+    t.m = (a->m + 7) / 8 * 8; t.n = (a->n + 7) / 8 * 8;
+    t.k = ((a->k + 7) / 8 * 24 + 63) / 64 * 64;
+    const bool bt = a->stride_bk == 1 && a->stride_bn != 1, at = !bt && a->stride_am == 1 && a->stride_ak != 1 && a->stride_bk != 1;
+    t.stride_am = at ? 1 : t.k; t.stride_ak = at ? t.m : 1;
+    t.stride_bk = bt ? 1 : t.n; t.stride_bn = bt ? t.k : 1;
+    const int st = tnx_gemm_default_config(&t);
+    a->block_m = t.block_m; a->block_n = t.block_n; a->block_k = t.block_k; a->group_m = t.group_m;
+    a->split_k = t.split_k; a->tail_tiles = t.tail_tiles; a->schedule = t.schedule;
+    a->num_stages = t.num_stages; a->num_warps = t.num_warps;
+    return st;
+  }
   const int es = elem_size(a->in_dtype);
   const int bk = es == 1 ? 128 : 64;   // 128 bytes of K per LDS row for either element size
   // Workgroups that run together: the CU count of the current device, or MI355X's 256 when no device can be asked
@@ -450,8 +488,8 @@ extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
   const int ncand = 8;
   // int8: rows of a 64-wide B tile are too short for the transposing read; the 192-wide tiles exist for it too
   // (3072 x 4096 x 4096: 53.6 -> 45.7 us with 192x256, 4096 x 3072 x 4096: 52.8 -> 47.3 us with 256x192)
-  // (a binary32 result exists on the tiles up to 128x128 only)
-  auto usable = [&](int i) { return (es == 2 || i != 4) && !(at && es == 1 && i == 3) && (a->out_dtype != TNX_F32 || (i >= 2 && i <= 4)); };
+  // (a binary32 result exists on the tiles up to 128x128 and on the eight-wave tiles of 192 and 256)
+  auto usable = [&](int i) { return (es == 2 || i != 4) && !(at && es == 1 && i == 3) && (a->out_dtype != TNX_F32 || i != 1); };
   const double cu_flops = 5.5e12 * (es == 1 ? 1.7 : 1.0);          // per CU with the largest tile
   const double launch = 3e-6, handover = 9e-6, readback = 60e9;
   const int64_t kt = (a->k + bk - 1) / bk;
@@ -493,6 +531,7 @@ extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
   // price of half again as many LDS reads, which is what loses on the long, power-limited 8192^3 loops.
   // (cut tiles too: 4096 x 5120 x 4096 with its last 64 tiles cut, 155 -> 140 us)
   if (es == 2 && bi == 0 && kt <= 64) a->num_warps = 8;
+  if (bi == 0 && a->out_dtype == TNX_F32) a->num_warps = 8;
   if (at && bi == 0) a->num_warps = 8;                               // the only 256x256 kernels built for an m-contiguous A
   a->split_k = bs;
   a->tail_tiles = btail;

@@ -130,6 +130,7 @@ struct GemmParams {
   int out_dtype;
   bool c_vec_ok;          // C takes 16-byte stores along n (stride_cn == 1, 16-byte aligned rows)
   bool c_row_ok;          // stride_cn == 1: rows of C take 16-byte stores at the element's own alignment
+  int64_t m_load, n_load; // DMA kernels: rows of an m-contiguous A and columns of B that may be loaded (>= m, n: operands padded to whole chunks)
   int tail_slab;          // DMA kernels: the last K slab (whole or partial) goes through the element-wise loader
   bool b_once;            // every element of B is read by exactly one workgroup (one tile row): stream it non-temporally
   int tile_order;         // 0: XCD remap + tl.swizzle2d(group_m); 1: 16x16 super-blocks in serpentine order (superblock_order)
@@ -997,11 +998,13 @@ template <int V> struct IntTag { static constexpr int value = V; };
 // t+2, before whose period nothing reads it.  16-bit types, stride_w == 1, k % BK == 0.
 // AT: A is m-contiguous (element (m, k) at a + k * stride_ak + m, the layout of `x.t() @ dy`): its slab sits in LDS as
 // BK rows of BM elements exactly like a row-major B slab, and its fragments are read with the transposing reads.
+// OUT32: the result is binary32 and nothing else.  (The tiles up to 128x128 carry both epilogues in one kernel, f32_out_tile;
+// in the 192- and 256-wide ones a second epilogue costs hundreds of spilled registers, so they have kernels of their own.)
 // GATHER (with BT): conv2d forward over a packed input (PackGeom): the rows of the k-contiguous B slab are the windows of
 // BN output pixels.  A lane's DMA ops fetch the same 16-byte k chunk of different pixels, so an op's offset is the
 // pixel's, kept in a register, plus the chunk's (filter tap, channels), read once per slab from a table in LDS.  Chunks
 // past the end of k get an offset outside the buffer and arrive as zeros.
-template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false, bool AT = false>
+template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false, bool AT = false, bool OUT32 = false>
 __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   constexpr int ES = C::ES, BM = C::BM, BN = C::BN, BK = C::BK, NW = C::NW, STAGES = C::STAGES;
   constexpr int MI = C::MI, TM = C::TM, TN = C::TN;
@@ -1188,7 +1191,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
           // rows of the slab are k, as in a row-major B slab: chunks past M as chunks past N there
           int row = P / AT_CPR, cs = P % AT_CPR;
           int c = cs ^ C::template swzT<AT_CPR>(row);
-          if (m0 + (int64_t)c * (16 / ES) >= p.m || (!p.tail_slab && m0 + (int64_t)(c + 1) * (16 / ES) > p.m)) c = 0;
+          if (m0 + (int64_t)c * (16 / ES) >= p.m_load || (!p.tail_slab && m0 + (int64_t)(c + 1) * (16 / ES) > p.m_load)) c = 0;
           a_voff[q] = (uint32_t)((int64_t)row * p.sak * ES + c * 16);
           continue;
         }
@@ -1253,7 +1256,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
           // column chunk past N: any valid address.  (A chunk that starts below N and ends above it -- tail_slab
           // launches only -- is loaded as it is: its upper elements come from the next k row, which exists because
           // the last slab is not loaded here, and belong to columns that are never stored.)
-          if (n0 + (int64_t)c * (16 / ES) >= p.n || (!p.tail_slab && n0 + (int64_t)(c + 1) * (16 / ES) > p.n)) c = 0;
+          if (n0 + (int64_t)c * (16 / ES) >= p.n_load || (!p.tail_slab && n0 + (int64_t)(c + 1) * (16 / ES) > p.n_load)) c = 0;
           b_voff[q] = (uint32_t)((int64_t)row * ldb * ES + c * 16);
         }
       }
@@ -2104,6 +2107,10 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
                                                 p.c_row_ok, p.epilogue);
       }
     };
+    if constexpr (OUT32) {
+      finish(TypeTag<OutF32>{});
+      return;
+    }
     if constexpr (f32_out_tile<T, C>()) {
       if (p.out_dtype == DT_F32) {
         finish(TypeTag<OutF32>{});

@@ -103,32 +103,6 @@ def drop_workspace(device, stream_ptr: int) -> None:
         _workspaces.pop(_workspace_key(device, stream_ptr, atomic), None)
 
 
-def split_f32_operands(bound: dict, stream: int) -> dict:
-    """A bound float32 call rewritten as the bf16 call that computes it.
-
-    The reference's kernels take float32 operands and multiply them in TF32 (tritonix/ops/matmul.py:98,
-    tritonix/ops/swiglu.py:89-93); gfx950 has no TF32 matrix instruction.  ``tnx_split_f32`` cuts each operand into a
-    bf16 head and a bf16 tail and lays out ``[hi | hi | lo]`` along the columns of A and ``[hi ; lo ; hi]`` along the
-    rows of B, so one bf16 GEMM with ``k' = 3k`` and an fp32 result is ``hi(a) hi(b) + hi(a) lo(b) + lo(a) hi(b)``: error
-    O(2^-16) per product, below TF32's.  The two scratch operands are contiguous, whatever strides the call had.
-    """
-    import torch
-
-    a, b = bound["a"], bound["b"]
-    m, n, k = int(bound["m"]), int(bound["n"]), int(bound["k"])
-    lib = _C.load()
-    a3 = torch.empty((m, 3 * k), dtype=torch.bfloat16, device=a.device)
-    b3 = torch.empty((3 * k, n), dtype=torch.bfloat16, device=a.device)
-    for src, rows, cols, sr, sc, dst, side in ((a, m, k, bound["stride_am"], bound["stride_ak"], a3, 0),
-                                               (b, k, n, bound["stride_bk"], bound["stride_bn"], b3, 1)):
-        status = lib.tnx_split_f32(src.data_ptr(), rows, cols, int(sr), int(sc), dst.data_ptr(), side, stream)
-        if status != _C.OK:
-            raise RuntimeError(f"tnx_split_f32: {_C.strerror(status)}")
-    out = dict(bound)
-    out.update(a=a3, b=b3, k=3 * k, stride_am=3 * k, stride_ak=1, stride_bk=n, stride_bn=1)
-    return out
-
-
 class _BoundLaunch:
     def __init__(self, kernel: "HipKernel", grid):
         self.kernel, self.grid = kernel, grid
@@ -228,8 +202,6 @@ class HipKernel:
         if a.dtype == torch.float32 and b.dtype == torch.float32:
             if c.dtype != torch.float32:
                 raise ValueError(f"{self.__name__}: float32 operands give a float32 result, got c of {c.dtype}")
-            with torch.cuda.device(a.device):
-                bound = split_f32_operands(bound, torch.cuda.current_stream(a.device).cuda_stream)
         g = self.make_args(bound)
         if a.device.index != torch.cuda.current_device():
             with torch.cuda.device(a.device):
@@ -245,12 +217,23 @@ class HipKernel:
 
         stream = torch.cuda.current_stream(device).cuda_stream
         g.stream = stream
+        scratch = None
+        if g.in_dtype == _C.F32:
+            # the reference's kernels take float32 operands and multiply them in TF32 (tritonix/ops/matmul.py:98,
+            # tritonix/ops/swiglu.py:89-93), for which gfx950 has no matrix instruction: the library cuts them into bf16
+            # heads and tails and multiplies those, with a float32 result
+            need = int(lib.tnx_gemm_f32_scratch_bytes(ctypes.byref(g)))
+            scratch = torch.empty(need, dtype=torch.uint8, device=device)
         if g.split_k > 1:
             need = int(lib.tnx_gemm_workspace_bytes(ctypes.byref(g)))
             if need:
                 ws = _workspace(device, stream, need, bool(g.schedule & _C.SCHED_ATOMIC_REDUCE))
                 g.workspace, g.workspace_bytes = ws.data_ptr(), ws.numel()
-        status = lib.tnx_gemm(ctypes.byref(g))
+        if scratch is None:
+            status = lib.tnx_gemm(ctypes.byref(g))
+        else:
+            status = lib.tnx_gemm_f32(ctypes.byref(g), scratch.data_ptr(), scratch.numel())
+            g.in_dtype = _C.BF16 if status else g.in_dtype          # what an error message has to describe
         if status == _C.E_HIP and g.split_k > 1:
             drop_workspace(device, stream)
         return status

@@ -22,7 +22,7 @@ Deliberate differences:
     HIP engine, which settles tile against K split in its own config memo) is
     timed, ``torch.matmul`` is registered un-raced, for ``force_backend``;
   * int8 inputs give an int32 result; float32 inputs run as a three-term bf16 split with an fp32 result
-    (``tritonix_amd.kernel.split_f32_operands``) where the reference multiplies them in TF32;
+    (``tnx_gemm_f32``) where the reference multiplies them in TF32;
   * split-K sums fp32 partials from a workspace and rounds once, where the
     reference rounds each partial to the output dtype and adds atomically
     (tritonix/ops/matmul.py:195-202); the ``_zero_output`` hook is gone with it.
@@ -211,7 +211,7 @@ def dma_operands(a, b):
 def _transposed_a(a, b) -> bool:
     """A column-major A (``x.t()`` of a row-major x) with a row-major B, of a type the transposing loader is built for."""
     return (a.stride(0) == 1 and a.stride(1) >= a.shape[0] and a.stride(1) != 1 and b.stride(1) == 1 and b.stride(0) >= b.shape[1]
-            and a.dtype in (torch.float16, torch.bfloat16, torch.int8))
+            and a.dtype in (torch.float16, torch.bfloat16, torch.int8, torch.float32))
 
 
 def engine_operands(a, b):
@@ -278,10 +278,9 @@ def default_config(a, b, split=False):
     g.m, g.k = a.shape
     g.n = b.shape[1]
     if a.dtype == torch.float32:
-        # what the launch turns a float32 problem into: contiguous bf16 operands, three terms along K, fp32 result
-        g.k = 3 * g.k
-        g.stride_am, g.stride_ak, g.stride_bk, g.stride_bn = g.k, 1, g.n, 1
-        g.in_dtype, g.out_dtype = _C.BF16, _C.F32
+        g.stride_am, g.stride_ak = a.stride()
+        g.stride_bk, g.stride_bn = b.stride()
+        g.in_dtype, g.out_dtype = _C.F32, _C.F32
     else:
         g.stride_am, g.stride_ak = a.stride()
         g.stride_bk, g.stride_bn = b.stride()
