@@ -409,6 +409,9 @@ extern "C" int tnx_gemm_static_workspace(const tnx_gemm_args* a) {
   return tnx_gemm(&t);
 }
 
+// large_f32: a binary32 result may go to the tiles beyond 128x128 that have one (tnx_gemm_f32's problems; bf16)
+static int default_config(tnx_gemm_args* a, bool large_f32);
+
 extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
   if (!a) return TNX_E_INVALID;
   if (a->in_dtype == TNX_F32) {
@@ -422,12 +425,16 @@ extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
     const bool bt = a->stride_bk == 1 && a->stride_bn != 1, at = !bt && a->stride_am == 1 && a->stride_ak != 1 && a->stride_bk != 1;
     t.stride_am = at ? 1 : t.k; t.stride_ak = at ? t.m : 1;
     t.stride_bk = bt ? 1 : t.n; t.stride_bn = bt ? t.k : 1;
-    const int st = tnx_gemm_default_config(&t);
+    const int st = default_config(&t, true);
     a->block_m = t.block_m; a->block_n = t.block_n; a->block_k = t.block_k; a->group_m = t.group_m;
     a->split_k = t.split_k; a->tail_tiles = t.tail_tiles; a->schedule = t.schedule;
     a->num_stages = t.num_stages; a->num_warps = t.num_warps;
     return st;
   }
+  return default_config(a, false);
+}
+
+static int default_config(tnx_gemm_args* a, bool large_f32) {
   const int es = elem_size(a->in_dtype);
   const int bk = es == 1 ? 128 : 64;   // 128 bytes of K per LDS row for either element size
   // Workgroups that run together: the CU count of the current device, or MI355X's 256 when no device can be asked
@@ -488,8 +495,8 @@ extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
   const int ncand = 8;
   // int8: rows of a 64-wide B tile are too short for the transposing read; the 192-wide tiles exist for it too
   // (3072 x 4096 x 4096: 53.6 -> 45.7 us with 192x256, 4096 x 3072 x 4096: 52.8 -> 47.3 us with 256x192)
-  // (a binary32 result exists on the tiles up to 128x128 and on the eight-wave tiles of 192 and 256)
-  auto usable = [&](int i) { return (es == 2 || i != 4) && !(at && es == 1 && i == 3) && (a->out_dtype != TNX_F32 || i != 1); };
+  // (a binary32 result exists on the tiles up to 128x128 and, for bf16, on the eight-wave tiles of 192 and 256)
+  auto usable = [&](int i) { return (es == 2 || i != 4) && !(at && es == 1 && i == 3) && (a->out_dtype != TNX_F32 || (i >= 2 && i <= 4) || (large_f32 && i != 1)); };
   const double cu_flops = 5.5e12 * (es == 1 ? 1.7 : 1.0);          // per CU with the largest tile
   const double launch = 3e-6, handover = 9e-6, readback = 60e9;
   const int64_t kt = (a->k + bk - 1) / bk;
