@@ -20,7 +20,7 @@ from typing import Dict, Optional, Tuple
 import torch
 
 from tritonix_amd import _C
-from tritonix_amd.kernel import cdiv
+from tritonix_amd.kernel import _stream_of, cdiv
 
 __all__ = ["conv2d_forward", "conv2d_forward_kernel", "torch_conv2d_forward", "output_size", "candidate_configs"]
 
@@ -292,7 +292,7 @@ def _launch_planned(input, weight, bias, stride, padding, dilation) -> Optional[
     if need:
         ws = torch.empty(need, dtype=torch.uint8, device=input.device)
         a.workspace, a.workspace_bytes = ws.data_ptr(), need
-    a.stream = torch.cuda.current_stream(dev).cuda_stream
+    a.stream = _stream_of(dev)
     if dev != torch.cuda.current_device():
         with torch.cuda.device(dev):
             status = lib.tnx_conv2d_forward(ctypes.byref(a))

@@ -35,7 +35,7 @@ import torch
 
 from tritonix_amd.autotune import Choice, PowerOfTwo, Range, tunable
 from tritonix_amd.dispatcher import dynamic_dispatch
-from tritonix_amd.kernel import HipKernel, cdiv, out_dtype_for
+from tritonix_amd.kernel import HipKernel, cdiv, keep_plan, out_dtype_for, plan_key, planned
 
 __all__ = ["matmul", "triton_matmul", "hip_matmul", "matmul_splitk", "matmul_skinny", "matmul_kernel", "gemm_splitk_kernel",
            "dma_layout", "dma_operands", "run_memoised",
@@ -349,15 +349,23 @@ def triton_matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     ``matmul`` refer to it.  ``hip_matmul`` is the same function.  For thin problems the tuned config may carry a
     K split (``_tile_or_split``).
     """
+    pkey = plan_key("matmul", a, b)
+    plan = planned(pkey, _matmul_cfg)
+    if plan is not None:
+        return plan(a, b)
     _check_2d(a, b)
+    given = (a, b)
     a, b, layout = engine_operands(a, b)
     m, k = a.shape
     _, n = b.shape
     key = (m, n, k, a.dtype, layout)
     if key not in _matmul_cfg:
         _matmul_cfg[key] = _tile_or_split(a, b, key)
-    return run_memoised(_matmul_cfg, "matmul", key, matmul_kernel, lambda cfg: _launch_matmul(a, b, cfg),
-                        lambda: default_config(a, b))
+    c = run_memoised(_matmul_cfg, "matmul", key, matmul_kernel, lambda cfg: _launch_matmul(a, b, cfg),
+                     lambda: default_config(a, b))
+    if a is given[0] and b is given[1]:          # operands that had to be copied first keep the long way
+        keep_plan(pkey, key, _matmul_cfg, matmul_kernel, a, b, c)
+    return c
 
 
 hip_matmul = triton_matmul
@@ -369,13 +377,21 @@ def matmul_splitk(a: torch.Tensor, b: torch.Tensor, split_k: int = 4) -> torch.T
     As in the reference (tritonix/ops/matmul.py:280-288) ``split_k`` only keys
     the config memo; the split factor launched is the one the tuner picked.
     """
+    pkey = plan_key(("splitk", split_k), a, b)
+    plan = planned(pkey, _splitk_cfg)
+    if plan is not None:
+        return plan(a, b)
     _check_2d(a, b)
+    given = (a, b)
     a, b, layout = engine_operands(a, b)
     m, k = a.shape
     _, n = b.shape
     key = (m, n, k, split_k, a.dtype, layout)
-    return run_memoised(_splitk_cfg, "matmul_splitk", key, gemm_splitk_kernel, lambda cfg: _launch_splitk(a, b, cfg),
-                        lambda: default_config(a, b, split=True))
+    c = run_memoised(_splitk_cfg, "matmul_splitk", key, gemm_splitk_kernel, lambda cfg: _launch_splitk(a, b, cfg),
+                     lambda: default_config(a, b, split=True))
+    if a is given[0] and b is given[1]:
+        keep_plan(pkey, key, _splitk_cfg, gemm_splitk_kernel, a, b, c)
+    return c
 
 
 # the m <= 16 kernel: eight waves of a workgroup each take an eighth of K and meet in LDS

@@ -20,7 +20,7 @@ from __future__ import annotations
 import torch
 
 from tritonix_amd.autotune import Choice, PowerOfTwo, Range, tunable
-from tritonix_amd.kernel import HipKernel, cdiv
+from tritonix_amd.kernel import HipKernel, cdiv, keep_plan, plan_key, planned
 import importlib
 
 _mm = importlib.import_module("tritonix_amd.ops.matmul")  # the module: the package attribute `matmul` is the dispatcher
@@ -167,18 +167,26 @@ _glu_cfg = {}
 
 def glu(x: torch.Tensor, w12: torch.Tensor, activation: str = "silu") -> torch.Tensor:
     """``act(x @ w12[:, 0::2]) * (x @ w12[:, 1::2])`` -> ``[m, n/2]``, tile config tuned once per shape."""
+    pkey = plan_key(("glu", activation), x, w12)
+    plan = planned(pkey, _glu_cfg)
+    if plan is not None:
+        return plan(x, w12)
     if x.dim() != 2 or w12.dim() != 2 or x.shape[1] != w12.shape[0]:
         raise ValueError(f"glu expects x[m,k] and w12[k,2n], got {tuple(x.shape)} and {tuple(w12.shape)}")
     if w12.shape[1] % 2:
         raise ValueError("the interleaved weight must have an even number of columns")
     if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
         raise ValueError(f"glu is built for float16, bfloat16 and float32, got {x.dtype}")
+    given = (x, w12)
     x, w12, layout = _mm.engine_operands(x, w12)
     m, k = x.shape
     n = w12.shape[1]
     key = (m, n, k, x.dtype, layout)
-    return _mm.run_memoised(_glu_cfg, "glu", key, glu_kernel, lambda cfg: _launch_glu(x, w12, cfg, activation),
-                            lambda: _mm.default_config(x, w12))
+    z = _mm.run_memoised(_glu_cfg, "glu", key, glu_kernel, lambda cfg: _launch_glu(x, w12, cfg, activation),
+                         lambda: _mm.default_config(x, w12))
+    if x is given[0] and w12 is given[1]:
+        keep_plan(pkey, key, _glu_cfg, glu_kernel, x, w12, z, activation=activation)
+    return z
 
 
 def swiglu(x: torch.Tensor, w12: torch.Tensor) -> torch.Tensor:
