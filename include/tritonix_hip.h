@@ -201,7 +201,8 @@ int tnx_split_f32(const float* src, int64_t rows, int64_t cols, int64_t stride_r
                   void* stream);
 
 /* A float32 product in two launches: both operands of `args` (in_dtype = out_dtype = TNX_F32; any strides) are cut into
- * those terms in one pass, then multiplied as the bf16 problem.  Tile, K cut and workspace are those of the bf16
+ * bf16 heads and tails in one pass, then multiplied with those three products in one sum (in the tiles the built-in
+ * choice names, head and tail of an operand are stored once; in every other tile as the three copies above).  Tile, K cut and workspace are those of the bf16
  * problem (tnx_gemm_default_config fills them for in_dtype = TNX_F32); GLU epilogues apply as in tnx_gemm.  scratch: at
  * least tnx_gemm_f32_scratch_bytes(args) bytes, 256-byte aligned, no initialisation needed; calls that share it must be
  * ordered.  Asynchronous, allocates nothing. */

@@ -338,9 +338,9 @@ def demangled_tile(name):
     m = re.search(r"gemm_tile_kernelINS_(\d)Tag(\w+?)ENS_7TileCfgIS1_Li(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)EEELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
     if not m:
         return None
-    _, tag, bm, bn, bk, nw, st, fast, persist, bt, conv, gather, at, out32 = m.groups()
+    _, tag, bm, bn, bk, nw, st, fast, persist, bt, conv, gather, at, pair = m.groups()
     kind = "at" if at == "1" else "packed conv" if gather == "1" else "conv" if conv == "1" else "bt" if bt == "1" else "persistent" if persist == "1" else "fast" if fast == "1" else "generic"
-    return f"{tag.lower()} {bm}x{bn}x{bk} w{nw} s{st} {kind}{' f32 out' if out32 == '1' else ''}"
+    return f"{tag.lower()} {bm}x{bn}x{bk} w{nw} s{st} {kind}{' f32 pair' if pair == '1' else ''}"
 
 
 def build(jobs=None, quick=False, verbose=True, force=True, only=None, out=None, defines=(), only_conv=None):

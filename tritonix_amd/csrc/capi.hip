@@ -59,7 +59,7 @@ static int64_t lds_bytes_of(const tnx_gemm_args* a) {
   return ring > strips ? ring : strips;
 }
 
-static int check_common(const tnx_gemm_args* a) {
+static int check_common(const tnx_gemm_args* a, bool pair) {
   if (!a) return TNX_E_INVALID;
   if (a->m < 0 || a->n < 0 || a->k < 0) return TNX_E_INVALID;
   if (a->in_dtype != TNX_F16 && a->in_dtype != TNX_BF16 && a->in_dtype != TNX_I8) return TNX_E_INVALID;
@@ -73,7 +73,7 @@ static int check_common(const tnx_gemm_args* a) {
   int want_out = a->in_dtype == TNX_I8 ? TNX_I32 : a->in_dtype;
   if (a->out_dtype != want_out) {
     const bool f32_out = a->out_dtype == TNX_F32 && a->in_dtype != TNX_I8 &&
-                         ((int64_t)a->block_m * a->block_n <= 128 * 128 || (find_entry(a) && find_entry(a)->out32[0])) &&
+                         ((int64_t)a->block_m * a->block_n <= 128 * 128 || pair) &&
                          !(a->schedule & TNX_SCHED_PERSISTENT) && !is_skinny_cfg(a);
     if (!f32_out) return TNX_E_UNSUPPORTED;
   }
@@ -150,11 +150,11 @@ extern "C" size_t tnx_gemm_workspace_bytes(const tnx_gemm_args* a) {
 }
 
 static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool* fast, bool inspect_ptrs, bool* bt = nullptr,
-                          bool* tail = nullptr, bool* at = nullptr, bool padded = false) {
+                          bool* tail = nullptr, bool* at = nullptr, GemmForm form = GEMM_PLAIN) {
   if (bt) *bt = false;
   if (at) *at = false;
   if (tail) *tail = false;
-  int st = check_common(a);
+  int st = check_common(a, form == GEMM_PAIR);
   if (st != TNX_OK) return st;
   int64_t lds = lds_bytes_of(a);
   if (lds > TNX_LDS_LIMIT_BYTES) return TNX_E_LDS;
@@ -178,11 +178,11 @@ static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool*
   if (!e) return TNX_E_UNSUPPORTED;
   tnx_gemm_args tmp = *a;
   if (!inspect_ptrs) { tmp.a = nullptr; tmp.b = nullptr; }
-  if (padded) { tmp.m = (tmp.m + 7) / 8 * 8; tmp.n = (tmp.n + 7) / 8 * 8; }    // 16-bit operands: chunks of 8 elements
+  if (form != GEMM_PLAIN) { tmp.m = (tmp.m + 7) / 8 * 8; tmp.n = (tmp.n + 7) / 8 * 8; }    // 16-bit operands: chunks of 8 elements
   bool tail_slab = false;
   // the persistent kernel keeps the strict layout
   const int layout = dma_layout(&tmp, (a->schedule & TNX_SCHED_PERSISTENT) ? nullptr : &tail_slab);
-  if (a->out_dtype == TNX_F32 && e->out32[0] && layout == 0) return TNX_E_UNSUPPORTED;   // DMA loaders only
+  if (form == GEMM_PAIR && (a->out_dtype != TNX_F32 || layout == 0 || tail_slab || !e->pair[layout - 1])) return TNX_E_UNSUPPORTED;
   bool f = layout == 1 || (layout == 2 && e->fast_bt) || (layout == 3 && e->fast_at);
   if (tail) *tail = f && tail_slab;
   if (!f && !e->generic) return TNX_E_UNSUPPORTED;
@@ -247,25 +247,26 @@ bool tnx::gemm_tile_for(int dtype, int bm, int bn, int bk, int* num_warps, int* 
   return true;
 }
 
-void tnx::gemm_tile_layouts(const tnx_gemm_args* a, bool* bt, bool* at) {
+void tnx::gemm_tile_layouts(const tnx_gemm_args* a, bool* pair, bool* bt, bool* at) {
   const KernelEntry* e = find_entry(a);
-  *bt = e && e->fast_bt;
-  *at = e && e->fast_at;
+  *pair = e && e->pair[0];
+  *bt = e && (*pair ? e->pair[1] : e->fast_bt);
+  *at = e && (*pair ? e->pair[2] : e->fast_at);
 }
 
-int tnx::gemm_check(const tnx_gemm_args* a, bool padded) {
-  const int st = supported_impl(a, nullptr, nullptr, true, nullptr, nullptr, nullptr, padded);
+int tnx::gemm_check(const tnx_gemm_args* a, GemmForm form) {
+  const int st = supported_impl(a, nullptr, nullptr, true, nullptr, nullptr, nullptr, form);
   if (st != TNX_OK) return st;
   const size_t need = tnx_gemm_workspace_bytes(a);
   return need > 0 && (!a->workspace || a->workspace_bytes < need || ((uintptr_t)a->workspace & 255)) ? TNX_E_WORKSPACE : TNX_OK;
 }
 
-int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, bool padded) {
+int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, GemmForm form) {
   const KernelEntry* e = nullptr;
   bool fast = false, bt = false, at = false, tail_slab = false;
-  int st = supported_impl(a, &e, &fast, true, &bt, &tail_slab, &at, padded);
+  int st = supported_impl(a, &e, &fast, true, &bt, &tail_slab, &at, form);
   if (st != TNX_OK) return st;
-  if (extra && (e->bm * e->bn > 128 * 128 || a->split_k != 1 || (a->schedule & TNX_SCHED_PERSISTENT) || is_skinny_cfg(a) || extra->batch < 1 ||
+  if (extra && (form == GEMM_PAIR || e->bm * e->bn > 128 * 128 || a->split_k != 1 || (a->schedule & TNX_SCHED_PERSISTENT) || is_skinny_cfg(a) || extra->batch < 1 ||
                 a->epilogue != TNX_EPI_NONE || (extra->bias && a->in_dtype == TNX_I8)))
     return TNX_E_UNSUPPORTED;
   if (!a->a || !a->b || !a->c) {
@@ -304,8 +305,8 @@ int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, bool padded
   p.c_vec_ok = a->stride_cn == 1 && ((a->stride_cm * es_out) % 16) == 0 && (((uintptr_t)a->c) % 16) == 0;
   p.c_row_ok = a->stride_cn == 1;
   p.tail_slab = tail_slab ? 1 : 0;
-  p.m_load = padded ? (a->m + 7) / 8 * 8 : a->m;
-  p.n_load = padded ? (a->n + 7) / 8 * 8 : a->n;
+  p.m_load = form != GEMM_PLAIN ? (a->m + 7) / 8 * 8 : a->m;
+  p.n_load = form != GEMM_PLAIN ? (a->n + 7) / 8 * 8 : a->n;
   int64_t problems = 1;
   if (extra) {
     p.batch = extra->batch;
@@ -329,8 +330,8 @@ int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, bool padded
     err = e->persist(p, (unsigned)(tiles < cus ? tiles : cus), stream);
   } else {
     unsigned grid = a->split_k > 1 ? (unsigned)(p.split_tile0 + ncut * a->split_k) : (unsigned)((int64_t)p.tiles_m * p.tiles_n * problems);
-    if (a->out_dtype == TNX_F32 && e->out32[0])
-      err = e->out32[at ? 2 : bt ? 1 : 0](p, grid, stream);
+    if (form == GEMM_PAIR)
+      err = e->pair[at ? 2 : bt ? 1 : 0](p, grid, stream);
     else
       err = (at ? e->fast_at : bt ? e->fast_bt : fast ? e->fast : e->generic)(p, grid, stream);
   }
@@ -409,19 +410,19 @@ extern "C" int tnx_gemm_static_workspace(const tnx_gemm_args* a) {
   return tnx_gemm(&t);
 }
 
-// large_f32: a binary32 result may go to the tiles beyond 128x128 that have one (tnx_gemm_f32's problems; bf16)
+// large_f32: a problem of tnx_gemm_f32 (heads and tails in bf16), which may also go to the tiles of 192 and 256
 static int default_config(tnx_gemm_args* a, bool large_f32);
 
 extern "C" int tnx_gemm_default_config(tnx_gemm_args* a) {
   if (!a) return TNX_E_INVALID;
   if (a->in_dtype == TNX_F32) {
-    // the bf16 problem tnx_gemm_f32 makes of it: three terms along k, aligned operands, k or the other dimension
+    // the bf16 problem tnx_gemm_f32 makes of it: heads and tails along k, aligned operands, k or the other dimension
     // contiguous as in the float32 operand
     tnx_gemm_args t = *a;
     t.in_dtype = TNX_BF16; t.out_dtype = TNX_F32;
     t.a = t.b = nullptr;
     t.m = (a->m + 7) / 8 * 8; t.n = (a->n + 7) / 8 * 8;
-    t.k = ((a->k + 7) / 8 * 24 + 63) / 64 * 64;
+    t.k = (a->k + 31) / 32 * 64;
     const bool bt = a->stride_bk == 1 && a->stride_bn != 1, at = !bt && a->stride_am == 1 && a->stride_ak != 1 && a->stride_bk != 1;
     t.stride_am = at ? 1 : t.k; t.stride_ak = at ? t.m : 1;
     t.stride_bk = bt ? 1 : t.n; t.stride_bn = bt ? t.k : 1;
@@ -495,7 +496,7 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
   const int ncand = 8;
   // int8: rows of a 64-wide B tile are too short for the transposing read; the 192-wide tiles exist for it too
   // (3072 x 4096 x 4096: 53.6 -> 45.7 us with 192x256, 4096 x 3072 x 4096: 52.8 -> 47.3 us with 256x192)
-  // (a binary32 result exists on the tiles up to 128x128 and, for bf16, on the eight-wave tiles of 192 and 256)
+  // (a binary32 result exists on the tiles up to 128x128 and, for float32 products, on the eight-wave tiles of 192 and 256)
   auto usable = [&](int i) { return (es == 2 || i != 4) && !(at && es == 1 && i == 3) && (a->out_dtype != TNX_F32 || (i >= 2 && i <= 4) || (large_f32 && i != 1)); };
   const double cu_flops = 5.5e12 * (es == 1 ? 1.7 : 1.0);          // per CU with the largest tile
   const double launch = 3e-6, handover = 9e-6, readback = 60e9;
@@ -533,6 +534,10 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
   // 2048^3 21.2 -> 19.6 us, 2048^2 x 512 9.4 -> 8.1 us, 1024^3 9.1 -> 7.9 us; int8 128x128 5-13 % on seven shapes,
   // int8 64x128 mixed).
   if (bi == 2 || (es == 2 && bi == 3)) a->num_warps = 8;
+  // (float32 products run three MFMA steps on the fragments of two, so fewer fragment reads decide: four waves, 2048^3
+  // 55.2 -> 54.1 us, 4096^3 333 -> 327 us; not for an m-contiguous A, whose transposing reads double the count: 57 us with
+  // eight, above 71 with four.)
+  if (bi == 2 && large_f32 && !at) a->num_warps = 4;
   // 16-bit problems with a short K loop (at most 64 slabs per tile) spend a visible share of every tile outside
   // it; two waves per SIMD cover that better than one (measured on 4096 x 28672 x 4096, gated: +2.4 %), at the
   // price of half again as many LDS reads, which is what loses on the long, power-limited 8192^3 loops.

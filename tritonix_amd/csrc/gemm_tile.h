@@ -998,13 +998,15 @@ template <int V> struct IntTag { static constexpr int value = V; };
 // t+2, before whose period nothing reads it.  16-bit types, stride_w == 1, k % BK == 0.
 // AT: A is m-contiguous (element (m, k) at a + k * stride_ak + m, the layout of `x.t() @ dy`): its slab sits in LDS as
 // BK rows of BM elements exactly like a row-major B slab, and its fragments are read with the transposing reads.
-// OUT32: the result is binary32 and nothing else.  (The tiles up to 128x128 carry both epilogues in one kernel, f32_out_tile;
-// in the 192- and 256-wide ones a second epilogue costs hundreds of spilled registers, so they have kernels of their own.)
+// PAIR: a float32 product.  A K slab of 64 holds the bf16 heads of 32 k (k step 0) and their tails (k step 1), and each
+// slab takes three MFMA steps from these two fragment sets -- head head, tail head, head tail -- where three copies laid
+// along k would read six; the result is binary32.  (Kernels of their own: a second epilogue and loop in one kernel cost
+// the 192- and 256-wide tiles hundreds of spilled registers.)
 // GATHER (with BT): conv2d forward over a packed input (PackGeom): the rows of the k-contiguous B slab are the windows of
 // BN output pixels.  A lane's DMA ops fetch the same 16-byte k chunk of different pixels, so an op's offset is the
 // pixel's, kept in a register, plus the chunk's (filter tap, channels), read once per slab from a table in LDS.  Chunks
 // past the end of k get an offset outside the buffer and arrive as zeros.
-template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false, bool AT = false, bool OUT32 = false>
+template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false, bool AT = false, bool PAIR = false>
 __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   constexpr int ES = C::ES, BM = C::BM, BN = C::BN, BK = C::BK, NW = C::NW, STAGES = C::STAGES;
   constexpr int MI = C::MI, TM = C::TM, TN = C::TN;
@@ -1015,12 +1017,13 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   static_assert(!BT || (FAST && (GATHER || C::B_LOADS % NW == 0)), "the k-contiguous B variant is built with the DMA loader only");
   static_assert(!CONV || (FAST && !PERSIST && !BT && ES == 2 && STAGES == 3 && MI == 16 && (NW * 64) % C::CPR_B == 0),
                 "the conv2d variant: DMA loader, 16-bit types, three ring slots");
+  static_assert(!PAIR || (FAST && !PERSIST && !CONV && !GATHER && C::KSTEPS == 2 && C::MMA_K == 32), "the float32 variant: DMA loader, slabs of 32 heads and 32 tails");
   typedef Mma<T, MI> MMA;
   typedef typename MMA::acc_t acc_t;
   typedef typename T::acc_s acc_s;
   // Several problems in one grid and a bias per row (GemmParams::batch, cv.bias) exist in the tiles up to 128x128:
   // the 256-wide tiles have no register to spare for the extra state (measured: 20 more spilled registers, -0.4 %).
-  constexpr bool MULTI = !PERSIST && !CONV && !GATHER && multi_problem_tile<C>();
+  constexpr bool MULTI = !PERSIST && !CONV && !GATHER && !PAIR && multi_problem_tile<C>();
 
   constexpr int AT_CPR = BM * ES / 16, AT_ROWB = BM * ES;    // AT: chunks and bytes of an A slab row
 
@@ -1092,7 +1095,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   // no multiple of BK, rows that are not 16-byte aligned or an N that ends inside a chunk, the host sets tail_slab
   // and the last slab of the K range (the only one whose chunks can cross the end of a row of A, or the end of the
   // last row of B) is left out of the ring and loaded element by element, zero-filled, after the K loop.
-  const bool tail_here = FAST && !PERSIST && !CONV && !GATHER && p.tail_slab != 0 && kt1 == kt_total && kt1 > kt0;
+  const bool tail_here = FAST && !PERSIST && !CONV && !GATHER && !PAIR && p.tail_slab != 0 && kt1 == kt_total && kt1 > kt0;
   const int KT = kt1 > kt0 ? kt1 - kt0 - (tail_here ? 1 : 0) : 0;          // slabs of this workgroup in the ring (per tile)
 
   // ---- the tile the loader works on: origin, DMA bases and per-lane byte offsets.
@@ -1681,12 +1684,15 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
       fa[set][i] = *TNX_LDS(i32x4, sa + a_koff[ks] + i * MI * C::ROWB_A);
     }
   };
+  auto mma_at = [&](int set_a, int set_b, int i, int j) __attribute__((always_inline)) {
+    i32x4 b4 = BT ? fbq[set_b][j] : i32x4{fb[set_b][j][0].x, fb[set_b][j][0].y, fb[set_b][j][1].x, fb[set_b][j][1].y};
+    i32x4 a4 = AT ? i32x4{fat[set_a][i][0].x, fat[set_a][i][0].y, fat[set_a][i][1].x, fat[set_a][i][1].y} : fa[set_a][i];
+    acc[i][j] = MMA::run(b4, a4, acc[i][j]);   // rows = n, cols = m: the tile comes out transposed
+  };
   auto mma_one = [&](int set, int idx) __attribute__((always_inline)) {
     int i = idx / TN, j = idx % TN;
     if (i & 1) j = TN - 1 - j;   // serpentine walk of the wave's MFMA tiles: one operand changes per instruction, never both
-    i32x4 b4 = BT ? fbq[set][j] : i32x4{fb[set][j][0].x, fb[set][j][0].y, fb[set][j][1].x, fb[set][j][1].y};
-    i32x4 a4 = AT ? i32x4{fat[set][i][0].x, fat[set][i][0].y, fat[set][i][1].x, fat[set][i][1].y} : fa[set][i];
-    acc[i][j] = MMA::run(b4, a4, acc[i][j]);   // rows = n, cols = m: the tile comes out transposed
+    mma_at(set, set, i, j);
   };
 
   // ---- pipeline ----------------------------------------------------------
@@ -1703,7 +1709,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   // first k step of the period instead.  The K loop is cut in three (refills
   // to issue / ring draining / final step) so the accumulators flow through
   // straight-line code.
-  constexpr int PERIOD = C::KSTEPS * NMMA;                       // MFMA slots per period
+  constexpr int PERIOD = (PAIR ? 3 : C::KSTEPS) * NMMA;            // MFMA slots per period
   // slots the refill is spread over.  Two-slab rings: the refill is due at the next barrier, so it
   // is front-loaded: over the first half of the period with one wave per SIMD (measured on 8192^3,
   // bf16 256x256x64: a quarter of the period 477, three eighths 853, half 1430, three quarters
@@ -1754,7 +1760,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
       int rd = 0;
 #pragma unroll
       for (int x = 0; x < NMMA; ++x)
-        slot_body((ks + P) & 1, x, (ks + 1 + P) & 1, rd, sa, sb, ks + 1, WITH_DMA, NMMA + ks * NMMA + x, dst);
+        slot_body((ks + P) & 1, x, (ks + 1 + P) & 1, rd, sa, sb, ks + 1, WITH_DMA, (PAIR ? 2 : 1) * NMMA + ks * NMMA + x, dst);
     }
   };
   // last k step of the slab whose fragments sit in set LAST; prefetches step 0 of the slab at (sa1, sb1)
@@ -1779,6 +1785,50 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   typedef BoolTag<true> Yes;
   typedef BoolTag<false> No;
   typedef IntTag<0> Par0;
+  // PAIR: what takes the place of the last k step.  Heads are in set 0, already multiplied with each other; the tails
+  // of the same 32 k have arrived in set 1.  First A's tails with B's heads column by column, then A's heads with B's
+  // tails row by row: so set 0 falls free one fragment after another, B's first, and the next slab's heads are read
+  // into it behind the MFMAs without a third set of registers (which the 256-wide tiles do not have).
+  auto cross_step = [&](uint32_t sa1, uint32_t sb1, auto with_reads, auto with_dma, uint32_t dst) __attribute__((always_inline)) {
+    constexpr bool READS = decltype(with_reads)::value, WITH_DMA = decltype(with_dma)::value;
+    constexpr int RB = BT ? 1 : 2, RA = AT ? 2 : 1;
+    auto read_b = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < RB; ++h) read_one(0, j * RB + h, sa1, sb1, 0);
+    };
+    auto read_a = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < RA; ++h) read_one(0, NBREAD + i * RA + h, sa1, sb1, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < 2 * NMMA; ++s) {
+      if (s < NMMA) {
+        const int j = s / TM, i = s % TM;
+        mma_at(1, 0, (j & 1) ? TM - 1 - i : i, j);
+      } else {
+        const int i = (s - NMMA) / TN, j = (s - NMMA) % TN;
+        mma_at(0, 1, i, (i & 1) ? TN - 1 - j : j);
+      }
+      int lo = 0, hi = 0;
+      if (WITH_DMA && s < SPAN) { lo = s * C::LPW / SPAN; hi = (s + 1) * C::LPW / SPAN; }
+      const bool rb = READS && s >= TM && s <= NMMA && s % TM == 0, ra = READS && s > NMMA && (s - NMMA) % TN == 0;
+      const bool paired = hi - lo == 1 && (rb || ra);
+      if (paired) dma_target(lo, dst);
+      if (rb) read_b(s / TM - 1);
+      if (ra) read_a((s - NMMA) / TN - 1);
+      if (paired) dma_go(lo);
+      else
+#pragma unroll
+        for (int q = lo; q < hi; ++q) dma_op(q, dst);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (READS) read_a(TM - 1);
+  };
+  // what follows a barrier: the end of the slab whose fragments are in registers
+  auto end_slab = [&](uint32_t sa1, uint32_t sb1, auto with_dma, uint32_t dst, auto par, auto swap) __attribute__((always_inline)) {
+    if constexpr (PAIR) cross_step(sa1, sb1, Yes{}, with_dma, dst);
+    else last_step(sa1, sb1, with_dma, dst, par, swap);
+  };
 
   // first STAGES slabs of the tile the loader stands on
   auto issue_prologue = [&]() __attribute__((always_inline)) {
@@ -1876,7 +1926,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
         conv_period_begin();
         const uint32_t dst = lds0 + (uint32_t)(j % STAGES) * C::STAGE_BYTES;
         const uint32_t sa1 = lds0 + (uint32_t)((j + 1) % STAGES) * C::STAGE_BYTES, sb1 = sa1 + C::A_BYTES;
-        last_step(sa1, sb1, Yes{}, dst, IntTag<P>{}, No{});
+        end_slab(sa1, sb1, Yes{}, dst, IntTag<P>{}, No{});
         inner_steps(sa1, sb1, Yes{}, dst, IntTag<(C::KSTEPS & 1) ? (P ^ 1) : 0>{});
         dma_advance();
       };
@@ -1903,7 +1953,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     const uint32_t dst = stage_of(t);
     const uint32_t sa1 = stage_of(t + 1), sb1 = sa1 + C::A_BYTES;
     if constexpr (FAST) {
-      last_step(sa1, sb1, Yes{}, dst, Par0{}, Yes{});
+      end_slab(sa1, sb1, Yes{}, dst, Par0{}, Yes{});
       inner_steps(sa1, sb1, Yes{}, dst, Par0{});
       dma_advance();
     } else {
@@ -1911,7 +1961,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
       // writes have to be in LDS before the next barrier lets anyone read them
       i32x4 ra[GEN_NA], rb[GEN_NB];
       gen_fetch(kt0 + t + STAGES, tid, ra, rb);
-      last_step(sa1, sb1, No{}, 0u, Par0{}, Yes{});
+      end_slab(sa1, sb1, No{}, 0u, Par0{}, Yes{});
       inner_steps(sa1, sb1, No{}, 0u, Par0{});
       gen_store(dst, tid, ra, rb);
       __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
@@ -1924,13 +1974,17 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     __builtin_amdgcn_sched_barrier(0);
     conv_fixup();      // CONV: the last slab that was issued has landed; nothing reads it before the next barrier
     const uint32_t sa1 = stage_of(t + 1), sb1 = sa1 + C::A_BYTES;
-    last_step(sa1, sb1, No{}, 0u, Par0{}, Yes{});
+    end_slab(sa1, sb1, No{}, 0u, Par0{}, Yes{});
     inner_steps(sa1, sb1, No{}, 0u, Par0{});
   }
   // (3) last k step of the final slab
   if (KT > 0) {
+    if constexpr (PAIR) {
+      cross_step(0u, 0u, No{}, No{}, 0u);
+    } else {
 #pragma unroll
-    for (int x = 0; x < NMMA; ++x) mma_one(LAST, x);
+      for (int x = 0; x < NMMA; ++x) mma_one(LAST, x);
+    }
   }
   };
 
@@ -2031,7 +2085,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     }
     if (PINGPONG_TILE && KT >= 2 && (KT & 1) == 0) pingpong_loop();
     else k_loop();
-    if constexpr (FAST && !CONV && !GATHER) {
+    if constexpr (FAST && !CONV && !GATHER && !PAIR) {
       if (tail_here) {
         // the left-out slab: every wave is done with the ring, slot 0 takes it, one slab of MFMAs follows
         __syncthreads();
@@ -2107,7 +2161,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
                                                 p.c_row_ok, p.epilogue);
       }
     };
-    if constexpr (OUT32) {
+    if constexpr (PAIR) {
       finish(TypeTag<OutF32>{});
       return;
     }

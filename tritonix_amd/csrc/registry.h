@@ -20,7 +20,7 @@ struct KernelEntry {
   launch_fn fast_bt;  // DMA loader for k-contiguous B (stride_bk == 1, the `x @ w.t()` layout); may be null
   launch_fn conv;     // conv2d forward on the DMA loader (GemmParams::cv); may be null
   launch_fn fast_at;  // DMA loader for m-contiguous A (stride_am == 1, the `x.t() @ dy` layout), row-major B; may be null
-  launch_fn out32[3];  // fast, fast_bt, fast_at with a binary32 result, of the tiles beyond 128x128; may be null
+  launch_fn pair[3];  // float32 products on head and tail slabs (gemm_tile_kernel<..., PAIR>): row-major B, k-contiguous B, m-contiguous A; may be null
 };
 
 // records the hipError_t behind a TNX_E_HIP for tnx_last_hip_error() (per thread)
@@ -35,13 +35,15 @@ struct GemmBatch {
   const void* bias;
   int bias_dtype;
 };
-// padded: the rows of B (and of an m-contiguous A) are followed by readable memory up to a whole 16-byte chunk, so an N
-// (M) that ends inside a chunk still takes the aligned loader
-int gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, bool padded = false);
+// What the operands of a launch are.  PADDED: the rows of B (and of an m-contiguous A) are followed by readable memory up
+// to a whole 16-byte chunk, so an N (M) that ends inside a chunk still takes the aligned loader.  PAIR: padded, and k
+// holds the heads and tails of a float32 product in blocks of 32 (KernelEntry::pair).
+enum GemmForm { GEMM_PLAIN = 0, GEMM_PADDED = 1, GEMM_PAIR = 2 };
+int gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, GemmForm form = GEMM_PLAIN);
 // the status gemm_launch would return for these arguments, the workspace included, without launching
-int gemm_check(const tnx_gemm_args* a, bool padded);
-// whether the tile of `a` has the k-contiguous-B and m-contiguous-A loaders
-void gemm_tile_layouts(const tnx_gemm_args* a, bool* bt, bool* at);
+int gemm_check(const tnx_gemm_args* a, GemmForm form);
+// whether the tile of `a` takes head and tail slabs, and whether it has the k-contiguous-B and m-contiguous-A loaders
+void gemm_tile_layouts(const tnx_gemm_args* a, bool* pair, bool* bt, bool* at);
 // waves and stages of a built tile with these dimensions that gemm_launch takes with a GemmBatch (eight waves and
 // two ring slots first); false: none built
 bool gemm_tile_for(int dtype, int bm, int bn, int bk, int* num_warps, int* num_stages);
@@ -62,10 +64,10 @@ struct KernelGroup {
 };
 
 template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false,
-          bool AT = false, bool OUT32 = false>
+          bool AT = false, bool PAIR = false>
 hipError_t launch_tile(const GemmParams& p, unsigned grid, hipStream_t stream) {
   static_assert(GATHER ? C::VALID_GATHER : C::VALID, "tile configuration is not buildable");
-  hipLaunchKernelGGL((gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV, GATHER, AT, OUT32>), dim3(grid), dim3(C::THREADS), 0, stream, p);
+  hipLaunchKernelGGL((gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV, GATHER, AT, PAIR>), dim3(grid), dim3(C::THREADS), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -126,25 +128,27 @@ template <class C> constexpr bool at_ok() {
           (C::BM == 64 && C::BN == 64 && C::NW == 4 && C::STAGES == 4) || (C::BM == 192 && C::BN == 192 && C::NW == 8 && C::STAGES == 3) ||
           ((C::BM == 192 || C::BN == 192) && C::BM != C::BN && C::NW == 8 && C::STAGES == 2));
 }
-template <class T, class C, bool OK = at_ok<C>()> struct AtLaunch {
+template <class T, class C, bool PAIR = false, bool OK = at_ok<C>()> struct AtLaunch {
   static constexpr launch_fn fn = nullptr;
 };
-template <class T, class C> struct AtLaunch<T, C, true> {
-  static constexpr launch_fn fn = &launch_tile<T, C, true, false, false, false, false, true>;
+template <class T, class C, bool PAIR> struct AtLaunch<T, C, PAIR, true> {
+  static constexpr launch_fn fn = &launch_tile<T, C, true, false, false, false, false, true, PAIR>;
 };
 
-// Binary32 results beyond 128x128 (float32 products, which run on bf16 terms): the eight-wave tiles of 192 and 256.
-template <class T, class C> constexpr bool out32_ok() {
-  return T::ID == DT_BF16 && C::NW == 8 && C::BK * C::ES == 128 && (C::BM == 256 || C::BM == 192) && (C::BN == 256 || C::BN == 192) &&
-         C::STAGES == (C::BM == 192 && C::BN == 192 ? 3 : 2);
+// The float32 variant exists for the tiles the built-in choice proposes for float32 problems.
+template <class T, class C> constexpr bool pair_ok() {
+  return T::ID == DT_BF16 && C::BK == 64 &&
+         ((C::NW == 8 && (C::BM == 256 || C::BM == 192) && (C::BN == 256 || C::BN == 192) && C::STAGES == (C::BM == 192 && C::BN == 192 ? 3 : 2)) ||
+          (C::BM == 128 && C::BN == 128 && C::STAGES == 3) || (C::NW == 8 && C::BM == 64 && C::BN == 128 && C::STAGES == 3) ||
+          (C::NW == 4 && C::BM == 64 && C::BN == 64 && C::STAGES == 4));
 }
-template <class T, class C, bool OK = out32_ok<T, C>()> struct Out32Launch {
+template <class T, class C, bool OK = pair_ok<T, C>()> struct PairLaunch {
   static constexpr launch_fn nn = nullptr, bt = nullptr, at = nullptr;
 };
-template <class T, class C> struct Out32Launch<T, C, true> {
+template <class T, class C> struct PairLaunch<T, C, true> {
   static constexpr launch_fn nn = &launch_tile<T, C, true, false, false, false, false, false, true>;
   static constexpr launch_fn bt = &launch_tile<T, C, true, false, true, false, false, false, true>;
-  static constexpr launch_fn at = &launch_tile<T, C, true, false, false, false, false, true, true>;
+  static constexpr launch_fn at = AtLaunch<T, C, true>::fn;
 };
 
 // The element-wise loader is built only for the tiles that ask for it (a conditional expression would instantiate
@@ -165,7 +169,7 @@ template <class T, class C> struct GenericLaunch<T, C, true> {
    GenericLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>, GENERIC>::fn,                                        \
    PersistLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::fn, BtLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::fn,     \
    ConvLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::fn, AtLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::fn,         \
-   {Out32Launch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::nn, Out32Launch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::bt,           \
-    Out32Launch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::at}}
+   {PairLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::nn, PairLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::bt,           \
+    PairLaunch<TAG, TileCfg<TAG, BM, BN, BK, NW, ST>>::at}}
 
 }  // namespace tnx
