@@ -461,14 +461,27 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
     at = layout == 3;         // ... except the 64-row int8 tiles, whose rows are too short to read an m-contiguous A from
   }
   if (a->m <= 64 && dma_ok && !(at && es == 1)) {
-    // skinny: B is streamed once; K is split until every CU owns one workgroup (measured on the
-    // M=16, N=4096, K=14336 shape: 8 waves, 3 stages, 256 workgroups stream at the HBM read limit)
-    a->block_m = 64; a->block_n = 128; a->num_stages = 3; a->num_warps = 8;
-    int64_t tiles = (a->n + a->block_n - 1) / a->block_n;
-    int64_t kt = (a->k + a->block_k - 1) / a->block_k;
+    // Skinny: B is streamed once, by at most one workgroup per CU, K cut further while that shortens the launch.
+    // 16-bit types: 64 columns per workgroup keep the chip busy with half the K cuts that 128 need, and the hand-over of
+    // the slices is a fixed cost per cut (16 x 4096 x 4096: 64 columns / 4 cuts 11.2 us, 128 / 8 12.7; 16 x 2048 x 4096
+    // 8.7 against 11.8; 64 x 2048 x 4096 11.3 against 17.0).  With a row-major B the wider rows stream better once
+    // there are enough bytes to stream, or enough columns for one round without a cut (64 x 8192 x 14336: 47.4 us with
+    // 128 columns, 52.9 with 64; 16 x 28672 x 4096: 38.5 against 44.1); rows of a k-contiguous B are k runs either way.
+    // Cutting s -> 2s saves kt / 2s slabs of the loop and costs s more slices: it pays while kt >= 1.75 s^2 (fitted to
+    // 51 shapes of bf16 and int8, n 1024 to 28672, k 1024 to 14336; kt / s >= 4 and up to 512 workgroups before: 1.14x in
+    // the mean).  Up to 32 rows a 32-row tile (not built for an m-contiguous A or for heads and tails), except where 128
+    // columns are cut: 16 x 4096 x 14336 24.1 us on 64 rows and eight waves, 24.7 on 32 and four.
+    const int64_t kt = (a->k + bk - 1) / bk;
+    const bool bt = a->stride_bk == 1 && a->stride_bn != 1;
+    const bool narrow = es == 2 && (bt || ((a->n + 63) / 64 <= cus && a->n * a->k <= 40000000));
+    a->block_n = narrow ? 64 : 128;
+    const int64_t tiles = (a->n + a->block_n - 1) / a->block_n;
     int s = 1;
-    while (tiles * s < cus && s * 2 <= 16 && kt / (s * 2) >= 4) s *= 2;
+    while (tiles * s * 2 <= cus && s < 16 && 4 * kt >= 7 * s * s) s *= 2;
     a->split_k = s;
+    a->block_m = es == 2 && a->m <= 32 && !at && !large_f32 && (narrow || s == 1) ? 32 : 64;
+    a->num_stages = narrow ? 4 : 3;
+    a->num_warps = narrow || a->block_m == 32 ? 4 : 8;
     return TNX_OK;
   }
   // operands the DMA loader cannot take (not row-major with unit inner strides, int8 rows that are not 16-byte
@@ -538,6 +551,12 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
   // 55.2 -> 54.1 us, 4096^3 333 -> 327 us; not for an m-contiguous A, whose transposing reads double the count: 57 us with
   // eight, above 71 with four.)
   if (bi == 2 && large_f32 && !at) a->num_warps = 4;
+  // A k-contiguous B on 64x128 tiles, one workgroup per CU: a fourth slot (the LDS holds six; five and six measured no
+  // better) covers the longer way of 128-byte runs.  512 x 4096 x 4096 24.5 -> 21.5 us, 1024 x 2048 x 4096 22.8 -> 21.3; with
+  // two workgroups on a CU three slots stay ahead (2048^3: 21.3 against 23.2 us), and with a row-major B they tie.
+  if (es == 2 && bi == 3 && !large_f32 && a->stride_bk == 1 && a->stride_bn != 1 &&
+      ((a->m + 63) / 64) * ((a->n + 127) / 128) * bs <= cus)
+    a->num_stages = 4;
   // 16-bit problems with a short K loop (at most 64 slabs per tile) spend a visible share of every tile outside
   // it; two waves per SIMD cover that better than one (measured on 4096 x 28672 x 4096, gated: +2.4 %), at the
   // price of half again as many LDS reads, which is what loses on the long, power-limited 8192^3 loops.
