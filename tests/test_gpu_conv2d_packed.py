@@ -29,6 +29,13 @@ CASES = {
     "one_output": (1, 64, 5, 5, 33, 5, 5, (1, 1), (0, 0), (1, 1)),
     "long_k_padded_table": (1, 468, 6, 6, 40, 7, 7, (1, 1), (3, 3), (1, 1)),   # offset table per slab only after rounding c_in up
     "cut_k": (1, 512, 7, 7, 512, 3, 3, (1, 1), (1, 1), (1, 1)),               # few tiles, long k: K slices meet in the workspace
+    # float32: blocks of 32 channels, whole and padded, on either side of where three terms are taken instead
+    "one_block": (2, 32, 9, 10, 40, 3, 3, (1, 1), (1, 1), (1, 1)),
+    "block_padded": (1, 25, 12, 9, 72, 3, 3, (2, 1), (1, 1), (1, 1)),
+    "three_terms_33": (2, 33, 9, 9, 24, 3, 3, (1, 1), (1, 1), (1, 1)),
+    "two_blocks_padded": (2, 51, 8, 11, 130, 2, 3, (1, 2), (1, 0), (2, 1)),
+    "blocks_1x1_stride_2": (3, 265, 15, 17, 64, 1, 1, (2, 2), (0, 0), (1, 1)),
+    "blocks_cut_k": (1, 512, 7, 9, 300, 3, 3, (1, 1), (1, 1), (1, 1)),
     "many_tiles": (16, 64, 57, 55, 256, 3, 3, (1, 1), (1, 1), (1, 1)),
 }
 
@@ -80,3 +87,23 @@ def test_a_non_finite_input_reaches_only_its_own_window(device, monkeypatch):
     hit = torch.zeros(2, 16, 9, 9, dtype=torch.bool)
     hit[1, :, 3:6, 3:6] = True
     assert bool(torch.isposinf(out[hit]).all()) and bool(torch.isfinite(out[~hit]).all())
+
+
+@pytest.mark.parametrize("c_in", [32, 33, 64])
+def test_non_finite_float32_elements(c_in, device, monkeypatch):
+    """Infinities and NaN of either operand fall where the float32 convolution has them, against partners whose bf16 tail is
+    zero or of the other sign, zeros, and each other."""
+    monkeypatch.setenv("TRITONIX_AUTOTUNE", "0")
+    g = torch.Generator().manual_seed(c_in)
+    inf, nan = float("inf"), float("nan")
+    x, wt = torch.randn(2, c_in, 8, 9, generator=g), torch.randn(20, c_in, 3, 3, generator=g)
+    x[:, :16], wt[:, :16] = x[:, :16].bfloat16().float(), wt[:, :16].bfloat16().float()
+    x[0, 3, 2, 2], x[0, c_in - 1, 6, 6], x[1, 5, 4, 4], x[1, 9, 0, 8] = inf, -inf, nan, inf
+    wt[4, 9, 1, 1], wt[7, 3, 0, 2], wt[11, c_in - 1, 2, 2], wt[13, 2, 1, 0] = inf, 0.0, -inf, nan
+    out = conv2d_forward(x.to(device), wt.to(device), None, (1, 1), (1, 1)).cpu()
+    # the float64 convolution pads with zeros that meet wt's infinities as well: so does every implementation
+    ref = torch.nn.functional.conv2d(x.double(), wt.double(), None, 1, 1)
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.isnan(out), torch.isnan(ref)) and torch.equal(torch.isposinf(out), torch.isposinf(ref))
+    assert torch.equal(torch.isneginf(out), torch.isneginf(ref))
+    assert ((out[fin] - ref[fin]).abs().max() / ref[fin].abs().max()).item() < 1e-4

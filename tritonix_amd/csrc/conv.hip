@@ -354,6 +354,8 @@ static void fill_dma(const tnx_conv2d_args* a, const Resolved& r, GemmParams* p,
 // the start and end of its tiles) on wide layers, by the two launches on small ones.  Measured against the kernels that
 // gather taps themselves, whole call, bf16/f16, 3x3: 256 channels of 56x56, batch 32: 155 -> 114 us (pass 18, GEMM 96:
 // 1230 TFLOP/s); 128 channels of 56x56, stride 2: 42.8 -> 22.8; 512 of 7x7, batch 8: 137 -> 23; float32, 256 of 14x14: 242 -> 23.
+// float32 with heads and tails in blocks of 32 channels instead of three terms (the GEMM reads a third less): 256 channels of
+// 56x56, batch 32: 319 -> 301 us; 512 of 28x28: 285 -> 261; 128 of 56x56, stride 2: 53 -> 47; 512 of 7x7, batch 8: 39 -> 30.
 // ---------------------------------------------------------------------------
 struct PackedPlan {
   const GatherEntry* e;
@@ -383,6 +385,8 @@ static const GatherCost* gather_cost(const GatherEntry& e) {
   return nullptr;
 }
 
+static constexpr double PAIR_SLAB = 1.3;
+
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
 static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p) {
@@ -409,8 +413,13 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p) {
   const int sh = a->filter_h == 1 ? 1 : a->stride_h, sw = a->filter_w == 1 ? 1 : a->stride_w;
   p->rows = (h_out - 1) * sh + (a->filter_h - 1) * a->dil_h + 1;
   p->cols = (w_out - 1) * sw + (a->filter_w - 1) * a->dil_w + 1;
-  p->terms = f32 ? 3 : 1;
   p->cp8 = (a->c_in + 7) / 8;
+  // float32: head and tail in blocks of 32 channels, one K slab each, or three terms of cp8 groups, 3/8 cp8 slabs.  A slab
+  // of heads and tails takes three MFMA steps for two and measures about PAIR_SLAB of an ordinary one.  (25 to 32,
+  // 49 to 64, 81 to 96, 105 to 128 and from 137 channels on.)
+  const int blocks32 = (p->cp8 + 3) / 4;
+  p->terms = !f32 ? 1 : PAIR_SLAB * blocks32 <= 0.375 * p->cp8 ? 2 : 3;
+  if (p->terms == 2) p->cp8 = blocks32 * 4;
   const int64_t taps = (int64_t)a->filter_h * a->filter_w * p->terms;
   // the kernel's offset table has one entry per k chunk (it reads one slab past the end), or one per slab where a filter
   // tap's channels are whole slabs: a long k is padded to that
@@ -446,7 +455,7 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p) {
         const int64_t slots = 256 * cost->per_cu, full = tiles * s / slots, rem = tiles * s % slots;
         double rounds = (double)full;
         if (rem) rounds += rem > 256 * (cost->per_cu - 1) ? 0.9 : 0.9 * (0.5 + 0.5 * (double)rem / (double)slots);
-        double c = rounds * (cost->fixed + cost->slab * (double)((kt + s - 1) / s));
+        double c = rounds * (cost->fixed + cost->slab * (p->terms == 2 ? PAIR_SLAB : 1.0) * (double)((kt + s - 1) / s));
         if (s > 1) c += 2.2 + 3.0 * s * area + 1.8 * area;
         if (c < best) { best = c; p->e = &e; p->split = s; }
       }
@@ -505,8 +514,9 @@ static int packed_forward(const tnx_conv2d_args* a, const PackedPlan& pl) {
   k.div_chunks = make_fastdiv((uint32_t)k.chunks_pad);
   const unsigned blocks = k.w_blocks + (unsigned)((waves + 3) / 4);
   hipStream_t stream = (hipStream_t)a->stream;
-  if (f32) hipLaunchKernelGGL((conv_pack_kernel<float>), dim3(blocks), dim3(256), 0, stream, k);
-  else hipLaunchKernelGGL((conv_pack_kernel<uint16_t>), dim3(blocks), dim3(256), 0, stream, k);
+  if (!f32) hipLaunchKernelGGL((conv_pack_kernel<uint16_t, 1>), dim3(blocks), dim3(256), 0, stream, k);
+  else if (pl.terms == 2) hipLaunchKernelGGL((conv_pack_kernel<float, 2>), dim3(blocks), dim3(256), 0, stream, k);
+  else hipLaunchKernelGGL((conv_pack_kernel<float, 3>), dim3(blocks), dim3(256), 0, stream, k);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) { note_hip_error((int)err); return TNX_E_HIP; }
 
@@ -541,7 +551,7 @@ static int packed_forward(const tnx_conv2d_args* a, const PackedPlan& pl) {
   q.tap_row_bytes = (uint32_t)a->dil_h * (uint32_t)pl.cols * px;
   q.tap_col_bytes = (uint32_t)a->dil_w * px;
   q.x_bytes = (uint32_t)pl.x_bytes;
-  err = e.launch(p, (unsigned)(tiles_m * tiles_n * pl.split), stream);
+  err = (pl.terms == 2 ? e.pair : e.launch)(p, (unsigned)(tiles_m * tiles_n * pl.split), stream);
   if (err != hipSuccess) { note_hip_error((int)err); return TNX_E_HIP; }
   return TNX_OK;
 }

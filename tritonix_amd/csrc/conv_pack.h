@@ -3,9 +3,11 @@
 //   input  [batch][c_in][h][w]        ->  [batch][rows][cols][terms * cp]   zero padding written out
 //   weight [c_out][c_in][fh][fw]      ->  [c_out][fh * fw][terms * cp], rows zero-filled to whole K slabs
 //
-// with cp = c_in rounded up to 8.  16-bit operands have one term; float32 operands are cut into bf16 terms -- input
-// [hi | hi' | lo], weight [hi | lo | hi'], hi' being hi without its infinities and NaNs -- so that the same kernel
-// computes hi hi + hi lo + lo hi (the split of tnx_split_f32).
+// with cp = c_in rounded up to 8.  16-bit operands have one term; float32 operands are cut into bf16 terms for
+// hi hi + hi lo + lo hi: as a head and a tail in blocks of 32 channels (two terms; the PAIR form of the GEMM kernel, a
+// non-finite element having +-1 for its head and itself for its tail), or, where padding the channels to 32 costs more
+// than the third copy, as three terms -- input [hi | hi' | lo], weight [hi | lo | hi'], hi' being hi without its
+// infinities and NaNs (the split of tnx_split_f32).
 //
 // What it buys: the im2col loaders gather the same input element once per filter tap with address arithmetic and edge
 // masks in the MFMA stream; after this pass a tap is a constant added to an address.  One launch does both operands.
@@ -42,8 +44,6 @@ struct PackParams {
   FastDiv div_cgb, div_row, div_wchunks, div_cpt, div_cp8, div_chunks, div_taps;
 };
 
-template <class E> struct PackTerms { static constexpr int N = sizeof(E) == 4 ? 3 : 1; };
-
 // one element as its bf16 (or 16-bit) terms; side 0: input order, side 1: weight order
 template <int SIDE> __device__ __forceinline__ void pack_terms(uint16_t v, uint16_t (&t)[1]) { t[0] = v; }
 template <int SIDE> __device__ __forceinline__ void pack_terms(float v, uint16_t (&t)[3]) {
@@ -55,10 +55,21 @@ template <int SIDE> __device__ __forceinline__ void pack_terms(float v, uint16_t
   t[SIDE == 0 ? 1 : 2] = fin ? h : (uint16_t)0;
   t[SIDE == 0 ? 2 : 1] = fin ? l : (uint16_t)0;
 }
+template <int SIDE> __device__ __forceinline__ void pack_terms(float v, uint16_t (&t)[2]) {
+  const __bf16 hi = (__bf16)v;
+  const float rest = v - (float)hi;
+  const bool fin = __builtin_isfinite(rest) && __builtin_isfinite((float)hi);
+  const __bf16 one = __builtin_signbit(v) ? (__bf16)-1.0f : (__bf16)1.0f;
+  t[0] = __builtin_bit_cast(uint16_t, fin ? hi : one);
+  t[1] = __builtin_bit_cast(uint16_t, fin ? (__bf16)rest : hi);
+}
+// chunk of term z of channel group cg among a pixel's (or filter tap's) chunks
+template <int NT> __device__ __forceinline__ int term_chunk(int z, int cg, int cp8) {
+  return NT == 2 ? (cg >> 2) * 8 + z * 4 + (cg & 3) : z * cp8 + cg;
+}
 
-template <class E>
+template <class E, int NT>
 __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
-  constexpr int NT = PackTerms<E>::N;
   const int tid = threadIdx.x;
   if (blockIdx.x < p.w_blocks) {
     const int item = blockIdx.x * 256 + tid;
@@ -78,7 +89,8 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
         tap = (int)fd_div((uint32_t)k8, p.div_cpt);
         r = k8 - tap * (p.cp8 * NT);
       }
-      const int term = NT == 1 ? 0 : (int)fd_div((uint32_t)r, p.div_cp8), cg = r - term * p.cp8;
+      const int term = NT == 1 ? 0 : NT == 2 ? (r >> 2) & 1 : (int)fd_div((uint32_t)r, p.div_cp8);
+      const int cg = NT == 2 ? (r >> 3) * 4 + (r & 3) : r - term * p.cp8;
       const E* src = (const E*)p.w + ((int64_t)co * p.c_in + cg * 8) * p.taps + tap;
       uint16_t o[8];
 #pragma unroll
@@ -86,6 +98,7 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
         uint16_t t[NT];
         pack_terms<1>(cg * 8 + e < p.c_in ? src[(int64_t)e * p.taps] : (E)0, t);
         o[e] = t[0];
+        if constexpr (NT == 2) o[e] = term == 0 ? t[0] : t[1];
         if constexpr (NT == 3) o[e] = term == 0 ? t[0] : term == 1 ? t[1] : t[2];
       }
       __builtin_memcpy(&v, o, 16);
@@ -147,7 +160,7 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
           if (c < nch && (uint32_t)(w0 + e * p.step_w) < (uint32_t)p.w_in) in[c][e] = src[o0 + c * plane + e * p.step_w];
     }
   }
-  uint8_t* dst = p.xp + (((int64_t)row_all * p.cols + col0) * (p.cp8 * NT) + cg) * 16;
+  uint8_t* dst = p.xp + ((int64_t)row_all * p.cols + col0) * (p.cp8 * NT) * 16;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     if (col0 + e >= p.cols) break;
@@ -163,17 +176,17 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
     for (int z = 0; z < NT; ++z) {
       i32x4 v;
       __builtin_memcpy(&v, o[z], 16);
-      *(i32x4*)(dst + ((int64_t)e * (p.cp8 * NT) + z * p.cp8) * 16) = v;
+      *(i32x4*)(dst + ((int64_t)e * (p.cp8 * NT) + term_chunk<NT>(z, cg, p.cp8)) * 16) = v;
     }
   }
   if (wc == 0)
     for (int col = -p.lead; col < 0; ++col)
 #pragma unroll
-      for (int z = 0; z < NT; ++z) *(i32x4*)(dst + ((int64_t)col * (p.cp8 * NT) + z * p.cp8) * 16) = i32x4{0, 0, 0, 0};
+      for (int z = 0; z < NT; ++z) *(i32x4*)(dst + ((int64_t)col * (p.cp8 * NT) + term_chunk<NT>(z, cg, p.cp8)) * 16) = i32x4{0, 0, 0, 0};
   if (wc == p.wchunks - 1)
     for (int col = 8; col0 + col < p.cols; ++col)
 #pragma unroll
-      for (int z = 0; z < NT; ++z) *(i32x4*)(dst + ((int64_t)col * (p.cp8 * NT) + z * p.cp8) * 16) = i32x4{0, 0, 0, 0};
+      for (int z = 0; z < NT; ++z) *(i32x4*)(dst + ((int64_t)col * (p.cp8 * NT) + term_chunk<NT>(z, cg, p.cp8)) * 16) = i32x4{0, 0, 0, 0};
 }
 
 }  // namespace tnx

@@ -1017,7 +1017,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   static_assert(!BT || (FAST && (GATHER || C::B_LOADS % NW == 0)), "the k-contiguous B variant is built with the DMA loader only");
   static_assert(!CONV || (FAST && !PERSIST && !BT && ES == 2 && STAGES == 3 && MI == 16 && (NW * 64) % C::CPR_B == 0),
                 "the conv2d variant: DMA loader, 16-bit types, three ring slots");
-  static_assert(!PAIR || (FAST && !PERSIST && !CONV && !GATHER && C::KSTEPS == 2 && C::MMA_K == 32), "the float32 variant: DMA loader, slabs of 32 heads and 32 tails");
+  static_assert(!PAIR || (FAST && !PERSIST && !CONV && C::KSTEPS == 2 && C::MMA_K == 32), "the float32 variant: DMA loader, slabs of 32 heads and 32 tails");
   typedef Mma<T, MI> MMA;
   typedef typename MMA::acc_t acc_t;
   typedef typename T::acc_s acc_s;
@@ -2129,6 +2129,10 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
           epilogue_store_conv<T, C, OT>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
         }
       };
+      if constexpr (PAIR) {
+        finish_conv(TypeTag<OutF32>{});
+        return;
+      }
       if (p.out_dtype == DT_F32) finish_conv(TypeTag<OutF32>{});
       else finish_conv(TypeTag<O>{});
       return;

@@ -52,6 +52,7 @@ bool gemm_tile_for(int dtype, int bm, int bn, int bk, int* num_warps, int* num_s
 struct GatherEntry {
   int dtype, bm, bn, nw, stages;
   launch_fn launch;
+  launch_fn pair;     // float32 operands as head and tail slabs; bf16 entries only
 };
 struct GatherGroup {
   GatherEntry* entries;
@@ -160,8 +161,16 @@ template <class T, class C> struct GenericLaunch<T, C, true> {
   static constexpr launch_fn fn = &launch_tile<T, C, false>;
 };
 
-#define TNX_GATHER_ENTRY(TAG, BM, BN, NW, ST) \
-  {TAG::ID, BM, BN, NW, ST, &launch_tile<TAG, TileCfg<TAG, BM, BN, 64, NW, ST>, true, false, true, false, true>}
+template <class T, class C, bool OK = T::ID == DT_BF16> struct GatherPairLaunch {
+  static constexpr launch_fn fn = nullptr;
+};
+template <class T, class C> struct GatherPairLaunch<T, C, true> {
+  static constexpr launch_fn fn = &launch_tile<T, C, true, false, true, false, true, false, true>;
+};
+
+#define TNX_GATHER_ENTRY(TAG, BM, BN, NW, ST)                                                                      \
+  {TAG::ID, BM, BN, NW, ST, &launch_tile<TAG, TileCfg<TAG, BM, BN, 64, NW, ST>, true, false, true, false, true>,  \
+   GatherPairLaunch<TAG, TileCfg<TAG, BM, BN, 64, NW, ST>>::fn}
 
 #define TNX_ENTRY(TAG, BM, BN, BK, NW, ST, GENERIC)                                                          \
   {TAG::ID, BM, BN, BK, NW, ST, TileCfg<TAG, BM, BN, BK, NW, ST>::LDS_BYTES,                                 \
