@@ -209,6 +209,12 @@ int tnx_split_f32(const float* src, int64_t rows, int64_t cols, int64_t stride_r
 size_t tnx_gemm_f32_scratch_bytes(const tnx_gemm_args* args);
 int tnx_gemm_f32(const tnx_gemm_args* args, void* scratch, size_t scratch_bytes);
 
+/* How many K slabs (of block_k) at the end of k a launch of `args` loads element by element, no access outside the
+ * operands: 0 where all of them go through the ring of whole 16-byte chunks, 1 where rows, base pointers or sizes are no
+ * whole chunks, all of them on the element-wise loader; -1 if tnx_gemm would refuse the arguments.  For tests and
+ * tooling: pure host arithmetic, of a and b only the alignment counts. */
+int tnx_gemm_tail_slabs(const tnx_gemm_args* args);
+
 /* Number of compiled tile kernels, and a description of the i-th one:
  * "dtype bm bn bk warps stages [generic] [persistent]" as a NUL-terminated string (static storage);
  * "generic": also built with the element-wise loader; "persistent": also built for TNX_SCHED_PERSISTENT. */

@@ -30,7 +30,7 @@ CONV_LOADER_AUTO, CONV_LOADER_REGISTERS, CONV_LOADER_DMA, CONV_LOADER_GEMM = 0, 
 
 EXPORTS = ("tnx_gemm", "tnx_gemm_static_workspace", "tnx_gemm_workspace_bytes", "tnx_gemm_lds_bytes", "tnx_gemm_supported",
            "tnx_gemm_default_config", "tnx_tile_coords", "tnx_split_f32", "tnx_gemm_f32_scratch_bytes",
-           "tnx_gemm_f32", "tnx_kernel_count", "tnx_kernel_name", "tnx_strerror",
+           "tnx_gemm_f32", "tnx_gemm_tail_slabs", "tnx_kernel_count", "tnx_kernel_name", "tnx_strerror",
            "tnx_last_hip_error", "tnx_version", "tnx_conv2d_forward", "tnx_conv2d_workspace_bytes", "tnx_conv2d_supported",
            "tnx_conv2d_output_size",
            "tnx_conv2d_default_config", "tnx_conv2d_kernel_count", "tnx_conv2d_kernel_name")
@@ -104,6 +104,8 @@ def load() -> ctypes.CDLL:
     lib.tnx_gemm_f32_scratch_bytes.restype = ctypes.c_size_t
     lib.tnx_gemm_f32.argtypes = [p, ctypes.c_void_p, ctypes.c_size_t]
     lib.tnx_gemm_f32.restype = ctypes.c_int
+    lib.tnx_gemm_tail_slabs.argtypes = [p]
+    lib.tnx_gemm_tail_slabs.restype = ctypes.c_int
     lib.tnx_kernel_count.argtypes = []
     lib.tnx_kernel_count.restype = ctypes.c_int
     lib.tnx_kernel_name.argtypes = [ctypes.c_int]

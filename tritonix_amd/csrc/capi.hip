@@ -82,25 +82,33 @@ static int check_common(const tnx_gemm_args* a, bool pair) {
   return TNX_OK;
 }
 
-// Which DMA loader the operands can take: 0 = none (element-wise loader only), 1 = row-major B
-// (stride_bn == 1), 2 = k-contiguous B (stride_bk == 1, the layout of x @ w.t()).  Both need row-major A,
-// 16-byte aligned rows and base pointers and k % block_k == 0.
-// 0: element-wise loader; 1: DMA loader, A and B row-major; 2: DMA loader, B k-contiguous; 3: DMA loader, A m-contiguous,
-// B row-major (only in the tiles built for it).
-// *tail (layout 1 only): the operands are row-major but not as the DMA loader likes them best -- K no multiple of
-// block_k, rows or base pointers not 16-byte aligned (the loads take any byte address: probed on the hardware),
-// N ending inside a 16-byte chunk -- so the last K slab, the only one whose chunks can cross the end of a row of A
-// or of the last row of B, is loaded element by element instead (GemmParams::tail_slab).
-static int dma_layout(const tnx_gemm_args* a, bool* tail = nullptr) {
+// Which DMA loader the operands can take.  0: none, the element-wise loader only; 1: A and B row-major; 2: row-major A,
+// k-contiguous B (stride_bk == 1, the layout of x @ w.t()); 3: m-contiguous A (stride_am == 1, x.t() @ dy), row-major B
+// (only in the tiles built for it).  All want 16-byte aligned rows and base pointers, k % block_k == 0 and rows of whole
+// 16-byte chunks.
+// *tail: the operands have such a layout but not as the DMA loader likes it best -- K no multiple of block_k, rows or
+// base pointers not 16-byte aligned (the loads take any byte address: probed on the hardware), N (layout 3: or M) ending
+// inside a 16-byte chunk -- so the last K slab, the only one whose chunks can cross the end of a row of A or of the last
+// row of B, is loaded element by element instead (GemmParams::tail_slab).
+// *narrow: the operands have such a layout, but rows shorter than a chunk and a last slab of few rows let a chunk of the
+// slab before it end past the operand (ring_chunks_inside): the layout is not taken.
+static int dma_layout(const tnx_gemm_args* a, bool* tail = nullptr, bool* narrow = nullptr) {
   const int es = elem_size(a->in_dtype);
   const int vec = 16 / es;
   if (tail) *tail = false;
+  if (narrow) *narrow = false;
+  const int64_t last_rows = a->k > 0 && a->block_k > 0 ? (a->k - 1) % a->block_k + 1 : 0;      // k rows of the last slab
+  const bool b_inside = ring_chunks_inside(last_rows, a->n, a->stride_bk, vec);
   if (a->stride_am == 1 && a->stride_ak != 1 && a->stride_bn == 1 && a->k > 0 && a->stride_ak >= a->m && a->stride_bk >= a->n &&
       (int64_t)a->block_k * a->stride_ak * es + (int64_t)a->block_m * es < (1ll << 32) &&
       (int64_t)a->block_k * a->stride_bk * es + (int64_t)a->block_n * es < (1ll << 32)) {
     const bool aligned = (a->stride_ak * es) % 16 == 0 && (a->stride_bk * es) % 16 == 0 && !((uintptr_t)a->a & 15) && !((uintptr_t)a->b & 15);
     if (aligned && a->k % a->block_k == 0 && a->m % vec == 0 && a->n % vec == 0) return 3;
     if (tail) {
+      if (!b_inside || !ring_chunks_inside(last_rows, a->m, a->stride_ak, vec)) {
+        if (narrow) *narrow = true;
+        return 0;
+      }
       *tail = true;
       return 3;
     }
@@ -114,10 +122,11 @@ static int dma_layout(const tnx_gemm_args* a, bool* tail = nullptr) {
     const bool strict = a_aligned && a->k % a->block_k == 0 && (a->stride_bk * es) % 16 == 0 && a->n % vec == 0 && a->n >= vec;
     if (strict) return 1;
     const bool loose_ok = tail && a->stride_am >= a->k && a->stride_bk >= a->n;
-    if (loose_ok) {
+    if (loose_ok && b_inside) {
       *tail = true;
       return 1;
     }
+    if (loose_ok && narrow) *narrow = true;
   }
   if (a->stride_bk == 1 && a->stride_bn >= 0 && (int64_t)a->block_n * a->stride_bn * es + (int64_t)a->block_k * es < (1ll << 32)) {
     if (a_aligned && a->k % a->block_k == 0 && (a->stride_bn * es) % 16 == 0) return 2;
@@ -149,11 +158,26 @@ extern "C" size_t tnx_gemm_workspace_bytes(const tnx_gemm_args* a) {
   return (size_t)WS_COUNTER_BYTES + (size_t)a->split_k * (size_t)cut_tiles(a) * (size_t)a->block_m * (size_t)a->block_n * 4;
 }
 
+// a tile that is built with the element-wise loader, for this problem's type and rows (null: none built)
+static const KernelEntry* elementwise_tile(const tnx_gemm_args* a) {
+  int ng = 0;
+  const KernelGroup* g = tnx_kernel_groups(&ng);
+  const KernelEntry* best = nullptr;
+  for (int i = 0; i < ng; ++i)
+    for (int j = 0; j < g[i].count; ++j) {
+      const KernelEntry& e = g[i].entries[j];
+      if (e.dtype != a->in_dtype || !e.generic || e.bm * e.bn > 128 * 128) continue;
+      if (!best || (a->m <= 64 ? e.bm < best->bm : e.bm > best->bm)) best = &e;
+    }
+  return best;
+}
+
 static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool* fast, bool inspect_ptrs, bool* bt = nullptr,
-                          bool* tail = nullptr, bool* at = nullptr, GemmForm form = GEMM_PLAIN) {
+                          bool* tail = nullptr, bool* at = nullptr, GemmForm form = GEMM_PLAIN, bool* other_tile = nullptr) {
   if (bt) *bt = false;
   if (at) *at = false;
   if (tail) *tail = false;
+  if (other_tile) *other_tile = false;
   int st = check_common(a, form == GEMM_PAIR);
   if (st != TNX_OK) return st;
   int64_t lds = lds_bytes_of(a);
@@ -179,13 +203,17 @@ static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool*
   tnx_gemm_args tmp = *a;
   if (!inspect_ptrs) { tmp.a = nullptr; tmp.b = nullptr; }
   if (form != GEMM_PLAIN) { tmp.m = (tmp.m + 7) / 8 * 8; tmp.n = (tmp.n + 7) / 8 * 8; }    // 16-bit operands: chunks of 8 elements
-  bool tail_slab = false;
+  bool tail_slab = false, narrow = false;
   // the persistent kernel keeps the strict layout
-  const int layout = dma_layout(&tmp, (a->schedule & TNX_SCHED_PERSISTENT) ? nullptr : &tail_slab);
+  const int layout = dma_layout(&tmp, (a->schedule & TNX_SCHED_PERSISTENT) ? nullptr : &tail_slab, &narrow);
   if (form == GEMM_PAIR && (a->out_dtype != TNX_F32 || layout == 0 || tail_slab || !e->pair[layout - 1])) return TNX_E_UNSUPPORTED;
   bool f = layout == 1 || (layout == 2 && e->fast_bt) || (layout == 3 && e->fast_at);
   if (tail) *tail = f && tail_slab;
-  if (!f && !e->generic) return TNX_E_UNSUPPORTED;
+  if (!f && narrow && !e->generic && (a->stride_ak == 1 || e->fast_at) && elementwise_tile(a)) {
+    if (other_tile) *other_tile = true;             // gemm_launch runs it on that tile
+  } else if (!f && !e->generic) {
+    return TNX_E_UNSUPPORTED;
+  }
   if (a->schedule & TNX_SCHED_PERSISTENT) {
     if (!e->persist || layout != 1 || a->split_k != 1 || a->k < (int64_t)a->num_stages * a->block_k) return TNX_E_UNSUPPORTED;
   }
@@ -218,6 +246,12 @@ static int compute_units(int* out) {
 }
 
 extern "C" int tnx_gemm_supported(const tnx_gemm_args* a) { return supported_impl(a, nullptr, nullptr, false); }
+
+extern "C" int tnx_gemm_tail_slabs(const tnx_gemm_args* a) {
+  bool fast = false, tail = false;
+  const int st = supported_impl(a, nullptr, &fast, true, nullptr, &tail);
+  return st != TNX_OK ? -1 : !fast ? (int)((a->k + a->block_k - 1) / a->block_k) : tail ? 1 : 0;
+}
 
 extern "C" int tnx_gemm(const tnx_gemm_args* a) { return tnx::gemm_launch(a, nullptr); }
 
@@ -263,8 +297,8 @@ int tnx::gemm_check(const tnx_gemm_args* a, GemmForm form) {
 
 int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, GemmForm form) {
   const KernelEntry* e = nullptr;
-  bool fast = false, bt = false, at = false, tail_slab = false;
-  int st = supported_impl(a, &e, &fast, true, &bt, &tail_slab, &at, form);
+  bool fast = false, bt = false, at = false, tail_slab = false, other_tile = false;
+  int st = supported_impl(a, &e, &fast, true, &bt, &tail_slab, &at, form, &other_tile);
   if (st != TNX_OK) return st;
   if (extra && (form == GEMM_PAIR || e->bm * e->bn > 128 * 128 || a->split_k != 1 || (a->schedule & TNX_SCHED_PERSISTENT) || is_skinny_cfg(a) || extra->batch < 1 ||
                 a->epilogue != TNX_EPI_NONE || (extra->bias && a->in_dtype == TNX_I8)))
@@ -277,6 +311,13 @@ int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, GemmForm fo
   if (tnx_gemm_workspace_bytes(a) > 0 &&
       (!a->workspace || a->workspace_bytes < tnx_gemm_workspace_bytes(a) || ((uintptr_t)a->workspace & 255)))
     return TNX_E_WORKSPACE;
+  if (other_tile) {
+    const KernelEntry* x = elementwise_tile(a);
+    tnx_gemm_args t = *a;
+    t.block_m = x->bm; t.block_n = x->bn; t.block_k = x->bk; t.num_warps = x->nw; t.num_stages = x->stages;
+    t.split_k = 1; t.tail_tiles = 0; t.schedule = TNX_SCHED_DEFAULT;
+    return gemm_launch(&t, extra, form);
+  }
 
   const int es_out = elem_size(a->out_dtype);
   GemmParams p;

@@ -186,6 +186,14 @@ template <> struct Mma<TagI8, 16> {
   }
 };
 
+// Whether the ring of a tail_slab launch stays inside an operand whose k rows have `len` elements at a pitch of
+// `pitch` >= len, `rows` of them in the slab that is left out: the last k row in the ring is loaded in whole chunks too,
+// and the rows left out have to reach the end of its last chunk.  They do, unless a row is shorter than a chunk (16-bit
+// types: up to 3 elements, int8: up to 7).
+__host__ __device__ inline bool ring_chunks_inside(int64_t rows, int64_t len, int64_t pitch, int vec) {
+  return rows * pitch + len >= (len + vec - 1) / vec * vec;
+}
+
 // ---------------------------------------------------------------------------
 // tile-id remap.  Workgroups are dealt round-robin to the 8 XCDs (each has its
 // own L2), so consecutive *logical* tile ids are first gathered per XCD, then
@@ -1257,8 +1265,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
           int row = P / C::CPR_B, cs = P % C::CPR_B;
           int c = cs ^ C::swzB(row);
           // column chunk past N: any valid address.  (A chunk that starts below N and ends above it -- tail_slab
-          // launches only -- is loaded as it is: its upper elements come from the next k row, which exists because
-          // the last slab is not loaded here, and belong to columns that are never stored.)
+          // launches only -- is loaded as it is: its upper elements come from the k rows after it, which reach that far
+          // because the last slab is not loaded here (ring_chunks_inside), and belong to columns that are never stored.)
           if (n0 + (int64_t)c * (16 / ES) >= p.n_load || (!p.tail_slab && n0 + (int64_t)(c + 1) * (16 / ES) > p.n_load)) c = 0;
           b_voff[q] = (uint32_t)((int64_t)row * ldb * ES + c * 16);
         }

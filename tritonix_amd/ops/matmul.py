@@ -208,9 +208,18 @@ def dma_operands(a, b):
     return a, b
 
 
+def _whole_chunks(length: int, pitch: int, k: int, es: int) -> bool:
+    """Whether k rows of ``length`` elements may be loaded in whole 16-byte chunks up to the last K slab (128 bytes of k) of
+    the 16-bit and int8 tiles: that slab's rows have to reach the end of the chunk before them, which rows shorter than a
+    chunk may not (``ring_chunks_inside`` in gemm_tile.h).  float32 operands are copied into padded rows anyway."""
+    vec, bk = 16 // es, 128 // es
+    return es == 4 or ((k - 1) % bk + 1) * pitch + length >= -(-length // vec) * vec
+
+
 def _transposed_a(a, b) -> bool:
     """A column-major A (``x.t()`` of a row-major x) with a row-major B, of a type the transposing loader is built for."""
     return (a.stride(0) == 1 and a.stride(1) >= a.shape[0] and a.stride(1) != 1 and b.stride(1) == 1 and b.stride(0) >= b.shape[1]
+            and _whole_chunks(a.shape[0], a.stride(1), a.shape[1], a.element_size())
             and a.dtype in (torch.float16, torch.bfloat16, torch.int8, torch.float32))
 
 
@@ -225,6 +234,10 @@ def engine_operands(a, b):
         # one row: its pitch means nothing, and one shorter than the row (the transpose of a [k, 1] matrix) would read as
         # overlapping rows, which only the element-wise loader takes (1 x 64 x 14144: 185 us, 8 us as a row)
         a = a.as_strided(a.shape, (a.shape[1], 1))
+    if b.stride(1) == 1 and b.stride(0) >= b.shape[1] and not _whole_chunks(b.shape[1], b.stride(0), b.shape[0], b.element_size()):
+        # a few columns: as k-contiguous runs instead of the element-wise loader, which would read all of A at a sixth of
+        # the speed for the sake of a B this small
+        b = b.t().contiguous().as_strided(b.shape, (1, b.shape[0]))
     if _transposed_a(a, b):
         es = a.element_size()
         aligned = ((a.stride(1) * es) % 16 == 0 and (b.stride(0) * es) % 16 == 0 and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
