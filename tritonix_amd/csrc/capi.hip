@@ -510,15 +510,30 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
     // 128 columns, 52.9 with 64; 16 x 28672 x 4096: 38.5 against 44.1); rows of a k-contiguous B are k runs either way.
     // Cutting s -> 2s saves kt / 2s slabs of the loop and costs s more slices: it pays while kt >= 1.75 s^2 (fitted to
     // 51 shapes of bf16 and int8, n 1024 to 28672, k 1024 to 14336; kt / s >= 4 and up to 512 workgroups before: 1.14x in
-    // the mean).  Up to 32 rows a 32-row tile (not built for an m-contiguous A or for heads and tails), except where 128
+    // the mean), once the loop is long enough to pay for the first cut's hand-over of 1.2 to 2.5 us: 18 slabs of the 16-bit
+    // types, 12 of int8, 14 of heads and tails (1,020 shapes, 1 to 64 slabs: the choice 1.01x the best cut in the mean, 1.14x
+    // with cuts from 2 slabs on; 48 x 4096 x 128 bf16 5.7 -> 3.9 us, 48 x 2048 x 384 int8 6.6 -> 4.6).  int8 of up to 16 rows
+    // hands less over and cuts from 1.25 s^2 on (8 x 256 x 10240 with a k-contiguous B: 9.3 us with 8 cuts, 8.1 with 16).
+    // A k-contiguous B whose slices are an odd multiple of 32 slabs takes one cut more: such slices are 4 KB runs, the
+    // workgroups all read at the same offsets modulo 4 KB, and halving them spreads the reads (16 x 8192 x 4096 bf16 16.2 ->
+    // 13.7 us, 16 x 4096 x 8192 16.4 -> 14.0, 16 x 12288 x 8192 int8 23.5 -> 20.7, 16 x 8192 x 6144 float32 113 -> 104; slices of
+    // 16, 24, 48 or 64 slabs lose 2 to 14 %).  Uncut it gains for int8 alone (16 x 28672 x 4096 24.3 -> 21.9).
+    // Up to 32 rows a 32-row tile (not built for an m-contiguous A or for heads and tails), except where 128
     // columns are cut: 16 x 4096 x 14336 24.1 us on 64 rows and eight waves, 24.7 on 32 and four.
     const int64_t kt = (a->k + bk - 1) / bk;
     const bool bt = a->stride_bk == 1 && a->stride_bn != 1;
-    const bool narrow = es == 2 && (bt || ((a->n + 63) / 64 <= cus && a->n * a->k <= 40000000));
+    // (A k-contiguous B of 200 MB or more, where 128 columns leave half a round and K is cut: 16 x 16384 x 14336 91 us with 64
+    // columns, 70 with 128; 16 x 12288 x 14336 75 against 60.  Heads and tails: where 64 columns are not cut and k is an odd
+    // multiple of 4 KB, see above: 16 x 16384 x 3072 float32 112 us with 64 columns, 104 with 128 cut in two.)
+    const bool wide_bt = (a->n + 127) / 128 * 2 <= cus &&
+                         (large_f32 ? (a->n + 63) / 64 * 2 > cus && kt % 64 == 32 : a->n * a->k >= 96000000);
+    const bool narrow = es == 2 && (bt ? !wide_bt : (a->n + 63) / 64 <= cus && a->n * a->k <= 40000000);
     a->block_n = narrow ? 64 : 128;
     const int64_t tiles = (a->n + a->block_n - 1) / a->block_n;
     int s = 1;
-    while (tiles * s * 2 <= cus && s < 16 && 4 * kt >= 7 * s * s) s *= 2;
+    if (kt >= (es == 1 ? 12 : large_f32 ? 14 : 18))
+      while (tiles * s * 2 <= cus && s < 16 && 4 * kt >= (es == 1 && a->m <= 16 ? 5 : 7) * s * s) s *= 2;
+    if (bt && s >= (es == 1 ? 1 : 2) && s < 8 && kt % (64 * s) == 32 * s) s *= 2;
     a->split_k = s;
     a->block_m = es == 2 && a->m <= 32 && !at && !large_f32 && (narrow || s == 1) ? 32 : 64;
     a->num_stages = narrow ? 4 : 3;
