@@ -52,3 +52,23 @@ def test_every_choice_for_few_rows_is_launchable():
                         g = _choice(dt, layout, m, n, k)
                         assert lib.tnx_gemm_supported(ctypes.byref(g)) == _C.OK, (dt, layout, m, n, k)
                         assert g.split_k <= max(1, -(-k // g.block_k) // 2)
+
+
+def test_int8_with_a_column_major_a():
+    """128-row tiles, K cut as the row-major choice cuts it; ragged rows are copied by the wrappers."""
+    import importlib
+
+    import torch
+
+    mm = importlib.import_module("tritonix_amd.ops.matmul")
+    for m, n, k, split in ((16, 4096, 4096, 8), (48, 8192, 4096, 4), (64, 512, 14336, 16), (16, 28672, 4096, 1), (48, 4096, 1536, 1)):
+        g = _choice("i8", "tn", m, n, k)
+        assert (g.block_m, g.block_n, g.num_warps, g.num_stages, g.split_k) == (128, 128, 8, 3, split), (m, n, k)
+    b = torch.zeros(256, 64, dtype=torch.int8)
+    for m, pitch, in_place in ((16, 16, True), (64, 64, True), (16, 24, False), (15, 16, False), (40, 48, False), (65, 65, False),
+                               (191, 191, False), (100, 100, True), (193, 193, True)):
+        a = torch.zeros(256, pitch, dtype=torch.int8)[:, :m].t()
+        x, _, layout = mm.engine_operands(a, b)
+        assert (x is a) == in_place and (layout in (5, 6)) == in_place, (m, pitch)
+    a = torch.zeros(256, 15, dtype=torch.bfloat16).t()
+    assert mm.engine_operands(a, b.bfloat16())[0] is a
