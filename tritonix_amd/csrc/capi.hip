@@ -579,7 +579,11 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
   // int8: rows of a 64-wide B tile are too short for the transposing read; the 192-wide tiles exist for it too
   // (3072 x 4096 x 4096: 53.6 -> 45.7 us with 192x256, 4096 x 3072 x 4096: 52.8 -> 47.3 us with 256x192)
   // (a binary32 result exists on the tiles up to 128x128 and, for float32 products, on the eight-wave tiles of 192 and 256)
-  auto usable = [&](int i) { return (es == 2 || i != 4) && !(at && es == 1 && i == 3) && (a->out_dtype != TNX_F32 || (i >= 2 && i <= 4) || (large_f32 && i != 1)); };
+  // (and only while a lane's 32-bit offset reaches from the first to the last of the tile's k-contiguous rows)
+  auto reach = [&](int i) {
+    return !large_f32 || ((at || cand[i][0] * a->k * 2 < (1ll << 32)) && (a->stride_bk != 1 || a->stride_bn == 1 || cand[i][1] * a->k * 2 < (1ll << 32)));
+  };
+  auto usable = [&](int i) { return reach(i) && (es == 2 || i != 4) && !(at && es == 1 && i == 3) && (a->out_dtype != TNX_F32 || (i >= 2 && i <= 4) || (large_f32 && i != 1)); };
   const double cu_flops = 5.5e12 * (es == 1 ? 1.7 : 1.0);          // per CU with the largest tile
   const double launch = 3e-6, handover = 9e-6, readback = 60e9;
   const int64_t kt = (a->k + bk - 1) / bk;

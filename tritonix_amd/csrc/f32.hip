@@ -32,7 +32,7 @@ struct SplitSide {
   int outer, inner;        // rows and columns of the source in that form
   int kp;                  // k rounded up to 8 (pairs: to 32)
   int groups;              // 16-byte chunks (8 elements) per row handled, padding included
-  int items;               // (row, chunk) pairs
+  int row0, items;         // first row of this launch, and its (row, chunk) pairs
   int64_t pitch;           // elements per scratch row
   int pad;                 // elements (k along the row) or rows (k planes) of zeros after the three terms
   bool planes;             // rows are k: one plane of kp8 rows per term
@@ -44,17 +44,17 @@ struct SplitSide {
 }  // namespace
 
 __device__ __forceinline__ void split_item(const SplitSide& s, int item) {
-  const int o = (int)fd_div((uint32_t)item, s.div), g = item - o * s.groups, j0 = g * 8;
+  const int q = (int)fd_div((uint32_t)item, s.div), g = item - q * s.groups, j0 = g * 8, o = s.row0 + q;
   float v[8];
   const float* src = s.src + (int64_t)o * s.so + (int64_t)j0 * s.si;
-  if (s.si == 1 && o < s.outer && j0 + 8 <= s.inner) {
+  if (s.si == 1 && o < s.outer && s.inner - j0 >= 8) {
     struct __attribute__((packed, aligned(4))) Run { float v[8]; };
     const Run r = *(const Run*)src;
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = r.v[e];
   } else {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = o < s.outer && j0 + e < s.inner ? src[(int64_t)e * s.si] : 0.0f;
+    for (int e = 0; e < 8; ++e) v[e] = o < s.outer && e < s.inner - j0 ? src[(int64_t)e * s.si] : 0.0f;
   }
   if (s.pair) {
     uint16_t hi[8], lo[8];
@@ -112,6 +112,10 @@ __global__ __launch_bounds__(256) void split_f32_pair_kernel(SplitSide a, SplitS
   }
 }
 
+// Pairs of one operand per launch: larger operands (2^30 elements, 4 GB of float32) take several, a millisecond each.  Both
+// operands' threads then stay within 32 bits, in the pair's number and in the grid.
+static constexpr int64_t MAX_ITEMS = 1ll << 27;
+
 static int64_t up(int64_t v, int64_t q) { return (v + q - 1) / q * q; }
 
 // The bf16 problem a float32 one becomes (pointers into `scratch`, which may be null for a size query), the two sides
@@ -119,7 +123,7 @@ static int64_t up(int64_t v, int64_t q) { return (v + q - 1) / q * q; }
 static int plan(const tnx_gemm_args* a, void* scratch, tnx_gemm_args* g, SplitSide* sa, SplitSide* sb, int64_t* bytes, bool* pair) {
   if (!a || a->in_dtype != TNX_F32 || a->m < 0 || a->n < 0 || a->k < 0 || a->block_k <= 0) return TNX_E_INVALID;
   if (a->out_dtype != TNX_F32) return TNX_E_UNSUPPORTED;
-  if (a->m > 0x7fffffff - 64 || a->n > 0x7fffffff - 64 || a->k > (0x7fffffff - 1024) / 3) return TNX_E_UNSUPPORTED;
+  if (a->m > 0x7fffffff || a->n > 0x7fffffff || a->k > (0x7fffffff - 1024) / 3) return TNX_E_UNSUPPORTED;
   *g = *a;
   g->in_dtype = TNX_BF16;
   bool tile_bt = false, tile_at = false;
@@ -145,15 +149,25 @@ static int plan(const tnx_gemm_args* a, void* scratch, tnx_gemm_args* g, SplitSi
     s->planes = planes; s->tail_second = tail_second;
     s->pitch = pitch;
     s->pad = *pair ? 0 : (int)(kt - 3 * kp);
-    const int64_t groups = planes ? pitch / 8 : kp / 8, items = (planes ? kp : rows) * groups;
-    s->groups = (int)groups; s->items = items > 0x7fffffff - 256 ? -1 : (int)items;
+    const int64_t groups = planes ? pitch / 8 : kp / 8;
+    s->groups = (int)groups;
+    s->row0 = s->items = 0;
     s->div = make_fastdiv((uint32_t)(groups > 0 ? groups : 1));
   };
   if (at) side(sa, a->a, true, a->k, a->m, a->stride_ak, a->stride_am, scratch, mp, false);
   else side(sa, a->a, false, a->m, a->k, a->stride_am, a->stride_ak, scratch, kt, false);
   if (bt) side(sb, a->b, false, a->n, a->k, a->stride_bn, a->stride_bk, (uint8_t*)scratch + a_bytes, kt, true);
   else side(sb, a->b, true, a->k, a->n, a->stride_bk, a->stride_bn, (uint8_t*)scratch + a_bytes, np, true);
-  return sa->items < 0 || sb->items < 0 ? TNX_E_UNSUPPORTED : TNX_OK;
+  return TNX_OK;
+}
+
+// moves a side to its next launch; false: nothing left (items 0)
+static bool next_rows(SplitSide* s) {
+  const int64_t rows = s->planes ? s->kp : s->outer, row0 = (int64_t)s->row0 + (s->groups > 0 ? s->items / s->groups : 0);
+  const int64_t most = s->groups > 0 ? (MAX_ITEMS > s->groups ? MAX_ITEMS / s->groups : 1) : 0, left = rows - row0;
+  s->row0 = (int)row0;
+  s->items = (int)((left < most ? left : most) * s->groups);
+  return s->items > 0;
 }
 
 extern "C" size_t tnx_gemm_f32_scratch_bytes(const tnx_gemm_args* a) {
@@ -181,9 +195,13 @@ extern "C" int tnx_gemm_f32(const tnx_gemm_args* a, void* scratch, size_t scratc
   st = gemm_check(&g, pair ? GEMM_PAIR : GEMM_PADDED); // refuse what the GEMM would refuse before anything is launched
   if (st != TNX_OK) return st;
   if (!scratch || scratch_bytes < (size_t)bytes || ((uintptr_t)scratch & 255)) return TNX_E_WORKSPACE;
-  const unsigned blocks_a = (unsigned)((sa.items + 255) / 256), blocks_b = (unsigned)((sb.items + 255) / 256);
-  hipLaunchKernelGGL(split_f32_pair_kernel, dim3(blocks_a + blocks_b), dim3(256), 0, (hipStream_t)a->stream, sa, sb, blocks_a);
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess) { note_hip_error((int)err); return TNX_E_HIP; }
+  for (;;) {
+    const bool more_a = next_rows(&sa), more_b = next_rows(&sb);
+    if (!more_a && !more_b) break;
+    const unsigned blocks_a = (unsigned)((sa.items + 255) / 256), blocks_b = (unsigned)((sb.items + 255) / 256);
+    hipLaunchKernelGGL(split_f32_pair_kernel, dim3(blocks_a + blocks_b), dim3(256), 0, (hipStream_t)a->stream, sa, sb, blocks_a);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) { note_hip_error((int)err); return TNX_E_HIP; }
+  }
   return gemm_launch(&g, nullptr, pair ? GEMM_PAIR : GEMM_PADDED);
 }
