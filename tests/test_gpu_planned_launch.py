@@ -108,3 +108,14 @@ def test_threads_with_streams_of_their_own_share_a_plan(device):
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_a_size_met_once_costs_no_plan(device):
+    """The first call of a size only notes it, the second keeps the launch, the third takes it."""
+    a, b = _ints((24, 128), torch.float16, 0).to(device), _ints((128, 64), torch.float16, 1).to(device)
+    first = mm.triton_matmul(a, b)
+    assert list(kernel._plans.values()) == [None]
+    second = mm.triton_matmul(a, b)
+    (plan, _), = kernel._plans.values()
+    assert isinstance(plan, kernel.PlannedLaunch)
+    assert torch.equal(second, first) and torch.equal(mm.triton_matmul(a, b), first)

@@ -239,14 +239,20 @@ def engine_operands(a, b):
     with the transposing loads a row-major B takes, at the speed of their row-major twins (4096 x 4096 x 2048 bf16:
     56-60 us either way), where the copy alone takes 37 us.  Its classes are 5 and, with the last K slab loaded chunk by
     chunk, 6."""
-    if a.shape[0] == 1 and a.stride(1) == 1 and a.stride(0) < a.shape[1]:
-        # one row: its pitch means nothing, and one shorter than the row (the transpose of a [k, 1] matrix) would read as
-        # overlapping rows, which only the element-wise loader takes (1 x 64 x 14144: 185 us, 8 us as a row)
-        a = a.as_strided(a.shape, (a.shape[1], 1))
+    layout = dma_layout(a, b)
+    if layout == 1 or layout == 2 or layout == 4:
+        return a, b, layout
     if b.stride(1) == 1 and b.stride(0) >= b.shape[1] and not _whole_chunks(b.shape[1], b.stride(0), b.shape[0], b.element_size()):
         # a few columns: as k-contiguous runs instead of the element-wise loader, which would read all of A at a sixth of
         # the speed for the sake of a B this small
         b = b.t().contiguous().as_strided(b.shape, (1, b.shape[0]))
+        layout = dma_layout(a, b)
+    if layout != 0:
+        return a, b, layout
+    if a.shape[0] == 1 and a.stride(1) == 1 and a.stride(0) < a.shape[1]:
+        # one row: its pitch means nothing, and one shorter than the row (the transpose of a [k, 1] matrix) would read as
+        # overlapping rows, which only the element-wise loader takes (1 x 64 x 14144: 185 us, 8 us as a row)
+        a = a.as_strided(a.shape, (a.shape[1], 1))
     if _transposed_a(a, b):
         es = a.element_size()
         aligned = ((a.stride(1) * es) % 16 == 0 and (b.stride(0) * es) % 16 == 0 and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
