@@ -88,6 +88,14 @@ def _raise_for_status(status: int, a: _C.Conv2dArgs) -> None:
     raise ValueError(f"{_C.strerror(status)}: conv2d")
 
 
+def _scratch(nbytes: int, device) -> Optional[torch.Tensor]:
+    """Scratch of the packed kernels, or None where the device has no room for it: the kernels that need none then run."""
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _args(out, input, weight, bias, batch, c_in, h_in, w_in, c_out, filter_h, filter_w, stride, padding, dilation,
           block_m: int, block_n: int, block_k: int, group_m: int, loader: int = 0) -> _C.Conv2dArgs:
     a = _C.Conv2dArgs()
@@ -97,8 +105,8 @@ def _args(out, input, weight, bias, batch, c_in, h_in, w_in, c_out, filter_h, fi
         a.stride_h, a.stride_w, a.pad_h, a.pad_w, a.dil_h, a.dil_w = *stride, *padding, *dilation
         a.dtype, a.out_f32 = _DTYPES[input.dtype], input.dtype == torch.float32
         need = _C.load().tnx_conv2d_workspace_bytes(ctypes.byref(a))
-        if need:
-            ws = torch.empty(need, dtype=torch.uint8, device=input.device)
+        ws = _scratch(need, input.device) if need else None
+        if ws is not None:
             a.workspace, a.workspace_bytes, a._keep = ws.data_ptr(), need, (ws,)
     if input.dtype == torch.float32 and not a.workspace:
         if not (input.is_cuda and weight.is_cuda and out.is_cuda):
@@ -257,7 +265,8 @@ _MAX_PLANS = 1024
 def _launch_planned(input, weight, bias, stride, padding, dilation) -> Optional[torch.Tensor]:
     """The library's own choice for a problem, launched from its remembered argument struct: a call then only fills in
     pointers (binding every argument by name anew costs 10 us of host time, twice what a small layer takes on the
-    GPU).  None: the ordinary path has to bind it (float32 without the packed kernels, arguments it has to refuse)."""
+    GPU).  None: the ordinary path has to bind it (float32 without the packed kernels or room for their scratch, arguments it
+    has to refuse)."""
     if bias is not None and not (bias.is_cuda and bias.is_contiguous()):
         return None
     dev = input.get_device()
@@ -290,8 +299,11 @@ def _launch_planned(input, weight, bias, stride, padding, dilation) -> Optional[
     if bias is not None:
         a.bias = bias.data_ptr()
     if need:
-        ws = torch.empty(need, dtype=torch.uint8, device=input.device)
-        a.workspace, a.workspace_bytes = ws.data_ptr(), need
+        ws = _scratch(need, input.device)
+        if ws is not None:
+            a.workspace, a.workspace_bytes = ws.data_ptr(), need
+        elif input.dtype == torch.float32:
+            return None
     a.stream = _stream_of(dev)
     if dev != torch.cuda.current_device():
         with torch.cuda.device(dev):
@@ -354,9 +366,12 @@ def conv2d_forward(
                 if t < best_time:
                     best_time, best = t, dict(BLOCK_SIZE_M=bm, BLOCK_SIZE_N=bn, BLOCK_SIZE_K=bk, GROUP_SIZE_M=g)
             # the library's own choice is one more candidate: with scratch it may be the packed kernels, which no tile names
-            t = _time_kernel(lambda: launch(0, 0, 0, 8))
-            if t < best_time:
-                best_time, best = t, dict(BLOCK_SIZE_M=0, BLOCK_SIZE_N=0, BLOCK_SIZE_K=0, GROUP_SIZE_M=8)
+            try:
+                t = _time_kernel(lambda: launch(0, 0, 0, 8))
+                if t < best_time:
+                    best_time, best = t, dict(BLOCK_SIZE_M=0, BLOCK_SIZE_N=0, BLOCK_SIZE_K=0, GROUP_SIZE_M=8)
+            except (ValueError, NotImplementedError, _C.OutOfResources, torch.OutOfMemoryError):
+                pass
             if (r, s) == (1, 1) and stride == (1, 1) and padding == (0, 0):
                 # a 1x1 layer is a plain GEMM per image: the library's GEMM route with its own tile is one more candidate
                 try:
