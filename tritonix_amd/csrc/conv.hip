@@ -386,6 +386,20 @@ static const GatherCost* gather_cost(const GatherEntry& e) {
 }
 
 static constexpr double PAIR_SLAB = 1.3;
+static constexpr double PASS_US = 9.0;     // the pass over the operands and the second launch, apart from the bytes
+
+// Modelled microseconds of the kernel a 16-bit layer has without scratch: rounds of workgroups x K slabs, constants fitted to
+// 636 layers of 3x3 and 5x5 filters (two tiles of the register-staged kernel per CU cost it a third of its slab rate).
+static double unpacked_time(const tnx_conv2d_args* a) {
+  Resolved r;
+  if (resolve(a, &r, false) != TNX_OK || r.gemm) return 1e300;
+  const int64_t cols = r.dma ? dma_cols(a, r.h_out, r.w_out) : (int64_t)a->batch * r.h_out * r.w_out;
+  const int64_t tiles = ((cols + r.bpix - 1) / r.bpix) * ((a->c_out + r.bcout - 1) / r.bcout);
+  const double kt = (double)(((int64_t)a->c_in * a->filter_h * a->filter_w + r.bk - 1) / r.bk);
+  if (r.dma) return 1.5 + (double)((tiles + 255) / 256) * (4.1 + (r.bcout > 128 ? 1.7 : 0.694) * kt);
+  const double slots = r.bcout > 64 ? 320.0 : 800.0, rounds = tiles > slots ? tiles / slots : 1.0;
+  return 4.0 + rounds * kt * (r.bcout > 64 ? 1.8 : tiles < 256 ? 1.15 + 0.4 * tiles / 256.0 : 1.55);
+}
 
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
@@ -461,6 +475,18 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p) {
       }
     }
   if (!p->e) return false;
+  // A wide padding (as a dilated filter has it) makes the packed image a multiple of the input, which the lines above do not
+  // know.  From twice the input on the pass is priced, at the 5 TB/s it moves (what does not fit the memory-side cache costs the
+  // GEMM twice its bytes more), against the kernel that needs none: 8 images of 2048 channels, 33x33 (packed 105x105), 256 out, 3x3:
+  // 227 us packed, 209 not; 128 of 512, 7x7 (127x127), 64 out: 415 and 87; 1 of 2048, 33x33 (177x177), 256 out, 5x5: 52 and
+  // 895.  On 636 layers of 1 to 6500 times the input, against the faster of the two: 0.4 % lost in the mean, 2.7 % without this
+  // rule.  float32 stays: its alternative is an extra pass too.
+  const double planes = (double)p->rows * p->cols / ((double)a->h_in * a->w_in);
+  if (!f32 && planes > 2.0) {
+    const double bytes = (double)p->x_bytes + 2.0 * a->batch * (double)a->c_in * a->h_in * a->w_in;
+    const double again = p->x_bytes > 200000000 ? 2.0 * ((double)p->x_bytes - 2.0e8) : 0.0;
+    if (best + PASS_US + (bytes + again) / 5.0e6 > unpacked_time(&t)) return false;
+  }
   const int64_t tiles = ((a->c_out + p->e->bm - 1) / p->e->bm) * ((p->n_total + p->e->bn - 1) / p->e->bn);
   if (tiles * p->split >= lim || (p->split > 1 && tiles > WS_MAX_TILES)) return false;
   p->slices_bytes = p->split > 1 ? WS_COUNTER_BYTES + (int64_t)p->split * tiles * p->e->bm * p->e->bn * 4 : 0;
