@@ -32,7 +32,10 @@
 extern "C" {
 #endif
 
-#define TNX_VERSION 1
+/* Raised whenever a struct below changes its layout: a program compares it with tnx_version() of the library it loaded
+ * before its first call, and does not call a library of another version, which would read fields its structs do not have.
+ * 2: tnx_conv2d_args ends in workspace and workspace_bytes. */
+#define TNX_VERSION 2
 
 /* element types */
 enum tnx_dtype {

@@ -210,3 +210,22 @@ def test_default_config_of_the_benchmark_shapes():
     assert picked == [_C.SCHED_SUPERBLOCK, _C.SCHED_SUPERBLOCK, _C.SCHED_SUPERBLOCK, 0, 0, 0, _C.SCHED_SUPERBLOCK]
 
 
+
+
+def test_struct_layouts_belong_to_the_version(monkeypatch):
+    """A library of another version is not called: its structs may be longer than the caller's.  A change of either size
+    raises TNX_VERSION and gets a line here."""
+    sizes = {1: (168, 128), 2: (168, 144)}
+    assert (ctypes.sizeof(_C.GemmArgs), ctypes.sizeof(_C.Conv2dArgs)) == sizes[_C.VERSION] and max(sizes) == _C.VERSION
+    header = open(os.path.join(ROOT, "include", "tritonix_hip.h")).read()
+    body = header[header.index("typedef struct tnx_conv2d_args {") + len("typedef struct tnx_conv2d_args {"):header.index("} tnx_conv2d_args;")]
+    names = []
+    for decl in re.sub(r"/\*.*?\*/", "", body, flags=re.S).split(";"):
+        decl = re.sub(r"^(const\s+)?(void|int32_t|size_t)\s*\*?", "", decl.strip())
+        names += [n.strip(" *") for n in decl.split(",") if n.strip(" *")]
+    assert names == [f[0] for f in _C.Conv2dArgs._fields_]
+    assert _C.load().tnx_version() == _C.VERSION
+    monkeypatch.setattr(_C, "_lib", None)
+    monkeypatch.setattr(_C, "VERSION", _C.VERSION - 1)
+    with pytest.raises(RuntimeError, match="version"):
+        _C.load()

@@ -16,6 +16,8 @@ from tritonix_amd.testing import LDS_LIMIT_BYTES, OutOfResources
 LIB_PATH = os.environ.get("TRITONIX_HIP_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)),
                                                               "libtritonix_hip.so")
 
+# TNX_VERSION of the header whose structs are restated here
+VERSION = 2
 # enum tnx_dtype
 F16, BF16, I8, I32, F32 = 0, 1, 2, 3, 4
 # enum tnx_epilogue
@@ -82,6 +84,10 @@ def load() -> ctypes.CDLL:
         raise RuntimeError(f"{LIB_PATH} is missing: build it with `python -m tritonix_amd.build` "
                            "(there is no non-HIP implementation to fall back to)")
     lib = ctypes.CDLL(LIB_PATH)
+    lib.tnx_version.argtypes, lib.tnx_version.restype = [], ctypes.c_int
+    if lib.tnx_version() != VERSION:
+        raise RuntimeError(f"{LIB_PATH} is of version {lib.tnx_version()}, this package of version {VERSION}: build it again with "
+                           "`python -m tritonix_amd.build`")
     p = ctypes.POINTER(GemmArgs)
     lib.tnx_gemm.argtypes = [p]
     lib.tnx_gemm.restype = ctypes.c_int
@@ -114,8 +120,6 @@ def load() -> ctypes.CDLL:
     lib.tnx_strerror.restype = ctypes.c_char_p
     lib.tnx_last_hip_error.argtypes = []
     lib.tnx_last_hip_error.restype = ctypes.c_int
-    lib.tnx_version.argtypes = []
-    lib.tnx_version.restype = ctypes.c_int
     cp = ctypes.POINTER(Conv2dArgs)
     for name in ("tnx_conv2d_forward", "tnx_conv2d_supported", "tnx_conv2d_default_config"):
         getattr(lib, name).argtypes = [cp]
