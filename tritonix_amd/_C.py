@@ -33,7 +33,8 @@ CONV_LOADER_AUTO, CONV_LOADER_REGISTERS, CONV_LOADER_DMA, CONV_LOADER_GEMM = 0, 
 EXPORTS = ("tnx_gemm", "tnx_gemm_static_workspace", "tnx_gemm_workspace_bytes", "tnx_gemm_lds_bytes", "tnx_gemm_supported",
            "tnx_gemm_default_config", "tnx_tile_coords", "tnx_split_f32", "tnx_gemm_f32_scratch_bytes",
            "tnx_gemm_f32", "tnx_gemm_tail_slabs", "tnx_kernel_count", "tnx_kernel_name", "tnx_strerror",
-           "tnx_last_hip_error", "tnx_version", "tnx_conv2d_forward", "tnx_conv2d_workspace_bytes", "tnx_conv2d_supported",
+           "tnx_last_hip_error", "tnx_version", "tnx_conv2d_forward", "tnx_conv2d_workspace_bytes",
+           "tnx_conv2d_packed_info", "tnx_conv2d_packed_forward", "tnx_conv2d_supported",
            "tnx_conv2d_output_size",
            "tnx_conv2d_default_config", "tnx_conv2d_kernel_count", "tnx_conv2d_kernel_name")
 
@@ -124,6 +125,10 @@ def load() -> ctypes.CDLL:
     for name in ("tnx_conv2d_forward", "tnx_conv2d_supported", "tnx_conv2d_default_config"):
         getattr(lib, name).argtypes = [cp]
         getattr(lib, name).restype = ctypes.c_int
+    lib.tnx_conv2d_packed_info.argtypes = [cp, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int32)]
+    lib.tnx_conv2d_packed_info.restype = ctypes.c_size_t
+    lib.tnx_conv2d_packed_forward.argtypes = [cp, ctypes.c_int, ctypes.c_int]
+    lib.tnx_conv2d_packed_forward.restype = ctypes.c_int
     lib.tnx_conv2d_workspace_bytes.argtypes = [cp]
     lib.tnx_conv2d_workspace_bytes.restype = ctypes.c_size_t
     lib.tnx_conv2d_output_size.argtypes = [cp, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]

@@ -403,7 +403,8 @@ static double unpacked_time(const tnx_conv2d_args* a) {
 
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
-static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p) {
+// tile >= 0: that tile of the type's table and that many K slices, whatever the rules below would choose
+static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, int split = 1) {
   if (!a || a->loader != TNX_CONV_LOADER_AUTO || a->block_cout || a->block_pixels || a->block_k) return false;
   tnx_conv2d_args t = *a;
   const bool f32 = a->dtype == TNX_F32;
@@ -418,7 +419,9 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p) {
   // (256 channels, 56x56: 20.0 / 24.0; 512, 28x28: 23.6 / 19.1).  float32 has three terms per element and its alternative
   // an extra pass over both operands.
   const int64_t macs = (int64_t)a->c_in * a->filter_h * a->filter_w;
-  if (f32 ? macs <= 48 : macs <= (a->filter_h * a->filter_w == 1 ? 256 : 144)) return false;
+  if (tile >= 0) {
+    if (split < 1 || split > 16) return false;
+  } else if (f32 ? macs <= 48 : macs <= (a->filter_h * a->filter_w == 1 ? 256 : 144)) return false;
   *p = PackedPlan{};
   p->h_out = h_out; p->w_out = w_out;
   // a filter one row high reads only every stride_h-th input row: only those are packed (likewise for columns)
@@ -454,12 +457,16 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p) {
   // triples on 120 layers; choosing by it costs 1.5 % against the best measured tile in the mean, 12 % at worst on
   // all but one.
   double best = 1e300;
-  int ng = 0;
+  int ng = 0, number = 0;
   const GatherGroup* const* g = tnx_gather_groups(&ng);
   for (int i = 0; i < ng; ++i)
     for (int j = 0; j < g[i]->count; ++j) {
       const GatherEntry& e = g[i]->entries[j];
       if (e.dtype != t.dtype) continue;
+      if (tile >= 0) {
+        if (number++ == tile) { p->e = &e; p->split = split; }
+        continue;
+      }
       const GatherCost* cost = gather_cost(e);
       if (!cost) continue;
       const int64_t tiles = ((a->c_out + e.bm - 1) / e.bm) * ((p->n_total + e.bn - 1) / e.bn);
@@ -482,7 +489,7 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p) {
   // 895.  On 636 layers of 1 to 6500 times the input, against the faster of the two: 0.4 % lost in the mean, 2.7 % without this
   // rule.  float32 stays: its alternative is an extra pass too.
   const double planes = (double)p->rows * p->cols / ((double)a->h_in * a->w_in);
-  if (!f32 && planes > 2.0) {
+  if (!f32 && tile < 0 && planes > 2.0) {
     const double bytes = (double)p->x_bytes + 2.0 * a->batch * (double)a->c_in * a->h_in * a->w_in;
     const double again = p->x_bytes > 200000000 ? 2.0 * ((double)p->x_bytes - 2.0e8) : 0.0;
     if (best + PASS_US + (bytes + again) / 5.0e6 > unpacked_time(&t)) return false;
@@ -582,6 +589,31 @@ static int packed_forward(const tnx_conv2d_args* a, const PackedPlan& pl) {
   return TNX_OK;
 }
 
+extern "C" size_t tnx_conv2d_packed_info(const tnx_conv2d_args* a, int tile, int split, int32_t* info) {
+  PackedPlan p;
+  if (!packed_plan(a, &p, tile, split)) return 0;
+  if (info) {
+    const int32_t v[6] = {p.e->bm, p.e->bn, p.e->nw, p.e->stages, p.split, p.terms};
+    memcpy(info, v, sizeof v);
+  }
+  return (size_t)p.total_bytes;
+}
+
+// the checks of a launch that has a plan and a workspace
+static int packed_launch(const tnx_conv2d_args* a, const PackedPlan& pl) {
+  if (!a->workspace || a->workspace_bytes < (size_t)pl.total_bytes || ((uintptr_t)a->workspace & 255)) return TNX_E_WORKSPACE;
+  const unsigned in_align = a->dtype == TNX_F32 ? 3 : 1, out_align = a->out_f32 ? 3 : 1;
+  if (!a->input || !a->weight || !a->output || ((uintptr_t)a->input & in_align) || ((uintptr_t)a->weight & in_align) ||
+      ((uintptr_t)a->output & out_align) || (a->bias && ((uintptr_t)a->bias & (a->bias_dtype == TNX_F32 ? 3 : 1))))
+    return TNX_E_INVALID;
+  return packed_forward(a, pl);
+}
+
+extern "C" int tnx_conv2d_packed_forward(const tnx_conv2d_args* a, int tile, int split) {
+  PackedPlan pl;
+  return packed_plan(a, &pl, tile, split) ? packed_launch(a, pl) : TNX_E_UNSUPPORTED;
+}
+
 extern "C" int tnx_conv2d_supported(const tnx_conv2d_args* a) {
   Resolved r;
   return resolve(a, &r, false);
@@ -605,14 +637,7 @@ extern "C" int tnx_conv2d_default_config(tnx_conv2d_args* a) {
 extern "C" int tnx_conv2d_forward(const tnx_conv2d_args* a) {
   if (a && a->workspace) {
     PackedPlan pl;
-    if (packed_plan(a, &pl)) {
-      if (a->workspace_bytes < (size_t)pl.total_bytes || ((uintptr_t)a->workspace & 255)) return TNX_E_WORKSPACE;
-      const unsigned in_align = a->dtype == TNX_F32 ? 3 : 1, out_align = a->out_f32 ? 3 : 1;
-      if (!a->input || !a->weight || !a->output || ((uintptr_t)a->input & in_align) || ((uintptr_t)a->weight & in_align) ||
-          ((uintptr_t)a->output & out_align) || (a->bias && ((uintptr_t)a->bias & (a->bias_dtype == TNX_F32 ? 3 : 1))))
-        return TNX_E_INVALID;
-      return packed_forward(a, pl);
-    }
+    if (packed_plan(a, &pl)) return packed_launch(a, pl);
   }
   Resolved r;
   const int st = resolve(a, &r, true);
