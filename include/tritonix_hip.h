@@ -229,8 +229,8 @@ const char* tnx_kernel_name(int i);
  * weight, NCHW output of the input's type, GEMM_M = batch * h_out * w_out, GEMM_N = c_out, GEMM_K = c_in *
  * filter_h * filter_w, zero padding, fp32 accumulation, optional bias added in fp32 before the one rounding.
  * block_pixels / block_cout / block_k / group_pixels are the reference's BLOCK_SIZE_M / BLOCK_SIZE_N /
- * BLOCK_SIZE_K / GROUP_SIZE_M.  dtype is TNX_F16 or TNX_BF16 (the reference's float32-with-TF32 mode has no
- * matrix instruction on gfx950 and is not built: TNX_E_UNSUPPORTED).  Limits: batch * h_out * w_out and the
+ * BLOCK_SIZE_K / GROUP_SIZE_M.  dtype is TNX_F16 or TNX_BF16, with a workspace also TNX_F32 (the reference's
+ * float32-with-TF32 mode has no matrix instruction on gfx950; without a workspace: TNX_E_UNSUPPORTED).  Limits: batch * h_out * w_out and the
  * element counts of input and weight below 2^31, h_in / w_in / pad / (filter - 1) * dilation at most 16384. */
 typedef struct tnx_conv2d_args {
   const void* input;   /* [batch, c_in, h_in, w_in]                                 */

@@ -625,8 +625,9 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
   // eight, above 71 with four.)
   if (bi == 2 && large_f32 && !at) a->num_warps = 4;
   // A k-contiguous B on 64x128 tiles, one workgroup per CU: a fourth slot (the LDS holds six; five and six measured no
-  // better) covers the longer way of 128-byte runs.  512 x 4096 x 4096 24.5 -> 21.5 us, 1024 x 2048 x 4096 22.8 -> 21.3; with
-  // two workgroups on a CU three slots stay ahead (2048^3: 21.3 against 23.2 us), and with a row-major B they tie.
+  // better) covers the longer way of 128-byte runs.  launches back to back: 512 x 4096 x 4096 23.6 -> 20.9 us, 1024 x 2048 x 4096
+  // 22.4 -> 20.1, 512 x 4096 x 2048 12.2 -> 11.2 (whole calls on changing operands, the first of them: 23.1 -> 21.2); with two
+  // workgroups on a CU three slots stay ahead (2048^3: 21.3 against 23.2 us), and with a row-major B they tie.
   if (es == 2 && bi == 3 && !large_f32 && a->stride_bk == 1 && a->stride_bn != 1 &&
       ((a->m + 63) / 64) * ((a->n + 127) / 128) * bs <= cus)
     a->num_stages = 4;

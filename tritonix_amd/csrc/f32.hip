@@ -5,7 +5,8 @@
 // gemm_tile.h); every other tile gets three copies of k, [hi | hi' | lo] against [hi | lo | hi'], as tnx_split_f32 lays
 // them out.  A non-finite element must not meet a tail that happens to be zero (inf * 0): in the three copies it is carried
 // by the first head alone; in the pairs its head is +-1 and its tail the element itself, so that against a finite or a
-// non-finite partner every product that is not finite has the right sign, and the finite ones vanish beside it.
+// non-finite partner every product that is not finite has the right sign, and the finite ones vanish beside it.  (Either
+// way a partner of at most 2^-134 has a zero head, and an infinity times it gives NaN where float32 gives the infinity.)
 // Where this pass writes follows the operand: an A with k along its rows and a B with k along its columns keep k
 // contiguous; the others keep their own contiguous dimension, k rows of it.  So every load and store is a run of the
 // operand's own rows, whichever way it is transposed, and the GEMM kernel has a loader for each form.  k is padded to

@@ -385,8 +385,7 @@ struct TileCfg {
   static constexpr int ES = T::ES;
   static constexpr int BM = BM_, BN = BN_, BK = BK_, NW = NW_, STAGES = STAGES_;
   static constexpr int THREADS = NW * 64;
-  // wave grid: 2 x 2 / 4 x 2 / 2 x 4; widths that no 16-column MFMA tile halves keep every wave on all columns
-  static constexpr int WGM = (NW == 4) ? ((BN / 2) % 16 ? 4 : 2) : (BM > BN ? 4 : 2);
+  static constexpr int WGM = (NW == 4) ? 2 : (BM > BN ? 4 : 2);  // wave grid
   static constexpr int WGN = NW / WGM;
   static constexpr int WTM = BM / WGM, WTN = BN / WGN;            // wave tile
   // MFMA shape: 16x16 (x32 for 16-bit, x64 for int8).  With operands that toggle like real data the part runs
@@ -465,8 +464,8 @@ struct OutF16 {
   static __device__ __forceinline__ raw cvt(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
 };
 // binary32 output of a 16-bit-float GEMM: the accumulator as it is.  It is what lets a float32 product run on the
-// bf16 matrix instructions as a three-term split (the host side cuts each operand into a bf16 head and a bf16 tail
-// and lays the terms out along K); built for the tiles up to 128x128 (f32_out_tile).
+// bf16 matrix instructions as a three-term split (each operand is cut into a bf16 head and a bf16 tail); built for the
+// tiles up to 128x128 (f32_out_tile), for the head-and-tail kernels of any width (PAIR) and for conv2d's.
 struct OutF32 {
   typedef float raw;
   static __device__ __forceinline__ raw cvt(float v) { return v; }

@@ -6,8 +6,7 @@ str_w, pad_h, pad_w, dil_h, dil_w, GEMM_M, GEMM_N, GEMM_K, BLOCK_SIZE_M=, BLOCK_
 GROUP_SIZE_M=, OUT_DTYPE=, USE_TF32=)`` keep the argument order and meaning of
 tritonix/ops/conv2d/forward.py:19-48 and :202-311; both end in one ``tnx_conv2d_forward`` through the C ABI on
 torch's current stream.  Float16 and bfloat16 are built; float32 tensors (the reference convolves them in TF32,
-which gfx950 has no matrix instruction for) run as a three-term bf16 convolution over 3 c_in channels with an fp32
-result.  Where no tile is named the library may copy the operands into a channels-last layout first and run the
+which gfx950 has no matrix instruction for) run as a three-term bf16 convolution with an fp32 result.  Where no tile is named the library may copy the operands into a channels-last layout first and run the
 k-contiguous GEMM kernel over that (``tnx_conv2d_workspace_bytes``; the scratch is allocated here, per call); float32
 operands are cut into their terms by that copy, or by ``_split_f32`` for the kernels that do not take it.
 """
@@ -77,8 +76,8 @@ def _raise_for_status(status: int, a: _C.Conv2dArgs) -> None:
     lib = _C.load()
     if status == _C.E_UNSUPPORTED:
         if a.dtype == _C.F32:
-            raise NotImplementedError("conv2d_forward is built for float16 and bfloat16; float32 (TF32) input has no "
-                                      "matrix instruction on gfx950")
+            raise NotImplementedError("conv2d_forward: this float32 problem is past what the packed kernels address; split along "
+                                      "the channels it runs as a bfloat16 one")
         raise ValueError(f"{_C.strerror(status)}: conv2d dtype={a.dtype} BLOCK_SIZE_M={a.block_pixels} "
                          f"BLOCK_SIZE_N={a.block_cout} BLOCK_SIZE_K={a.block_k}")
     if status == _C.E_LDS:
