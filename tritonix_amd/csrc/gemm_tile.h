@@ -137,6 +137,8 @@ struct GemmParams {
   int atomic_reduce;      // split-K: slices are added into one fp32/int32 copy with device-scope atomics instead of being kept apart
   int batch;              // uncut, non-persistent launches of tiles up to 128x128: the grid holds `batch` problems that share A (0 or 1: one problem);
   int64_t b_batch_bytes, c_batch_bytes;   // problem i reads B + i * b_batch_bytes and writes C + i * c_batch_bytes
+  FastDiv div_tiles, div_cut;             // by tiles_m * tiles_n and by the number of cut tiles
+  FastDiv div_group, div_rows, div_rows_last;   // by group_m * tiles_n, by the rows of a group and by those of the last, shorter one
   ConvGeom cv;            // read by the CONV kernels; cv.bias / cv.bias_dtype also by the plain epilogue (a bias per row of C)
   PackGeom pk;            // read by the GATHER kernels (with cv's output side)
 };
@@ -216,6 +218,32 @@ __host__ __device__ inline void swizzle2d(int i, int j, int size_i, int size_j, 
   int r = ij % size_gj;
   *oi = off_i + r % g;
   *oj = r / g;
+}
+
+// The divisors of the tile-id arithmetic, filled in by the launch.  Five divisions by run-time numbers, one after another
+// and 30 instructions each, stood before a workgroup's first load (0.1 us of a launch of 64x64 tiles).
+inline void set_order_divisors(GemmParams* p) {
+  const int64_t tiles = (int64_t)p->tiles_m * p->tiles_n, cut = tiles - p->split_tile0;
+  const int last = p->tiles_m % p->group_m;
+  p->div_tiles = make_fastdiv((uint32_t)tiles);
+  p->div_cut = make_fastdiv((uint32_t)(cut > 0 ? cut : 1));
+  // (a group of more tiles than the grid has is the only group: no tile id reaches the divisor)
+  const int64_t group = (int64_t)p->group_m * p->tiles_n;
+  p->div_group = make_fastdiv((uint32_t)(group < 0x7fffffff ? group : 0x7fffffff));
+  p->div_rows = make_fastdiv((uint32_t)p->group_m);
+  p->div_rows_last = make_fastdiv((uint32_t)(last ? last : p->group_m));
+}
+// swizzle2d of tile id `ij` by these divisors (the same map)
+__device__ __forceinline__ void swizzle2d(int ij, const GemmParams& p, int* oi, int* oj) {
+  const int group_id = (int)fd_div((uint32_t)ij, p.div_group);
+  const int off_i = group_id * p.group_m;
+  const bool last = p.tiles_m - off_i < p.group_m;
+  const int g = last ? p.tiles_m - off_i : p.group_m;
+  const int r = ij - group_id * p.group_m * p.tiles_n;
+  const FastDiv d = last ? p.div_rows_last : p.div_rows;
+  const int q = (int)fd_div((uint32_t)r, d);
+  *oi = off_i + r - q * g;
+  *oj = q;
 }
 
 // Chip-level tile order for grids much larger than the CU count.  The 256 workgroups that run
@@ -354,9 +382,18 @@ __device__ __forceinline__ float quad_swap1(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
 }
 
-__device__ __forceinline__ float glu_gate(float g, int epi) {
+// ROUNDED: the result is rounded to 16 bits, so the reciprocal instruction (1 ulp of binary32) takes the place of the
+// division and its eleven instructions; arguments past 2^96 are scaled, since its subnormal results are flushed.
+template <bool ROUNDED> __device__ __forceinline__ float glu_gate(float g, int epi) {
   if (epi == EPI_GLU_IDENTITY) return g;
-  float s = 1.0f / (1.0f + __expf(-g));
+  const float d = 1.0f + __expf(-g);
+  float s;
+  if constexpr (ROUNDED) {
+    const float c = d > 0x1p96f ? 0x1p-32f : 1.0f;
+    s = __builtin_amdgcn_rcpf(d * c) * c;
+  } else {
+    s = 1.0f / d;
+  }
   return epi == EPI_GLU_SILU ? g * s : s;
 }
 
@@ -452,6 +489,10 @@ struct TileCfg {
   }
 };
 
+template <class X> struct TypeTag { typedef X type; };
+template <bool B> struct BoolTag { static constexpr bool value = B; };
+template <int V> struct IntTag { static constexpr int value = V; };
+
 // ---------------------------------------------------------------------------
 // output conversion and the store of a wave's accumulators
 // ---------------------------------------------------------------------------
@@ -476,16 +517,32 @@ template <> struct OutOf<TagF16> { typedef OutF16 type; };
 template <> struct OutOf<TagI8> { typedef int type; };
 
 
-// LDS one wave needs to pass one row-block (MI rows) of its accumulators through LDS: raw
-// 32-bit values, rows padded by 16 bytes to spread the banks.
+// LDS one wave needs to pass one row-block (MI rows) of its outputs through LDS: up to 32 bits per accumulator, rows
+// padded by 16 bytes to spread the banks.
 template <class C> struct EpiStage {
   static constexpr int PITCH = C::WTN * 4 + 16;
-  // row-blocks per pass.  Two (32 rows per pass, half as many passes) was measured on the gated 4096x28672x4096
-  // problem and lost 2-3 %: the longer read-back of a pass delays the first stores.
-  static constexpr int RB = 1;
-  static constexpr int ROWS = RB * C::MI;
+  static constexpr int ROWS = C::MI;
   static constexpr int WAVE_BYTES = ROWS * PITCH;
   static constexpr int BYTES = C::NW * WAVE_BYTES;
+};
+
+// Outputs of four accumulators of one row (four consecutive columns; GLU: two gate / linear pairs), as they go to the strip.
+template <class O, class S, bool GLU> struct Quad;
+template <class O, bool GLU> struct Quad<O, float, GLU> {
+  typedef typename O::raw raw;
+  static constexpr int N = GLU ? 2 : 4;
+  typedef raw vec __attribute__((ext_vector_type(N)));
+  static __device__ __forceinline__ vec run(float a, float b, float c, float d, int epi) {
+    constexpr bool ROUNDED = sizeof(raw) == 2;
+    if constexpr (GLU) return vec{O::cvt(glu_gate<ROUNDED>(a, epi) * b), O::cvt(glu_gate<ROUNDED>(c, epi) * d)};
+    else return vec{O::cvt(a), O::cvt(b), O::cvt(c), O::cvt(d)};
+  }
+};
+template <bool GLU> struct Quad<int, int, GLU> {
+  typedef int raw;
+  static constexpr int N = 4;
+  typedef int vec __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ vec run(int a, int b, int c, int d, int) { return vec{a, b, c, d}; }
 };
 
 // 16 bytes of output from NF accumulator values that sit row-major in LDS.
@@ -496,7 +553,7 @@ template <class O, bool GLU> struct Pack16<O, float, GLU> {   // 16-bit float ou
   static constexpr int OUTV = 8, NF = GLU ? 16 : 8;
   static __device__ __forceinline__ void run(const float* f, int epi, raw* out) {
 #pragma unroll
-    for (int x = 0; x < OUTV; ++x) out[x] = O::cvt(GLU ? glu_gate(f[2 * x], epi) * f[2 * x + 1] : f[x]);
+    for (int x = 0; x < OUTV; ++x) out[x] = O::cvt(GLU ? glu_gate<true>(f[2 * x], epi) * f[2 * x + 1] : f[x]);
   }
 };
 template <bool GLU> struct Pack16<OutF32, float, GLU> {       // binary32 outputs: 4 per lane
@@ -504,7 +561,7 @@ template <bool GLU> struct Pack16<OutF32, float, GLU> {       // binary32 output
   static constexpr int OUTV = 4, NF = GLU ? 8 : 4;
   static __device__ __forceinline__ void run(const float* f, int epi, raw* out) {
 #pragma unroll
-    for (int x = 0; x < OUTV; ++x) out[x] = GLU ? glu_gate(f[2 * x], epi) * f[2 * x + 1] : f[x];
+    for (int x = 0; x < OUTV; ++x) out[x] = GLU ? glu_gate<false>(f[2 * x], epi) * f[2 * x + 1] : f[x];
   }
 };
 template <bool GLU> struct Pack16<int, int, GLU> {            // int32 outputs: 4 per lane
@@ -527,56 +584,67 @@ struct SliceSrc {
   bool rezero;             // atomic reduction: the one slice holds the finished sums; it is cleared again after the read
 };
 
-// Sum of the split-K slices of one row-block of a wave, group by group, into the wave's LDS
-// strip (same places the accumulators of an uncut tile go).  ZB slices of G = 32 / ZB groups
-// are fetched together; slices are added in slice order whatever ZB is.
-// largest batch of groups <= cap that divides the nq groups of a row-block (nq is 6 for the 192-wide tiles)
-constexpr int slice_batch(int nq, int cap) {
-  int g = cap < nq ? cap : nq;
-  while (nq % g) --g;
+// largest divisor of n that is <= cap
+constexpr int slice_batch(int n, int cap) {
+  int g = cap < n ? cap : n;
+  while (n % g) --g;
   return g;
 }
-template <class ACC4, int ZB, int NQ, int MI, int NGRP>
-__device__ __forceinline__ void sum_slices(__amdgpu_buffer_rsrc_t win, uint32_t q0, const SliceSrc& src, uint32_t wbase,
-                                           bool row_ok) {
-  constexpr int G = slice_batch(NQ, 32 / ZB);
-  static_assert(NQ % G == 0, "groups per row-block must be a multiple of the batch");
-#pragma unroll 1
-  for (int jg0 = 0; jg0 < NQ; jg0 += G) {
-    ACC4 v[G];
+
+// The split-K slices of one wave's part of a tile, added in slice order into the accumulators (which an uncut tile
+// would hold there), whatever workgroup does it.  Bound by the latency of device-scope loads and, from 64 KiB of slices on,
+// by the 64 bytes per cycle a CU takes in: ZB slices of CG groups, 16 to 32 loads per lane, are in flight together, across
+// row-blocks, and nothing is loaded past the last slice or row-block (a load from an empty window costs as much).
+template <class C, class ACC>
+__device__ __forceinline__ void collect_slices(ACC (&acc)[C::TM][C::TN], const SliceSrc& src, int lane, int64_t rows_left) {
+  constexpr int NGRP = C::ACC_N / 4, NQ = C::TN * NGRP, G = C::TM * NQ;
+  constexpr int CG = slice_batch(G, G == 32 ? 8 : 16), ZB = G > 8 ? 2 : G == 8 ? 4 : 8;
+  typedef std::remove_reference_t<decltype(acc[0][0][0])> acc_s;
+  typedef acc_s acc4 __attribute__((ext_vector_type(4)));
+  const __amdgpu_buffer_rsrc_t win = agent_window(src.base);
+  const int row_blocks = rows_left >= C::WTM ? C::TM : (int)((rows_left + C::MI - 1) / C::MI);
 #pragma unroll
-    for (int x = 0; x < G; ++x) v[x] = ACC4{0, 0, 0, 0};
-    // lanes whose row lies past the last row of the problem were not stored and are not read
-#pragma unroll 1
-    for (int z0 = 0; row_ok && z0 < src.nslices; z0 += ZB) {
-      i32x4 w[G * ZB];
+  for (int c0 = 0; c0 < G; c0 += CG) {
+    acc4 v[CG];
 #pragma unroll
-      for (int x = 0; x < G; ++x)
+    for (int x = 0; x < CG; ++x) v[x] = acc4{0, 0, 0, 0};
+    if (c0 / NQ < row_blocks) {
+#pragma unroll 1
+      for (int z0 = 0; z0 < src.nslices; z0 += ZB) {
+        i32x4 w[ZB * CG];
 #pragma unroll
         for (int u = 0; u < ZB; ++u) {
-          const int z = z0 + u < src.nslices ? z0 + u : src.nslices - 1;
-          w[x * ZB + u] = load16_agent(win, q0 + (uint32_t)(jg0 + x) * 1024u + (uint32_t)z * src.slice_stride);
+          if (z0 + u >= src.nslices) break;
+#pragma unroll
+          for (int x = 0; x < CG; ++x) {
+            // (row-block by row-block in the tiles of few groups; a branch more in the others keeps the compiler from
+            // having the loads in flight together at all)
+            if (G <= 8 && (c0 + x) / NQ >= row_blocks) break;
+            w[u * CG + x] = load16_agent(win, (uint32_t)lane * 16u + (uint32_t)(c0 + x) * 1024u + (uint32_t)(z0 + u) * src.slice_stride);
+          }
         }
-      if (src.rezero) {
-        // atomic reduction: what was just read is the sum; leave zeros behind for the next launch
 #pragma unroll
-        for (int x = 0; x < G; ++x) store16_agent(win, q0 + (uint32_t)(jg0 + x) * 1024u, i32x4{0, 0, 0, 0});
-      }
+        for (int u = 0; u < ZB; ++u) {
+          if (z0 + u >= src.nslices) break;
 #pragma unroll
-      for (int x = 0; x < G; ++x)
-#pragma unroll
-        for (int u = 0; u < ZB; ++u)
-          if (z0 + u < src.nslices) {
-            ACC4 t;
-            __builtin_memcpy(&t, &w[x * ZB + u], 16);
+          for (int x = 0; x < CG; ++x) {
+            acc4 t;
+            __builtin_memcpy(&t, &w[u * CG + x], 16);
             v[x] += t;
           }
+        }
+      }
     }
 #pragma unroll
-    for (int x = 0; x < G; ++x) {
-      const int j = (jg0 + x) / NGRP, g = (jg0 + x) % NGRP;
-      *TNX_LDS(ACC4, wbase + (j * MI + g * 8) * 4) = v[x];
-    }
+    for (int x = 0; x < CG; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[(c0 + x) / NQ][(c0 + x) % NQ / NGRP][(c0 + x) % NGRP * 4 + e] = v[x][e];
+  }
+  if (src.rezero) {
+    // atomic reduction: what was just read is the sum; leave zeros behind for the next launch
+    TNX_WAIT_VM(0);
+#pragma unroll 1
+    for (int q = 0; q < G; ++q) store16_agent(win, (uint32_t)lane * 16u + (uint32_t)q * 1024u, i32x4{0, 0, 0, 0});
   }
 }
 
@@ -590,133 +658,122 @@ __device__ __forceinline__ float bias_value(const uint8_t* bias, int row, int dt
   return __builtin_bit_cast(float, (uint32_t)((const uint16_t*)bias)[row] << 16);
 }
 
+// How the lanes of a wave share the 16-byte output chunks of one row-block (ROWS rows of CPRW chunks each), 64 chunks per
+// pass.  EVEN: a lane's chunk column is the same in every pass and its row RSTEP further on.
+template <int ROWS, int CPRW> struct RowPasses {
+  static constexpr int ITERS = (ROWS * CPRW + 63) / 64;
+  static constexpr bool EVEN = 64 % CPRW == 0;
+  static constexpr int RSTEP = EVEN ? 64 / CPRW : 0;
+  static constexpr int NL = EVEN ? 1 : ITERS;           // distinct (row, column) places of a lane
+  // passes whose LDS reads are in flight together; the rest, if any, in a rolled loop where the places allow it
+  static constexpr int UNR = ITERS <= 4 ? ITERS : (ITERS % 4 == 0 ? 4 : ITERS % 3 == 0 ? 3 : ITERS % 2 == 0 ? 2 : 1);
+};
+
 // The MFMA result is C^T: lane l owns output row m = l % MI and, per group of four accumulator
 // registers, four consecutive columns n.  Each wave passes one row-block at a time through its
-// private LDS strip: raw accumulators in (one ds_write_b128 per group), then a plain loop reads
-// the strip row-major, converts / gates, and stores 16 bytes per lane, so every row of C
-// receives full contiguous runs.  Keeping the conversion out of the unrolled part keeps the
-// epilogue variants of a 256x256 tile inside the instruction cache.
-// FROM_WS: the values do not come from this wave's registers but from the split-K slices in
-// the workspace, added in slice order (the result does not depend on which workgroup does it).
-template <class T, class C, class O, bool GLU, bool FROM_WS, bool BIAS = false, class ACC>
-__device__ __forceinline__ void epilogue_store(ACC (&acc)[C::TM][C::TN], const SliceSrc& src, uint8_t* cbase,
-                                               uint32_t lds_strip, int lane, int64_t gm0, int64_t gc0, int64_t m,
-                                               int64_t ncols, int64_t scm, int64_t scn, bool vec_ok, int epi,
-                                               const uint8_t* bias = nullptr, int bias_dtype = 0) {
+// private LDS strip: gated and rounded outputs in (one write per group), then the strip is read
+// row-major and stored 16 bytes per lane, so every row of C receives full contiguous runs.
+// Bound, on launches of a round or two of tiles, by its own instructions and LDS traffic: so the outputs are rounded before
+// the strip (half the bytes, a quarter for a gated pair), a lane's place in C and in the strip is worked out once, a pass
+// adds a scalar, and the next row-block is written to the strip behind the reads of the present one, before its stores
+// (a wave's LDS operations are carried out in order: no wait is needed between them).  Sums through the strip, rounded
+// after it, with every address worked out anew: 4 tiles of 128x256 and 4 K slabs 7.7 us a launch, now 7.1; of 128x128 5.6, now 5.3;
+// the gated 4096 x 28672 x 4096 with its division by a reciprocal too (7 rounds) 1.5 % of the feed-forward block.
+template <class T, class C, class O, bool GLU, bool BIAS = false, class ACC>
+__device__ __forceinline__ void epilogue_store(ACC (&acc)[C::TM][C::TN], uint8_t* cbase, uint32_t lds_strip, int lane,
+                                               int64_t gm0, int64_t gc0, int64_t m, int64_t ncols, int64_t scm, int64_t scn,
+                                               bool vec_ok, int epi, const uint8_t* bias = nullptr, int bias_dtype = 0) {
   typedef typename T::acc_s acc_s;
-  typedef Pack16<O, acc_s, GLU> PK;
-  typedef typename PK::raw raw;
-  typedef acc_s acc4 __attribute__((ext_vector_type(4)));
+  typedef std::conditional_t<std::is_same<acc_s, int>::value, Quad<int, int, GLU>, Quad<O, acc_s, GLU>> QD;
+  typedef typename QD::raw raw;
   constexpr int MI = C::MI;
   constexpr int NGRP = C::ACC_N / 4;                    // groups of four consecutive columns per accumulator tile
-  constexpr int PITCH = EpiStage<C>::PITCH;
-  constexpr int RB = EpiStage<C>::RB, ROWS = EpiStage<C>::ROWS;   // a pass moves RB row-blocks = ROWS rows
+  constexpr int OUTV = 16 / sizeof(raw);
   constexpr int WCOLS = GLU ? C::WTN / 2 : C::WTN;      // output columns of the wave tile
-  constexpr int CPRW = WCOLS / PK::OUTV;                // 16-byte output chunks per strip row
-  constexpr int ITERS = (ROWS * CPRW + 63) / 64;
-  constexpr int UNR = ITERS % 4 == 0 ? 4 : (ITERS % 2 == 0 ? 2 : 1);   // read-back rows in flight together
-  static_assert(WCOLS % PK::OUTV == 0, "wave tile too narrow for 16-byte stores");
-  raw* cp = (raw*)cbase;
-  const uint32_t wbase0 = lds_strip + (lane % MI) * PITCH + (lane / MI) * 16;
-  // A bias per row of C (conv2d's 1x1 layers): lane l fetches the values of rows l, l + 64, .. of the wave tile now,
-  // so that the loads fly under the first pass through the strip; the row loop below picks its value from the lane that holds it.
+  constexpr int PITCH = WCOLS * sizeof(raw) + 16;
+  constexpr int CPRW = WCOLS / OUTV;                    // 16-byte output chunks per strip row
+  typedef RowPasses<MI, CPRW> RP;
+  static_assert(WCOLS % OUTV == 0, "wave tile too narrow for 16-byte stores");
+  static_assert(PITCH <= EpiStage<C>::PITCH, "strip too small");
+  const uint32_t wbase = lds_strip + (lane % MI) * PITCH + (lane / MI) * (QD::N * sizeof(raw));
+  if (gm0 >= m) return;
+  const int rows_left = m - gm0 < C::WTM ? (int)(m - gm0) : C::WTM;
+  // A bias per row of C (conv2d's 1x1 layers): a lane's row in every row-block is lane % MI.
   constexpr bool WITH_BIAS = BIAS && std::is_same<acc_s, float>::value && !GLU;
-  constexpr int NBR = (C::WTM + 63) / 64;
-  float bias_rows[NBR] = {};
+  float bias_rows[WITH_BIAS ? C::TM : 1] = {};
   if constexpr (WITH_BIAS) {
     if (bias) {
 #pragma unroll
-      for (int r = 0; r < NBR; ++r) {
-        const int64_t g = gm0 + r * 64 + lane;
-        if (r * 64 + lane < C::WTM && g < m) bias_rows[r] = bias_value(bias, (int)g, bias_dtype);
-      }
+      for (int i = 0; i < C::TM; ++i)
+        if (i * MI + lane % MI < rows_left) bias_rows[i] = bias_value(bias, (int)gm0 + i * MI + lane % MI, bias_dtype);
     }
   }
+  // this lane's places: row of the row-block, columns of the chunk that exist, strip address, address in C
+  int l_row[RP::NL], l_cols[RP::NL];
+  uint32_t l_lds[RP::NL];
+  raw* l_dst[RP::NL];
 #pragma unroll
-  for (int i0 = 0; i0 < C::TM; i0 += RB) {
-    if (gm0 + i0 * MI >= m) break;                      // row-blocks past the last row hold nothing
+  for (int t = 0; t < RP::NL; ++t) {
+    const int q = t * 64 + lane, row = q / CPRW, cc = q % CPRW;
+    const int64_t left = ncols - (gc0 + cc * OUTV);
+    const bool idle = MI * CPRW % 64 != 0 && row >= MI;
+    l_row[t] = row;
+    l_cols[t] = idle || left <= 0 ? 0 : left < OUTV ? (int)left : OUTV;
+    l_lds[t] = lds_strip + (idle ? MI - 1 : row) * PITCH + cc * 16;
+    l_dst[t] = (raw*)cbase + (gm0 + row) * scm + (gc0 + cc * OUTV) * scn;
+  }
+  auto put = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-    for (int ii = 0; ii < RB; ++ii) {
-      const int i = i0 + ii;
-      const uint32_t wbase = wbase0 + ii * MI * PITCH;
-      if constexpr (!FROM_WS) {
+    for (int j = 0; j < C::TN; ++j)
 #pragma unroll
-        for (int j = 0; j < C::TN; ++j)
+      for (int g = 0; g < NGRP; ++g) {
+        acc_s v[4] = {acc[i][j][4 * g + 0], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+        if constexpr (WITH_BIAS) {                      // added to the finished fp32 sum before the one rounding
 #pragma unroll
-          for (int g = 0; g < NGRP; ++g)
-            // (typed vector store: __builtin_bit_cast on an ext-vector element reads element 0)
-            *TNX_LDS(acc4, wbase + (j * MI + g * 8) * 4) =
-                acc4{acc[i][j][4 * g + 0], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-      } else {
-        // 32 loads per lane in flight (G groups x ZB slices): the hand-over is latency-bound otherwise
-        const __amdgpu_buffer_rsrc_t win = agent_window(src.base);
-        const uint32_t q0 = (uint32_t)i * (C::TN * NGRP) * 1024u + lane * 16u;
-        const bool row_ok = gm0 + i * MI + lane % MI < m;
-        if (src.nslices <= 2)
-          sum_slices<acc4, 2, C::TN * NGRP, MI, NGRP>(win, q0, src, wbase, row_ok);
-        else if (src.nslices <= 4)
-          sum_slices<acc4, 4, C::TN * NGRP, MI, NGRP>(win, q0, src, wbase, row_ok);
-        else
-          sum_slices<acc4, 8, C::TN * NGRP, MI, NGRP>(win, q0, src, wbase, row_ok);
+          for (int e = 0; e < 4; ++e) v[e] += bias_rows[i];
+        }
+        // (typed vector store: __builtin_bit_cast on an ext-vector element reads element 0)
+        *TNX_LDS(typename QD::vec, wbase + (j * MI + g * 8) * (QD::N * sizeof(raw) / 4)) = QD::run(v[0], v[1], v[2], v[3], epi);
       }
-    }
-    // the strip is private to this wave: its own LDS writes are ordered before its reads
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-#pragma unroll 1
-    for (int it0 = 0; it0 < ITERS; it0 += UNR) {
-      // UNR rows of LDS reads are issued together, then converted and stored one after the other
-      acc_s f[UNR][PK::NF];
-      float bv[UNR] = {};
+  };
+  put(0);
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        const int q = (it0 + u) * 64 + lane;
-        int row = q / CPRW;
-        const int cc = q % CPRW;
-        if (ROWS * CPRW % 64 != 0 && row >= ROWS) row = ROWS - 1;
-        if constexpr (WITH_BIAS) {
-          const int rt = i0 * MI + row;                 // row of the wave tile: held by lane rt % 64 in bias_rows[rt / 64]
-          if (bias)
+  for (int i = 0; i < C::TM; ++i) {
+    if (i * MI >= rows_left) break;                     // row-blocks past the last row hold nothing
+    // UNR passes from `it0` on: strip reads together, then one store after the other
+    auto passes = [&](int it0, auto last) __attribute__((always_inline)) {
+      i32x4 v[RP::UNR];
 #pragma unroll
-          for (int r = 0; r < NBR; ++r) {
-            const float t = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((rt & 63) * 4, __builtin_bit_cast(int, bias_rows[r])));
-            if ((rt >> 6) == r) bv[u] = t;
-          }
-        }
+      for (int u = 0; u < RP::UNR; ++u)
+        v[u] = *TNX_LDS(i32x4, l_lds[RP::EVEN ? 0 : it0 + u] + (RP::EVEN ? (it0 + u) * RP::RSTEP : 0) * PITCH);
+      if constexpr (decltype(last)::value)
+        if (i + 1 < C::TM) put(i + 1 < C::TM ? i + 1 : i);
 #pragma unroll
-        for (int x = 0; x < PK::NF / 4; ++x) {
-          const i32x4 v = *TNX_LDS(i32x4, lds_strip + row * PITCH + (cc * PK::NF + 4 * x) * 4);
-          __builtin_memcpy(&f[u][4 * x], &v, 16);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        const int q = (it0 + u) * 64 + lane;
-        const int row = q / CPRW, cc = q % CPRW;
-        const int64_t gm = gm0 + i0 * MI + row;
-        const int64_t gc = gc0 + cc * PK::OUTV;
-        if ((ROWS * CPRW % 64 != 0 && row >= ROWS) || gm >= m) continue;
-        if constexpr (WITH_BIAS) {
-          // added to the finished fp32 sum before the one rounding
-          if (bias)
-#pragma unroll
-            for (int x = 0; x < PK::NF; ++x) f[u][x] += bv[u];
-        }
-        raw out[PK::OUTV];
-        PK::run(f[u], epi, out);
-        raw* dst = cp + gm * scm + gc * scn;
-        if (vec_ok && gc + PK::OUTV <= ncols) {
-          i32x4 v;
-          __builtin_memcpy(&v, out, 16);
-          store16_stream_loose(dst, v);                 // rows of C need not be 16-byte aligned
+      for (int u = 0; u < RP::UNR; ++u) {
+        const int t = RP::EVEN ? 0 : it0 + u, step = RP::EVEN ? (it0 + u) * RP::RSTEP : 0;
+        if (l_row[t] >= rows_left - (i * MI + step) || l_cols[t] == 0) continue;
+        raw* dst = l_dst[t] + (int64_t)(i * MI + step) * scm;
+        if (vec_ok && l_cols[t] == OUTV) {
+          store16_stream_loose(dst, v[u]);              // rows of C need not be 16-byte aligned
         } else {
+          raw out[OUTV];
+          __builtin_memcpy(out, &v[u], 16);
 #pragma unroll 1
-          for (int x = 0; x < PK::OUTV; ++x)
-            if (gc + x < ncols) dst[x * scn] = out[x];
+          for (int x = 0; x < l_cols[t]; ++x) dst[x * scn] = out[x];
         }
       }
+    };
+    if constexpr (RP::ITERS == RP::UNR) {
+      passes(0, BoolTag<true>{});
+    } else if constexpr (RP::EVEN) {
+#pragma unroll 1
+      for (int it0 = 0; it0 < RP::ITERS; it0 += RP::UNR) passes(it0, BoolTag<false>{});
+      if (i + 1 < C::TM) put(i + 1 < C::TM ? i + 1 : i);
+    } else {
+#pragma unroll
+      for (int it0 = 0; it0 < RP::ITERS; it0 += RP::UNR) passes(it0, BoolTag<false>{});
+      if (i + 1 < C::TM) put(i + 1 < C::TM ? i + 1 : i);
     }
-    // the next pass overwrites the strip: wait for the reads above
-    __builtin_amdgcn_s_waitcnt(0xC07F);
   }
 }
 
@@ -823,9 +880,10 @@ constexpr int WS_MAX_TILES = WS_COUNTER_BYTES / 4;
 // all slices back with device-scope loads and runs the ordinary epilogue on their sum.
 // Whole-L2 write-backs and invalidates (what a device-scope fence costs on a part with eight
 // L2s) are avoided on purpose: they cost more than the GEMM.
-template <class T, class C, class ACC>
-__device__ __forceinline__ bool splitk_arrive(ACC (&acc)[C::TM][C::TN], uint8_t* wave_slice, uint32_t lds_strip, int lane,
-                                              int64_t gm0, int64_t m, int* counter, int* flag, int nslices, bool atomic) {
+// FLAG_APART: the flag's LDS word is not part of the epilogue strips that are written next.
+template <class T, class C, bool FLAG_APART, class ACC>
+__device__ __forceinline__ bool splitk_arrive(ACC (&acc)[C::TM][C::TN], uint8_t* wave_slice, int lane, int64_t gm0, int64_t m,
+                                              int* counter, int* flag, int nslices, bool atomic) {
   typedef typename T::acc_s acc_s;
   typedef acc_s acc4 __attribute__((ext_vector_type(4)));
   constexpr int NGRP = C::ACC_N / 4;
@@ -834,37 +892,29 @@ __device__ __forceinline__ bool splitk_arrive(ACC (&acc)[C::TM][C::TN], uint8_t*
 #pragma unroll
   for (int i = 0; i < C::TM; ++i) {
     if (gm0 + i * C::MI >= m) break;
+    if (gm0 + i * C::MI + lane % C::MI >= m) continue;   // a lane is one row: rows past the problem are not stored
     if (atomic) {
       // every slice adds into the same copy (wave_slice is slice 0 for all of them); same element order as a stored slice
-      if (gm0 + i * C::MI + lane % C::MI < m) {
-        acc_s* dst = (acc_s*)(wave_slice + (int64_t)i * NQ * 1024 + lane * 16);
+      acc_s* dst = (acc_s*)(wave_slice + (int64_t)i * NQ * 1024 + lane * 16);
 #pragma unroll
-        for (int j = 0; j < C::TN; ++j)
+      for (int j = 0; j < C::TN; ++j)
 #pragma unroll
-          for (int g = 0; g < NGRP; ++g)
+        for (int g = 0; g < NGRP; ++g)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              __hip_atomic_fetch_add(dst + (j * NGRP + g) * 256 + e, acc[i][j][4 * g + e], __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
-      }
-      continue;
+          for (int e = 0; e < 4; ++e)
+            __hip_atomic_fetch_add(dst + (j * NGRP + g) * 256 + e, acc[i][j][4 * g + e], __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+#pragma unroll
+      for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+        for (int g = 0; g < NGRP; ++g) {
+          const acc4 v = {acc[i][j][4 * g + 0], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+          i32x4 w;
+          __builtin_memcpy(&w, &v, 16);
+          store16_agent(win, (uint32_t)lane * 16u + (uint32_t)(i * NQ + j * NGRP + g) * 1024u, w);
+        }
     }
-    // registers -> LDS -> registers keeps the copy loop rolled (the accumulators may sit in AGPRs,
-    // which a 16-byte device-scope store cannot name directly)
-#pragma unroll
-    for (int j = 0; j < C::TN; ++j)
-#pragma unroll
-      for (int g = 0; g < NGRP; ++g)
-        *TNX_LDS(acc4, lds_strip + (j * NGRP + g) * 1024 + lane * 16) =
-            acc4{acc[i][j][4 * g + 0], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    const uint32_t dst = (uint32_t)i * NQ * 1024u + lane * 16u;
-    if (gm0 + i * C::MI + lane % C::MI < m) {            // a lane is one row: rows past the problem are not stored
-#pragma unroll 4
-      for (int q = 0; q < NQ; ++q)
-        store16_agent(win, dst + q * 1024u, *TNX_LDS(i32x4, lds_strip + q * 1024 + lane * 16));
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
   }
   // device-scope stores: once they are acknowledged they are visible to every XCD, so the
   // arrival count may follow
@@ -878,7 +928,7 @@ __device__ __forceinline__ bool splitk_arrive(ACC (&acc)[C::TM][C::TN], uint8_t*
   }
   __syncthreads();
   const bool last = *flag == nslices - 1;
-  __syncthreads();                                      // the flag's LDS word is reused by the epilogue strips
+  if constexpr (!FLAG_APART) __syncthreads();
   return last;
 }
 
@@ -889,103 +939,96 @@ struct __attribute__((packed, aligned(2))) Loose16 {
 
 
 // Epilogue of the CONV kernels: rows are output channels, columns are pixels of the padded pixel index space.  Same
-// pass through the wave's LDS strip as epilogue_store; a 16-byte chunk is 8 pixels of one output row, so it is one
-// run of the NCHW output (cut at w_out: the pixels past it exist only in the index space).  Bias is added in fp32.
-// FROM_WS: the values are the sum of the split-K slices in the workspace, as in epilogue_store.
-template <class T, class C, class O, bool FROM_WS = false, class ACC>
+// pass through the wave's LDS strip as epilogue_store; a chunk is 8 pixels of one output row, so it is one
+// run of the NCHW output (cut at w_out: the pixels past it exist only in the index space).  Bias is added in fp32; it is
+// fetched up front (a load per row-block in the middle of the loop put a memory round trip on each of up to eight), and
+// a chunk's place in the output is worked out once per lane.
+template <class T, class C, class O, class ACC>
 __device__ __forceinline__ void epilogue_store_conv(ACC (&acc)[C::TM][C::TN], uint8_t* ybase, uint32_t lds_strip, int lane,
-                                                    int gm0, int gn0, const ConvGeom& g, const SliceSrc& src = SliceSrc{nullptr, 0, 0, false}) {
+                                                    int gm0, int gn0, const ConvGeom& g) {
+  typedef Quad<O, float, false> QD;
   typedef typename O::raw raw;                          // 16-bit outputs, or binary32 (the fp32 sums + bias as they are)
-  typedef float acc4 __attribute__((ext_vector_type(4)));
   constexpr int MI = C::MI;
   constexpr int NGRP = C::ACC_N / 4;
-  constexpr int PITCH = EpiStage<C>::PITCH;
-  constexpr int ROWS = EpiStage<C>::ROWS;
+  constexpr int PITCH = C::WTN * sizeof(raw) + 16;
   constexpr int CPRW = C::WTN / 8;                       // a lane handles 8 pixels: one 16-byte chunk of the im2col slab
-  constexpr int ITERS = (ROWS * CPRW + 63) / 64;
-  constexpr int UNR = ITERS % 4 == 0 ? 4 : ITERS <= 7 ? ITERS : (ITERS % 2 == 0 ? 2 : 1);
-  static_assert(EpiStage<C>::RB == 1 && C::WTN % 8 == 0, "one row-block per pass, 8 outputs per chunk");
-  raw* yp = (raw*)ybase;
-  const uint32_t wbase = lds_strip + (lane % MI) * PITCH + (lane / MI) * 16;
+  typedef RowPasses<MI, CPRW> RP;
+  static_assert(PITCH <= EpiStage<C>::PITCH && C::WTN % 8 == 0 && RP::ITERS == RP::UNR, "one row-block per pass, 8 outputs per chunk");
+  const uint32_t wbase = lds_strip + (lane % MI) * PITCH + (lane / MI) * (4 * sizeof(raw));
+  if (gm0 >= g.c_out) return;
+  const int rows_left = g.c_out - gm0 < C::WTM ? g.c_out - gm0 : C::WTM;
+  float bias_rows[C::TM] = {};
+  if (g.bias) {
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i)
+      if (i * MI + lane % MI < rows_left) bias_rows[i] = bias_value(g.bias, gm0 + i * MI + lane % MI, g.bias_dtype);
+  }
+  const int64_t plane = (int64_t)g.h_out * g.w_out;
+  // this lane's places: row of the row-block, pixels of the chunk that exist, strip address, address in the output
+  int l_row[RP::NL], l_valid[RP::NL];
+  uint32_t l_lds[RP::NL];
+  raw* l_dst[RP::NL];
+#pragma unroll
+  for (int t = 0; t < RP::NL; ++t) {
+    const int q = t * 64 + lane, row = q / CPRW, cc = q % CPRW;
+    const bool idle = MI * CPRW % 64 != 0 && row >= MI;
+    const int gc = gn0 + cc * 8;
+    const int img = (int)fd_div((uint32_t)gc, g.div_hwp);
+    const int r = gc - img * (g.h_out * g.wp);
+    const int ho = (int)fd_div((uint32_t)r, g.div_wp);
+    const int wq = r - ho * g.wp;
+    const int valid = g.w_out - wq;                     // pixels of this chunk that exist
+    l_row[t] = row;
+    l_valid[t] = idle || gc >= g.n_total || valid <= 0 ? 0 : valid < 8 ? valid : 8;
+    l_lds[t] = lds_strip + (idle ? MI - 1 : row) * PITCH + cc * (8 * sizeof(raw));
+    l_dst[t] = (raw*)ybase + ((int64_t)img * g.c_out + gm0 + row) * plane + (int64_t)ho * g.w_out + wq;
+  }
+  auto put = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+      for (int q = 0; q < NGRP; ++q)
+        *TNX_LDS(typename QD::vec, wbase + (j * MI + q * 8) * sizeof(raw)) =
+            QD::run(acc[i][j][4 * q + 0] + bias_rows[i], acc[i][j][4 * q + 1] + bias_rows[i], acc[i][j][4 * q + 2] + bias_rows[i],
+                    acc[i][j][4 * q + 3] + bias_rows[i], 0);
+  };
+  put(0);
 #pragma unroll
   for (int i = 0; i < C::TM; ++i) {
-    if (gm0 + i * MI >= g.c_out) break;
-    if constexpr (!FROM_WS) {
+    if (i * MI >= rows_left) break;
+    constexpr int H = sizeof(raw) / 2;                  // 16-byte halves of a chunk
+    i32x4 v[RP::UNR][H];
 #pragma unroll
-      for (int j = 0; j < C::TN; ++j)
+    for (int u = 0; u < RP::UNR; ++u)
 #pragma unroll
-        for (int q = 0; q < NGRP; ++q)
-          *TNX_LDS(acc4, wbase + (j * MI + q * 8) * 4) =
-              acc4{acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-    } else {
-      const __amdgpu_buffer_rsrc_t win = agent_window(src.base);
-      const uint32_t q0 = (uint32_t)i * (C::TN * NGRP) * 1024u + lane * 16u;
-      const bool row_ok = gm0 + i * MI + lane % MI < g.c_out;
-      if (src.nslices <= 2) sum_slices<acc4, 2, C::TN * NGRP, MI, NGRP>(win, q0, src, wbase, row_ok);
-      else if (src.nslices <= 4) sum_slices<acc4, 4, C::TN * NGRP, MI, NGRP>(win, q0, src, wbase, row_ok);
-      else sum_slices<acc4, 8, C::TN * NGRP, MI, NGRP>(win, q0, src, wbase, row_ok);
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-#pragma unroll 1
-    for (int it0 = 0; it0 < ITERS; it0 += UNR) {
-      float f[UNR][8];
+      for (int h = 0; h < H; ++h) v[u][h] = *TNX_LDS(i32x4, l_lds[RP::EVEN ? 0 : u] + (RP::EVEN ? u * RP::RSTEP : 0) * PITCH + 16 * h);
+    if (i + 1 < C::TM) put(i + 1 < C::TM ? i + 1 : i);
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        const int q = (it0 + u) * 64 + lane;
-        int row = q / CPRW;
-        const int cc = q % CPRW;
-        if (ROWS * CPRW % 64 != 0 && row >= ROWS) row = ROWS - 1;
+    for (int u = 0; u < RP::UNR; ++u) {
+      const int t = RP::EVEN ? 0 : u, step = RP::EVEN ? u * RP::RSTEP : 0;
+      if (l_row[t] >= rows_left - (i * MI + step) || l_valid[t] == 0) continue;
+      raw* dst = l_dst[t] + (int64_t)(i * MI + step) * plane;
+      if (l_valid[t] == 8) {
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
-          const i32x4 v = *TNX_LDS(i32x4, lds_strip + row * PITCH + (cc * 8 + 4 * x) * 4);
-          __builtin_memcpy(&f[u][4 * x], &v, 16);
+        for (int h = 0; h < H; ++h) {                   // element-aligned: w_out need not be a multiple of 8
+          // binary32: the two stores of a lane interleave with its neighbours', so each fills half of every cache line;
+          // kept in the L2 the halves meet there, hinted they go out one by one (1984 channels of 17x17, batch 64:
+          // 116 -> 64 us)
+          if constexpr (H == 2) *(i32x4_loose*)((uint8_t*)dst + 16 * h) = v[u][h];
+          else store16_stream_loose(dst, v[u][h]);
         }
-      }
-#pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        const int q = (it0 + u) * 64 + lane;
-        const int row = q / CPRW, cc = q % CPRW;
-        const int gm = gm0 + i * MI + row;
-        const int gc = gn0 + cc * 8;
-        if ((ROWS * CPRW % 64 != 0 && row >= ROWS) || gm >= g.c_out || gc >= g.n_total) continue;
-        const int img = (int)fd_div((uint32_t)gc, g.div_hwp);
-        const int r = gc - img * (g.h_out * g.wp);
-        const int ho = (int)fd_div((uint32_t)r, g.div_wp);
-        const int wq = r - ho * g.wp;
-        const int valid = g.w_out - wq;              // pixels of this chunk that exist
-        if (valid <= 0) continue;
-        const float bv = g.bias ? bias_value(g.bias, gm, g.bias_dtype) : 0.0f;
+      } else {
         raw out[8];
-#pragma unroll
-        for (int x = 0; x < 8; ++x) out[x] = O::cvt(f[u][x] + bv);
-        raw* dst = yp + (((int64_t)img * g.c_out + gm) * g.h_out + ho) * g.w_out + wq;
-        if (valid >= 8) {
-          i32x4 v[sizeof(raw) / 2];
-          __builtin_memcpy(v, out, 8 * sizeof(raw));
-#pragma unroll
-          for (int h = 0; h < (int)sizeof(raw) / 2; ++h) {         // element-aligned: w_out need not be a multiple of 8
-            // binary32: the two stores of a lane interleave with its neighbours', so each fills half of every cache line;
-            // kept in the L2 the halves meet there, hinted they go out one by one (1984 channels of 17x17, batch 64:
-            // 116 -> 64 us)
-            if constexpr (sizeof(raw) == 4) *(i32x4_loose*)((uint8_t*)dst + 16 * h) = v[h];
-            else store16_stream_loose((uint8_t*)dst + 16 * h, v[h]);
-          }
-        } else {
+        __builtin_memcpy(out, v[u], 8 * sizeof(raw));
 #pragma unroll 1
-          for (int x = 0; x < valid; ++x) dst[x] = out[x];
-        }
+        for (int x = 0; x < l_valid[t]; ++x) dst[x] = out[x];
       }
     }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
   }
 }
 
 // GATHER: the table of k-chunk offsets behind the ring
 constexpr int GATHER_TABLE_BYTES = 8192;
-
-template <class X> struct TypeTag { typedef X type; };
-template <bool B> struct BoolTag { static constexpr bool value = B; };
-template <int V> struct IntTag { static constexpr int value = V; };
 
 // ---------------------------------------------------------------------------
 // the kernel
@@ -1064,7 +1107,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
       superblock_order(id, p.tiles_m, p.tiles_n, pid_m, pid_n);
     } else {
       const int lg = xcd_remap(id, ntiles, 8);
-      swizzle2d(lg / p.tiles_n, lg % p.tiles_n, p.tiles_m, p.tiles_n, p.group_m, pid_m, pid_n);
+      swizzle2d(lg, p, pid_m, pid_n);
     }
   };
   int pid_m, pid_n;
@@ -1073,7 +1116,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     if constexpr (MULTI) {
       // several problems with one A in one grid (conv2d's 1x1 layers: one per image): problem after problem
       if (p.batch > 1) {
-        const int img = bid / ntiles;
+        const int img = (int)fd_div((uint32_t)bid, p.div_tiles);
         bid -= img * ntiles;
         p.b += (int64_t)img * p.b_batch_bytes;
         p.c += (int64_t)img * p.c_batch_bytes;
@@ -1086,12 +1129,12 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
     } else {
       const int ncut = ntiles - p.split_tile0;
       int t = blockIdx.x - p.split_tile0;
-      split = t / ncut;
+      split = (int)fd_div((uint32_t)t, p.div_cut);
       t -= split * ncut;
       logical = p.split_tile0 + xcd_remap(t, ncut, 8);
       cut = true;
     }
-    swizzle2d(logical / p.tiles_n, logical % p.tiles_n, p.tiles_m, p.tiles_n, p.group_m, &pid_m, &pid_n);
+    swizzle2d(logical, p, &pid_m, &pid_n);
   }
 
   const int kt_total = (int)((p.k + BK - 1) / BK);
@@ -2120,69 +2163,47 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
       else epilogue_store_conv<T, C, O>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
       return;
     }
-    if constexpr (GATHER) {
-      auto finish_conv = [&](auto otag) __attribute__((always_inline)) {
+    // `sums`: the wave's accumulators, or what the slices of a cut tile add up to.  The output type: the input's own
+    // 16-bit type (int32 for int8), or binary32 where that epilogue is built.
+    auto finish = [&](auto& sums) __attribute__((always_inline)) {
+      auto as = [&](auto otag) __attribute__((always_inline)) {
         typedef typename decltype(otag)::type OT;
-        if (cut) {
-          const int ncut = ntiles - p.split_tile0, ctile = logical - p.split_tile0;
-          const int64_t slice_stride = (int64_t)ncut * BM * BN * 4;
-          uint8_t* wave0 = p.ws + WS_COUNTER_BYTES + ((int64_t)ctile * NW + wave) * (C::WTM * C::WTN * 4);
-          if (!splitk_arrive<T, C>(acc, wave0 + split * slice_stride, strip, lane, gm0, p.m, (int*)p.ws + ctile, (int*)smem,
-                                   p.split_k, false))
-            return;
-          epilogue_store_conv<T, C, OT, true>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv,
-                                              SliceSrc{wave0, (uint32_t)slice_stride, p.split_k, false});
-        } else {
-          epilogue_store_conv<T, C, OT>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
-        }
+        if constexpr (GATHER)
+          epilogue_store_conv<T, C, OT>(sums, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
+        else if (p.epilogue == EPI_NONE)
+          epilogue_store<T, C, OT, false, MULTI>(sums, p.c, strip, lane, gm0, gn0, p.m, p.n, p.scm, p.scn, p.c_row_ok, 0,
+                                                 p.cv.bias, p.cv.bias_dtype);
+        else
+          epilogue_store<T, C, OT, true>(sums, p.c, strip, lane, gm0, gn0 >> 1, p.m, p.n >> 1, p.scm, p.scn, p.c_row_ok,
+                                         p.epilogue);
       };
       if constexpr (PAIR) {
-        finish_conv(TypeTag<OutF32>{});
-        return;
+        as(TypeTag<OutF32>{});
+      } else if constexpr (GATHER || f32_out_tile<T, C>()) {
+        if (p.out_dtype == DT_F32) as(TypeTag<OutF32>{});
+        else as(TypeTag<O>{});
+      } else {
+        as(TypeTag<O>{});
       }
-      if (p.out_dtype == DT_F32) finish_conv(TypeTag<OutF32>{});
-      else finish_conv(TypeTag<O>{});
-      return;
-    }
-    // the output type: the input's own 16-bit type (int32 for int8), or binary32 where that epilogue is built
-    auto finish = [&](auto otag) __attribute__((always_inline)) {
-      typedef typename decltype(otag)::type OT;
+    };
+    if constexpr (!CONV) {
       if (cut) {
         // workspace after the counters: [slice][cut tile][wave][group][lane] 16-byte elements
+        constexpr bool APART = RING_OR_STRIPS >= EpiStage<C>::BYTES + 16;
         const int ncut = ntiles - p.split_tile0, ctile = logical - p.split_tile0;
         const int64_t slice_stride = (int64_t)ncut * BM * BN * 4;
         uint8_t* wave0 = p.ws + WS_COUNTER_BYTES + ((int64_t)ctile * NW + wave) * (C::WTM * C::WTN * 4);
-        const bool atomic = p.atomic_reduce != 0;
-        if (!splitk_arrive<T, C>(acc, wave0 + (atomic ? 0 : split * slice_stride), strip, lane, gm0, p.m, (int*)p.ws + ctile,
-                                 (int*)smem, p.split_k, atomic))
+        const bool atomic = !GATHER && p.atomic_reduce != 0;
+        if (!splitk_arrive<T, C, APART>(acc, wave0 + (atomic ? 0 : split * slice_stride), lane, gm0, p.m, (int*)p.ws + ctile,
+                                        (int*)(smem + (APART ? EpiStage<C>::BYTES : 0)), p.split_k, atomic))
           return;
-        const SliceSrc src = {wave0, (uint32_t)slice_stride, atomic ? 1 : p.split_k, atomic};
-        if (p.epilogue == EPI_NONE)
-          epilogue_store<T, C, OT, false, true>(acc, src, p.c, strip, lane, gm0, gn0, p.m, p.n, p.scm, p.scn, p.c_row_ok, 0);
-        else
-          epilogue_store<T, C, OT, true, true>(acc, src, p.c, strip, lane, gm0, gn0 >> 1, p.m, p.n >> 1, p.scm, p.scn,
-                                               p.c_row_ok, p.epilogue);
-      } else {
-        const SliceSrc none = {nullptr, 0, 0, false};
-        if (p.epilogue == EPI_NONE)
-          epilogue_store<T, C, OT, false, false, MULTI>(acc, none, p.c, strip, lane, gm0, gn0, p.m, p.n, p.scm, p.scn, p.c_row_ok, 0,
-                                                        p.cv.bias, p.cv.bias_dtype);
-        else
-          epilogue_store<T, C, OT, true, false>(acc, none, p.c, strip, lane, gm0, gn0 >> 1, p.m, p.n >> 1, p.scm, p.scn,
-                                                p.c_row_ok, p.epilogue);
-      }
-    };
-    if constexpr (PAIR) {
-      finish(TypeTag<OutF32>{});
-      return;
-    }
-    if constexpr (f32_out_tile<T, C>()) {
-      if (p.out_dtype == DT_F32) {
-        finish(TypeTag<OutF32>{});
+        acc_t sums[TM][TN];          // (not `acc`: two definitions that meet again spill in the tiles that use every register)
+        collect_slices<C>(sums, SliceSrc{wave0, (uint32_t)slice_stride, atomic ? 1 : p.split_k, atomic}, lane, p.m - gm0);
+        finish(sums);
         return;
       }
     }
-    finish(TypeTag<O>{});
+    finish(acc);
   } else {
     // ---- persistent: this workgroup walks tiles blockIdx.x, blockIdx.x + gridDim.x, ... ------------
     // The host launches it only with KT >= STAGES.  While the epilogue of a tile runs, the first

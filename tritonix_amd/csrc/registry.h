@@ -68,7 +68,9 @@ template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bo
           bool AT = false, bool PAIR = false>
 hipError_t launch_tile(const GemmParams& p, unsigned grid, hipStream_t stream) {
   static_assert(GATHER ? C::VALID_GATHER : C::VALID, "tile configuration is not buildable");
-  hipLaunchKernelGGL((gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV, GATHER, AT, PAIR>), dim3(grid), dim3(C::THREADS), 0, stream, p);
+  GemmParams q = p;
+  set_order_divisors(&q);
+  hipLaunchKernelGGL((gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV, GATHER, AT, PAIR>), dim3(grid), dim3(C::THREADS), 0, stream, q);
   return hipGetLastError();
 }
 
