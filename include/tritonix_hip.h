@@ -208,9 +208,14 @@ int tnx_split_f32(const float* src, int64_t rows, int64_t cols, int64_t stride_r
  * choice names, head and tail of an operand are stored once; in every other tile as the three copies above).  Tile, K cut and workspace are those of the bf16
  * problem (tnx_gemm_default_config fills them for in_dtype = TNX_F32); GLU epilogues apply as in tnx_gemm.  scratch: at
  * least tnx_gemm_f32_scratch_bytes(args) bytes, 256-byte aligned, no initialisation needed; calls that share it must be
- * ordered.  Asynchronous, allocates nothing. */
+ * ordered.  Asynchronous, allocates nothing.
+ * Three tiles (block_k = 32: 32x64 and 64x64 with 4 waves and 4 slots, 32x128 with 4 and 3) multiply the operands as they are,
+ * on the binary32 matrix instruction, where a dimension of each is contiguous: one launch, no scratch (the size query
+ * returns 0).  tnx_gemm_f32_config fills in one of them where it is modelled to be faster -- small products and few rows --
+ * and the built-in choice elsewhere. */
 size_t tnx_gemm_f32_scratch_bytes(const tnx_gemm_args* args);
 int tnx_gemm_f32(const tnx_gemm_args* args, void* scratch, size_t scratch_bytes);
+int tnx_gemm_f32_config(tnx_gemm_args* args);
 
 /* How many K slabs (of block_k) at the end of k a launch of `args` loads element by element, no access outside the
  * operands: 0 where all of them go through the ring of whole 16-byte chunks, 1 where rows, base pointers or sizes are no

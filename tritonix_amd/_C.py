@@ -31,7 +31,7 @@ STATIC_WORKSPACE_BYTES = 65536 + (32 << 20)
 CONV_LOADER_AUTO, CONV_LOADER_REGISTERS, CONV_LOADER_DMA, CONV_LOADER_GEMM = 0, 1, 2, 3
 
 EXPORTS = ("tnx_gemm", "tnx_gemm_static_workspace", "tnx_gemm_workspace_bytes", "tnx_gemm_lds_bytes", "tnx_gemm_supported",
-           "tnx_gemm_default_config", "tnx_tile_coords", "tnx_split_f32", "tnx_gemm_f32_scratch_bytes",
+           "tnx_gemm_default_config", "tnx_gemm_f32_config", "tnx_tile_coords", "tnx_split_f32", "tnx_gemm_f32_scratch_bytes",
            "tnx_gemm_f32", "tnx_gemm_tail_slabs", "tnx_kernel_count", "tnx_kernel_name", "tnx_strerror",
            "tnx_last_hip_error", "tnx_version", "tnx_conv2d_forward", "tnx_conv2d_workspace_bytes",
            "tnx_conv2d_packed_info", "tnx_conv2d_packed_forward", "tnx_conv2d_supported",
@@ -102,6 +102,8 @@ def load() -> ctypes.CDLL:
     lib.tnx_gemm_supported.restype = ctypes.c_int
     lib.tnx_gemm_default_config.argtypes = [p]
     lib.tnx_gemm_default_config.restype = ctypes.c_int
+    lib.tnx_gemm_f32_config.argtypes = [p]
+    lib.tnx_gemm_f32_config.restype = ctypes.c_int
     lib.tnx_tile_coords.argtypes = [ctypes.c_int] * 5 + [ctypes.POINTER(ctypes.c_int)] * 2
     lib.tnx_tile_coords.restype = ctypes.c_int
     lib.tnx_split_f32.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,

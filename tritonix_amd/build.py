@@ -36,7 +36,9 @@ DEVICE_FLAGS = ["-O3", f"--offload-arch={ARCH}", "-fPIC", "-std=c++17",
                 "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option"]
 
 LDS_LIMIT = 160 * 1024
-TAGS = {"bf16": ("TagBF16", 2), "f16": ("TagF16", 2), "i8": ("TagI8", 1)}
+TAGS = {"bf16": ("TagBF16", 2), "f16": ("TagF16", 2), "i8": ("TagI8", 1), "f32": ("TagF32", 4)}
+# tiles of float32 operands on the binary32 matrix instruction (tnx_gemm_f32), block_k = 32: (block_m, block_n, waves, ring slots)
+F32_TILES = ((32, 64, 4, 4), (64, 64, 4, 4), (32, 128, 4, 3))
 
 
 def tile_valid(es, bm, bn, bk, nw, stages):
@@ -89,6 +91,9 @@ def instance_list(quick=False):
     """(dtype, bm, bn, bk, nw, stages, generic) for every kernel to build."""
     out = []
     for dt, (_, es) in TAGS.items():
+        if dt == "f32":
+            out += [(dt, bm, bn, 32, nw, st, False) for bm, bn, nw, st in F32_TILES]
+            continue
         bks = (32, 64) if es == 2 else (64, 128)
         for bm in (32, 64, 128, 256):
             for bn in (64, 128, 256):

@@ -4,6 +4,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <cmath>
 #include <mutex>
 
 #include "../../include/tritonix_hip.h"
@@ -59,10 +60,12 @@ static int64_t lds_bytes_of(const tnx_gemm_args* a) {
   return ring > strips ? ring : strips;
 }
 
-static int check_common(const tnx_gemm_args* a, bool pair) {
+static int check_common(const tnx_gemm_args* a, GemmForm form) {
+  const bool pair = form == GEMM_PAIR;
   if (!a) return TNX_E_INVALID;
   if (a->m < 0 || a->n < 0 || a->k < 0) return TNX_E_INVALID;
-  if (a->in_dtype != TNX_F16 && a->in_dtype != TNX_BF16 && a->in_dtype != TNX_I8) return TNX_E_INVALID;
+  if (a->in_dtype != TNX_F16 && a->in_dtype != TNX_BF16 && a->in_dtype != TNX_I8 && !(form == GEMM_F32 && a->in_dtype == TNX_F32))
+    return TNX_E_INVALID;
   if (a->epilogue < TNX_EPI_NONE || a->epilogue > TNX_EPI_GLU_IDENTITY) return TNX_E_INVALID;
   if (a->block_m <= 0 || a->block_n <= 0 || a->block_k <= 0 || a->group_m <= 0 || a->split_k <= 0 ||
       a->num_stages <= 0 || a->num_warps <= 0 || a->tail_tiles < 0 || a->schedule < 0 ||
@@ -178,7 +181,7 @@ static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool*
   if (at) *at = false;
   if (tail) *tail = false;
   if (other_tile) *other_tile = false;
-  int st = check_common(a, form == GEMM_PAIR);
+  int st = check_common(a, form);
   if (st != TNX_OK) return st;
   int64_t lds = lds_bytes_of(a);
   if (lds > TNX_LDS_LIMIT_BYTES) return TNX_E_LDS;
@@ -202,7 +205,8 @@ static int supported_impl(const tnx_gemm_args* a, const KernelEntry** out, bool*
   if (!e) return TNX_E_UNSUPPORTED;
   tnx_gemm_args tmp = *a;
   if (!inspect_ptrs) { tmp.a = nullptr; tmp.b = nullptr; }
-  if (form != GEMM_PLAIN) { tmp.m = (tmp.m + 7) / 8 * 8; tmp.n = (tmp.n + 7) / 8 * 8; }    // 16-bit operands: chunks of 8 elements
+  const bool padded = form == GEMM_PADDED || form == GEMM_PAIR;
+  if (padded) { tmp.m = (tmp.m + 7) / 8 * 8; tmp.n = (tmp.n + 7) / 8 * 8; }    // 16-bit operands: chunks of 8 elements
   bool tail_slab = false, narrow = false;
   // the persistent kernel keeps the strict layout
   const int layout = dma_layout(&tmp, (a->schedule & TNX_SCHED_PERSISTENT) ? nullptr : &tail_slab, &narrow);
@@ -281,6 +285,11 @@ bool tnx::gemm_tile_for(int dtype, int bm, int bn, int bk, int* num_warps, int* 
   return true;
 }
 
+bool tnx::gemm_f32_direct(const tnx_gemm_args* a) {
+  const KernelEntry* e = nullptr;
+  return a && a->in_dtype == TNX_F32 && a->k > 0 && supported_impl(a, &e, nullptr, true, nullptr, nullptr, nullptr, GEMM_F32) == TNX_OK && e;
+}
+
 void tnx::gemm_tile_layouts(const tnx_gemm_args* a, bool* pair, bool* bt, bool* at) {
   const KernelEntry* e = find_entry(a);
   *pair = e && e->pair[0];
@@ -346,8 +355,9 @@ int tnx::gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, GemmForm fo
   p.c_vec_ok = a->stride_cn == 1 && ((a->stride_cm * es_out) % 16) == 0 && (((uintptr_t)a->c) % 16) == 0;
   p.c_row_ok = a->stride_cn == 1;
   p.tail_slab = tail_slab ? 1 : 0;
-  p.m_load = form != GEMM_PLAIN ? (a->m + 7) / 8 * 8 : a->m;
-  p.n_load = form != GEMM_PLAIN ? (a->n + 7) / 8 * 8 : a->n;
+  const bool padded = form == GEMM_PADDED || form == GEMM_PAIR;
+  p.m_load = padded ? (a->m + 7) / 8 * 8 : a->m;
+  p.n_load = padded ? (a->n + 7) / 8 * 8 : a->n;
   int64_t problems = 1;
   if (extra) {
     p.batch = extra->batch;
@@ -451,6 +461,157 @@ extern "C" int tnx_gemm_static_workspace(const tnx_gemm_args* a) {
   return tnx_gemm(&t);
 }
 
+// Modelled microseconds of a launch of one tile, fitted per tile and element size (16-bit, int8, float32).
+//   start      launch, first slab and epilogue of a workgroup          turn    what every further workgroup on a CU adds
+//   slab       a K slab of one workgroup per CU                        shared  a slab of as many as share a CU, against one
+//   step       what part of such a round the first workgroup in it costs (the rest grows with their number)
+//   crowd      slab's growth from few workgroups to one on every CU    bt      its growth for a k-contiguous B
+//   a_off, b_off  ... for rows of A, of B that are not 16-byte aligned  tail    the last slab, where it goes chunk by chunk
+//   cut, cut_slice, cut_all  K cut: fixed, per slice of 64 KiB, and per 16 MiB of slices in all
+//   store      C, in units of 0.2 us per MB
+struct TileCost {
+  int bm, bn, nw, stages;
+  double start, turn, slab, shared, step, crowd, cut, cut_slice, a_off, b_off, tail, store, cut_all, bt;
+};
+static const TileCost COST16[] = {
+    {256, 256, 8, 2, 4.16, 0.00108, 1.18, 1.89, 0.746, 0.278, 2.83, 0.129, 0.11, 0.159, 2.8, 1.08, 4.01, 0},
+    {256, 256, 4, 2, 7.61, 1.54, 1.17, 1.16, 0.703, 0.337, 2.5, 0.232, 0.144, 0.227, 5.69, 1.39, 3.89, 0},
+    {256, 192, 8, 2, 4.16, 0.586, 0.929, 51.7, 0.739, 0.305, 2.53, 0.244, 0.152, 0.184, 2.69, 0.986, 3.57, 0.0163},
+    {192, 256, 8, 2, 4.01, 0.785, 0.932, 44.5, 0.736, 0.305, 2.46, 0.248, 0.11, 0.205, 2.38, 0.85, 3.64, 0.0384},
+    {192, 192, 8, 3, 4.54, 1.15, 0.621, 43.7, 0.712, 0.406, 2.59, 0.248, 0.134, 0.191, 2.08, 1.46, 3.9, 0.0314},
+    {256, 128, 8, 3, 4.24, 0.735, 0.575, 5.24, 0.711, 0.439, 2.27, 0.257, 0.266, 0.164, 2.3, 1.14, 3.74, 0},
+    {256, 128, 4, 3, 5.25, 1.57, 0.585, 7.21, 0.694, 0.399, 2.84, 0.206, 0.29, 0.224, 3.63, 1.21, 4, 0},
+    {128, 256, 8, 3, 4.5, 1.7, 0.574, 17.8, 0.666, 0.442, 2.25, 0.389, 0.135, 0.231, 2.08, 0.845, 3.5, 0.00578},
+    {128, 128, 8, 3, 3.91, 0.51, 0.356, 2.18, 0.752, 0.439, 1.73, 0.358, 0.196, 0.215, 1.32, 1.45, 4.14, 0},
+    {128, 128, 8, 2, 3.12, 0.0154, 0.551, 0.877, 0.795, 0.356, 1.55, 0.351, 0.158, 0.186, 1.14, 1.33, 3.93, 0},
+    {64, 256, 8, 3, 4.15, 1.62, 0.489, 3.44, 0.84, 0.0951, 2.1, 0.584, 0.131, 0.341, 1.14, 0.887, 3.96, 0},
+    {128, 64, 8, 3, 3.42, 0.296, 0.271, 0.952, 0.875, 0.359, 1.26, 0.422, 0.267, 0.197, 0.911, 2.27, 5.21, 0},
+    {64, 128, 8, 3, 3.63, 1.11, 0.328, 0.975, 0.896, 0.0551, 1.28, 0.648, 0.171, 0.3, 0.653, 1.35, 5.83, 0},
+    {64, 128, 8, 4, 3.61, 1.22, 0.316, 0.6, 0.865, 0.052, 1.35, 0.633, 0.188, 0.327, 0.758, 1.28, 5.97, 0},
+    {64, 64, 4, 4, 3.62, 0.794, 0.203, 0.493, 0.919, 0.308, 1.69, 0.884, 0.288, 0.366, 0.896, 0.0846, 2.06, 0},
+    {32, 128, 4, 3, 3.81, 0.918, 0.259, 0.495, 0.874, 0.171, 1.73, 1.06, 0.127, 0.432, 0.983, 0.0198, 1.81, 0},
+    {32, 64, 4, 4, 3.48, 0.431, 0.151, 1.1, 0.893, 0.276, 1.39, 1.51, 0.152, 0.472, 0.682, 0.103, 1.79, 0}};
+static const TileCost COST8[] = {
+    {256, 256, 8, 2, 4.92, 2.97, 1.16, 1.33, 0.673, 0.206, 2.71, 0.119, 0.141, 0.316, 2.63, 0.884, 3.56, 0.014},
+    {256, 256, 4, 2, 8.13, 2.65, 1.16, 41.3, 33.4, 0.117, 2.41, 0.148, 0.182, 0.357, 4.58, 1.21, 4.01, 0.0384},
+    {256, 192, 8, 2, 5.08, 3.12, 0.93, 45.5, 0.674, 0.228, 2.28, 0.209, 0.171, 0.325, 2.52, 0.785, 3.13, 0.00399},
+    {192, 256, 8, 2, 4.56, 2.83, 0.93, 64, 0.74, 0.188, 2.06, 0.227, 0.13, 0.379, 2.43, 0.812, 3.65, 0.0327},
+    {192, 192, 8, 3, 4.66, 2.92, 0.652, 42.1, 0.713, 0.309, 2.11, 0.328, 0.188, 0.323, 2.15, 0.927, 3.51, 0.0156},
+    {256, 128, 8, 3, 4.26, 1.9, 0.621, 173, 0.698, 0.279, 1.78, 0.302, 0.29, 0.276, 2.04, 0.973, 3.52, 0.000823},
+    {128, 256, 8, 3, 4.62, 2.87, 0.588, 16.7, 0.638, 0.326, 2.03, 0.414, 0.189, 0.387, 2.06, 0.807, 3.27, 0.0633},
+    {128, 128, 8, 3, 3.7, 0.56, 0.377, 1.02, 0.917, 0.271, 1.47, 0.465, 0.303, 0.374, 1.42, 1.16, 4.28, 0},
+    {128, 128, 8, 2, 3.25, 0.175, 0.498, 0.887, 0.757, 0.405, 1.36, 0.379, 0.253, 0.342, 1.39, 1.07, 4.12, 0},
+    {64, 256, 8, 3, 4.09, 1.59, 0.477, 22.8, 0.853, 0.126, 1.47, 0.575, 0.198, 0.541, 1.52, 0.878, 4.04, 0.0117},
+    {64, 128, 8, 3, 3.54, 1.24, 0.298, 0.883, 0.914, 0.175, 1.16, 0.614, 0.272, 0.453, 1.04, 0.996, 5.44, 0},
+    {64, 128, 8, 4, 3.52, 1.28, 0.296, 0.6, 0.843, 0.128, 1.11, 0.623, 0.288, 0.477, 1.06, 1.04, 5.6, 0},
+    {32, 128, 4, 3, 3.53, 0.276, 0.271, 0.628, 0.976, 0.00642, 1.1, 1.06, 0.264, 0.674, 1.18, 1.14, 4.32, 0}};
+// ... of float32 operands as they are (TagF32)
+static const TileCost COST32[] = {
+    {64, 64, 4, 4, 3.78, 0.00146, 0.508, 0.815, 0.924, 0.00596, 1.19, 0.628, 0.0157, 0.0607, 0.611, 1.72, 5.8, 0},
+    {32, 128, 4, 3, 4.29, 1.2, 0.535, 0.695, 0.752, 0.151, 1.58, 0.711, 0.0186, 0.0689, 0.782, 0.485, 1.38, 0},
+    {32, 64, 4, 4, 3.68, 0.0338, 0.279, 1.48, 0.782, 0.133, 1.11, 1.04, 0.0341, 0.0867, 0.498, 1.33, 5.28, 0}};
+
+struct Priced {
+  int64_t m, n, kt, cus;
+  bool a_off, b_off, ragged, bt;
+  double c_mb, ab_mb;              // bytes of C, of A and B together, in MB
+};
+// s slices of K for every tile (tail 0) or for the last `tail` tiles
+static double tile_time(const TileCost& t, const Priced& p, int s, int64_t tail) {
+  const int64_t lds = (int64_t)(t.bm + t.bn) * 128 * t.stages, fit = TNX_LDS_LIMIT_BYTES / lds, most = t.nw == 8 ? 2 : 3;
+  const int64_t c = fit < 1 ? 1 : fit < most ? fit : most;              // workgroups that share a CU
+  const double cus = (double)p.cus, g = c > 1 ? 1.0 + t.shared : 1.0;
+  const double slab = t.slab * (1.0 + (p.a_off ? t.a_off : 0.0)) * (1.0 + (p.b_off ? t.b_off : 0.0));
+  auto of = [&](int64_t n) { return n <= 0 ? 0.0 : 1.0 + (g - 1.0) * (double)(n - 1) / (double)(c > 1 ? c - 1 : 1); };
+  const double q = t.step < 1.0 ? t.step : 1.0;
+  auto rounds = [&](int64_t groups, double slabs) {
+    const int64_t full = groups / (p.cus * c), rem = groups - full * p.cus * c, n = (rem + p.cus - 1) / p.cus;
+    const double fill = (double)groups / cus, frac = (double)rem / cus - (double)(n - 1);
+    const double crowd = (groups <= p.cus ? 1.0 + t.crowd * fill * fill : 1.0 + t.crowd) * (p.bt ? 1.0 + t.bt : 1.0);
+    double last = 0.0;
+    if (rem > 0) last = n == 1 ? (full > 0 ? q + (1.0 - q) * frac : 1.0) : of(n - 1) + (of(n) - of(n - 1)) * (q + (1.0 - q) * frac);
+    return (double)(full * c + n - 1) * t.turn + slab * slabs * crowd * ((double)full * g + last);
+  };
+  const int64_t tiles = ((p.m + t.bm - 1) / t.bm) * ((p.n + t.bn - 1) / t.bn), per = (p.kt + s - 1) / s;
+  const double area = t.bm * t.bn / 16384.0;
+  double us = tail > 0 ? rounds(tiles - tail, (double)p.kt) + t.turn + slab * (double)per * (1.0 + t.crowd) : rounds(tiles * s, (double)per);
+  if (s > 1) us += t.cut + t.cut_slice * s * area + t.cut_all * (double)(tail > 0 ? tail : tiles) * s * area / 256.0;
+  us += t.start + (p.ragged ? t.tail : 0.0) + t.store * p.c_mb / 5.0;
+  const double stream = p.ab_mb / 6.0 + 2.0;
+  return us > stream ? us : stream;
+}
+
+// The tile, its waves and slots, and the K cut with the smallest modelled time.  The constants are a least-squares fit of the
+// logarithm to 273,000 launches: 3,979 problems of 17 to 8192 rows, 64 to 28672 columns and k of 64 to 14336 in bf16, f16
+// and int8, nn, nt and tn, gated and not, odd sizes among them, on every tile here uncut and cut in 2 to 16, ten launches
+// each in a graph.  Against the fastest of them the choice takes 1.021x the time in the mean (int8 1.027x), the one before
+// (six tiles at fixed relative rates, cuts of 2, 4, 8 and 16 at 9 us each) 1.088x (int8 1.13x): on problems of 33 to 256 rows
+// 0.88 to 0.90 of its time, to 1024 rows 0.94, above 0.96, int8 0.83 to 0.90; 4 % of the problems lose more than 5 %, 40 %
+// gain more.  Slices are kept within what tnx_gemm_static_workspace holds.
+// only_cut > 0: that many slices and no other number.
+static double price_tiles(tnx_gemm_args* a, int es, bool at, int64_t cus, int only_cut = 0) {
+  const int vec = 16 / es, bk = 128 / es;
+  a->block_k = bk;
+  Priced p;
+  p.m = a->m; p.n = a->n; p.kt = (a->k + bk - 1) / bk; p.cus = cus;
+  p.bt = a->stride_bk == 1 && a->stride_bn != 1;
+  const int64_t ra = at ? a->stride_ak : a->stride_am, rb = p.bt ? a->stride_bn : a->stride_bk;
+  p.a_off = ra % vec != 0 || ((uintptr_t)a->a & 15) != 0;
+  p.b_off = rb % vec != 0 || ((uintptr_t)a->b & 15) != 0;
+  p.ragged = p.a_off || p.b_off || a->k % bk != 0 || a->n % vec != 0;
+  p.c_mb = (double)a->m * (double)(a->epilogue == TNX_EPI_NONE ? a->n : a->n / 2) * (es == 2 ? 2 : 4) * 1e-6;
+  p.ab_mb = ((double)a->m + (double)a->n) * (double)a->k * es * 1e-6;
+  const TileCost* table = es == 1 ? COST8 : es == 4 ? COST32 : COST16;
+  const int type = a->in_dtype == TNX_I8 ? 2 : a->in_dtype == TNX_F16 ? 1 : a->in_dtype == TNX_F32 ? 3 : 0;
+  static const int cuts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
+  struct Entries {                 // the kernels behind the tables (looking one up takes a third of a microsecond)
+    const KernelEntry* of[4][sizeof COST16 / sizeof *COST16];
+    int count[4];
+    Entries() {
+      static_assert(sizeof COST8 <= sizeof COST16 && sizeof COST32 <= sizeof COST16, "one array holds any table");
+      for (int d = 0; d < 4; ++d) {
+        count[d] = (int)((d == 3 ? sizeof COST32 : d == 2 ? sizeof COST8 : sizeof COST16) / sizeof *COST16);
+        for (int i = 0; i < count[d]; ++i) {
+          const TileCost& t = (d == 3 ? COST32 : d == 2 ? COST8 : COST16)[i];
+          tnx_gemm_args q = {};
+          q.in_dtype = d == 3 ? TNX_F32 : d == 2 ? TNX_I8 : d == 1 ? TNX_F16 : TNX_BF16;
+          q.block_m = t.bm; q.block_n = t.bn; q.block_k = d == 3 ? 32 : d == 2 ? 128 : 64; q.num_warps = t.nw; q.num_stages = t.stages;
+          of[d][i] = find_entry(&q);
+        }
+      }
+    }
+  };
+  static const Entries entries;
+  double best = 1e300;
+  const TileCost* pick = nullptr;
+  int best_s = 1, best_tail = 0;
+  for (int i = 0; i < entries.count[type]; ++i) {
+    const TileCost& t = table[i];
+    // 256x256: two waves per SIMD cover the start and end of a short K loop, at half again as many LDS reads, which lose on the
+    // long, power-limited ones (8192^3: 2 %; 4096 x 28672 x 4096, gated: 2.4 % the other way)
+    if (t.bm == 256 && t.bn == 256 && t.nw != ((es == 2 && p.kt <= 64) || at ? 8 : 4)) continue;
+    const KernelEntry* e = entries.of[type][i];
+    if (!e || (at ? !e->fast_at : p.bt ? !e->fast_bt : !e->fast)) continue;
+    const int64_t tiles = ((a->m + t.bm - 1) / t.bm) * ((a->n + t.bn - 1) / t.bn);
+    if ((double)t.bm * t.bn * (double)tiles > 5.0 * (double)a->m * (double)a->n + 4.0 * 65536) continue;
+    for (int s : cuts) {
+      if (only_cut > 0 && s != only_cut) continue;
+      const bool last_only = s > 1 && tiles > cus && tiles % cus != 0;         // only the tiles of the partial round are cut
+      const int64_t tail = last_only ? tiles % cus : 0, ncut = s == 1 ? 0 : last_only ? tail : tiles;
+      if (s > 1 && (p.kt / s < 2 || ncut > WS_MAX_TILES || ncut * s > (last_only ? 2 : 3) * cus ||
+                    ncut * s * t.bm * t.bn * 4 > TNX_STATIC_WORKSPACE_BYTES - WS_COUNTER_BYTES))
+        break;
+      // (what is modelled to be even goes to the fewer slices: 4 % per doubling, 83 instead of 104 of 2,866 problems lose 5 %)
+      const double us = tile_time(t, p, s, tail) * (1.0 + 0.04 * log2((double)s));
+      if (us < best) { best = us; pick = &t; best_s = s; best_tail = (int)tail; }
+    }
+  }
+  if (!pick) { a->block_m = 128; a->block_n = 128; a->num_stages = 3; a->num_warps = 8; return 1e300; }
+  a->block_m = pick->bm; a->block_n = pick->bn; a->num_stages = pick->stages; a->num_warps = pick->nw;
+  a->split_k = best_s; a->tail_tiles = best_tail;
+  return best;
+}
+
 // large_f32: a problem of tnx_gemm_f32 (heads and tails in bf16), which may also go to the tiles of 192 and 256
 static int default_config(tnx_gemm_args* a, bool large_f32);
 
@@ -538,6 +699,13 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
     a->block_m = es == 2 && a->m <= 32 && !at && !large_f32 && (narrow || s == 1) ? 32 : 64;
     a->num_stages = narrow ? 4 : 3;
     a->num_warps = narrow || a->block_m == 32 ? 4 : 8;
+    // 33 to 64 rows: the tile by modelled time (two rounds of 32 rows, three of which share a CU, mostly: 64 x 3840 x 6272
+    // 16.9 -> 14.1 us), the cut as above -- an m-contiguous A then gives the bits of its row-major copy (434 problems: 0.89
+    // of the time of the tiles above, 0.85 with the best cut too)
+    if (es == 2 && !large_f32 && a->out_dtype != TNX_F32 && !at && a->m > 32) {
+      tnx_gemm_args t = *a;
+      if (price_tiles(&t, es, at, cus, s) < 1e300) *a = t;
+    }
     return TNX_OK;
   }
   if (a->m <= 64 && at) {
@@ -559,7 +727,17 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
     a->block_m = a->m <= 64 ? 64 : 128; a->block_n = 128; a->num_stages = 2; a->num_warps = 4;
     return TNX_OK;
   }
-  // Pick the tile and the K cut with the smallest modelled time.  A wave is 256 workgroups (one per CU); a tile
+  // 16-bit and int8 results
+  // (two rounds and more of 256x256 tiles with long K loops run against the power limit, which the rates below are from and the
+  // fitted launches, ten in a row, hardly meet)
+  const bool powered = ((a->m + 255) / 256) * ((a->n + 255) / 256) >= 2 * cus && a->k >= 64 * bk;
+  if (!large_f32 && a->out_dtype != TNX_F32 && !powered) {
+    price_tiles(a, es, at, cus);
+    const int64_t tm = (a->m + a->block_m - 1) / a->block_m, tn = (a->n + a->block_n - 1) / a->block_n;
+    if (a->split_k == 1 && tm >= 16 && tn >= 16) a->schedule = TNX_SCHED_SUPERBLOCK;
+    return TNX_OK;
+  }
+  // those, and binary32 results: pick the tile and the K cut with the smallest modelled time.  A wave is 256 workgroups (one per CU); a tile
   // costs its multiply-adds over the rate a CU sustains with that tile (relative rates measured on 8192^3 and
   // 2048^2 x 8192: 256x256 1.0, 256x128 0.9, 128x128 0.75); a last, partial wave costs 0.75 of a full one (the
   // part is power-limited: fewer busy CUs clock higher; measured 0.70-0.80 on 6144^3, 5120^2 x 8192,
@@ -652,6 +830,44 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
   return TNX_OK;
 }
 
+// tnx_gemm_default_config for a float32 product, or a tile that multiplies its operands as they are (TagF32) instead of heads
+// and tails where that is modelled to be faster.
+// The binary32 instruction has a sixteenth of bf16's rate where the split takes three bf16 products, but the split reads both
+// operands once more, writes and reads their terms, and is a launch of its own: up to 64 rows the direct product is ahead
+// everywhere (16 x 10112 x 7616 with a k-contiguous B: 176 -> 55 us, 5 x 7664 x 4992 87 -> 31), and so is one of up to 3e8
+// operations (7.0 -> 4.9 us); from 3e9 on and 256 rows the split.  Split: a pass at 0.39 us per MB of operands and 5.4 us of
+// its own and the second launch, then rounds of workgroups; constants from 2,900 problems, on which the choice takes 0.71x the
+// split's time in the mean and loses more than 5 percent on 24.  Its sums are closer to the float64 product (2e-7 to 2e-6)
+// than the split's (5e-6).
+extern "C" int tnx_gemm_f32_config(tnx_gemm_args* a) {
+  if (!a || a->in_dtype != TNX_F32) return TNX_E_INVALID;
+  const int st = tnx_gemm_default_config(a);
+  if (st != TNX_OK) return st;
+  const tnx_gemm_args split = *a;
+  tnx_gemm_args t = *a;
+  t.a = t.b = nullptr;
+  if (t.stride_ak == 0 && t.stride_bn == 0) { t.stride_am = t.k; t.stride_ak = 1; t.stride_bk = t.n; t.stride_bn = 1; }
+  t.block_m = 64; t.block_n = 128; t.block_k = 32;
+  bool tail_slab = false;
+  const int layout = t.k > 0 ? dma_layout(&t, &tail_slab) : 0;
+  if (layout == 0) return TNX_OK;
+  int64_t cus = 256;
+  int n = 0;
+  if (compute_units(&n) == TNX_OK && n > 0) cus = n;
+  t.group_m = 8; t.split_k = 1; t.tail_tiles = 0; t.schedule = TNX_SCHED_DEFAULT;
+  const double direct = price_tiles(&t, 4, layout == 3, cus);
+  const double kt = (double)((a->k + 31) / 32), s = split.split_k, area = split.block_m * split.block_n / 16384.0;
+  const double tiles = (double)((a->m + split.block_m - 1) / split.block_m) * (double)((a->n + split.block_n - 1) / split.block_n);
+  const double rounds = ceil(tiles * (split.tail_tiles ? 1.0 : s) / (double)cus), per = split.tail_tiles ? kt : ceil(kt / s);
+  const double in_mb = ((double)a->m + (double)a->n) * (double)a->k * 4e-6, out_mb = (double)a->m * (double)a->n * 4e-6;
+  const double both = 5.44 + 0.388 * in_mb + 0.337 * out_mb + rounds * (0.37 + per * (0.14 + 0.373 * area)) + (s > 1 ? 1.58 + 0.663 * s * area : 0.0);
+  if (direct * 1.03 > both) return TNX_OK;
+  a->block_m = t.block_m; a->block_n = t.block_n; a->block_k = t.block_k; a->group_m = t.group_m;
+  a->split_k = t.split_k; a->tail_tiles = t.tail_tiles; a->schedule = t.schedule;
+  a->num_stages = t.num_stages; a->num_warps = t.num_warps;
+  return TNX_OK;
+}
+
 // ---------------------------------------------------------------------------
 // float32 operands as bf16 head and tail (see tnx_split_f32 in the header)
 // ---------------------------------------------------------------------------
@@ -711,7 +927,8 @@ extern "C" int tnx_tile_coords(int schedule, int id, int tiles_m, int tiles_n, i
 extern "C" int tnx_kernel_count(void) {
   int ng = 0, n = 0;
   const KernelGroup* g = tnx_kernel_groups(&ng);
-  for (int i = 0; i < ng; ++i) n += g[i].count;
+  for (int i = 0; i < ng; ++i)
+    for (int j = 0; j < g[i].count; ++j) n += g[i].entries[j].dtype != TNX_F32;    // (those are tnx_gemm_f32's own)
   return n;
 }
 
@@ -720,6 +937,7 @@ extern "C" const char* tnx_kernel_name(int idx) {
   int ng = 0;
   const KernelGroup* g = tnx_kernel_groups(&ng);
   for (int i = 0; i < ng; ++i) {
+    if (g[i].count > 0 && g[i].entries[0].dtype == TNX_F32) continue;              // groups hold one type
     if (idx < g[i].count) {
       const KernelEntry& e = g[i].entries[idx];
       const char* dn = e.dtype == TNX_F16 ? "f16" : e.dtype == TNX_BF16 ? "bf16" : "i8";

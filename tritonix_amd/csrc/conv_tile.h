@@ -291,7 +291,7 @@ __global__ __launch_bounds__(C::THREADS, TNX_CONV_OCC) void conv2d_tile_kernel(C
         const int colb = b_colb0 + j * MI * ES;
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          fb[j][h] = lds_read_tr<ES>(sb + (b_krow + ks * C::MMA_K + h * 4) * C::ROWB_B + (((colb >> 4) ^ b_sw) << 4) + (colb & 15));
+          fb[j][h] = lds_read_tr<ES, 0>(sb + (b_krow + ks * C::MMA_K + h * 4) * C::ROWB_B + (((colb >> 4) ^ b_sw) << 4) + (colb & 15));
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i)

@@ -16,6 +16,9 @@
 // Bound by memory: 4 bytes read and 4 (three copies: 6) written per element.  2048^3: 13 us for both operands (64 MB, 5 TB/s),
 // the product from 61.3 us (three copies) to 52.4; its GEMM, 64 slabs of 0.64 us, is bound by filling the slabs from the L2
 // and by the MFMAs (0.45 us of a slab).  3072 x 3200 x 2822: 162 -> 145 us.
+//
+// Small products and few rows skip all that: the binary32 matrix instruction on the operands as they are (TagF32 in
+// gemm_tile.h, chosen by tnx_gemm_f32_config), one launch, no scratch.
 #include <hip/hip_runtime.h>
 #include <string.h>
 
@@ -172,6 +175,7 @@ static bool next_rows(SplitSide* s) {
 }
 
 extern "C" size_t tnx_gemm_f32_scratch_bytes(const tnx_gemm_args* a) {
+  if (gemm_f32_direct(a)) return 0;
   tnx_gemm_args g;
   SplitSide sa, sb;
   int64_t bytes = 0;
@@ -187,6 +191,10 @@ extern "C" int tnx_gemm_f32(const tnx_gemm_args* a, void* scratch, size_t scratc
   int st = plan(a, scratch, &g, &sa, &sb, &bytes, &pair);
   if (st != TNX_OK) return st;
   if (a->m == 0 || a->n == 0) return TNX_OK;
+  if (gemm_f32_direct(a)) {
+    if (!a->a || !a->b || !a->c || (((uintptr_t)a->a | (uintptr_t)a->b | (uintptr_t)a->c) & 3)) return TNX_E_INVALID;
+    return gemm_launch(a, nullptr, GEMM_F32);
+  }
   if (a->k == 0) {                          // nothing to cut: the GEMM writes zeros
     g.k = 0;
     return gemm_launch(&g, nullptr, pair ? GEMM_PAIR : GEMM_PADDED);

@@ -81,8 +81,8 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(GemmParams p
     const i32x4 af = *TNX_LDS(i32x4, slot + a_off);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const i32x2 lo = lds_read_tr<2>(slot + b_off[j][0]);
-      const i32x2 hi = lds_read_tr<2>(slot + b_off[j][1]);
+      const i32x2 lo = lds_read_tr<2, 0>(slot + b_off[j][0]);
+      const i32x2 hi = lds_read_tr<2, 0>(slot + b_off[j][1]);
       acc[j] = MMA::run(i32x4{lo.x, lo.y, hi.x, hi.y}, af, acc[j]);   // rows = n, cols = m
     }
   };

@@ -149,6 +149,8 @@ struct GemmParams {
 struct TagF16 { static constexpr int ES = 2; static constexpr int ID = DT_F16; typedef float acc_s; };
 struct TagBF16 { static constexpr int ES = 2; static constexpr int ID = DT_BF16; typedef float acc_s; };
 struct TagI8 { static constexpr int ES = 1; static constexpr int ID = DT_I8; typedef int acc_s; };
+// float32 operands as they are, on the binary32 matrix instruction (a sixteenth of bf16's rate)
+struct TagF32 { static constexpr int ES = 4; static constexpr int ID = DT_F32; typedef float acc_s; };
 
 template <class T, int MI> struct Mma;
 template <> struct Mma<TagBF16, 32> {
@@ -173,6 +175,17 @@ template <> struct Mma<TagF16, 16> {
   typedef f32x4 acc_t;
   static __device__ __forceinline__ acc_t run(i32x4 a, i32x4 b, acc_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+};
+// 16 k: four instructions of four k.  Lane group g holds k = 4 g .. 4 g + 3 of a 16-byte fragment and gives instruction e
+// its element e, so the instructions take the k in another order than they lie in, A and B alike.
+template <> struct Mma<TagF32, 16> {
+  typedef f32x4 acc_t;
+  static __device__ __forceinline__ acc_t run(i32x4 a, i32x4 b, acc_t c) {
+    const f32x4 fa = __builtin_bit_cast(f32x4, a), fb = __builtin_bit_cast(f32x4, b);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], c, 0, 0, 0);
+    return c;
   }
 };
 template <> struct Mma<TagI8, 32> {
@@ -366,15 +379,16 @@ __device__ __forceinline__ i32x4 load16_agent(__amdgpu_buffer_rsrc_t w, uint32_t
 // stores into one and drops the hint, measured as the full loss of the gain.)
 typedef i32x4 __attribute__((aligned(2))) i32x4_loose;
 typedef i32x4 __attribute__((aligned(1))) i32x4_bytes;
+typedef i32x4 __attribute__((aligned(4))) i32x4_words;
 __device__ __forceinline__ void store16_stream(void* dst, i32x4 v) { __builtin_nontemporal_store(v, (i32x4*)dst); }
 __device__ __forceinline__ void store16_stream_loose(void* dst, i32x4 v) { __builtin_nontemporal_store(v, (i32x4_loose*)dst); }
 
-template <int ES> __device__ __forceinline__ i32x2 lds_read_tr(uint32_t addr);
-template <> __device__ __forceinline__ i32x2 lds_read_tr<2>(uint32_t addr) {
-  return __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(TNX_LDS(i16x4, addr)));
-}
-template <> __device__ __forceinline__ i32x2 lds_read_tr<1>(uint32_t addr) {
-  return __builtin_amdgcn_ds_read_tr8_b64_v2i32(TNX_LDS(i32x2, addr));
+// half a fragment from a slab of k rows, ROWB bytes each: 8 bytes along k per lane.  Transposing reads for 16-bit and int8
+// elements, two words for 32-bit ones.
+template <int ES, int ROWB> __device__ __forceinline__ i32x2 lds_read_tr(uint32_t addr) {
+  if constexpr (ES == 2) return __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(TNX_LDS(i16x4, addr)));
+  else if constexpr (ES == 1) return __builtin_amdgcn_ds_read_tr8_b64_v2i32(TNX_LDS(i32x2, addr));
+  else return i32x2{*TNX_LDS(int, addr), *TNX_LDS(int, addr + ROWB)};
 }
 
 __device__ __forceinline__ float quad_swap1(float v) {
@@ -431,6 +445,7 @@ struct TileCfg {
   // which outweighs their four points of extra issue overhead.  The 32x32 code paths below stay usable
   // (MI = 32 needs WTM % 32 == 0 && WTN % 32 == 0).
   static constexpr int MI = 16;
+  static_assert(ES != 4 || MI == 16, "binary32 operands: 16x16 shapes only");
   static constexpr int TM = WTM / MI, TN = WTN / MI;
   static constexpr int KB = (MI == 32) ? 32 : 64;                 // k bytes one MFMA consumes
   static constexpr int MMA_K = KB / ES;
@@ -477,6 +492,9 @@ struct TileCfg {
       const int pass = MI == 16 ? (((row >> 3) ^ (row >> 4)) & 1) << 1 : 0;
       if (CPR % 16 == 0) { int k = row & 3; return ((2 * k + (k >> 1)) << 1) ^ pass; }
       return ((row & 3) << 1) ^ pass;       // stays inside a group of 8 chunks: also for rows of 24 chunks (BN = 192)
+    } else if (ES == 4) {
+      // a read is 16 neighbouring words (4 chunks) of one k row per lane group, the groups 4 rows apart
+      return ((row >> 2) & (CPR % 16 == 0 ? 3 : 1)) << 2;
     } else {
       const int pass = MI == 16 ? ((row >> 4) ^ (row >> 5)) & 1 : 0;
       if (CPR % 16 == 0) { int k = row & 7; return (2 * k + (k >> 2)) ^ pass; }
@@ -515,6 +533,7 @@ template <class T> struct OutOf;
 template <> struct OutOf<TagBF16> { typedef OutBF16 type; };
 template <> struct OutOf<TagF16> { typedef OutF16 type; };
 template <> struct OutOf<TagI8> { typedef int type; };
+template <> struct OutOf<TagF32> { typedef OutF32 type; };
 
 
 // LDS one wave needs to pass one row-block (MI rows) of its outputs through LDS: up to 32 bits per accumulator, rows
@@ -1328,8 +1347,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   constexpr int GEN_B_ROWS = BT ? BN : BK, GEN_B_CPR = BT ? C::CPR_A : C::CPR_B;
   constexpr int GEN_NA = (BM * C::CPR_A + C::THREADS - 1) / C::THREADS;
   constexpr int GEN_NB = (GEN_B_ROWS * GEN_B_CPR + C::THREADS - 1) / C::THREADS;
-  typedef typename std::conditional<ES == 2, uint16_t, uint8_t>::type gen_elem_t;
-  typedef typename std::conditional<ES == 2, i32x4_loose, i32x4_bytes>::type gen_chunk_t;
+  typedef std::conditional_t<ES == 4, uint32_t, std::conditional_t<ES == 2, uint16_t, uint8_t>> gen_elem_t;
+  typedef std::conditional_t<ES == 4, i32x4_words, std::conditional_t<ES == 2, i32x4_loose, i32x4_bytes>> gen_chunk_t;
   constexpr int EPC = 16 / ES;                           // elements per chunk
   // chunk idx of the A part of slab kt_global: row idx / CPR_A, k chunk idx % CPR_A
   auto gen_fetch_a = [&](int kt_global, int idx) __attribute__((always_inline)) -> i32x4 {
@@ -1654,8 +1673,9 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
 
   const int blk = lane >> 4, li = lane & 15;
   const int b_kg = (MI == 32) ? (blk >> 1) : blk;
-  const int b_sub = (ES == 2) ? (li >> 2) : (li >> 1);               // k row inside the transposed block
-  const int b_colb0 = (wx * C::WTN + ((MI == 32) ? 16 * (blk & 1) : 0)) * ES + ((ES == 2) ? 8 * (li & 3) : 8 * (li & 1));
+  const int b_sub = (ES == 4) ? 0 : (ES == 2) ? (li >> 2) : (li >> 1);               // k row inside the transposed block
+  const int b_col = (ES == 4) ? 4 * li : (ES == 2) ? 8 * (li & 3) : 8 * (li & 1);    // byte of the block's row
+  const int b_colb0 = (wx * C::WTN + ((MI == 32) ? 16 * (blk & 1) : 0)) * ES + b_col;
   constexpr int RPR = 8 / ES;                                       // k rows one transposing read covers
   const int b_sw = C::swzB((16 / ES) * b_kg + b_sub);     // the same for every k step and both halves of a fragment
   uint32_t b_joff[TN];          // byte offset inside the B slab, per column block
@@ -1666,7 +1686,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
   }
 
   // m-contiguous A: as a row-major B slab
-  const int at_colb0 = (wy * C::WTM) * ES + ((ES == 2) ? 8 * (li & 3) : 8 * (li & 1));
+  const int at_colb0 = (wy * C::WTM) * ES + b_col;
   const int at_sw = C::template swzT<AT_CPR>((16 / ES) * b_kg + b_sub);
   uint32_t at_off[TM];
 #pragma unroll
@@ -1717,17 +1737,17 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
       int j = idx >> 1, h = idx & 1;
       if constexpr (XOR_OFFS) {
         if (h == 0) xo_b = xor_off(sb + b_joff[0], j * MI * ES);
-        fb[set][j][h] = lds_read_tr<ES>(xo_b + ks * C::MMA_K * C::ROWB_B + h * RPR * C::ROWB_B);
+        fb[set][j][h] = lds_read_tr<ES, C::ROWB_B>(xo_b + ks * C::MMA_K * C::ROWB_B + h * RPR * C::ROWB_B);
       } else {
-        fb[set][j][h] = lds_read_tr<ES>(sb + b_joff[j] + ks * C::MMA_K * C::ROWB_B + h * RPR * C::ROWB_B);
+        fb[set][j][h] = lds_read_tr<ES, C::ROWB_B>(sb + b_joff[j] + ks * C::MMA_K * C::ROWB_B + h * RPR * C::ROWB_B);
       }
     } else if (AT) {
       int i = (idx - NBREAD) >> 1, h = (idx - NBREAD) & 1;
       if constexpr (XOR_OFFS) {
         if (h == 0) xo_at = xor_off(sa + at_off[0], i * MI * ES);
-        fat[set][i][h] = lds_read_tr<ES>(xo_at + ks * C::MMA_K * AT_ROWB + h * RPR * AT_ROWB);
+        fat[set][i][h] = lds_read_tr<ES, AT_ROWB>(xo_at + ks * C::MMA_K * AT_ROWB + h * RPR * AT_ROWB);
       } else {
-        fat[set][i][h] = lds_read_tr<ES>(sa + at_off[i] + ks * C::MMA_K * AT_ROWB + h * RPR * AT_ROWB);
+        fat[set][i][h] = lds_read_tr<ES, AT_ROWB>(sa + at_off[i] + ks * C::MMA_K * AT_ROWB + h * RPR * AT_ROWB);
       }
     } else {
       int i = idx - NBREAD;

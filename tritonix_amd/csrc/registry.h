@@ -38,10 +38,13 @@ struct GemmBatch {
 // What the operands of a launch are.  PADDED: the rows of B (and of an m-contiguous A) are followed by readable memory up
 // to a whole 16-byte chunk, so an N (M) that ends inside a chunk still takes the aligned loader.  PAIR: padded, and k
 // holds the heads and tails of a float32 product in blocks of 32 (KernelEntry::pair).
-enum GemmForm { GEMM_PLAIN = 0, GEMM_PADDED = 1, GEMM_PAIR = 2 };
+// F32: float32 operands as they are, on the binary32 matrix instruction.
+enum GemmForm { GEMM_PLAIN = 0, GEMM_PADDED = 1, GEMM_PAIR = 2, GEMM_F32 = 3 };
 int gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, GemmForm form = GEMM_PLAIN);
 // the status gemm_launch would return for these arguments, the workspace included, without launching
 int gemm_check(const tnx_gemm_args* a, GemmForm form);
+// whether the tile of `a` and the layout of its float32 operands have a kernel that multiplies them as they are
+bool gemm_f32_direct(const tnx_gemm_args* a);
 // whether the tile of `a` takes head and tail slabs, and whether it has the k-contiguous-B and m-contiguous-A loaders
 void gemm_tile_layouts(const tnx_gemm_args* a, bool* pair, bool* bt, bool* at);
 // waves and stages of a built tile with these dimensions that gemm_launch takes with a GemmBatch (eight waves and
@@ -126,7 +129,7 @@ template <class T, class C> struct ConvLaunch<T, C, true> {
 // spills.)
 template <class C> constexpr bool at_ok() {
   return C::BK * C::ES == 128 && C::VALID_AT &&
-         ((C::BM == 256 && C::BN == 256 && C::NW == 8 && C::STAGES == 2) || (C::BM == 256 && C::BN == 128 && C::NW == 4 && C::STAGES == 3) ||
+         (C::ES == 4 || (C::BM == 256 && C::BN == 256 && C::NW == 8 && C::STAGES == 2) || (C::BM == 256 && C::BN == 128 && C::NW == 4 && C::STAGES == 3) ||
           (C::BM == 128 && C::BN == 128 && C::NW == 8 && C::STAGES == 3) || (C::BM == 64 && C::BN == 128 && C::NW == 8 && C::STAGES == 3) ||
           (C::BM == 64 && C::BN == 64 && C::NW == 4 && C::STAGES == 4) || (C::BM == 192 && C::BN == 192 && C::NW == 8 && C::STAGES == 3) ||
           ((C::BM == 192 || C::BN == 192) && C::BM != C::BN && C::NW == 8 && C::STAGES == 2));

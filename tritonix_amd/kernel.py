@@ -157,8 +157,8 @@ class PlannedLaunch:
         if g.in_dtype == _C.F32:
             import torch
 
-            scratch = torch.empty(self.scratch, dtype=torch.uint8, device=device)
-            status = self.lib.tnx_gemm_f32(ctypes.byref(g), scratch.data_ptr(), self.scratch)
+            scratch = torch.empty(self.scratch, dtype=torch.uint8, device=device) if self.scratch else None
+            status = self.lib.tnx_gemm_f32(ctypes.byref(g), scratch.data_ptr() if self.scratch else None, self.scratch)
             g.in_dtype = _C.BF16 if status else g.in_dtype          # what an error message has to describe
         else:
             status = self.lib.tnx_gemm(ctypes.byref(g))
@@ -320,6 +320,7 @@ class HipKernel:
             # the reference's kernels take float32 operands and multiply them in TF32 (tritonix/ops/matmul.py:98,
             # tritonix/ops/swiglu.py:89-93), for which gfx950 has no matrix instruction: the library cuts them into bf16
             # heads and tails and multiplies those, with a float32 result
+            # -- or, for small products and few rows, multiplies them as they are, without scratch
             need = int(lib.tnx_gemm_f32_scratch_bytes(ctypes.byref(g)))
             scratch = torch.empty(need, dtype=torch.uint8, device=device)
         if g.split_k > 1:

@@ -316,7 +316,8 @@ def default_config(a, b, split=False):
         # base-pointer alignment decides between the two loaders; CPU tensors (host-side planning) count as aligned
         g.a = a.data_ptr() if a.is_cuda else None
         g.b = b.data_ptr() if b.is_cuda else None
-    _C.load().tnx_gemm_default_config(ctypes.byref(g))
+    lib = _C.load()
+    (lib.tnx_gemm_f32_config if a.dtype == torch.float32 else lib.tnx_gemm_default_config)(ctypes.byref(g))
     cfg = {"block_m": g.block_m, "block_n": g.block_n, "block_k": g.block_k, "group_m": g.group_m,
            "num_stages": g.num_stages, "num_warps": g.num_warps}
     if split:
