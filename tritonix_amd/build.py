@@ -365,6 +365,8 @@ def build(jobs=None, quick=False, verbose=True, force=True, only=None, out=None,
         GATHER_TILES if not (only or only_conv) or only == "gather" else (), os.path.join(BUILD, "gen")) + [
         os.path.join(CSRC, "capi.hip"), os.path.join(CSRC, "skinny.hip"),
         os.path.join(CSRC, "conv.hip"), os.path.join(CSRC, "f32.hip")]
+    if lib == LIB:
+        build_launch(verbose)
     objdir = os.path.join(BUILD, "obj")
     os.makedirs(objdir, exist_ok=True)
     objs = [os.path.join(objdir, os.path.basename(s)[:-4] + ".o") for s in srcs]
@@ -388,6 +390,28 @@ def build(jobs=None, quick=False, verbose=True, force=True, only=None, out=None,
         print(f"linked {lib} in {time.time() - t0:.1f}s; no compiler-generated use of M0; "
               f"kernel resources in {os.path.join(BUILD, 'kernel_resources.json')}", flush=True)
     return lib
+
+
+def build_launch(verbose=True):
+    """tritonix_amd/_launch.so: the host side of repeated calls (csrc/launch.cpp), against torch's C++ interface."""
+    import sysconfig
+
+    import torch
+
+    t0 = time.time()
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    out = os.path.join(HERE, "_launch.so")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
+           os.path.join(CSRC, "launch.cpp"), "-o", out + ".tmp", f"-L{root}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for launch.cpp:\n{r.stderr[-4000:]}")
+    os.replace(out + ".tmp", out)
+    if verbose:
+        print(f"linked {out} in {time.time() - t0:.1f}s", flush=True)
+    return out
 
 
 def main(argv=None):

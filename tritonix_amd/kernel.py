@@ -167,9 +167,62 @@ class PlannedLaunch:
         return status
 
 
+class _Plans(dict):
+    """The kept launches; what the native side holds of them goes with them."""
+
+    def clear(self) -> None:
+        super().clear()
+        if _launch is not None:
+            _launch.forget()
+
+
 # by everything a launch depends on but its pointers (None: met once so far); bounded, dropped whole when full
-_plans: dict = {}
+_plans: dict = _Plans()
 _MAX_PLANS = 1024
+
+# tritonix_amd/_launch.so (csrc/launch.cpp), which repeats a kept launch without the interpreter; loaded with the first of them
+_launch = None
+_tags: dict = {"matmul": 0}
+
+
+def product(tag: int, a, b, memo: dict, hooks: list):
+    """The product of ``a`` and ``b`` by a kept launch of the native side, or None.  (Replaced by ``_launch.product`` once there
+    is such a launch.)"""
+    return None
+
+
+def plan_tag(tag) -> int:
+    """A number for the operation of a plan key."""
+    n = _tags.get(tag)
+    if n is None:
+        if len(_tags) >= _MAX_PLANS:
+            _plans.clear()
+            _tags.clear()
+            _tags["matmul"] = 0
+        n = _tags[tag] = len(_tags)
+    return n
+
+
+def _workspace_of(index: int, stream: int, nbytes: int, atomic: int):
+    import torch
+
+    ws = _workspace(torch.device("cuda", index), stream, nbytes, bool(atomic))
+    return ws.data_ptr(), ws.numel()
+
+
+def launch_module():
+    """``_launch``, bound to the loaded library; a missing build raises, as for the library itself."""
+    global _launch, product
+    if _launch is None:
+        lib = _C.load()
+        try:
+            from tritonix_amd import _launch as module
+        except ImportError as err:
+            raise RuntimeError(f"tritonix_amd/_launch.so cannot be loaded ({err}): build it with `python -m tritonix_amd.build`") from err
+        at = [ctypes.cast(fn, ctypes.c_void_p).value for fn in (lib.tnx_gemm, lib.tnx_gemm_f32, lib.tnx_conv2d_forward)]
+        module.bind(*at, _workspace_of)
+        _launch, product = module, module.product
+    return _launch
 
 
 def plan_key(tag, a, b) -> tuple:
@@ -187,9 +240,12 @@ def planned(key: tuple, memo: dict) -> Optional[PlannedLaunch]:
     return hit[0]
 
 
-def keep_plan(key: tuple, memo_key: tuple, memo: dict, kernel, a, b, c, **extra) -> None:
-    """Remember the launch that just gave ``c``, the second time it is met: making it ready takes 9 us, which a program that
+def keep_plan(key: tuple, memo_key: tuple, memo: dict, kernel, a, b, c, given, **extra) -> None:
+    """Operands that had to be copied first keep the long way; views of the ``given`` ones (a row with another pitch) do not.
+    Remember the launch that just gave ``c``, the second time it is met: making it ready takes 9 us, which a program that
     never meets a size twice would pay for nothing (first call of a 16-bit product 34 us with it, 26 without)."""
+    if a.data_ptr() != given[0].data_ptr() or b.data_ptr() != given[1].data_ptr():
+        return
     if key not in _plans:
         if len(_plans) >= _MAX_PLANS:
             _plans.clear()
@@ -198,7 +254,9 @@ def keep_plan(key: tuple, memo_key: tuple, memo: dict, kernel, a, b, c, **extra)
     kernel = getattr(kernel, "kernel", kernel)                # the launch object behind its tunable wrapper
     if a.get_device() < 0 or memo_key not in memo or not isinstance(kernel, HipKernel):
         return
-    _plans[key] = (PlannedLaunch(kernel, a, b, c, memo[memo_key], extra), memo_key)
+    plan = PlannedLaunch(kernel, a, b, c, memo[memo_key], extra)
+    _plans[key] = (plan, memo_key)
+    launch_module().keep(plan_tag(key[0]), *given, c, bytes(plan.template), plan.scratch, plan.slices, plan.atomic, memo_key, plan.cfg)
 
 
 class _BoundLaunch:

@@ -18,7 +18,7 @@ from typing import Dict, Optional, Tuple
 
 import torch
 
-from tritonix_amd import _C
+from tritonix_amd import _C, kernel as _kernel
 from tritonix_amd.kernel import _stream_of, cdiv
 
 __all__ = ["conv2d_forward", "conv2d_forward_kernel", "torch_conv2d_forward", "output_size", "candidate_configs"]
@@ -93,6 +93,9 @@ def _scratch(nbytes: int, device) -> Optional[torch.Tensor]:
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
     except torch.OutOfMemoryError:
         return None
+
+
+_own_scratch = _scratch
 
 
 def _args(out, input, weight, bias, batch, c_in, h_in, w_in, c_out, filter_h, filter_w, stride, padding, dilation,
@@ -290,7 +293,10 @@ def _launch_planned(input, weight, bias, stride, padding, dilation) -> Optional[
             return None
         if len(_PLANS) >= _MAX_PLANS:
             _PLANS.clear()
+            if _kernel._launch is not None:
+                _kernel._launch.forget_convs()
         plan = _PLANS[key] = (a, (n, c_out, h_out, w_out), need)
+        _kernel.launch_module().keep_conv(input, weight, bias, stride, padding, dilation, bytes(a), plan[1], need)
     template, shape, need = plan
     a = _C.Conv2dArgs.from_buffer_copy(template)          # its own copy: calls from several threads share the template
     out = input.new_empty(shape)
@@ -330,6 +336,12 @@ def conv2d_forward(
     does (with ``TRITONIX_AUTOTUNE=0`` in the environment it launches the library's built-in choice instead); ``config={"BLOCK_SIZE_M", "BLOCK_SIZE_N", "BLOCK_SIZE_K"[, "GROUP_SIZE_M"][, "LOADER"]}`` launches that tile
     (all three sizes 0: the library's own choice; ``LOADER`` is "auto", "registers", "dma" or "gemm").
     Returns a new [N, C_OUT, H_OUT, W_OUT] tensor of the input's dtype."""
+    # the library's own choice for sizes met before: one call of the native side, which answers None to anything out of the
+    # ordinary (and where the scratch is somebody else's business)
+    if config is None and _kernel._launch is not None and _scratch is _own_scratch and os.environ.get("TRITONIX_AUTOTUNE", "1") in ("0", "false", "False"):
+        out = _kernel._launch.conv(input, weight, bias, stride, padding, dilation)
+        if out is not None:
+            return out
     assert input.is_contiguous(), "Input must be contiguous NCHW"
     assert weight.is_contiguous(), "Weight must be contiguous KCRS"
     n, c_in, h_in, w_in = input.shape

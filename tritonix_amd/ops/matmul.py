@@ -33,6 +33,7 @@ import os
 
 import torch
 
+from tritonix_amd import kernel as _kernel
 from tritonix_amd.autotune import Choice, PowerOfTwo, Range, tunable
 from tritonix_amd.dispatcher import dynamic_dispatch
 from tritonix_amd.kernel import HipKernel, cdiv, keep_plan, out_dtype_for, plan_key, planned
@@ -378,6 +379,9 @@ def triton_matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     ``matmul`` refer to it.  ``hip_matmul`` is the same function.  For thin problems the tuned config may carry a
     K split (``_tile_or_split``).
     """
+    c = _kernel.product(0, a, b, _matmul_cfg, matmul_kernel.kernel.pre_run_hooks)
+    if c is not None:
+        return c
     pkey = plan_key("matmul", a, b)
     plan = planned(pkey, _matmul_cfg)
     if plan is not None:
@@ -392,8 +396,7 @@ def triton_matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
         _matmul_cfg[key] = _tile_or_split(a, b, key)
     c = run_memoised(_matmul_cfg, "matmul", key, matmul_kernel, lambda cfg: _launch_matmul(a, b, cfg),
                      lambda: default_config(a, b))
-    if a is given[0] and b is given[1]:          # operands that had to be copied first keep the long way
-        keep_plan(pkey, key, _matmul_cfg, matmul_kernel, a, b, c)
+    keep_plan(pkey, key, _matmul_cfg, matmul_kernel, a, b, c, given)
     return c
 
 
@@ -406,6 +409,9 @@ def matmul_splitk(a: torch.Tensor, b: torch.Tensor, split_k: int = 4) -> torch.T
     As in the reference (tritonix/ops/matmul.py:280-288) ``split_k`` only keys
     the config memo; the split factor launched is the one the tuner picked.
     """
+    c = _kernel.product(_kernel.plan_tag(("splitk", split_k)), a, b, _splitk_cfg, gemm_splitk_kernel.kernel.pre_run_hooks)
+    if c is not None:
+        return c
     pkey = plan_key(("splitk", split_k), a, b)
     plan = planned(pkey, _splitk_cfg)
     if plan is not None:
@@ -418,8 +424,7 @@ def matmul_splitk(a: torch.Tensor, b: torch.Tensor, split_k: int = 4) -> torch.T
     key = (m, n, k, split_k, a.dtype, layout)
     c = run_memoised(_splitk_cfg, "matmul_splitk", key, gemm_splitk_kernel, lambda cfg: _launch_splitk(a, b, cfg),
                      lambda: default_config(a, b, split=True))
-    if a is given[0] and b is given[1]:
-        keep_plan(pkey, key, _splitk_cfg, gemm_splitk_kernel, a, b, c)
+    keep_plan(pkey, key, _splitk_cfg, gemm_splitk_kernel, a, b, c, given)
     return c
 
 

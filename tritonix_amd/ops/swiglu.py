@@ -19,6 +19,7 @@ from __future__ import annotations
 
 import torch
 
+from tritonix_amd import kernel as _kernel
 from tritonix_amd.autotune import Choice, PowerOfTwo, Range, tunable
 from tritonix_amd.kernel import HipKernel, cdiv, keep_plan, plan_key, planned
 import importlib
@@ -167,6 +168,9 @@ _glu_cfg = {}
 
 def glu(x: torch.Tensor, w12: torch.Tensor, activation: str = "silu") -> torch.Tensor:
     """``act(x @ w12[:, 0::2]) * (x @ w12[:, 1::2])`` -> ``[m, n/2]``, tile config tuned once per shape."""
+    z = _kernel.product(_kernel.plan_tag(("glu", activation)), x, w12, _glu_cfg, glu_kernel.kernel.pre_run_hooks)
+    if z is not None:
+        return z
     pkey = plan_key(("glu", activation), x, w12)
     plan = planned(pkey, _glu_cfg)
     if plan is not None:
@@ -184,8 +188,7 @@ def glu(x: torch.Tensor, w12: torch.Tensor, activation: str = "silu") -> torch.T
     key = (m, n, k, x.dtype, layout)
     z = _mm.run_memoised(_glu_cfg, "glu", key, glu_kernel, lambda cfg: _launch_glu(x, w12, cfg, activation),
                          lambda: _mm.default_config(x, w12))
-    if x is given[0] and w12 is given[1]:
-        keep_plan(pkey, key, _glu_cfg, glu_kernel, x, w12, z, activation=activation)
+    keep_plan(pkey, key, _glu_cfg, glu_kernel, x, w12, z, given, activation=activation)
     return z
 
 
