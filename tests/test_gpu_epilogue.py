@@ -83,3 +83,22 @@ def test_edges_of_a_wave_tile(tile, cut):
         assert torch.equal(got[1:m + 1, 1:n + 1], want), (m, n)
         got[1:m + 1, 1:n + 1] = 7.0
         assert bool((got == 7.0).all()), f"written outside C at {(m, n)}"
+
+
+@pytest.mark.parametrize("cut", [2, 4, 7, 9])
+@pytest.mark.parametrize("tile", [(32, 64, 4, 2), (32, 128, 4, 2), (64, 64, 4, 2), (64, 128, 8, 2), (128, 64, 4, 2), (128, 128, 8, 2)])
+def test_slices_of_tiles_that_share_a_compute_unit(tile, cut):
+    """Tiles of few registers add the slices of a cut in small batches: slice counts around a batch, bit for bit (small
+    integers, exact in every partial sum), with rows that end inside the first and the last row-block."""
+    from tritonix_amd.ops.matmul import matmul_kernel
+
+    bm, bn, nw, st = tile
+    gen = torch.Generator("cpu").manual_seed(bm + bn + cut)
+    k, n = 64 * 2 * cut, 2 * bn - 8
+    for m in (3, bm, bm + 17):
+        a = torch.randint(-2, 3, (m, k), generator=gen).bfloat16()
+        b = torch.randint(-1, 2, (k, n), generator=gen).bfloat16()
+        c = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+        matmul_kernel[(1, 1)](a.cuda(), b.cuda(), c, m, n, k, k, 1, n, 1, n, 1, block_m=bm, block_n=bn, block_k=64, group_m=8,
+                              num_stages=st, num_warps=nw, split_k=cut)
+        assert torch.equal(c.cpu(), (a.float() @ b.float()).bfloat16()), m

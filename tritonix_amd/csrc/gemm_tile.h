@@ -603,6 +603,28 @@ struct SliceSrc {
   bool rezero;             // atomic reduction: the one slice holds the finished sums; it is cleared again after the read
 };
 
+// Workgroups of a tile that a CU is to hold at once, as many as the ring's LDS allows, and the registers a lane may then
+// use.  Left to itself the compiler takes all that the hand-over of cut tiles can use (its loads in flight), which the
+// launches that cut nothing pay for too: 64x128 tiles of 8 waves on 152 registers, one workgroup on a CU instead of two,
+// ran conv2d's 1x1 layer of 1088 -> 320 channels on 14x14, batch 32, in 28.5 us; on 110 registers in 20.5.  NEED: accumulators,
+// two sets of fragments and what addresses take; a tile that needs more than its share keeps fewer workgroups resident
+// (no tile spills for it).
+template <class C> struct Residency {
+  static constexpr int LDS = C::LDS_BYTES > EpiStage<C>::BYTES ? C::LDS_BYTES : EpiStage<C>::BYTES;
+  static constexpr int ACC = C::TM * C::TN * C::ACC_N;
+  static constexpr int NEED = ACC + ACC / 8 + (C::TM + C::TN) * 8 + 24;
+  static constexpr int regs_of(int wgs) { return 512 / (wgs * C::NW / 4) / 8 * 8; }
+  static constexpr int fit() {
+    int r = 163840 / LDS;
+    if (r * C::NW > 32) r = 32 / C::NW;
+    while (r > 1 && regs_of(r) < NEED) --r;
+    return r;
+  }
+  static constexpr int WGS = fit();
+  static constexpr int WAVES = WGS * C::NW / 4;         // per SIMD
+  static constexpr int REGS = regs_of(WGS);
+};
+
 // largest divisor of n that is <= cap
 constexpr int slice_batch(int n, int cap) {
   int g = cap < n ? cap : n;
@@ -617,7 +639,10 @@ constexpr int slice_batch(int n, int cap) {
 template <class C, class ACC>
 __device__ __forceinline__ void collect_slices(ACC (&acc)[C::TM][C::TN], const SliceSrc& src, int lane, int64_t rows_left) {
   constexpr int NGRP = C::ACC_N / 4, NQ = C::TN * NGRP, G = C::TM * NQ;
-  constexpr int CG = slice_batch(G, G == 32 ? 8 : 16), ZB = G > 8 ? 2 : G == 8 ? 4 : 8;
+  constexpr int CG = slice_batch(G, G == 32 ? 8 : 16);
+  constexpr int ROOM = (Residency<C>::REGS - 32) / (4 * CG) - 1;        // slices of CG groups beside their sums
+  constexpr int ZCAP = G > 8 ? 2 : G == 8 ? 4 : 8;
+  constexpr int ZB = ROOM >= ZCAP ? ZCAP : ROOM >= 4 ? 4 : ROOM >= 2 ? 2 : 1;
   typedef std::remove_reference_t<decltype(acc[0][0][0])> acc_s;
   typedef acc_s acc4 __attribute__((ext_vector_type(4)));
   const __amdgpu_buffer_rsrc_t win = agent_window(src.base);
@@ -1076,7 +1101,7 @@ constexpr int GATHER_TABLE_BYTES = 8192;
 // pixel's, kept in a register, plus the chunk's (filter tap, channels), read once per slab from a table in LDS.  Chunks
 // past the end of k get an offset outside the buffer and arrive as zeros.
 template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false, bool AT = false, bool PAIR = false>
-__global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(GemmParams p) {
+__global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void gemm_tile_kernel(GemmParams p) {
   constexpr int ES = C::ES, BM = C::BM, BN = C::BN, BK = C::BK, NW = C::NW, STAGES = C::STAGES;
   constexpr int MI = C::MI, TM = C::TM, TN = C::TN;
   static_assert(GATHER ? C::VALID_GATHER : C::VALID, "tile configuration not supported by this kernel");
