@@ -289,7 +289,7 @@ int tnx_conv2d_forward(const tnx_conv2d_args* args);
 size_t tnx_conv2d_workspace_bytes(const tnx_conv2d_args* args);
 
 /* For tests and tooling: the packed route with tile number `tile` of the type's table (bfloat16's for TNX_F32; counted from
- * 0) and `split` K slices (1 to 16) instead of the library's choice, on any layer the route can lay out; tile < 0 asks for
+ * 0, the tiles of 32 output channels and of small rings from 32) and `split` K slices (1 to 16) instead of the library's choice, on any layer the route can lay out; tile < 0 asks for
  * that choice.  _info: its scratch bytes, or 0 where there is none, and in info[6] output channels and pixels per
  * tile, waves, ring slots, K slices, and bf16 terms per element.  _forward: launches it in args->workspace. */
 size_t tnx_conv2d_packed_info(const tnx_conv2d_args* args, int tile, int split, int32_t* info);

@@ -153,7 +153,9 @@ def conv_instance_list(quick=False):
 # pixels: what divides a layer into whole rounds of the 256 CUs (256 channels, batch 32, 56x56: 392 tiles of 256 pixels,
 # 448 of 224: two rounds each, the second shorter).
 GATHER_TILES = ((256, 256, 8, 2), (256, 224, 8, 2), (256, 192, 8, 2), (256, 128, 8, 3), (128, 256, 8, 3), (128, 128, 8, 3), (128, 128, 8, 2),
-                (64, 256, 8, 3), (64, 128, 8, 3), (64, 128, 4, 3), (64, 64, 4, 4))
+                (64, 256, 8, 3), (64, 128, 8, 3), (64, 128, 4, 3), (64, 64, 4, 4),
+                # layers of few channels and launches of many short tiles, two to four workgroups on a CU
+                (32, 64, 4, 4), (32, 128, 4, 3), (32, 128, 4, 2), (32, 256, 4, 2), (64, 64, 4, 2), (64, 128, 8, 2))
 
 
 def generate_gather(tiles, gen):

@@ -369,16 +369,25 @@ struct PackedPlan {
   int64_t total_bytes;
 };
 
-// microseconds per round of workgroups and per K slab of one, and workgroups that share a CU, per packed tile
+// What a packed tile costs, in microseconds: `fixed` at its start and end, `slab` per K slab alone on its CU; of `per_cu`
+// that share one, each one more adds `share` of the slabs' time; after whole rounds, a last one of few workgroups costs `last`
+// of a whole one at least.
 struct GatherCost {
-  int bm, bn, nw, stages;
-  double fixed, slab;
-  int per_cu;
+  int bm, bn, nw, stages, per_cu;
+  double fixed, slab, share, last;
 };
 static const GatherCost GATHER_COST[] = {
-    {256, 256, 8, 2, 9.5, 1.12, 1}, {256, 224, 8, 2, 8.2, 1.03, 1}, {256, 192, 8, 2, 5.8, 0.92, 1}, {256, 128, 8, 3, 5.2, 0.555, 1},
-    {128, 256, 8, 3, 5.1, 0.584, 1}, {128, 128, 8, 3, 3.1, 0.341, 1}, {128, 128, 8, 2, 2.9, 0.935, 2}, {64, 256, 8, 3, 2.8, 0.422, 1},
-    {64, 128, 8, 3, 1.8, 0.483, 2}, {64, 128, 4, 3, 2.6, 0.481, 2}, {64, 64, 4, 4, 1.3, 0.272, 2}};
+    {256, 256, 8, 2, 1, 2.24, 1.127, 0.00, 1.00}, {256, 224, 8, 2, 1, 2.90, 1.033, 0.00, 0.92},
+    {256, 192, 8, 2, 1, 2.57, 0.888, 0.00, 0.85}, {256, 128, 8, 3, 1, 2.26, 0.572, 0.00, 1.00},
+    {128, 256, 8, 3, 1, 2.42, 0.610, 0.00, 0.88}, {128, 128, 8, 3, 1, 1.70, 0.331, 0.00, 1.00},
+    {128, 128, 8, 2, 2, 0.87, 0.522, 0.30, 0.80}, {64, 256, 8, 3, 1, 1.90, 0.388, 0.00, 0.92},
+    {64, 128, 8, 3, 2, 1.01, 0.251, 0.70, 0.74}, {64, 128, 8, 2, 2, 0.59, 0.440, 0.04, 0.97},
+    {64, 128, 4, 3, 2, 1.18, 0.258, 0.58, 0.70}, {32, 256, 4, 2, 2, 0.86, 0.581, 0.01, 0.83},
+    {64, 64, 4, 4, 2, 0.87, 0.132, 0.89, 1.00}, {64, 64, 4, 2, 4, 0.31, 0.380, 0.10, 0.81},
+    {32, 128, 4, 3, 2, 0.87, 0.208, 0.51, 0.94}, {32, 128, 4, 2, 3, 0.37, 0.406, 0.11, 0.75},
+    {32, 64, 4, 4, 2, 0.68, 0.105, 0.77, 1.00}};
+// tile numbers of tnx_conv2d_packed_info / _forward: the first tiles of the table from 0, those of few channels or small rings from 32
+static constexpr int FIRST_SMALL = 11, SMALL_FROM = 32;
 static const GatherCost* gather_cost(const GatherEntry& e) {
   for (const GatherCost& c : GATHER_COST)
     if (c.bm == e.bm && c.bn == e.bn && c.nw == e.nw && c.stages == e.stages) return &c;
@@ -387,6 +396,24 @@ static const GatherCost* gather_cost(const GatherEntry& e) {
 
 static constexpr double PAIR_SLAB = 1.3;
 static constexpr double PASS_US = 9.0;     // the pass over the operands and the second launch, apart from the bytes
+
+// Modelled microseconds of the GEMM over packed operands: `tiles` tiles of kt K slabs, cut `s` ways; `bytes` of input, as given
+// and packed (what the caches cannot hold arrives up to a fifth slower).
+static double gather_time(const GatherCost& c, int64_t tiles, int64_t kt, int s, bool pair, double bytes) {
+  const double slow = 1.0 + 0.2 * (bytes < 3.0e8 ? bytes / 3.0e8 : 1.0);
+  const double k = (double)((kt + s - 1) / s) * c.slab * (pair ? 1.04 : 1.0) * slow, area = c.bm * c.bn / 16384.0;
+  const double fixed = c.fixed * (pair ? 1.62 : 1.0);
+  auto together = [&](double n) { return fixed + k * (1.0 + (n - 1.0) * c.share); };
+  const int64_t slots = 256 * c.per_cu, full = tiles * s / slots, rem = tiles * s % slots;
+  double t = (double)full * together(c.per_cu);
+  if (rem && !full) t = together((double)((rem + 255) / 256));
+  else if (rem) {
+    const double n = (double)rem / 256.0;
+    t += n < 1.0 ? together(1.0) * (c.last + (1.0 - c.last) * n) : together(n);
+  }
+  if (s > 1) t += 2.2 + 0.27 * s * area + 2.9 * (double)(tiles * s) * area / 256.0;
+  return t;
+}
 
 // Modelled microseconds of the kernel a 16-bit layer has without scratch: rounds of workgroups x K slabs, constants fitted to
 // 636 layers of 3x3 and 5x5 filters (two tiles of the register-staged kernel per CU cost it a third of its slab rate).
@@ -401,6 +428,36 @@ static double unpacked_time(const tnx_conv2d_args* a) {
   return 4.0 + rounds * kt * (r.bcout > 64 ? 1.8 : tiles < 256 ? 1.15 + 0.4 * tiles / 256.0 : 1.55);
 }
 
+// Layers of few multiply-adds per output (packed_plan: `priced`): the packed route, its GEMM modelled at gemm_us, against the
+// kernels that gather for themselves.  Both sides are least-squares fits to 782 such layers (10 % rms each); the choice costs
+// 1.3 % against the better of the two in the mean, the line drawn at the multiply-adds alone cost 10 %.  Few channels out of
+// a small plane stay with the one launch (3 channels of 17x17, 3x3, 45 out: 6.0 us, packed 9.6), many outputs do not (64 images of 3
+// channels, 112x112, 3x3, 64 out: 115 us, packed 55; 128 of 36 channels, 56x56, 1x1 stride 2, 960 out: 200 and 79; float32,
+// 64 of 19 channels, 17x17, 1x1, 1088 out: 49 and 36).  A call of two launches takes the host 11 to 12 us, one launch half of it: 16-bit
+// layers under 12 us keep the one.  The float32 alternative is three launches on operands cut by two of them, 35 us and more
+// for the host: below that it is never the faster call.
+static bool few_taps_packed(const tnx_conv2d_args* a, const PackedPlan& p, double gemm_us, int h_out, int w_out) {
+  const bool f32 = a->dtype == TNX_F32;
+  const double es = f32 ? 4.0 : 2.0;
+  const double out = (double)a->batch * a->c_out * h_out * w_out * es / 5.0e6;                 // in 5 MB: a microsecond of traffic
+  const double in = (double)a->batch * a->c_in * a->h_in * a->w_in * es / 5.0e6;
+  const double moved = (double)p.x_bytes / 5.0e6 + in / p.step_h, weight = (double)p.w_bytes / 5.0e6;
+  const double packed = f32 ? 12.2 + 0.94 * gemm_us + 1.14 * out + 1.30 * moved + 1.04 * weight
+                            : 8.7 + 0.92 * gemm_us + 1.12 * out + 1.62 * moved + 1.15 * weight;
+  tnx_conv2d_args t = *a;
+  if (f32) { t.dtype = TNX_BF16; t.c_in = 3 * a->c_in; }
+  Resolved r;
+  if (resolve(&t, &r, false) != TNX_OK) return true;
+  if (f32 && packed <= 35.0) return true;
+  if (r.gemm) return packed < 9.7 + 1.25 * out + 4.67 * in;
+  const bool wide = r.bcout > 64;
+  const int64_t tiles = (((int64_t)a->batch * h_out * w_out + r.bpix - 1) / r.bpix) * ((a->c_out + r.bcout - 1) / r.bcout);
+  const double k32 = (double)(((int64_t)t.c_in * a->filter_h * a->filter_w + r.bk - 1) / r.bk * r.bk / 32);
+  const double slots = 256.0 * (wide ? 1.53 : f32 ? 3.1 : 2.69), rounds = tiles > slots ? (double)tiles / slots : 1.0;
+  const double alone = f32 ? (wide ? 9.9 : 7.8) + rounds * ((wide ? 0.0 : 1.8) + (wide ? 1.58 : 0.87) * k32) + 1.25 * out + 4.67 * in
+                           : (wide ? 5.95 : 4.55) + rounds * ((wide ? 0.86 : 0.26) + (wide ? 0.80 : 0.84) * k32) + 3.06 * out + 0.57 * in;
+  return packed < 0.95 * alone && alone >= 12.0;
+}
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
 // tile >= 0: that tile of the type's table and that many K slices, whatever the rules below would choose
@@ -412,16 +469,12 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, 
   int32_t h_out = 0, w_out = 0;
   if (check_problem(&t, &h_out, &w_out) != TNX_OK) return false;
   if (f32 ? a->out_f32 == 0 : gemm_problem_ok(a)) return false;
-  // The pass over the operands costs about 4 us of its own, which a short K loop does not pay back: measured on 120 layers,
-  // the kernels that gather for themselves win below 145 multiply-adds per output (3 channels 3x3: 6.4-8.7 against
-  // 10.2-11.7 us; 16 channels 3x3: 8.8 / 11.7), the packed route above (17 channels: 15.5 / 11.9, 24: 13.0 / 11.9, 64 at
-  // 56x56: 38 / 31).  A 1x1 filter (here with a stride) reads every input element once either way, so its line lies higher
-  // (256 channels, 56x56: 20.0 / 24.0; 512, 28x28: 23.6 / 19.1).  float32 has three terms per element and its alternative
-  // an extra pass over both operands.
+  // The pass over the operands and a second launch do not always pay.  From 145 multiply-adds per output on (257 for a 1x1
+  // filter, here with a stride, which reads every input element once either way) they did on all but 0.2 % of 654 layers; below
+  // that the route is priced against the kernels that gather for themselves, further down.
   const int64_t macs = (int64_t)a->c_in * a->filter_h * a->filter_w;
-  if (tile >= 0) {
-    if (split < 1 || split > 16) return false;
-  } else if (f32 ? macs <= 48 : macs <= (a->filter_h * a->filter_w == 1 ? 256 : 144)) return false;
+  const bool priced = tile < 0 && macs <= (f32 ? 48 : a->filter_h * a->filter_w == 1 ? 256 : 144);
+  if (tile >= 0 && (split < 1 || split > 16)) return false;
   *p = PackedPlan{};
   p->h_out = h_out; p->w_out = w_out;
   // a filter one row high reads only every stride_h-th input row: only those are packed (likewise for columns)
@@ -451,11 +504,12 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, 
   const int64_t lim = (1ll << 31) - 4096;
   if (p->n_total >= lim || p->x_bytes >= lim || p->w_bytes >= lim || (int64_t)a->c_out * kt * 8 >= lim) return false;
 
-  // Tile and K cut with the smallest modelled time: rounds of workgroups x (fixed + per K slab), with the constants of
-  // GATHER_COST; a round is one workgroup per CU, two where two fit its LDS, and a last, partial one costs 0.9 of a
-  // full one.  A K cut adds its hand-over.  Constants and form are a least-squares fit to 1,500 measured (layer, tile, cut)
-  // triples on 120 layers; choosing by it costs 1.5 % against the best measured tile in the mean, 12 % at worst on
-  // all but one.
+  // Tile and K cut with the smallest modelled time (gather_time): constants and form are a least-squares fit to 82,000 measured
+  // (layer, tile, cut) triples on 2,200 layers; choosing by it costs 1.5 % against the best measured tile in the mean.
+  // The tiles of 32 channels and those of two slots, several of which share a CU, win on layers of up to 64 channels and on
+  // launches of many short tiles: 128 images of 64 channels, 28x28, 29 out: 28.5 -> 22 us, by 7 % on layers of up to 32
+  // channels in the mean, by 3 % on the others.
+  const double in_bytes = (double)p->x_bytes + (double)a->batch * a->c_in * a->h_in * a->w_in * (f32 ? 4 : 2) / p->step_h;
   double best = 1e300;
   int ng = 0, number = 0;
   const GatherGroup* const* g = tnx_gather_groups(&ng);
@@ -464,24 +518,21 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, 
       const GatherEntry& e = g[i]->entries[j];
       if (e.dtype != t.dtype) continue;
       if (tile >= 0) {
+        if (number == FIRST_SMALL) number = SMALL_FROM;
         if (number++ == tile) { p->e = &e; p->split = split; }
         continue;
       }
       const GatherCost* cost = gather_cost(e);
       if (!cost) continue;
       const int64_t tiles = ((a->c_out + e.bm - 1) / e.bm) * ((p->n_total + e.bn - 1) / e.bn);
-      const double area = e.bm * e.bn / 65536.0;
-      for (int s = 1; s <= 16; s *= 2) {
-        if (s > 1 && (kt / s < 4 || tiles * s > 512)) break;
-        const int64_t slots = 256 * cost->per_cu, full = tiles * s / slots, rem = tiles * s % slots;
-        double rounds = (double)full;
-        if (rem) rounds += rem > 256 * (cost->per_cu - 1) ? 0.9 : 0.9 * (0.5 + 0.5 * (double)rem / (double)slots);
-        double c = rounds * (cost->fixed + cost->slab * (p->terms == 2 ? PAIR_SLAB : 1.0) * (double)((kt + s - 1) / s));
-        if (s > 1) c += 2.2 + 3.0 * s * area + 1.8 * area;
+      for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        if (s > 1 && (kt / s < 3 || tiles * s > 800)) break;
+        const double c = gather_time(*cost, tiles, kt, s, p->terms == 2, in_bytes);
         if (c < best) { best = c; p->e = &e; p->split = s; }
       }
     }
   if (!p->e) return false;
+  if (priced && !few_taps_packed(a, *p, best, h_out, w_out)) return false;
   // A wide padding (as a dilated filter has it) makes the packed image a multiple of the input, which the lines above do not
   // know.  From twice the input on the pass is priced, at the 5 TB/s it moves (what does not fit the memory-side cache costs the
   // GEMM twice its bytes more), against the kernel that needs none: 8 images of 2048 channels, 33x33 (packed 105x105), 256 out, 3x3:
