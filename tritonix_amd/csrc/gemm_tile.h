@@ -702,6 +702,23 @@ __device__ __forceinline__ float bias_value(const uint8_t* bias, int row, int dt
   return __builtin_bit_cast(float, (uint32_t)((const uint16_t*)bias)[row] << 16);
 }
 
+// The bias of a lane's row in each of TM row-blocks, for rows_left >= 1 rows (rows past them get the last one's).  All the loads
+// are under way before the first value is converted: one memory round trip, where a value at a time took TM of them.
+template <int TM, int MI>
+__device__ __forceinline__ void bias_of_rows(const uint8_t* bias, int dtype, int row0, int rows_left, int lane, float (&out)[TM]) {
+  uint32_t raw[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int r = i * MI + lane % MI, row = row0 + (r < rows_left ? r : rows_left - 1);
+    raw[i] = dtype == DT_F32 ? ((const uint32_t*)bias)[row] : (uint32_t)((const uint16_t*)bias)[row];
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+    out[i] = dtype == DT_F32   ? __builtin_bit_cast(float, raw[i])
+             : dtype == DT_F16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)raw[i])
+                               : __builtin_bit_cast(float, raw[i] << 16);
+}
+
 // How the lanes of a wave share the 16-byte output chunks of one row-block (ROWS rows of CPRW chunks each), 64 chunks per
 // pass.  EVEN: a lane's chunk column is the same in every pass and its row RSTEP further on.
 template <int ROWS, int CPRW> struct RowPasses {
@@ -746,11 +763,7 @@ __device__ __forceinline__ void epilogue_store(ACC (&acc)[C::TM][C::TN], uint8_t
   constexpr bool WITH_BIAS = BIAS && std::is_same<acc_s, float>::value && !GLU;
   float bias_rows[WITH_BIAS ? C::TM : 1] = {};
   if constexpr (WITH_BIAS) {
-    if (bias) {
-#pragma unroll
-      for (int i = 0; i < C::TM; ++i)
-        if (i * MI + lane % MI < rows_left) bias_rows[i] = bias_value(bias, (int)gm0 + i * MI + lane % MI, bias_dtype);
-    }
+    if (bias) bias_of_rows<C::TM, MI>(bias, bias_dtype, (int)gm0, rows_left, lane, bias_rows);
   }
   // this lane's places: row of the row-block, columns of the chunk that exist, strip address, address in C
   int l_row[RP::NL], l_cols[RP::NL];
@@ -1002,11 +1015,7 @@ __device__ __forceinline__ void epilogue_store_conv(ACC (&acc)[C::TM][C::TN], ui
   if (gm0 >= g.c_out) return;
   const int rows_left = g.c_out - gm0 < C::WTM ? g.c_out - gm0 : C::WTM;
   float bias_rows[C::TM] = {};
-  if (g.bias) {
-#pragma unroll
-    for (int i = 0; i < C::TM; ++i)
-      if (i * MI + lane % MI < rows_left) bias_rows[i] = bias_value(g.bias, gm0 + i * MI + lane % MI, g.bias_dtype);
-  }
+  if (g.bias) bias_of_rows<C::TM, MI>(g.bias, g.bias_dtype, gm0, rows_left, lane, bias_rows);
   const int64_t plane = (int64_t)g.h_out * g.w_out;
   // this lane's places: row of the row-block, pixels of the chunk that exist, strip address, address in the output
   int l_row[RP::NL], l_valid[RP::NL];
