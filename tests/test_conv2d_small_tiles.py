@@ -71,3 +71,22 @@ def test_few_multiply_adds(layer, dtype, device, monkeypatch):
     bound = unit * ref.abs() + (c * r * s * 2.0 ** -24 + (2.0 ** -16 if dtype == torch.float32 else 0.0)) * mag + 1e-7
     out = conv2d_forward(x.to(device), wt.to(device), b.to(device), stride, padding, dilation)
     assert ((out.cpu().double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("layer", [(3, 200, 14, 14, 30), (2, 64, 33, 33, 640), (5, 23, 17, 17, 70), (1, 130, 7, 7, 129), (16, 3, 33, 33, 515),
+                                   (9, 1000, 9, 11, 61)])
+def test_images_of_a_1x1_layer(layer, dtype, device, monkeypatch):
+    """1x1 layers on every kind of tile the choice gives them: channels, pixels and planes that end inside a tile."""
+    from tritonix.ops.conv2d import conv2d_forward
+
+    monkeypatch.setenv("TRITONIX_AUTOTUNE", "0")
+    n, c, h, w, k = layer
+    g = torch.Generator().manual_seed(n + c)
+    x, wt, b = torch.randn(n, c, h, w, generator=g).to(dtype), (torch.randn(k, c, 1, 1, generator=g) / c ** 0.5).to(dtype), torch.randn(k, generator=g).to(dtype)
+    ref = torch.nn.functional.conv2d(x.double(), wt.double(), b.double())
+    mag = torch.nn.functional.conv2d(x.double().abs(), wt.double().abs(), b.double().abs())
+    bound = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype] * ref.abs() + c * 2.0 ** -24 * mag + 1e-7
+    out = conv2d_forward(x.to(device), wt.to(device), b.to(device))
+    assert ((out.cpu().double() - ref).abs() <= bound).all()

@@ -176,8 +176,49 @@ static bool gemm_problem_ok(const tnx_conv2d_args* a) {
   return a->filter_h == 1 && a->filter_w == 1 && a->stride_h == 1 && a->stride_w == 1 && a->pad_h == 0 && a->pad_w == 0;
 }
 
-// Built-in tile for that GEMM: 128 x 128, narrowed to 64 channels or 64 pixels where the layer is that small or the
-// grid would leave CUs idle (measured on the 1x1 layers of a ResNet-50 at batch 8, 32 and 128).
+// What a tile of that GEMM costs, in microseconds: `fixed` at its start and end, `slab` per K slab alone on its CU; of
+// `per_cu` that share one, each one more adds `share` of the slabs' time; after whole rounds, a last one of few workgroups costs `last` of
+// a whole one at least; `tail` for a last slab that is not whole; per 5 MB of output `store`, and `odd` more where rows of
+// the output start off 16 bytes (narrow tiles then write more pieces of cache lines).
+struct ImageCost {
+  int bm, bn, nw, stages, per_cu;
+  double fixed, slab, share, last, tail, store, odd;
+};
+static const ImageCost IMAGE_COST[] = {
+    {128, 128, 8, 2, 2, 1.70, 0.408, 0.69, 0.97, 0.53, 0.69, 1.37},
+    {128, 128, 8, 3, 1, 2.17, 0.323, 0.00, 1.00, 0.24, 0.97, 1.35},
+    {64, 256, 8, 2, 2, 1.95, 0.611, 0.55, 0.77, 0.34, 0.44, 0.81},
+    {128, 64, 8, 2, 3, 1.11, 0.271, 0.66, 0.95, 0.45, 0.97, 1.12},
+    {128, 64, 8, 3, 2, 1.46, 0.200, 1.14, 0.90, 0.27, 1.06, 1.01},
+    {64, 128, 8, 2, 3, 1.35, 0.398, 0.49, 0.83, 0.26, 0.74, 0.92},
+    {64, 128, 8, 3, 2, 1.73, 0.301, 0.80, 0.72, 0.10, 0.75, 0.92},
+    {64, 64, 4, 3, 3, 1.42, 0.227, 0.60, 0.76, 0.30, 0.67, 1.07},
+    {32, 128, 4, 2, 4, 1.40, 0.346, 0.40, 0.84, 0.56, 0.40, 1.13},
+    {32, 64, 4, 2, 6, 0.85, 0.206, 0.44, 0.66, 0.32, 1.05, 1.03},
+    {32, 64, 4, 4, 3, 1.15, 0.142, 0.79, 0.63, 0.15, 0.89, 1.60}};
+
+static double image_time(const ImageCost& c, const tnx_conv2d_args* a) {
+  const int64_t hw = (int64_t)a->h_in * a->w_in, kt = (a->c_in + 63) / 64;
+  const int64_t tiles = (((int64_t)a->c_out + c.bm - 1) / c.bm) * ((hw + c.bn - 1) / c.bn) * a->batch;
+  const double k = (double)kt * c.slab * (a->c_in % 8 ? 1.23 : 1.0) * (hw % 8 ? 1.58 : 1.0);
+  const double fixed = c.fixed + (a->c_in % 64 ? c.tail : 0.0);
+  auto together = [&](double n) { return fixed + k * (1.0 + (n - 1.0) * c.share); };
+  const int64_t slots = 256 * c.per_cu, full = tiles / slots, rem = tiles % slots;
+  double t = (double)full * together(c.per_cu);
+  if (rem && !full) t = together((double)((rem + 255) / 256));
+  else if (rem) {
+    const double n = (double)rem / 256.0;
+    t += n < 1.0 ? together(1.0) * (c.last + (1.0 - c.last) * n) : together(n);
+  }
+  const double in = (double)a->batch * a->c_in * (double)hw * 2 / 5.0e6, out = (double)a->batch * a->c_out * (double)hw * (a->out_f32 ? 4 : 2) / 5.0e6;
+  return 3.3 + 0.52 * in + t + (c.store + (hw % 8 ? c.odd : 0.0)) * out;
+}
+
+// Built-in tile for that GEMM.  128 x 128, narrowed to 64 channels or 64 pixels where the layer is that small or the grid would
+// leave CUs idle, stays unless another one's modelled time is 5 % under its own: a least-squares fit to 11,720
+// launches of 700 layers (1 to 128 images of 7x7 to 112x112, 3 to 2048 channels).  Measured on them it takes 0.927x the time
+// of the first rule alone, 34 are slower by 3 % or more, 406 faster by 5 % or more: 16 images of 2034 channels, 14x14, 64 out:
+// 23.7 -> 14.4 us (32x64 tiles, three on a CU); 128 of 23 channels, 33x33, 640 out: 136 -> 82 (64x256: longer runs of a row).
 static bool builtin_gemm_tile(const tnx_conv2d_args* a, int* bcout, int* bpix, int* bk, int* nw, int* st) {
   const int64_t hw = (int64_t)a->h_in * a->w_in;
   int bm = a->c_out <= 64 ? 64 : 128, bn = hw <= 64 ? 64 : 128;
@@ -185,7 +226,17 @@ static bool builtin_gemm_tile(const tnx_conv2d_args* a, int* bcout, int* bpix, i
   if (tiles(bm, bn) < 256 && bm > 64) bm = 64;
   if (tiles(bm, bn) < 256 && bn > 64) bn = 64;
   *bcout = bm; *bpix = bn; *bk = 64;
-  return gemm_tile_for(a->dtype, bm, bn, 64, nw, st);
+  if (!gemm_tile_for(a->dtype, bm, bn, 64, nw, st)) return false;
+  // up to 16 channels out of one K slab in a round of tiles: every tile takes 4.5 to 5 us
+  if (a->c_out <= 16 && a->c_in <= 64 && tiles(bm, bn) <= 256) return true;
+  double best = 0.0;
+  for (const ImageCost& c : IMAGE_COST)
+    if (c.bm == bm && c.bn == bn && c.nw == *nw && c.stages == *st) best = 0.95 * image_time(c, a);
+  for (const ImageCost& c : IMAGE_COST) {
+    const double t = image_time(c, a);
+    if (t < best) { best = t; *bcout = c.bm; *bpix = c.bn; *nw = c.nw; *st = c.stages; }
+  }
+  return true;
 }
 
 static void fill_gemm(const tnx_conv2d_args* a, const Resolved& r, tnx_gemm_args* g, GemmBatch* x) {
