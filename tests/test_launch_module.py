@@ -1,6 +1,7 @@
 """tritonix_amd/_launch.so (csrc/launch.cpp): repeated calls without the interpreter.  It may answer only what the ordinary path
 would do alike; everything else is None and goes the long way."""
 import importlib
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 import torch
@@ -90,3 +91,30 @@ def test_split_gated_and_conv_calls(built_in, device):
         assert (y.double() - ref).norm() <= 2 ** -10 * ref.norm()
     with pytest.raises(AssertionError):
         conv.conv2d_forward(x.transpose(2, 3), w, bias, (1, 1), (1, 1), (1, 1))
+
+
+@pytest.mark.gpu
+def test_threads_repeat_kept_calls_on_streams_of_their_own(built_in, device):
+    """The interpreter lock is given back around the launch, so calls of several threads interleave there: same bits, plans kept
+    and dropped meanwhile."""
+    gen = torch.Generator(device).manual_seed(2)
+    a, b = torch.randn(16, 4096, generator=gen, device=device).bfloat16(), torch.randn(4096, 256, generator=gen, device=device).bfloat16()
+    f, g = torch.randn(300, 640, generator=gen, device=device), torch.randn(640, 320, generator=gen, device=device)
+    x, w = torch.randn(2, 24, 14, 14, generator=gen, device=device).half(), torch.randn(32, 24, 3, 3, generator=gen, device=device).half()
+    calls = [lambda: mm.matmul_splitk(a, b), lambda: mm.triton_matmul(f, g), lambda: conv.conv2d_forward(x, w, None, (1, 1), (1, 1), (1, 1))]
+    want = [_met(c) for c in calls]
+    torch.cuda.synchronize()
+
+    def work(turn):
+        stream, wrong = torch.cuda.Stream(device), 0
+        with torch.cuda.stream(stream):
+            for i in range(60):
+                got = calls[(turn + i) % 3]()
+                stream.synchronize()
+                wrong += not torch.equal(got, want[(turn + i) % 3])
+                if turn == 0 and i % 20 == 10:
+                    kernel._plans.clear()
+        return wrong
+
+    with ThreadPoolExecutor(4) as pool:
+        assert list(pool.map(work, range(4))) == [0] * 4

@@ -8,7 +8,8 @@
 // The entry points are looked up in the library that tritonix_amd/_C.py has loaded (their addresses are handed to bind()), the
 // structs are the header's.  Every function answers None where the ordinary path has to take the call: a size not kept, a hook,
 // a replaced config, a tensor on another than the current device, a subclass that dispatches in Python, an allocation that
-// failed, a status other than TNX_OK.  That path then raises what is to be raised.  All state is guarded by the interpreter lock.
+// failed, a status other than TNX_OK.  That path then raises what is to be raised.  All state is guarded by the interpreter lock,
+// which no entry of the tables is read without.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -101,11 +102,18 @@ bool operand_key(int64_t tag, const at::Tensor& a, const at::Tensor& b, Key* k) 
   return b.get_device() == k->device;
 }
 
-at::Tensor fresh(at::IntArrayRef shape, at::ScalarType type, const at::Tensor& like) {
-  return at::empty(shape, at::TensorOptions().dtype(type).device(like.device()));
+at::Tensor fresh(at::IntArrayRef shape, at::ScalarType type, c10::DeviceIndex device) {
+  return at::empty(shape, at::TensorOptions().dtype(type).device(c10::Device(c10::DeviceType::CUDA, device)));
 }
 
 bool tensor_arg(PyObject* o) { return THPVariable_Check(o); }
+
+// The interpreter lock is given back while memory is allocated and the launch is queued: both may wait for the GPU (an allocation
+// that frees cached blocks, a full queue), and what the GPU waits for may be a host function or a thread that needs the lock.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
 
 PyObject* none() {
   PyErr_Clear();
@@ -169,7 +177,8 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (products.empty() || !plain(a, 2) || !plain(b, 2) || !operand_key(tag, a, b, &k)) Py_RETURN_NONE;
     const auto hit = products.find(k);
     if (hit == products.end()) Py_RETURN_NONE;
-    // by value: the comparison below and the workspace call run Python, behind which the entry may be forgotten
+    // by value: the comparison and the workspace call below run Python, and the lock is given back, behind which the entry may be
+    // forgotten
     const Product& kept = hit->second;
     const struct { int64_t rows, cols; at::ScalarType type; int64_t scratch, slices; bool atomic; } p = {
         kept.rows, kept.cols, kept.type, kept.scratch, kept.slices, kept.atomic};
@@ -181,8 +190,7 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (PyObject_RichCompareBool(now, config.p, Py_EQ) != 1) return none();
     const c10::DeviceIndex device = (c10::DeviceIndex)k.device;
     if (c10::hip::current_device() != device) Py_RETURN_NONE;
-    const at::Tensor c = fresh({p.rows, p.cols}, p.type, a);
-    g.a = a.data_ptr(); g.b = b.data_ptr(); g.c = c.data_ptr();
+    g.a = a.data_ptr(); g.b = b.data_ptr();
     g.stream = c10::hip::getCurrentHIPStream(device).stream();
     if (p.slices > 0) {
       PyObject* ws = PyObject_CallFunction(fn_workspace, "iKLi", (int)device, (unsigned long long)(uintptr_t)g.stream, (long long)p.slices, (int)p.atomic);
@@ -194,13 +202,19 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t n) {
       g.workspace = (void*)(uintptr_t)ptr;
       g.workspace_bytes = bytes;
     }
+    at::Tensor c;
     int status;
-    if (g.in_dtype == TNX_F32) {
-      at::Tensor scratch;
-      if (p.scratch > 0) scratch = fresh({p.scratch}, at::kByte, a);
-      status = fn_gemm_f32(&g, p.scratch > 0 ? scratch.data_ptr() : nullptr, (size_t)p.scratch);
-    } else {
-      status = fn_gemm(&g);
+    {
+      const Unlocked unlocked;
+      c = fresh({p.rows, p.cols}, p.type, device);
+      g.c = c.data_ptr();
+      if (g.in_dtype == TNX_F32) {
+        at::Tensor scratch;
+        if (p.scratch > 0) scratch = fresh({p.scratch}, at::kByte, device);
+        status = fn_gemm_f32(&g, p.scratch > 0 ? scratch.data_ptr() : nullptr, (size_t)p.scratch);
+      } else {
+        status = fn_gemm(&g);
+      }
     }
     if (status != TNX_OK) Py_RETURN_NONE;
     return THPVariable_Wrap(c);
@@ -271,22 +285,29 @@ PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!conv_key(args, &k)) Py_RETURN_NONE;
     const auto hit = convs.find(k);
     if (hit == convs.end()) Py_RETURN_NONE;
-    const Conv& p = hit->second;
+    const Conv p = hit->second;
     const c10::DeviceIndex device = (c10::DeviceIndex)k.device;
     if (c10::hip::current_device() != device) Py_RETURN_NONE;
     const at::Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]);
     tnx_conv2d_args a = p.args;
-    const at::Tensor y = fresh({p.shape[0], p.shape[1], p.shape[2], p.shape[3]}, x.scalar_type(), x);
-    at::Tensor scratch;
-    if (p.scratch > 0) {
-      scratch = fresh({p.scratch}, at::kByte, x);
-      a.workspace = scratch.data_ptr();
-      a.workspace_bytes = (size_t)p.scratch;
-    }
-    a.input = x.data_ptr(); a.weight = w.data_ptr(); a.output = y.data_ptr();
+    a.input = x.data_ptr(); a.weight = w.data_ptr();
     a.bias = args[2] == Py_None ? nullptr : THPVariable_Unpack(args[2]).data_ptr();
     a.stream = c10::hip::getCurrentHIPStream(device).stream();
-    if (fn_conv(&a) != TNX_OK) Py_RETURN_NONE;
+    at::Tensor y;
+    int status;
+    {
+      const Unlocked unlocked;
+      y = fresh({p.shape[0], p.shape[1], p.shape[2], p.shape[3]}, (at::ScalarType)k.type_a, device);
+      at::Tensor scratch;
+      if (p.scratch > 0) {
+        scratch = fresh({p.scratch}, at::kByte, device);
+        a.workspace = scratch.data_ptr();
+        a.workspace_bytes = (size_t)p.scratch;
+      }
+      a.output = y.data_ptr();
+      status = fn_conv(&a);
+    }
+    if (status != TNX_OK) Py_RETURN_NONE;
     return THPVariable_Wrap(y);
   } catch (...) {
     return none();
