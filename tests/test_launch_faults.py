@@ -1,0 +1,61 @@
+"""What a kept launch (tritonix_amd/_launch.so, tritonix_amd/kernel.py) leaves to go wrong around it: buffers of other threads,
+numbers of operations, launches that fail, a module that is not there."""
+import ctypes
+import importlib
+import weakref
+
+import pytest
+import torch
+
+import tritonix_amd.kernel as kernel
+from tritonix_amd import _C
+
+mm = importlib.import_module("tritonix_amd.ops.matmul")
+GEMM = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p)
+
+
+def test_the_native_side_is_given_the_buffer_itself(monkeypatch):
+    """A pointer alone keeps nothing alive while the interpreter lock is given back."""
+    buf = torch.zeros(64, dtype=torch.uint8)
+    monkeypatch.setattr(kernel, "_workspace", lambda device, stream, nbytes, atomic: buf)
+    assert kernel._workspace_of(0, 0, 64, 0) is buf
+
+
+@pytest.fixture
+def kept_split(monkeypatch, device):
+    """Operands of a K-split product whose launch is kept, and a way to repeat it with other entry points."""
+    monkeypatch.setenv("TRITONIX_AUTOTUNE", "0")
+    kernel._plans.clear()
+    gen = torch.Generator(device).manual_seed(1)
+    a, b = torch.randn(16, 4096, generator=gen, device=device).bfloat16(), torch.randn(4096, 256, generator=gen, device=device).bfloat16()
+    want = [mm.matmul_splitk(a, b) for _ in range(3)][-1]
+    torch.cuda.synchronize()
+    hooks = mm.gemm_splitk_kernel.kernel.pre_run_hooks
+
+    def repeat(gemm, workspace=kernel._workspace_of):
+        kernel._bind(kernel._launch, gemm, workspace)
+        return kernel._launch.product(kernel.plan_tag(("splitk", 4)), a, b, mm._splitk_cfg, hooks)
+
+    yield repeat, want
+    kernel._bind(kernel._launch, _C.load().tnx_gemm)
+
+
+@pytest.mark.gpu
+def test_a_replaced_workspace_lives_until_its_launch_is_queued(kept_split, device):
+    repeat, want = kept_split
+    refs, at_launch = [], []
+
+    def given_away(index, stream, nbytes, atomic):
+        buf = torch.zeros(nbytes, dtype=torch.uint8, device=device)      # (nothing else refers to it: replaced by another thread)
+        refs.append(weakref.ref(buf))
+        return buf
+
+    def launch(p):
+        g = _C.GemmArgs.from_address(p)
+        buf = refs[-1]()
+        at_launch.append(buf is not None and (g.workspace, g.workspace_bytes) == (buf.data_ptr(), buf.numel()))
+        return _C.OK
+
+    assert repeat(GEMM(launch), given_away).shape == want.shape and at_launch == [True]
+    assert refs[-1]() is None
+    assert torch.equal(repeat(_C.load().tnx_gemm), want)

@@ -28,7 +28,7 @@ namespace {
 int (*fn_gemm)(const tnx_gemm_args*) = nullptr;
 int (*fn_gemm_f32)(const tnx_gemm_args*, void*, size_t) = nullptr;
 int (*fn_conv)(const tnx_conv2d_args*) = nullptr;
-PyObject* fn_workspace = nullptr;       // (device index, stream, bytes, atomic) -> (pointer, bytes)
+PyObject* fn_workspace = nullptr;       // (device index, stream, bytes, atomic) -> tensor
 
 // What a launch depends on but its pointers.  Compared and hashed as bytes: zero-filled before it is written.
 struct Key {
@@ -61,6 +61,12 @@ struct Object {                          // a Python reference that goes with it
   Object& operator=(Object&& o) noexcept { std::swap(p, o.p); return *this; }
   ~Object() { Py_XDECREF(p); }
 };
+
+Object taken(PyObject* o) {              // a new reference
+  Object t;
+  t.p = o;
+  return t;
+}
 
 struct Product {
   tnx_gemm_args args;
@@ -192,15 +198,15 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (c10::hip::current_device() != device) Py_RETURN_NONE;
     g.a = a.data_ptr(); g.b = b.data_ptr();
     g.stream = c10::hip::getCurrentHIPStream(device).stream();
+    // held until the launch is queued: while the lock is given back another thread may have the buffer replaced by a larger one
+    // or evicted, and a block that goes back to the stream's pool before then is handed out again -- to the result below, even
+    Object workspace;
     if (p.slices > 0) {
-      PyObject* ws = PyObject_CallFunction(fn_workspace, "iKLi", (int)device, (unsigned long long)(uintptr_t)g.stream, (long long)p.slices, (int)p.atomic);
-      if (!ws) return none();
-      unsigned long long ptr = 0, bytes = 0;
-      const int ok = PyArg_ParseTuple(ws, "KK", &ptr, &bytes);
-      Py_DECREF(ws);
-      if (!ok) return none();
-      g.workspace = (void*)(uintptr_t)ptr;
-      g.workspace_bytes = bytes;
+      workspace = taken(PyObject_CallFunction(fn_workspace, "iKLi", (int)device, (unsigned long long)(uintptr_t)g.stream, (long long)p.slices, (int)p.atomic));
+      if (!workspace.p || !tensor_arg(workspace.p)) return none();
+      const at::Tensor& ws = THPVariable_Unpack(workspace.p);
+      g.workspace = ws.data_ptr();
+      g.workspace_bytes = (size_t)ws.nbytes();
     }
     at::Tensor c;
     int status;

@@ -204,10 +204,10 @@ def plan_tag(tag) -> int:
 
 
 def _workspace_of(index: int, stream: int, nbytes: int, atomic: int):
+    """The buffer itself, for the caller to hold until its launch is queued."""
     import torch
 
-    ws = _workspace(torch.device("cuda", index), stream, nbytes, bool(atomic))
-    return ws.data_ptr(), ws.numel()
+    return _workspace(torch.device("cuda", index), stream, nbytes, bool(atomic))
 
 
 def launch_module():
@@ -219,10 +219,15 @@ def launch_module():
             from tritonix_amd import _launch as module
         except ImportError as err:
             raise RuntimeError(f"tritonix_amd/_launch.so cannot be loaded ({err}): build it with `python -m tritonix_amd.build`") from err
-        at = [ctypes.cast(fn, ctypes.c_void_p).value for fn in (lib.tnx_gemm, lib.tnx_gemm_f32, lib.tnx_conv2d_forward)]
-        module.bind(*at, _workspace_of)
+        _bind(module, lib.tnx_gemm)
         _launch, product = module, module.product
     return _launch
+
+
+def _bind(module, gemm, workspace=_workspace_of) -> None:
+    """Hand the native side its entry points: the library's, with ``gemm`` for 16-bit and int8 products."""
+    lib = _C.load()
+    module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (gemm, lib.tnx_gemm_f32, lib.tnx_conv2d_forward)), workspace)
 
 
 def plan_key(tag, a, b) -> tuple:
