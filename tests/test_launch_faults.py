@@ -2,6 +2,8 @@
 numbers of operations, launches that fail, a module that is not there."""
 import ctypes
 import importlib
+import threading
+import time
 import weakref
 
 import pytest
@@ -19,6 +21,40 @@ def test_the_native_side_is_given_the_buffer_itself(monkeypatch):
     buf = torch.zeros(64, dtype=torch.uint8)
     monkeypatch.setattr(kernel, "_workspace", lambda device, stream, nbytes, atomic: buf)
     assert kernel._workspace_of(0, 0, 64, 0) is buf
+
+
+class _Slow(dict):
+    """Lets the other threads in between a read and what is made of it."""
+
+    def __len__(self):
+        n = super().__len__()
+        time.sleep(0.005)
+        return n
+
+
+def test_operations_asked_for_at_once_get_numbers_of_their_own(monkeypatch):
+    monkeypatch.setattr(kernel, "_tags", _Slow(matmul=0))
+    start, got = threading.Barrier(8), {}
+
+    def ask(i):
+        start.wait()
+        got[i] = (kernel.plan_tag(("at once", i)), kernel.plan_tag(("at once", 0)))
+
+    threads = [threading.Thread(target=ask, args=(i,)) for i in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len({n for n, _ in got.values()}) == 8 and {n for _, n in got.values()} == {got[0][0]}
+    assert all(kernel.plan_tag(("at once", i)) == n for i, (n, _) in got.items())
+
+
+def test_a_number_is_not_given_twice_when_the_tags_are_dropped(monkeypatch):
+    monkeypatch.setattr(kernel, "_tags", {"matmul": 0})
+    monkeypatch.setattr(kernel, "_plans", kernel._Plans())
+    monkeypatch.setattr(kernel, "_MAX_PLANS", 4)
+    numbers = [kernel.plan_tag(("dropped", i)) for i in range(12)]
+    assert len(set(numbers)) == 12 and 0 not in numbers and kernel.plan_tag("matmul") == 0
 
 
 @pytest.fixture

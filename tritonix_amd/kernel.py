@@ -12,6 +12,8 @@ derives its own 1-D grid from the shape and the tile.
 from __future__ import annotations
 
 import ctypes
+import itertools
+import threading
 from collections import OrderedDict
 from typing import Callable, List, Optional, Tuple
 
@@ -183,6 +185,8 @@ _MAX_PLANS = 1024
 # tritonix_amd/_launch.so (csrc/launch.cpp), which repeats a kept launch without the interpreter; loaded with the first of them
 _launch = None
 _tags: dict = {"matmul": 0}
+_tag_numbers = itertools.count(1)
+_tags_lock = threading.Lock()
 
 
 def product(tag: int, a, b, memo: dict, hooks: list):
@@ -192,14 +196,18 @@ def product(tag: int, a, b, memo: dict, hooks: list):
 
 
 def plan_tag(tag) -> int:
-    """A number for the operation of a plan key."""
+    """A number for the operation of a plan key, never another one's: not where threads ask at once, and not after the tags have
+    been dropped, when a thread may still hold an old number."""
     n = _tags.get(tag)
     if n is None:
-        if len(_tags) >= _MAX_PLANS:
-            _plans.clear()
-            _tags.clear()
-            _tags["matmul"] = 0
-        n = _tags[tag] = len(_tags)
+        with _tags_lock:
+            n = _tags.get(tag)
+            if n is None:
+                if len(_tags) >= _MAX_PLANS:
+                    _plans.clear()
+                    _tags.clear()
+                    _tags["matmul"] = 0
+                n = _tags[tag] = next(_tag_numbers)
     return n
 
 
