@@ -57,6 +57,19 @@ def test_a_number_is_not_given_twice_when_the_tags_are_dropped(monkeypatch):
     assert len(set(numbers)) == 12 and 0 not in numbers and kernel.plan_tag("matmul") == 0
 
 
+def test_a_failed_launch_drops_its_workspace_and_raises(monkeypatch):
+    device, buf = torch.device("cuda", 0), torch.zeros(64, dtype=torch.uint8)
+    monkeypatch.setattr(kernel, "_workspaces", type(kernel._workspaces)({kernel._workspace_key(device, 7, False): buf, kernel._workspace_key(device, 8, False): buf}))
+    g = _C.GemmArgs()
+    g.in_dtype, g.split_k = _C.BF16, 4
+    with pytest.raises(RuntimeError):
+        kernel._launch_failed(0, 7, _C.E_WORKSPACE, bytes(g))
+    assert len(kernel._workspaces) == 2                      # refused before anything ran
+    with pytest.raises(RuntimeError):
+        kernel._launch_failed(0, 7, _C.E_HIP, bytes(g))
+    assert list(kernel._workspaces) == [kernel._workspace_key(device, 8, False)]
+
+
 @pytest.fixture
 def kept_split(monkeypatch, device):
     """Operands of a K-split product whose launch is kept, and a way to repeat it with other entry points."""
@@ -94,4 +107,36 @@ def test_a_replaced_workspace_lives_until_its_launch_is_queued(kept_split, devic
 
     assert repeat(GEMM(launch), given_away).shape == want.shape and at_launch == [True]
     assert refs[-1]() is None
+    assert torch.equal(repeat(_C.load().tnx_gemm), want)
+
+
+@pytest.mark.gpu
+def test_a_launch_that_fails_is_raised_and_not_repeated(kept_split, device):
+    repeat, want = kept_split
+    key = kernel._workspace_key(device, kernel._stream_of(0), False)
+    asked = []
+
+    def launch(p):
+        asked.append(_C.GemmArgs.from_address(p).workspace)
+        return _C.E_HIP
+
+    buf = kernel._workspaces[key]
+    with pytest.raises(RuntimeError):
+        repeat(GEMM(launch))
+    assert asked == [buf.data_ptr()] and key not in kernel._workspaces
+    assert torch.equal(repeat(_C.load().tnx_gemm), want) and kernel._workspaces[key] is not buf
+
+
+@pytest.mark.gpu
+def test_an_interrupt_is_not_swallowed(kept_split, device):
+    repeat, want = kept_split
+
+    def raising(error):
+        def workspace(*_):
+            raise error
+        return workspace
+
+    assert repeat(_C.load().tnx_gemm, raising(torch.OutOfMemoryError())) is None          # the ordinary path meets it again
+    with pytest.raises(KeyboardInterrupt):
+        repeat(_C.load().tnx_gemm, raising(KeyboardInterrupt()))
     assert torch.equal(repeat(_C.load().tnx_gemm), want)

@@ -8,8 +8,9 @@
 // The entry points are looked up in the library that tritonix_amd/_C.py has loaded (their addresses are handed to bind()), the
 // structs are the header's.  Every function answers None where the ordinary path has to take the call: a size not kept, a hook,
 // a replaced config, a tensor on another than the current device, a subclass that dispatches in Python, an allocation that
-// failed, a status other than TNX_OK.  That path then raises what is to be raised.  All state is guarded by the interpreter lock,
-// which no entry of the tables is read without.
+// failed, a conv2d status other than TNX_OK.  That path then raises what is to be raised.  A product's status is raised here: its
+// launch may have left counters set in the workspace, which is not to be launched over again.  All state is guarded by the
+// interpreter lock, which no entry of the tables is read without.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -29,6 +30,7 @@ int (*fn_gemm)(const tnx_gemm_args*) = nullptr;
 int (*fn_gemm_f32)(const tnx_gemm_args*, void*, size_t) = nullptr;
 int (*fn_conv)(const tnx_conv2d_args*) = nullptr;
 PyObject* fn_workspace = nullptr;       // (device index, stream, bytes, atomic) -> tensor
+PyObject* fn_failed = nullptr;          // (device index, stream, status, argument struct): raises
 
 // What a launch depends on but its pointers.  Compared and hashed as bytes: zero-filled before it is written.
 struct Key {
@@ -121,22 +123,24 @@ struct Unlocked {
   ~Unlocked() { PyEval_RestoreThread(state); }
 };
 
+// None, whatever Exception is set (the ordinary path meets its cause again); an interrupt or an exit goes on its way
 PyObject* none() {
+  if (PyErr_Occurred() && !PyErr_ExceptionMatches(PyExc_Exception)) return nullptr;
   PyErr_Clear();
   Py_RETURN_NONE;
 }
 
-// bind(tnx_gemm, tnx_gemm_f32, tnx_conv2d_forward, workspace): addresses of the entry points
+// bind(tnx_gemm, tnx_gemm_f32, tnx_conv2d_forward, workspace, failed): addresses of the entry points
 PyObject* bind(PyObject*, PyObject* args) {
   unsigned long long g, f, c;
-  PyObject* w;
-  if (!PyArg_ParseTuple(args, "KKKO", &g, &f, &c, &w)) return nullptr;
+  PyObject *w, *e;
+  if (!PyArg_ParseTuple(args, "KKKOO", &g, &f, &c, &w, &e)) return nullptr;
   fn_gemm = (decltype(fn_gemm))(uintptr_t)g;
   fn_gemm_f32 = (decltype(fn_gemm_f32))(uintptr_t)f;
   fn_conv = (decltype(fn_conv))(uintptr_t)c;
-  Py_INCREF(w);
-  Py_XDECREF(fn_workspace);
-  fn_workspace = w;
+  Object workspace(w), failed(e);
+  std::swap(fn_workspace, workspace.p);
+  std::swap(fn_failed, failed.p);
   Py_RETURN_NONE;
 }
 
@@ -222,7 +226,10 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t n) {
         status = fn_gemm(&g);
       }
     }
-    if (status != TNX_OK) Py_RETURN_NONE;
+    if (status != TNX_OK) {
+      taken(PyObject_CallFunction(fn_failed, "iKiy#", (int)device, (unsigned long long)(uintptr_t)g.stream, status, (const char*)&g, (Py_ssize_t)sizeof g));
+      return PyErr_Occurred() ? nullptr : none();
+    }
     return THPVariable_Wrap(c);
   } catch (...) {
     return none();

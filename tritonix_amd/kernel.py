@@ -218,6 +218,17 @@ def _workspace_of(index: int, stream: int, nbytes: int, atomic: int):
     return _workspace(torch.device("cuda", index), stream, nbytes, bool(atomic))
 
 
+def _launch_failed(index: int, stream: int, status: int, args: bytes) -> None:
+    """What ``PlannedLaunch`` does about a launch that reported an error."""
+    import torch
+
+    g = _C.GemmArgs.from_buffer_copy(args)
+    if status == _C.E_HIP and g.split_k > 1:
+        drop_workspace(torch.device("cuda", index), stream)
+    g.in_dtype = _C.BF16 if g.in_dtype == _C.F32 else g.in_dtype
+    _C.raise_for_status(status, g)
+
+
 def launch_module():
     """``_launch``, bound to the loaded library; a missing build raises, as for the library itself."""
     global _launch, product
@@ -235,7 +246,7 @@ def launch_module():
 def _bind(module, gemm, workspace=_workspace_of) -> None:
     """Hand the native side its entry points: the library's, with ``gemm`` for 16-bit and int8 products."""
     lib = _C.load()
-    module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (gemm, lib.tnx_gemm_f32, lib.tnx_conv2d_forward)), workspace)
+    module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (gemm, lib.tnx_gemm_f32, lib.tnx_conv2d_forward)), workspace, _launch_failed)
 
 
 def plan_key(tag, a, b) -> tuple:
