@@ -4,6 +4,7 @@ import ctypes
 import importlib
 import threading
 import time
+import types
 import weakref
 
 import pytest
@@ -68,6 +69,31 @@ def test_a_failed_launch_drops_its_workspace_and_raises(monkeypatch):
     with pytest.raises(RuntimeError):
         kernel._launch_failed(0, 7, _C.E_HIP, bytes(g))
     assert list(kernel._workspaces) == [kernel._workspace_key(device, 8, False)]
+
+
+def _without_module(monkeypatch, how):
+    """``kernel`` as in a process in which the module cannot be had."""
+    import sys
+
+    import tritonix_amd
+
+    stand_in = None if how == "missing" else types.SimpleNamespace(torch_version="1.0.0")
+    monkeypatch.setitem(sys.modules, "tritonix_amd._launch", stand_in)
+    if how == "missing":
+        monkeypatch.delattr(tritonix_amd, "_launch", raising=False)
+    else:
+        monkeypatch.setattr(tritonix_amd, "_launch", stand_in, raising=False)
+    monkeypatch.setattr(kernel, "_launch", None)
+    monkeypatch.setattr(kernel, "_launch_missing", False, raising=False)
+    monkeypatch.setattr(kernel, "product", lambda *_: None)
+
+
+@pytest.mark.parametrize("how", ["missing", "another torch"])
+def test_without_the_module_the_ordinary_path_stays(monkeypatch, how):
+    _without_module(monkeypatch, how)
+    with pytest.warns(RuntimeWarning):
+        assert kernel.launch_module() is None
+    assert kernel.launch_module() is None and kernel._launch is None          # said once
 
 
 @pytest.fixture
@@ -140,3 +166,19 @@ def test_an_interrupt_is_not_swallowed(kept_split, device):
     with pytest.raises(KeyboardInterrupt):
         repeat(_C.load().tnx_gemm, raising(KeyboardInterrupt()))
     assert torch.equal(repeat(_C.load().tnx_gemm), want)
+
+
+@pytest.mark.gpu
+def test_calls_without_the_module(device, monkeypatch):
+    _without_module(monkeypatch, "missing")
+    monkeypatch.setenv("TRITONIX_AUTOTUNE", "0")
+    kernel._plans.clear()
+    conv = importlib.import_module("tritonix_amd.ops.conv2d.forward")
+    monkeypatch.setattr(conv, "_PLANS", {})
+    a, b = torch.randn(40, 96, device=device).half(), torch.randn(96, 72, device=device).half()
+    x, w = torch.randn(2, 24, 14, 14, device=device).half(), torch.randn(32, 24, 3, 3, device=device).half()
+    with pytest.warns(RuntimeWarning):
+        products = [mm.triton_matmul(a, b) for _ in range(4)]
+        layers = [conv.conv2d_forward(x, w, None, (1, 1), (1, 1), (1, 1)) for _ in range(3)]
+    assert all(torch.equal(p, products[0]) for p in products) and all(torch.equal(y, layers[0]) for y in layers)
+    assert kernel._launch is None and any(plan for plan in kernel._plans.values())

@@ -18,6 +18,7 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/headeronly/version.h>
 
 #include <cstring>
 #include <unordered_map>
@@ -359,4 +360,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", nullptr, -1, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__launch() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__launch() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) {      // whose classes it was compiled against
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

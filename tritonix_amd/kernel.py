@@ -14,6 +14,7 @@ from __future__ import annotations
 import ctypes
 import itertools
 import threading
+import warnings
 from collections import OrderedDict
 from typing import Callable, List, Optional, Tuple
 
@@ -184,6 +185,7 @@ _MAX_PLANS = 1024
 
 # tritonix_amd/_launch.so (csrc/launch.cpp), which repeats a kept launch without the interpreter; loaded with the first of them
 _launch = None
+_launch_missing = False
 _tags: dict = {"matmul": 0}
 _tag_numbers = itertools.count(1)
 _tags_lock = threading.Lock()
@@ -230,15 +232,22 @@ def _launch_failed(index: int, stream: int, status: int, args: bytes) -> None:
 
 
 def launch_module():
-    """``_launch``, bound to the loaded library; a missing build raises, as for the library itself."""
-    global _launch, product
-    if _launch is None:
-        lib = _C.load()
+    """``_launch``, bound to the loaded library, or None where it was not built or was built against another torch: it only
+    repeats what the ordinary path does, which then takes every call."""
+    global _launch, product, _launch_missing
+    if _launch is None and not _launch_missing:
         try:
+            import torch
             from tritonix_amd import _launch as module
-        except ImportError as err:
-            raise RuntimeError(f"tritonix_amd/_launch.so cannot be loaded ({err}): build it with `python -m tritonix_amd.build`") from err
-        _bind(module, lib.tnx_gemm)
+
+            if module.torch_version != torch.__version__.split("+")[0]:
+                raise ImportError(f"built against torch {module.torch_version}, this is {torch.__version__}")
+        except (ImportError, AttributeError) as err:
+            _launch_missing = True
+            warnings.warn(f"tritonix_amd/_launch.so cannot be used ({err}): repeated calls take the interpreter's path, a few "
+                          "microseconds longer; `python -m tritonix_amd.build` builds it", RuntimeWarning, stacklevel=2)
+            return None
+        _bind(module, _C.load().tnx_gemm)
         _launch, product = module, module.product
     return _launch
 
@@ -280,7 +289,9 @@ def keep_plan(key: tuple, memo_key: tuple, memo: dict, kernel, a, b, c, given, *
         return
     plan = PlannedLaunch(kernel, a, b, c, memo[memo_key], extra)
     _plans[key] = (plan, memo_key)
-    launch_module().keep(plan_tag(key[0]), *given, c, bytes(plan.template), plan.scratch, plan.slices, plan.atomic, memo_key, plan.cfg)
+    native = launch_module()
+    if native is not None:
+        native.keep(plan_tag(key[0]), *given, c, bytes(plan.template), plan.scratch, plan.slices, plan.atomic, memo_key, plan.cfg)
 
 
 class _BoundLaunch:

@@ -296,7 +296,9 @@ def _launch_planned(input, weight, bias, stride, padding, dilation) -> Optional[
             if _kernel._launch is not None:
                 _kernel._launch.forget_convs()
         plan = _PLANS[key] = (a, (n, c_out, h_out, w_out), need)
-        _kernel.launch_module().keep_conv(input, weight, bias, stride, padding, dilation, bytes(a), plan[1], need)
+        native = _kernel.launch_module()
+        if native is not None:
+            native.keep_conv(input, weight, bias, stride, padding, dilation, bytes(a), plan[1], need)
     template, shape, need = plan
     a = _C.Conv2dArgs.from_buffer_copy(template)          # its own copy: calls from several threads share the template
     out = input.new_empty(shape)
