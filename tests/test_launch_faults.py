@@ -182,3 +182,25 @@ def test_calls_without_the_module(device, monkeypatch):
         layers = [conv.conv2d_forward(x, w, None, (1, 1), (1, 1), (1, 1)) for _ in range(3)]
     assert all(torch.equal(p, products[0]) for p in products) and all(torch.equal(y, layers[0]) for y in layers)
     assert kernel._launch is None and any(plan for plan in kernel._plans.values())
+
+
+class _Tagged(torch.Tensor):
+    """A subclass like those that carry metadata: results of its methods are of its type."""
+
+
+@pytest.mark.gpu
+def test_a_subclass_keeps_its_type_on_repeated_calls(device, monkeypatch):
+    monkeypatch.setenv("TRITONIX_AUTOTUNE", "0")
+    kernel._plans.clear()
+    conv = importlib.import_module("tritonix_amd.ops.conv2d.forward")
+    x, w = torch.randn(2, 24, 14, 14, device=device).half(), torch.randn(32, 24, 3, 3, device=device).half()
+    want = [conv.conv2d_forward(x, w, None, (1, 1), (1, 1), (1, 1)) for _ in range(3)][-1]
+    for _ in range(3):
+        y = conv.conv2d_forward(x.as_subclass(_Tagged), w, None, (1, 1), (1, 1), (1, 1))
+        assert type(y) is _Tagged and torch.equal(y.as_subclass(torch.Tensor), want)
+    assert type(conv.conv2d_forward(x, torch.nn.Parameter(w), None, (1, 1), (1, 1), (1, 1))) is torch.Tensor
+    a, b = torch.randn(40, 96, device=device).half(), torch.randn(96, 72, device=device).half()
+    want = [mm.triton_matmul(a, b) for _ in range(3)][-1]
+    hooks = mm.matmul_kernel.kernel.pre_run_hooks
+    assert kernel._launch.product(0, a.as_subclass(_Tagged), b, mm._matmul_cfg, hooks) is None
+    assert torch.equal(kernel._launch.product(0, torch.nn.Parameter(a), b, mm._matmul_cfg, hooks), want)

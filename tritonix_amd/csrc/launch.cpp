@@ -7,7 +7,7 @@
 //
 // The entry points are looked up in the library that tritonix_amd/_C.py has loaded (their addresses are handed to bind()), the
 // structs are the header's.  Every function answers None where the ordinary path has to take the call: a size not kept, a hook,
-// a replaced config, a tensor on another than the current device, a subclass that dispatches in Python, an allocation that
+// a replaced config, a tensor on another than the current device, a subclass of torch.Tensor (but Parameter), an allocation that
 // failed, a conv2d status other than TNX_OK.  That path then raises what is to be raised.  A product's status is raised here: its
 // launch may have left counters set in the workspace, which is not to be launched over again.  All state is guarded by the
 // interpreter lock, which no entry of the tables is read without.
@@ -116,6 +116,9 @@ at::Tensor fresh(at::IntArrayRef shape, at::ScalarType type, c10::DeviceIndex de
 }
 
 bool tensor_arg(PyObject* o) { return THPVariable_Check(o); }
+// a torch.Tensor or Parameter itself: a subclass may answer the Python path's calls in its own way, and gives its type to a result
+// that comes from one of its methods (new_empty)
+bool own_tensor(PyObject* o) { return THPVariable_CheckExact(o); }
 
 // The interpreter lock is given back while memory is allocated and the launch is queued: both may wait for the GPU (an allocation
 // that frees cached blocks, a full queue), and what the GPU waits for may be a host function or a thread that needs the lock.
@@ -160,7 +163,7 @@ PyObject* keep(PyObject*, PyObject* args) {
   try {
     const at::Tensor &ta = THPVariable_Unpack(a), &tb = THPVariable_Unpack(b), &tc = THPVariable_Unpack(c);
     Key k;
-    if (!plain(ta, 2) || !plain(tb, 2) || !operand_key(tag, ta, tb, &k)) Py_RETURN_NONE;
+    if (!own_tensor(a) || !own_tensor(b) || !plain(ta, 2) || !plain(tb, 2) || !operand_key(tag, ta, tb, &k)) Py_RETURN_NONE;
     Product p;
     std::memcpy(&p.args, bytes, sizeof p.args);
     p.rows = tc.size(0); p.cols = tc.size(1);
@@ -177,7 +180,7 @@ PyObject* keep(PyObject*, PyObject* args) {
 
 // product(tag, a, b, memo, hooks) -> c, or None
 PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n != 5 || !tensor_arg(args[1]) || !tensor_arg(args[2]) || !PyDict_Check(args[3]) || !PyList_Check(args[4]) ||
+  if (n != 5 || !own_tensor(args[1]) || !own_tensor(args[2]) || !PyDict_Check(args[3]) || !PyList_Check(args[4]) ||
       PyList_GET_SIZE(args[4]) != 0)
     Py_RETURN_NONE;
   const long long tag = PyLong_AsLongLong(args[0]);
@@ -249,7 +252,7 @@ bool pair_of(PyObject* t, int64_t* out) {
 
 // (input, weight, bias or None, stride, padding, dilation) -> key; false: the ordinary path
 bool conv_key(PyObject* const* args, Key* k) {
-  if (!tensor_arg(args[0]) || !tensor_arg(args[1]) || !(args[2] == Py_None || tensor_arg(args[2]))) return false;
+  if (!own_tensor(args[0]) || !own_tensor(args[1]) || !(args[2] == Py_None || own_tensor(args[2]))) return false;
   const at::Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]);
   if (!plain(x, 4) || !plain(w, 4) || !x.is_contiguous() || !w.is_contiguous()) return false;
   std::memset(k, 0, sizeof *k);
