@@ -211,7 +211,7 @@ int tnx_split_f32(const float* src, int64_t rows, int64_t cols, int64_t stride_r
  * ordered.  Asynchronous, allocates nothing.
  * Three tiles (block_k = 32: 32x64 and 64x64 with 4 waves and 4 slots, 32x128 with 4 and 3) multiply the operands as they are,
  * on the binary32 matrix instruction, where a dimension of each is contiguous: one launch, no scratch (the size query
- * returns 0).  tnx_gemm_f32_config fills in one of them where it is modelled to be faster -- small products and few rows --
+ * returns 0, unless rows overlap: the base pointers, which it does not look at, then decide).  tnx_gemm_f32_config fills in one of them where it is modelled to be faster -- small products and few rows --
  * and the built-in choice elsewhere. */
 size_t tnx_gemm_f32_scratch_bytes(const tnx_gemm_args* args);
 int tnx_gemm_f32(const tnx_gemm_args* args, void* scratch, size_t scratch_bytes);

@@ -295,9 +295,13 @@ bool tnx::gemm_tile_for(int dtype, int bm, int bn, int bk, int* num_warps, int* 
   return true;
 }
 
-bool tnx::gemm_f32_direct(const tnx_gemm_args* a) {
+// any_base: whatever the base pointers are (as if they were off 16 bytes, which refuses rows that overlap).
+bool tnx::gemm_f32_direct(const tnx_gemm_args* a, bool any_base) {
+  if (!a || a->in_dtype != TNX_F32 || a->k <= 0) return false;
+  tnx_gemm_args t = *a;
+  if (any_base) t.a = t.b = (const void*)4;
   const KernelEntry* e = nullptr;
-  return a && a->in_dtype == TNX_F32 && a->k > 0 && supported_impl(a, &e, nullptr, true, nullptr, nullptr, nullptr, GEMM_F32) == TNX_OK && e;
+  return supported_impl(&t, &e, nullptr, true, nullptr, nullptr, nullptr, GEMM_F32) == TNX_OK && e;
 }
 
 void tnx::gemm_tile_layouts(const tnx_gemm_args* a, bool* pair, bool* bt, bool* at) {
@@ -855,12 +859,13 @@ extern "C" int tnx_gemm_f32_config(tnx_gemm_args* a) {
   if (st != TNX_OK) return st;
   const tnx_gemm_args split = *a;
   tnx_gemm_args t = *a;
-  t.a = t.b = nullptr;
+  t.a = t.b = (const void*)4;               // whatever the base pointers will be
   if (t.stride_ak == 0 && t.stride_bn == 0) { t.stride_am = t.k; t.stride_ak = 1; t.stride_bk = t.n; t.stride_bn = 1; }
   t.block_m = 64; t.block_n = 128; t.block_k = 32;
   bool tail_slab = false;
   const int layout = t.k > 0 ? dma_layout(&t, &tail_slab) : 0;
   if (layout == 0) return TNX_OK;
+  t.a = t.b = nullptr;
   int64_t cus = 256;
   int n = 0;
   if (compute_units(&n) == TNX_OK && n > 0) cus = n;

@@ -175,7 +175,8 @@ static bool next_rows(SplitSide* s) {
 }
 
 extern "C" size_t tnx_gemm_f32_scratch_bytes(const tnx_gemm_args* a) {
-  if (gemm_f32_direct(a)) return 0;
+  // (asked before there are pointers, or with others: no scratch only where none of them would need any)
+  if (gemm_f32_direct(a, true)) return 0;
   tnx_gemm_args g;
   SplitSide sa, sb;
   int64_t bytes = 0;
@@ -191,7 +192,7 @@ extern "C" int tnx_gemm_f32(const tnx_gemm_args* a, void* scratch, size_t scratc
   int st = plan(a, scratch, &g, &sa, &sb, &bytes, &pair);
   if (st != TNX_OK) return st;
   if (a->m == 0 || a->n == 0) return TNX_OK;
-  if (gemm_f32_direct(a)) {
+  if (gemm_f32_direct(a, false)) {
     if (!a->a || !a->b || !a->c || (((uintptr_t)a->a | (uintptr_t)a->b | (uintptr_t)a->c) & 3)) return TNX_E_INVALID;
     return gemm_launch(a, nullptr, GEMM_F32);
   }

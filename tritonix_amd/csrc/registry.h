@@ -44,7 +44,7 @@ int gemm_launch(const tnx_gemm_args* a, const GemmBatch* extra, GemmForm form = 
 // the status gemm_launch would return for these arguments, the workspace included, without launching
 int gemm_check(const tnx_gemm_args* a, GemmForm form);
 // whether the tile of `a` and the layout of its float32 operands have a kernel that multiplies them as they are
-bool gemm_f32_direct(const tnx_gemm_args* a);
+bool gemm_f32_direct(const tnx_gemm_args* a, bool any_base);
 // whether the tile of `a` takes head and tail slabs, and whether it has the k-contiguous-B and m-contiguous-A loaders
 void gemm_tile_layouts(const tnx_gemm_args* a, bool* pair, bool* bt, bool* at);
 // waves and stages of a built tile with these dimensions that gemm_launch takes with a GemmBatch (eight waves and
