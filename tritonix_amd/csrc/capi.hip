@@ -525,6 +525,13 @@ static const TileCost COST32[] = {
     {32, 128, 4, 3, 4.29, 1.2, 0.535, 0.695, 0.752, 0.151, 1.58, 0.711, 0.0186, 0.0689, 0.782, 0.485, 1.38, 0},
     {32, 64, 4, 4, 3.68, 0.0338, 0.279, 1.48, 0.782, 0.133, 1.11, 1.04, 0.0341, 0.0867, 0.498, 1.33, 5.28, 0}};
 
+// `s` slices of K, or as many as the same runs of slabs fill: kt = 81 cut in 10 is nine runs of nine, and the tenth slice would be a
+// workgroup that stores a tile of zeros for the last one to read back.
+static int filled_slices(int64_t kt, int s) {
+  const int64_t per = (kt + s - 1) / s;
+  return per > 0 ? (int)((kt + per - 1) / per) : 1;
+}
+
 struct Priced {
   int64_t m, n, kt, cus;
   bool a_off, b_off, ragged, bt;
@@ -608,8 +615,9 @@ static double price_tiles(tnx_gemm_args* a, int es, bool at, int64_t cus, int on
     if (!e || (at ? !e->fast_at : p.bt ? !e->fast_bt : !e->fast)) continue;
     const int64_t tiles = ((a->m + t.bm - 1) / t.bm) * ((a->n + t.bn - 1) / t.bn);
     if ((double)t.bm * t.bn * (double)tiles > 5.0 * (double)a->m * (double)a->n + 4.0 * 65536) continue;
-    for (int s : cuts) {
-      if (only_cut > 0 && s != only_cut) continue;
+    for (int cut : cuts) {
+      if (only_cut > 0 && cut > 1) break;
+      const int s = filled_slices(p.kt, only_cut > 0 ? only_cut : cut);
       const bool last_only = s > 1 && tiles > cus && tiles % cus != 0;         // only the tiles of the partial round are cut
       const int64_t tail = last_only ? tiles % cus : 0, ncut = s == 1 ? 0 : last_only ? tail : tiles;
       if (s > 1 && (p.kt / s < 2 || ncut > WS_MAX_TILES || ncut * s > (last_only ? 2 : 3) * cus ||
@@ -709,6 +717,7 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
     if (kt >= (es == 1 ? 12 : large_f32 ? 14 : 18))
       while (tiles * s * 2 <= cus && s < 16 && 4 * kt >= (es == 1 && a->m <= 16 ? 5 : 7) * s * s) s *= 2;
     if (bt && s >= (es == 1 ? 1 : 2) && s < 8 && kt % (64 * s) == 32 * s) s *= 2;
+    s = filled_slices(kt, s);
     a->split_k = s;
     a->block_m = es == 2 && a->m <= 32 && !at && !large_f32 && (narrow || s == 1) ? 32 : 64;
     a->num_stages = narrow ? 4 : 3;
@@ -732,7 +741,7 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
     int s = 1;
     if (kt >= 16)
       while (tiles * s * 2 <= cus && s < 16 && 4 * kt >= 7 * s * s) s *= 2;
-    a->split_k = s;
+    a->split_k = filled_slices(kt, s);
     return TNX_OK;
   }
   // operands the DMA loader cannot take (not row-major with unit inner strides, int8 rows that are not 16-byte
@@ -830,7 +839,7 @@ static int default_config(tnx_gemm_args* a, bool large_f32) {
   if (es == 2 && bi == 0 && kt <= 64) a->num_warps = 8;
   if (bi == 0 && a->out_dtype == TNX_F32) a->num_warps = 8;
   if (at && bi == 0) a->num_warps = 8;                               // the only 256x256 kernels built for an m-contiguous A
-  a->split_k = bs;
+  a->split_k = filled_slices(kt, bs);
   a->tail_tiles = btail;
   // Grids of several rounds of 256 tiles in both directions: the super-block order keeps what one round reads
   // to 16 + 16 operand panels and lets consecutive rounds share half of them (measured on 8192^3: int8 +4 %,

@@ -576,8 +576,10 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, 
       const GatherCost* cost = gather_cost(e);
       if (!cost) continue;
       const int64_t tiles = ((a->c_out + e.bm - 1) / e.bm) * ((p->n_total + e.bn - 1) / e.bn);
-      for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
-        if (s > 1 && (kt / s < 3 || tiles * s > 800)) break;
+      for (int cut : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        if (cut > 1 && (kt / cut < 3 || tiles * cut > 800)) break;
+        const int64_t per = (kt + cut - 1) / cut;
+        const int s = (int)((kt + per - 1) / per);          // (no slice without a slab)
         const double c = gather_time(*cost, tiles, kt, s, p->terms == 2, in_bytes);
         if (c < best) { best = c; p->e = &e; p->split = s; }
       }
