@@ -638,57 +638,78 @@ constexpr int slice_batch(int n, int cap) {
   return g;
 }
 
-// The split-K slices of one wave's part of a tile, added in slice order into the accumulators (which an uncut tile
-// would hold there), whatever workgroup does it.  Bound by the latency of device-scope loads and, from 64 KiB of slices on,
-// by the 64 bytes per cycle a CU takes in: ZB slices of CG groups, 16 to 32 loads per lane, are in flight together, across
-// row-blocks, and nothing is loaded past the last slice or row-block (a load from an empty window costs as much).
-template <class C, class ACC>
-__device__ __forceinline__ void collect_slices(ACC (&acc)[C::TM][C::TN], const SliceSrc& src, int lane, int64_t rows_left) {
+// Sums of the slices of CG groups, from group c0 of the wave's part on, into the accumulators of those groups; ZB slices in flight
+// together, in slice order whatever ZB is.
+template <class C, int CG, int ZB, class ACC>
+__device__ __forceinline__ void collect_groups(ACC (&acc)[C::TM][C::TN], __amdgpu_buffer_rsrc_t win, const SliceSrc& src, int lane, int c0,
+                                               int row_blocks) {
   constexpr int NGRP = C::ACC_N / 4, NQ = C::TN * NGRP, G = C::TM * NQ;
-  constexpr int CG = slice_batch(G, G == 32 ? 8 : 16);
-  constexpr int ROOM = (Residency<C>::REGS - 32) / (4 * CG) - 1;        // slices of CG groups beside their sums
-  constexpr int ZCAP = G > 8 ? 2 : G == 8 ? 4 : 8;
-  constexpr int ZB = ROOM >= ZCAP ? ZCAP : ROOM >= 4 ? 4 : ROOM >= 2 ? 2 : 1;
   typedef std::remove_reference_t<decltype(acc[0][0][0])> acc_s;
   typedef acc_s acc4 __attribute__((ext_vector_type(4)));
-  const __amdgpu_buffer_rsrc_t win = agent_window(src.base);
-  const int row_blocks = rows_left >= C::WTM ? C::TM : (int)((rows_left + C::MI - 1) / C::MI);
+  acc4 v[CG];
 #pragma unroll
-  for (int c0 = 0; c0 < G; c0 += CG) {
-    acc4 v[CG];
-#pragma unroll
-    for (int x = 0; x < CG; ++x) v[x] = acc4{0, 0, 0, 0};
-    if (c0 / NQ < row_blocks) {
+  for (int x = 0; x < CG; ++x) v[x] = acc4{0, 0, 0, 0};
+  if (c0 / NQ < row_blocks) {
 #pragma unroll 1
-      for (int z0 = 0; z0 < src.nslices; z0 += ZB) {
-        i32x4 w[ZB * CG];
+    for (int z0 = 0; z0 < src.nslices; z0 += ZB) {
+      i32x4 w[ZB * CG];
 #pragma unroll
-        for (int u = 0; u < ZB; ++u) {
-          if (z0 + u >= src.nslices) break;
+      for (int u = 0; u < ZB; ++u) {
+        if (z0 + u >= src.nslices) break;
 #pragma unroll
-          for (int x = 0; x < CG; ++x) {
-            // (row-block by row-block in the tiles of few groups; a branch more in the others keeps the compiler from
-            // having the loads in flight together at all)
-            if (G <= 8 && (c0 + x) / NQ >= row_blocks) break;
-            w[u * CG + x] = load16_agent(win, (uint32_t)lane * 16u + (uint32_t)(c0 + x) * 1024u + (uint32_t)(z0 + u) * src.slice_stride);
-          }
+        for (int x = 0; x < CG; ++x) {
+          // (row-block by row-block in the tiles of few groups; a branch more in the others keeps the compiler from
+          // having the loads in flight together at all)
+          if (G <= 8 && (c0 + x) / NQ >= row_blocks) break;
+          w[u * CG + x] = load16_agent(win, (uint32_t)lane * 16u + (uint32_t)(c0 + x) * 1024u + (uint32_t)(z0 + u) * src.slice_stride);
         }
+      }
 #pragma unroll
-        for (int u = 0; u < ZB; ++u) {
-          if (z0 + u >= src.nslices) break;
+      for (int u = 0; u < ZB; ++u) {
+        if (z0 + u >= src.nslices) break;
 #pragma unroll
-          for (int x = 0; x < CG; ++x) {
-            acc4 t;
-            __builtin_memcpy(&t, &w[u * CG + x], 16);
-            v[x] += t;
-          }
+        for (int x = 0; x < CG; ++x) {
+          acc4 t;
+          __builtin_memcpy(&t, &w[u * CG + x], 16);
+          v[x] += t;
         }
       }
     }
+  }
 #pragma unroll
-    for (int x = 0; x < CG; ++x)
+  for (int x = 0; x < CG; ++x)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[(c0 + x) / NQ][(c0 + x) % NQ / NGRP][(c0 + x) % NGRP * 4 + e] = v[x][e];
+    for (int e = 0; e < 4; ++e) acc[(c0 + x) / NQ][(c0 + x) % NQ / NGRP][(c0 + x) % NGRP * 4 + e] = v[x][e];
+}
+
+// The split-K slices of one wave's part of a tile, added in slice order into the accumulators (which an uncut tile
+// would hold there), whatever workgroup does it.  Bound by the latency of device-scope loads and, from 64 KiB of slices on,
+// by the 64 bytes per cycle a CU takes in: ZB slices of CG groups, 16 to 32 loads per lane, are in flight together, across
+// row-blocks.  Nothing is loaded past the last slice (a load from an empty window costs as much) nor, in the tiles of few groups,
+// past the last row-block.  What is loaded beyond the problem's rows -- the other lanes of a row-block, the other row-blocks of a batch
+// of groups -- was never written: it lies inside the slice, stays in the lane of its row, and no epilogue stores it.
+// One row-block alone has fewer groups, so more of its slices fit the same registers: 8 x 2048 x 10240 int8, sixteen cuts, 11.5 us with
+// four slices of two row-blocks in flight, 10.8 with eight of one.
+template <class C, class ACC>
+__device__ __forceinline__ void collect_slices(ACC (&acc)[C::TM][C::TN], const SliceSrc& src, int lane, int64_t rows_left) {
+  constexpr int NQ = C::TN * (C::ACC_N / 4), G = C::TM * NQ;
+  constexpr int CG = slice_batch(G, G >= 32 ? 8 : 16);
+  constexpr int ROOM = (Residency<C>::REGS - 32) / (4 * CG) - 1;        // slices of CG groups beside their sums
+  constexpr int ZCAP = G > 8 ? 2 : G == 8 ? 4 : 8;
+  constexpr int ZB = ROOM >= ZCAP ? ZCAP : ROOM >= 4 ? 4 : ROOM >= 2 ? 2 : 1;
+  constexpr int ZB1 = ZB * CG / NQ < 8 ? ZB * CG / NQ : 8;              // of the first row-block alone
+  constexpr bool FEW = G <= 8 && C::TM > 1 && CG > NQ && ZB1 > ZB;
+  const __amdgpu_buffer_rsrc_t win = agent_window(src.base);
+  const int row_blocks = rows_left >= C::WTM ? C::TM : (int)((rows_left + C::MI - 1) / C::MI);
+  if (FEW && row_blocks <= 1) {
+#pragma unroll
+    for (int i = 1; i < C::TM; ++i)
+#pragma unroll
+      for (int j = 0; j < C::TN; ++j) acc[i][j] = {};
+    collect_groups<C, FEW ? NQ : CG, FEW ? ZB1 : ZB>(acc, win, src, lane, 0, row_blocks);
+  } else {
+#pragma unroll
+    for (int c0 = 0; c0 < G; c0 += CG) collect_groups<C, CG, ZB>(acc, win, src, lane, c0, row_blocks);
   }
   if (src.rezero) {
     // atomic reduction: what was just read is the sum; leave zeros behind for the next launch
