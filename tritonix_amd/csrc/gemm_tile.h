@@ -1791,9 +1791,25 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
     asm volatile("v_xor_b32 %0, %1, %2" : "=v"(r) : "i"(bits), "v"(base));
     return r;
   };
+  // Likewise the 256-wide float32 pairs of a k-contiguous B: an offset for each operand, k step and slot, kept in registers, takes
+  // eight where the loop has two to spare (packed conv2d: 96 registers spilled, 21 reloads per two slabs; now one).  The k step is
+  // again a bit to XOR in, the slot is added in the same instruction.
+  constexpr bool SLOT_OFFS = BT && PAIR && C::STAGE_BYTES >= 65536;
+  static_assert(!SLOT_OFFS || (MI == 16 && C::BK * ES == 128), "the k step is one bit of the chunk index");
+  uint32_t so_a = 0, so_b = 0;
+  auto slot_off = [&](uint32_t slot, uint32_t off, int ks) __attribute__((always_inline)) {
+    uint32_t r;
+    asm volatile("v_xad_u32 %0, %1, %2, %3" : "=v"(r) : "v"(off), "i"(ks * C::KB), "s"(slot));
+    return r;
+  };
   auto read_one = [&](int set, int idx, uint32_t sa, uint32_t sb, int ks) __attribute__((always_inline)) {
     if (BT && idx < NBREAD) {
-      fbq[set][idx] = *TNX_LDS(i32x4, sb + bt_koff[ks] + idx * MI * C::ROWB_A);
+      if constexpr (SLOT_OFFS) {
+        if (idx == 0) so_b = slot_off(sb, bt_koff[0], ks);
+        fbq[set][idx] = *TNX_LDS(i32x4, so_b + idx * MI * C::ROWB_A);
+      } else {
+        fbq[set][idx] = *TNX_LDS(i32x4, sb + bt_koff[ks] + idx * MI * C::ROWB_A);
+      }
     } else if (idx < NBREAD) {
       int j = idx >> 1, h = idx & 1;
       if constexpr (XOR_OFFS) {
@@ -1812,7 +1828,12 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
       }
     } else {
       int i = idx - NBREAD;
-      fa[set][i] = *TNX_LDS(i32x4, sa + a_koff[ks] + i * MI * C::ROWB_A);
+      if constexpr (SLOT_OFFS) {
+        if (i == 0) so_a = slot_off(sa, a_koff[0], ks);
+        fa[set][i] = *TNX_LDS(i32x4, so_a + i * MI * C::ROWB_A);
+      } else {
+        fa[set][i] = *TNX_LDS(i32x4, sa + a_koff[ks] + i * MI * C::ROWB_A);
+      }
     }
   };
   auto mma_at = [&](int set_a, int set_b, int i, int j) __attribute__((always_inline)) {
@@ -2239,9 +2260,14 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
     const int64_t gm0 = m0 + wy * C::WTM;
     const int64_t gn0 = n0 + wx * C::WTN;
     const uint32_t strip = lds0 + wave * EpiStage<C>::WAVE_BYTES;
+    // Float32 pairs: the lane again, from nothing that is older.  What the epilogue works out from it is else worked out before the K
+    // loop, whose operands share a part of it, and carried through -- 256x256, k-contiguous B: 52 registers spilled, seven reloads per
+    // two slabs, 3019 x 6592 x 5248 555 us; now none, 479.  (Tiles with registers to spare lose by it: 4032 x 1696 x 1536 bf16 on 128x256
+    // 22.5 -> 23.7; so does the one of four waves that spills outside its loop: 8192^3 698 -> 717.)
+    const int elane = PAIR ? __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane;
     if constexpr (CONV) {
-      if (p.out_dtype == DT_F32) epilogue_store_conv<T, C, OutF32>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
-      else epilogue_store_conv<T, C, O>(acc, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
+      if (p.out_dtype == DT_F32) epilogue_store_conv<T, C, OutF32>(acc, p.c, strip, elane, (int)gm0, (int)gn0, p.cv);
+      else epilogue_store_conv<T, C, O>(acc, p.c, strip, elane, (int)gm0, (int)gn0, p.cv);
       return;
     }
     // `sums`: the wave's accumulators, or what the slices of a cut tile add up to.  The output type: the input's own
@@ -2250,12 +2276,12 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
       auto as = [&](auto otag) __attribute__((always_inline)) {
         typedef typename decltype(otag)::type OT;
         if constexpr (GATHER)
-          epilogue_store_conv<T, C, OT>(sums, p.c, strip, lane, (int)gm0, (int)gn0, p.cv);
+          epilogue_store_conv<T, C, OT>(sums, p.c, strip, elane, (int)gm0, (int)gn0, p.cv);
         else if (p.epilogue == EPI_NONE)
-          epilogue_store<T, C, OT, false, MULTI>(sums, p.c, strip, lane, gm0, gn0, p.m, p.n, p.scm, p.scn, p.c_row_ok, 0,
+          epilogue_store<T, C, OT, false, MULTI>(sums, p.c, strip, elane, gm0, gn0, p.m, p.n, p.scm, p.scn, p.c_row_ok, 0,
                                                  p.cv.bias, p.cv.bias_dtype);
         else
-          epilogue_store<T, C, OT, true>(sums, p.c, strip, lane, gm0, gn0 >> 1, p.m, p.n >> 1, p.scm, p.scn, p.c_row_ok,
+          epilogue_store<T, C, OT, true>(sums, p.c, strip, elane, gm0, gn0 >> 1, p.m, p.n >> 1, p.scm, p.scn, p.c_row_ok,
                                          p.epilogue);
       };
       if constexpr (PAIR) {
@@ -2275,11 +2301,11 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
         const int64_t slice_stride = (int64_t)ncut * BM * BN * 4;
         uint8_t* wave0 = p.ws + WS_COUNTER_BYTES + ((int64_t)ctile * NW + wave) * (C::WTM * C::WTN * 4);
         const bool atomic = !GATHER && p.atomic_reduce != 0;
-        if (!splitk_arrive<T, C, APART>(acc, wave0 + (atomic ? 0 : split * slice_stride), lane, gm0, p.m, (int*)p.ws + ctile,
+        if (!splitk_arrive<T, C, APART>(acc, wave0 + (atomic ? 0 : split * slice_stride), elane, gm0, p.m, (int*)p.ws + ctile,
                                         (int*)(smem + (APART ? EpiStage<C>::BYTES : 0)), p.split_k, atomic))
           return;
         acc_t sums[TM][TN];          // (not `acc`: two definitions that meet again spill in the tiles that use every register)
-        collect_slices<C>(sums, SliceSrc{wave0, (uint32_t)slice_stride, atomic ? 1 : p.split_k, atomic}, lane, p.m - gm0);
+        collect_slices<C>(sums, SliceSrc{wave0, (uint32_t)slice_stride, atomic ? 1 : p.split_k, atomic}, elane, p.m - gm0);
         finish(sums);
         return;
       }
