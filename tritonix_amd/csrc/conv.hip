@@ -179,7 +179,9 @@ static bool gemm_problem_ok(const tnx_conv2d_args* a) {
 // What a tile of that GEMM costs, in microseconds: `fixed` at its start and end, `slab` per K slab alone on its CU; of
 // `per_cu` that share one, each one more adds `share` of the slabs' time; after whole rounds, a last one of few workgroups costs `last` of
 // a whole one at least; `tail` for a last slab that is not whole; per 5 MB of output `store`, and `odd` more where rows of
-// the output start off 16 bytes (narrow tiles then write more pieces of cache lines).
+// the output start off 16 bytes (narrow tiles then write more pieces of cache lines).  These loops are short: a CU that is done takes the
+// next workgroup while others run, so a last round is counted at the mean number on a CU; counted at the most (last_round, further
+// down) the choice measured 1.0210x the best tile on 1,500 layers, this way 1.0205x.
 struct ImageCost {
   int bm, bn, nw, stages, per_cu;
   double fixed, slab, share, last, tail, store, odd;
@@ -421,22 +423,21 @@ struct PackedPlan {
 };
 
 // What a packed tile costs, in microseconds: `fixed` at its start and end, `slab` per K slab alone on its CU; of `per_cu`
-// that share one, each one more adds `share` of the slabs' time; after whole rounds, a last one of few workgroups costs `last`
-// of a whole one at least.
+// that share one, each one more adds `share` of the slabs' time; `last` as in last_round.
 struct GatherCost {
   int bm, bn, nw, stages, per_cu;
   double fixed, slab, share, last;
 };
 static const GatherCost GATHER_COST[] = {
-    {256, 256, 8, 2, 1, 2.24, 1.127, 0.00, 1.00}, {256, 224, 8, 2, 1, 2.90, 1.033, 0.00, 0.92},
-    {256, 192, 8, 2, 1, 2.57, 0.888, 0.00, 0.85}, {256, 128, 8, 3, 1, 2.26, 0.572, 0.00, 1.00},
-    {128, 256, 8, 3, 1, 2.42, 0.610, 0.00, 0.88}, {128, 128, 8, 3, 1, 1.70, 0.331, 0.00, 1.00},
-    {128, 128, 8, 2, 2, 0.87, 0.522, 0.30, 0.80}, {64, 256, 8, 3, 1, 1.90, 0.388, 0.00, 0.92},
-    {64, 128, 8, 3, 2, 1.01, 0.251, 0.70, 0.74}, {64, 128, 8, 2, 2, 0.59, 0.440, 0.04, 0.97},
-    {64, 128, 4, 3, 2, 1.18, 0.258, 0.58, 0.70}, {32, 256, 4, 2, 2, 0.86, 0.581, 0.01, 0.83},
-    {64, 64, 4, 4, 2, 0.87, 0.132, 0.89, 1.00}, {64, 64, 4, 2, 4, 0.31, 0.380, 0.10, 0.81},
-    {32, 128, 4, 3, 2, 0.87, 0.208, 0.51, 0.94}, {32, 128, 4, 2, 3, 0.37, 0.406, 0.11, 0.75},
-    {32, 64, 4, 4, 2, 0.68, 0.105, 0.77, 1.00}};
+    {256, 256, 8, 2, 1, 2.45, 1.163, 0.00, 0.96}, {256, 224, 8, 2, 1, 2.95, 1.058, 0.00, 0.91},
+    {256, 192, 8, 2, 1, 2.51, 0.908, 0.00, 0.85}, {256, 128, 8, 3, 1, 2.15, 0.602, 0.00, 1.00},
+    {128, 256, 8, 3, 1, 2.28, 0.620, 0.00, 0.92}, {128, 128, 8, 3, 1, 1.60, 0.350, 0.00, 1.00},
+    {128, 128, 8, 2, 2, 0.79, 0.545, 0.31, 0.87}, {64, 256, 8, 3, 1, 1.80, 0.383, 0.00, 0.93},
+    {64, 128, 8, 3, 2, 1.01, 0.258, 0.64, 0.78}, {64, 128, 8, 2, 2, 0.55, 0.459, 0.03, 0.95},
+    {64, 128, 4, 3, 2, 1.17, 0.262, 0.55, 0.73}, {32, 256, 4, 2, 2, 0.89, 0.629, 0.02, 0.83},
+    {64, 64, 4, 4, 2, 0.92, 0.141, 0.76, 0.90}, {64, 64, 4, 2, 4, 0.39, 0.386, 0.09, 0.87},
+    {32, 128, 4, 3, 2, 0.89, 0.218, 0.45, 0.86}, {32, 128, 4, 2, 3, 0.43, 0.417, 0.10, 0.68},
+    {32, 64, 4, 4, 2, 0.66, 0.119, 0.56, 1.00}};
 // tile numbers of tnx_conv2d_packed_info / _forward: the first tiles of the table from 0, those of few channels or small rings from 32
 static constexpr int FIRST_SMALL = 11, SMALL_FROM = 32;
 static const GatherCost* gather_cost(const GatherEntry& e) {
@@ -448,21 +449,29 @@ static const GatherCost* gather_cost(const GatherEntry& e) {
 static constexpr double PAIR_SLAB = 1.3;
 static constexpr double PASS_US = 9.0;     // the pass over the operands and the second launch, apart from the bytes
 
+// Time of the last, partial round of `rem` workgroups: the CU that holds the most of them sets it.  After whole rounds, what it adds over
+// a CU with one fewer counts from `last` (few such CUs) to whole (all of them).  (Counted at the mean number on a CU,
+// 272 were 1.06 workgroups' time after a whole round and two workgroups' alone: 64 images of 256 channels, 28x28, 5x5, 62 out then
+// took 784 tiles of 64x64 in place of 196 of 64x256, 74 us in place of 58.)
+template <class F> static double last_round(F together, int64_t rem, bool after_whole, double last) {
+  const int64_t most = (rem + 255) / 256;
+  const double all = together((double)most);
+  if (!after_whole) return all;
+  const double fewer = most > 1 ? together((double)(most - 1)) : 0.0, part = (double)rem / 256.0 - (double)(most - 1);
+  return fewer + (all - fewer) * (last + (1.0 - last) * part);
+}
+
 // Modelled microseconds of the GEMM over packed operands: `tiles` tiles of kt K slabs, cut `s` ways; `bytes` of input, as given
-// and packed (what the caches cannot hold arrives up to a fifth slower).
+// and packed (what the caches cannot hold arrives up to a tenth slower).
 static double gather_time(const GatherCost& c, int64_t tiles, int64_t kt, int s, bool pair, double bytes) {
-  const double slow = 1.0 + 0.2 * (bytes < 3.0e8 ? bytes / 3.0e8 : 1.0);
-  const double k = (double)((kt + s - 1) / s) * c.slab * (pair ? 1.04 : 1.0) * slow, area = c.bm * c.bn / 16384.0;
-  const double fixed = c.fixed * (pair ? 1.62 : 1.0);
+  const double slow = 1.0 + 0.09 * (bytes < 3.0e8 ? bytes / 3.0e8 : 1.0);
+  const double k = (double)((kt + s - 1) / s) * c.slab * (pair ? 1.05 : 1.0) * slow, area = c.bm * c.bn / 16384.0;
+  const double fixed = c.fixed * (pair ? 1.98 : 1.0);
   auto together = [&](double n) { return fixed + k * (1.0 + (n - 1.0) * c.share); };
   const int64_t slots = 256 * c.per_cu, full = tiles * s / slots, rem = tiles * s % slots;
   double t = (double)full * together(c.per_cu);
-  if (rem && !full) t = together((double)((rem + 255) / 256));
-  else if (rem) {
-    const double n = (double)rem / 256.0;
-    t += n < 1.0 ? together(1.0) * (c.last + (1.0 - c.last) * n) : together(n);
-  }
-  if (s > 1) t += 2.2 + 0.27 * s * area + 2.9 * (double)(tiles * s) * area / 256.0;
+  if (rem) t += last_round(together, rem, full > 0, c.last);
+  if (s > 1) t += 1.6 + (0.13 + 0.42 * area) * s + 3.0 * (double)(tiles * s) * area / 256.0;
   return t;
 }
 
@@ -555,8 +564,9 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, 
   const int64_t lim = (1ll << 31) - 4096;
   if (p->n_total >= lim || p->x_bytes >= lim || p->w_bytes >= lim || (int64_t)a->c_out * kt * 8 >= lim) return false;
 
-  // Tile and K cut with the smallest modelled time (gather_time): constants and form are a least-squares fit to 82,000 measured
-  // (layer, tile, cut) triples on 2,200 layers; choosing by it costs 1.5 % against the best measured tile in the mean.
+  // Tile and K cut with the smallest modelled time (gather_time): constants and form are a least-squares fit to 112,000 measured
+  // (layer, tile, cut) triples on 2,500 layers; on 1,600 others choosing by it costs 1.2 % against the best measured tile in the mean,
+  // 7 % of them lose more than 5 %.
   // The tiles of 32 channels and those of two slots, several of which share a CU, win on layers of up to 64 channels and on
   // launches of many short tiles: 128 images of 64 channels, 28x28, 29 out: 28.5 -> 22 us, by 7 % on layers of up to 32
   // channels in the mean, by 3 % on the others.
