@@ -491,15 +491,15 @@ static const TileCost COST16[] = {
     {256, 256, 8, 2, 4.16, 0.00108, 1.18, 1.89, 0.746, 0.278, 2.83, 0.129, 0.11, 0.159, 2.8, 1.08, 4.01, 0},
     {256, 256, 4, 2, 7.61, 1.54, 1.17, 1.16, 0.703, 0.337, 2.5, 0.232, 0.144, 0.227, 5.69, 1.39, 3.89, 0},
     {256, 192, 8, 2, 4.16, 0.586, 0.929, 51.7, 0.739, 0.305, 2.53, 0.244, 0.152, 0.184, 2.69, 0.986, 3.57, 0.0163},
-    {192, 256, 8, 2, 4.01, 0.785, 0.932, 44.5, 0.736, 0.305, 2.46, 0.248, 0.11, 0.205, 2.38, 0.85, 3.64, 0.0384},
+    {192, 256, 8, 2, 4.01, 0.785, 0.951, 44.5, 0.736, 0.305, 2.46, 0.248, 0.11, 0.205, 2.38, 0.85, 3.64, 0.0384},
     {192, 192, 8, 3, 4.54, 1.15, 0.621, 43.7, 0.712, 0.406, 2.59, 0.248, 0.134, 0.191, 2.08, 1.46, 3.9, 0.0314},
     {256, 128, 8, 3, 4.24, 0.735, 0.575, 5.24, 0.711, 0.439, 2.27, 0.257, 0.266, 0.164, 2.3, 1.14, 3.74, 0},
     {256, 128, 4, 3, 5.25, 1.57, 0.585, 7.21, 0.694, 0.399, 2.84, 0.206, 0.29, 0.224, 3.63, 1.21, 4, 0},
     {128, 256, 8, 3, 4.5, 1.7, 0.574, 17.8, 0.666, 0.442, 2.25, 0.389, 0.135, 0.231, 2.08, 0.845, 3.5, 0.00578},
     {128, 128, 8, 3, 3.91, 0.51, 0.356, 2.18, 0.752, 0.439, 1.73, 0.358, 0.196, 0.215, 1.32, 1.45, 4.14, 0},
     {128, 128, 8, 2, 3.12, 0.0154, 0.551, 0.877, 0.795, 0.356, 1.55, 0.351, 0.158, 0.186, 1.14, 1.33, 3.93, 0},
-    {64, 256, 8, 3, 4.15, 1.62, 0.489, 3.44, 0.84, 0.0951, 2.1, 0.584, 0.131, 0.341, 1.14, 0.887, 3.96, 0},
-    {128, 64, 8, 3, 3.42, 0.296, 0.271, 0.952, 0.875, 0.359, 1.26, 0.422, 0.267, 0.197, 0.911, 2.27, 5.21, 0},
+    {64, 256, 8, 3, 4.15, 1.62, 0.509, 3.44, 0.84, 0.0951, 2.1, 0.584, 0.131, 0.341, 1.14, 0.887, 3.96, 0},
+    {128, 64, 8, 3, 3.42, 0.296, 0.298, 0.952, 0.875, 0.359, 1.26, 0.422, 0.267, 0.197, 0.911, 2.27, 5.21, 0},
     {64, 128, 8, 3, 3.63, 1.11, 0.328, 0.975, 0.896, 0.0551, 1.28, 0.648, 0.171, 0.3, 0.653, 1.35, 5.83, 0},
     {64, 128, 8, 4, 3.61, 1.22, 0.316, 0.6, 0.865, 0.052, 1.35, 0.633, 0.188, 0.327, 0.758, 1.28, 5.97, 0},
     {64, 64, 4, 4, 3.62, 0.794, 0.203, 0.493, 0.919, 0.308, 1.69, 0.884, 0.288, 0.366, 0.896, 0.0846, 2.06, 0},
@@ -568,7 +568,12 @@ static double tile_time(const TileCost& t, const Priced& p, int s, int64_t tail)
 // each in a graph.  Against the fastest of them the choice takes 1.021x the time in the mean (int8 1.027x), the one before
 // (six tiles at fixed relative rates, cuts of 2, 4, 8 and 16 at 9 us each) 1.088x (int8 1.13x): on problems of 33 to 256 rows
 // 0.88 to 0.90 of its time, to 1024 rows 0.94, above 0.96, int8 0.83 to 0.90; 4 % of the problems lose more than 5 %, 40 %
-// gain more.  Slices are kept within what tnx_gemm_static_workspace holds.
+// gain more.  Slices are kept within what tnx_gemm_static_workspace holds (3136 x 1344 x 11632 with a k-contiguous B would want 35 MB
+// of them: 102 us on 192x192 cut in two, 154 uncut).
+// Three slabs of the 16-bit table are above the fit, by what 8,200 further problems measured: 128x64 by a tenth (column tiles of one row
+// panel land on different L2s, which a tall A of long rows pays for: 3776 x 72 x 5952 16 -> 21 us where it took the place of 64x128),
+// 64x256 by 4 % and 192x256 by 2 % (near ties with 128x128 and 256x256: 1024 x 13122 x 64 15 -> 21).  Of the choices that differ from
+// the one before, 116 instead of 153 of 2,800 now lose 3 %, 29 instead of 51 lose 10 %.
 // only_cut > 0: that many slices and no other number.
 static double price_tiles(tnx_gemm_args* a, int es, bool at, int64_t cus, int only_cut = 0) {
   const int vec = 16 / es, bk = 128 / es;
