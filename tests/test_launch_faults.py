@@ -204,3 +204,35 @@ def test_a_subclass_keeps_its_type_on_repeated_calls(device, monkeypatch):
     hooks = mm.matmul_kernel.kernel.pre_run_hooks
     assert kernel._launch.product(0, a.as_subclass(_Tagged), b, mm._matmul_cfg, hooks) is None
     assert torch.equal(kernel._launch.product(0, torch.nn.Parameter(a), b, mm._matmul_cfg, hooks), want)
+
+
+@pytest.mark.gpu
+def test_a_kept_conv2d_call_without_room_for_its_scratch(device, monkeypatch):
+    """The native side answers None, and the ordinary path runs the kernel that needs none."""
+    monkeypatch.setenv("TRITONIX_AUTOTUNE", "0")
+    conv = importlib.import_module("tritonix_amd.ops.conv2d.forward")
+    gen = torch.Generator(device).manual_seed(4)
+    x, w = torch.randn(64, 256, 56, 56, generator=gen, device=device).bfloat16(), torch.randn(64, 256, 3, 3, generator=gen, device=device).bfloat16()
+    args = (x, w, None, (1, 1), (1, 1), (1, 1))
+    packed = [conv.conv2d_forward(*args) for _ in range(2)][-1]
+    assert kernel._launch.conv(*args) is not None
+    asked = []
+    scratch = conv._scratch
+    monkeypatch.setattr(conv, "_scratch", lambda nbytes, dev: asked.append(nbytes) or scratch(nbytes, dev))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(device).total_memory
+    held = []
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (60 << 20)) / total)     # the result is 25 MB, the scratch 110
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                held.append(torch.empty(100 << 20, dtype=torch.uint8, device=device))                       # what the allocator keeps
+        answered = kernel._launch.conv(*args) is not None
+        bare = conv.conv2d_forward(*args)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert not answered
+    assert asked and asked[0] > 100 << 20
+    assert (bare.double() - packed.double()).norm() <= 2 ** -8 * packed.double().norm()
+    assert torch.equal(conv.conv2d_forward(*args), packed) and len(asked) == 1                             # natively again

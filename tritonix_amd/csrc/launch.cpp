@@ -339,7 +339,6 @@ PyObject* forget_convs(PyObject*, PyObject*) {
   convs.clear();
   Py_RETURN_NONE;
 }
-PyObject* kept(PyObject*, PyObject*) { return Py_BuildValue("nn", (Py_ssize_t)products.size(), (Py_ssize_t)convs.size()); }
 
 // the stream a launch on the device would go to, for tests
 PyObject* stream_of(PyObject*, PyObject* arg) {
@@ -356,7 +355,6 @@ PyMethodDef methods[] = {
     {"conv", (PyCFunction)(void (*)(void))conv, METH_FASTCALL, nullptr},
     {"forget", forget, METH_NOARGS, nullptr},
     {"forget_convs", forget_convs, METH_NOARGS, nullptr},
-    {"kept", kept, METH_NOARGS, nullptr},
     {"stream_of", stream_of, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

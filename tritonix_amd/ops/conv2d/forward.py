@@ -95,9 +95,6 @@ def _scratch(nbytes: int, device) -> Optional[torch.Tensor]:
         return None
 
 
-_own_scratch = _scratch
-
-
 def _args(out, input, weight, bias, batch, c_in, h_in, w_in, c_out, filter_h, filter_w, stride, padding, dilation,
           block_m: int, block_n: int, block_k: int, group_m: int, loader: int = 0) -> _C.Conv2dArgs:
     a = _C.Conv2dArgs()
@@ -339,8 +336,8 @@ def conv2d_forward(
     (all three sizes 0: the library's own choice; ``LOADER`` is "auto", "registers", "dma" or "gemm").
     Returns a new [N, C_OUT, H_OUT, W_OUT] tensor of the input's dtype."""
     # the library's own choice for sizes met before: one call of the native side, which answers None to anything out of the
-    # ordinary (and where the scratch is somebody else's business)
-    if config is None and _kernel._launch is not None and _scratch is _own_scratch and os.environ.get("TRITONIX_AUTOTUNE", "1") in ("0", "false", "False"):
+    # ordinary, and where the device has no room for the scratch
+    if config is None and _kernel._launch is not None and os.environ.get("TRITONIX_AUTOTUNE", "1") in ("0", "false", "False"):
         out = _kernel._launch.conv(input, weight, bias, stride, padding, dilation)
         if out is not None:
             return out
