@@ -24,6 +24,33 @@ def test_the_native_side_is_given_the_buffer_itself(monkeypatch):
     assert kernel._workspace_of(0, 0, 64, 0) is buf
 
 
+def test_threads_that_evict_each_others_workspaces(monkeypatch):
+    """A buffer may be evicted between its lookup and its move to the end of the list: nobody's call fails for it."""
+
+    class Slow(type(kernel._workspaces)):
+        def move_to_end(self, key):
+            time.sleep(0.002)
+            super().move_to_end(key)
+
+    monkeypatch.setattr(kernel, "_workspaces", Slow())
+    monkeypatch.setattr(kernel, "_MAX_WORKSPACES", 1)
+    device, errors = torch.device("cpu", 0), []
+
+    def ask(stream):
+        try:
+            for _ in range(10):
+                assert kernel._workspace(device, stream, 64).numel() >= 64
+        except Exception as err:                             # noqa: BLE001
+            errors.append(err)
+
+    threads = [threading.Thread(target=ask, args=(i,)) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+
+
 class _Slow(dict):
     """Lets the other threads in between a read and what is made of it."""
 

@@ -33,6 +33,7 @@ _ACTIVATIONS = {"silu": _C.EPI_GLU_SILU, "sigmoid": _C.EPI_GLU_SIGMOID}
 
 # split-K scratch buffers, most recently used last; at most _MAX_WORKSPACES are kept alive
 _workspaces: "OrderedDict[Tuple[int, int], object]" = OrderedDict()
+_workspaces_lock = threading.RLock()           # (an allocation may run other Python code of its thread)
 _MAX_WORKSPACES = 8
 
 
@@ -71,20 +72,21 @@ def _workspace(device, stream_ptr: int, nbytes: int, atomic: bool = False):
     # launches that reduce with atomics need their sum region zero and leave it zero; ordered launches leave
     # slices behind: the two modes never share a buffer
     key = _workspace_key(device, stream_ptr, atomic)
-    buf = _workspaces.get(key)
-    if buf is None or buf.numel() < nbytes:
-        buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _workspaces[key] = buf
-    _workspaces.move_to_end(key)
-    if _capturing():
-        # A launch recorded into a HIP graph bakes this pointer into the graph: the buffer must outlive every
-        # replay, so it is never released (not by the eviction below, not when a later call needs a larger one).
-        if not any(kept is buf for kept in _captured_workspaces):
-            _captured_workspaces.append(buf)
+    with _workspaces_lock:              # a thread that evicts between another one's lookup and its move to the end
+        buf = _workspaces.get(key)
+        if buf is None or buf.numel() < nbytes:
+            buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            _workspaces[key] = buf
+        _workspaces.move_to_end(key)
+        if _capturing():
+            # A launch recorded into a HIP graph bakes this pointer into the graph: the buffer must outlive every
+            # replay, so it is never released (not by the eviction below, not when a later call needs a larger one).
+            if not any(kept is buf for kept in _captured_workspaces):
+                _captured_workspaces.append(buf)
+            return buf
+        while len(_workspaces) > _MAX_WORKSPACES:
+            _workspaces.popitem(last=False)       # launches already enqueued keep their buffer alive through the allocator's stream ordering
         return buf
-    while len(_workspaces) > _MAX_WORKSPACES:
-        _workspaces.popitem(last=False)       # launches already enqueued keep their buffer alive through the allocator's stream ordering
-    return buf
 
 
 # scratch buffers handed to launches that were recorded into a HIP graph: alive until the process ends
@@ -102,8 +104,9 @@ def _capturing() -> bool:
 
 def drop_workspace(device, stream_ptr: int) -> None:
     """Forget the scratch of (device, stream): called when a launch on it reported an error."""
-    for atomic in (False, True):
-        _workspaces.pop(_workspace_key(device, stream_ptr, atomic), None)
+    with _workspaces_lock:
+        for atomic in (False, True):
+            _workspaces.pop(_workspace_key(device, stream_ptr, atomic), None)
 
 
 def _stream_of(index: int) -> int:
