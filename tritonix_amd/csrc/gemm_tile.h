@@ -613,8 +613,8 @@ struct SliceSrc {
 // use.  Left to itself the compiler takes all that the hand-over of cut tiles can use (its loads in flight), which the
 // launches that cut nothing pay for too: 64x128 tiles of 8 waves on 152 registers, one workgroup on a CU instead of two,
 // ran conv2d's 1x1 layer of 1088 -> 320 channels on 14x14, batch 32, in 28.5 us; on 110 registers in 20.5.  NEED: accumulators,
-// two sets of fragments and what addresses take; a tile that needs more than its share keeps fewer workgroups resident
-// (no tile spills for it).
+// two sets of fragments and what addresses take; a tile that needs more than its share keeps fewer workgroups resident.  (25 of the
+// 681 kernels spill, all of them 256x256 tiles, which one workgroup fills whatever is stated here.)
 template <class C> struct Residency {
   static constexpr int LDS = C::LDS_BYTES > EpiStage<C>::BYTES ? C::LDS_BYTES : EpiStage<C>::BYTES;
   static constexpr int ACC = C::TM * C::TN * C::ACC_N;
@@ -2262,9 +2262,12 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
     const uint32_t strip = lds0 + wave * EpiStage<C>::WAVE_BYTES;
     // Float32 pairs: the lane again, from nothing that is older.  What the epilogue works out from it is else worked out before the K
     // loop, whose operands share a part of it, and carried through -- 256x256, k-contiguous B: 52 registers spilled, seven reloads per
-    // two slabs, 3019 x 6592 x 5248 555 us; now none, 479.  (Tiles with registers to spare lose by it: 4032 x 1696 x 1536 bf16 on 128x256
-    // 22.5 -> 23.7; so does the one of four waves that spills outside its loop: 8192^3 698 -> 717.)
-    const int elane = PAIR ? __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane;
+    // two slabs, 3019 x 6592 x 5248 555 us; now none, 479.  Likewise the 256x256 tiles of four waves and one k step per slab (16-bit, four
+    // slots: 4096^3 164 -> 141 us, three: 125 -> 120, two: even; int8 with two: 165 -> 118, with three and four 1 and 5 % the other way).
+    // Tiles with registers to spare lose by it (4032 x 1696 x 1536 bf16 on 128x256 22.5 -> 23.7), and so does the one of four waves and
+    // two k steps, which spills outside its loop only (8192^3 698 -> 717).
+    constexpr bool NEW_LANE = PAIR || (C::KSTEPS == 1 && NW == 4 && BM == 256 && BN == 256 && (ES == 2 || STAGES == 2));
+    const int elane = NEW_LANE ? __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane;
     if constexpr (CONV) {
       if (p.out_dtype == DT_F32) epilogue_store_conv<T, C, OutF32>(acc, p.c, strip, elane, (int)gm0, (int)gn0, p.cv);
       else epilogue_store_conv<T, C, O>(acc, p.c, strip, elane, (int)gm0, (int)gn0, p.cv);
