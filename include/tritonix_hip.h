@@ -44,8 +44,8 @@ enum tnx_dtype {
   TNX_I8 = 2,   /* signed 8-bit */
   TNX_I32 = 3,  /* signed 32-bit (output of the int8 path) */
   TNX_F32 = 4   /* binary32: the type of split-K slices in the workspace, and an output type: a bf16 / f16 GEMM on
-                   a tile of at most 128x128 may write its fp32 sums unrounded (out_dtype = TNX_F32).  No kernel
-                   takes binary32 operands; tnx_split_f32 turns them into bf16 operands of a three-term product */
+                   a tile of at most 128x128 may write its fp32 sums unrounded (out_dtype = TNX_F32).  As an
+                   operand type it is tnx_gemm_f32's: tnx_gemm refuses it */
 };
 
 /* epilogues fused after the K loop (tritonix/ops/swiglu.py:98-104).

@@ -212,7 +212,8 @@ def dma_operands(a, b):
 def _whole_chunks(length: int, pitch: int, k: int, es: int) -> bool:
     """Whether k rows of ``length`` elements may be loaded in whole 16-byte chunks up to the last K slab (128 bytes of k) of
     the 16-bit and int8 tiles: that slab's rows have to reach the end of the chunk before them, which rows shorter than a
-    chunk may not (``ring_chunks_inside`` in gemm_tile.h).  float32 operands are copied into padded rows anyway."""
+    chunk may not (``ring_chunks_inside`` in gemm_tile.h).  float32 operands that cannot be go through
+    the split, which writes padded rows."""
     vec, bk = 16 // es, 128 // es
     return es == 4 or ((k - 1) % bk + 1) * pitch + length >= -(-length // vec) * vec
 
