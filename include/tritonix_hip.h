@@ -284,14 +284,17 @@ int tnx_conv2d_forward(const tnx_conv2d_args* args);
  * does not take it: input and weight are copied into a channels-last layout with the zero padding written out, and
  * the convolution is one GEMM launch over that -- any stride, padding, dilation and channel count.  Give a workspace
  * of at least this size (no initialisation needed) in args->workspace and tnx_conv2d_forward takes the route; without one it
- * runs the kernels above.  With a workspace, dtype may be TNX_F32 (input, weight and output binary32, out_f32 set):
+ * runs the kernels above.  Within that workspace it may also lay out the weight alone and take every input window straight from
+ * the tensor into LDS (filters of two rows and columns or more, 16-bit types).  With a workspace, dtype may be TNX_F32 (input, weight and output binary32, out_f32 set):
  * the copy then cuts the operands into their bf16 terms.  Calls that share a workspace must be ordered. */
 size_t tnx_conv2d_workspace_bytes(const tnx_conv2d_args* args);
 
 /* For tests and tooling: the packed route with tile number `tile` of the type's table (bfloat16's for TNX_F32; counted from
  * 0, the tiles of 32 output channels and of small rings from 32) and `split` K slices (1 to 16) instead of the library's choice, on any layer the route can lay out; tile < 0 asks for
  * that choice.  _info: its scratch bytes, or 0 where there is none, and in info[6] output channels and pixels per
- * tile, waves, ring slots, K slices, and bf16 terms per element.  _forward: launches it in args->workspace. */
+ * tile, waves, ring slots, K slices, and bf16 terms per element.  _forward: launches it in args->workspace.
+ * Tiles from 64 on are those that take their windows from the tensor: `split` - 1 is by how many groups of 8 pixels a tile is narrower
+ * than it can be, and info[4] and info[5] are the rows of the largest window and a workgroup's LDS bytes. */
 size_t tnx_conv2d_packed_info(const tnx_conv2d_args* args, int tile, int split, int32_t* info);
 int tnx_conv2d_packed_forward(const tnx_conv2d_args* args, int tile, int split);
 

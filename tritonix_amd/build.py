@@ -159,6 +159,36 @@ GATHER_TILES = ((256, 256, 8, 2), (256, 224, 8, 2), (256, 192, 8, 2), (256, 128,
                 (32, 64, 4, 4), (32, 128, 4, 3), (32, 128, 4, 2), (32, 256, 4, 2), (64, 64, 4, 2), (64, 128, 8, 2))
 
 
+# (block_cout, block_pixels, k steps of a period, periods in the ring, bytes of a pixel slot) of the conv2d kernels that keep their input window in LDS
+# (conv_halo.h), eight waves
+HALO_TILES = ((256, 224, 2, 2, 96), (128, 192, 4, 2, 96), (128, 128, 4, 2, 96), (64, 256, 4, 2, 96), (64, 128, 4, 2, 96), (64, 64, 4, 2, 96),
+              (32, 256, 4, 2, 96), (32, 128, 4, 2, 96), (128, 256, 2, 2, 64), (128, 128, 2, 3, 64), (128, 128, 4, 2, 64), (64, 256, 4, 2, 64),
+              (64, 128, 4, 2, 64), (64, 64, 4, 2, 64), (32, 256, 4, 2, 64), (32, 128, 4, 2, 64))
+
+
+def generate_halo(tiles, gen):
+    """Instance files of those kernels (one per dtype and tile) and their table."""
+    files, names = [], []
+    for dt in ("bf16", "f16"):
+        for bm, bn, ksp, ring, slot in tiles:
+            name = f"halo_{dt}_c{bm}_p{bn}_k{ksp}_r{ring}_s{slot}"
+            text = (f'// generated by tritonix_amd/build.py -- do not edit\n#include "{CSRC}/conv_halo.h"\n'
+                    f"namespace tnx {{\nHaloEntry k_{name} = TNX_HALO_ENTRY({TAGS[dt][0]}, {bm}, {bn}, {ksp}, {ring}, {slot});\n}}\n")
+            path = os.path.join(gen, name + ".hip")
+            write_if_changed(path, text)
+            files.append(path)
+            names.append(name)
+    decl = "\n".join(f"extern HaloEntry k_{n};" for n in names)
+    ptrs = ", ".join(f"&k_{n}" for n in names) or "nullptr"
+    text = (f'// generated by tritonix_amd/build.py -- do not edit\n#include "{CSRC}/conv_halo.h"\nnamespace tnx {{\n{decl}\n}}\n'
+            f"using namespace tnx;\n"
+            f'extern "C" const HaloEntry* const* tnx_halo_entries(int* n) {{\n'
+            f"  static const HaloEntry* const all[] = {{{ptrs}}};\n  *n = {len(names)};\n  return all;\n}}\n")
+    path = os.path.join(gen, "halo_entries.hip")
+    write_if_changed(path, text)
+    return files + [path]
+
+
 def generate_gather(tiles, gen):
     """Instance files of the packed conv2d kernels (one per dtype and tile) and their table."""
     files, names = [], []
@@ -319,6 +349,7 @@ _resources = {}
 def _compile(src, obj, verbose, force=True):
     deps = [src, os.path.join(CSRC, "gemm_tile.h"), os.path.join(CSRC, "gemm_skinny.h"), os.path.join(CSRC, "registry.h"),
             os.path.join(CSRC, "conv_tile.h"), os.path.join(CSRC, "conv_pack.h"),
+            *([os.path.join(CSRC, "conv_halo.h")] if os.path.basename(src).startswith(("halo_", "conv.hip")) else []),
             os.path.join(ROOT, "include", "tritonix_hip.h"), os.path.abspath(__file__)]
     if not force and os.path.exists(obj) and os.path.getmtime(obj) > max(os.path.getmtime(d) for d in deps):
         return obj
@@ -365,7 +396,8 @@ def build(jobs=None, quick=False, verbose=True, force=True, only=None, out=None,
         BUILD = os.path.join(ROOT, "build", "dev_" + os.path.basename(lib).replace(".", "_"))
     DEVICE_FLAGS.extend(f"-D{d}" for d in defines)
     srcs = generate(instances) + generate_conv(conv_instances, os.path.join(BUILD, "gen")) + generate_gather(
-        GATHER_TILES if not (only or only_conv) or only == "gather" else (), os.path.join(BUILD, "gen")) + [
+        GATHER_TILES if not (only or only_conv) or only == "gather" else (), os.path.join(BUILD, "gen")) + generate_halo(
+        HALO_TILES if not (only or only_conv) or only == "gather" else (), os.path.join(BUILD, "gen")) + [
         os.path.join(CSRC, "capi.hip"), os.path.join(CSRC, "skinny.hip"),
         os.path.join(CSRC, "conv.hip"), os.path.join(CSRC, "f32.hip")]
     if lib == LIB:

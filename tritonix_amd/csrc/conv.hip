@@ -5,6 +5,7 @@
 #include <string.h>
 
 #include "../../include/tritonix_hip.h"
+#include "conv_halo.h"
 #include "conv_pack.h"
 #include "conv_tile.h"
 #include "registry.h"
@@ -14,6 +15,7 @@ using namespace tnx;
 extern "C" const ConvGroup* tnx_conv_groups(int* ngroups);      // generated
 extern "C" const KernelGroup* tnx_kernel_groups(int* ngroups);  // generated
 extern "C" const GatherGroup* const* tnx_gather_groups(int* ngroups);  // generated
+extern "C" const HaloEntry* const* tnx_halo_entries(int* n);    // generated
 
 // The GEMM kernel's conv2d variant for this tile (three ring slots), or null.  Eight waves are preferred (and the
 // only ones built): the loader's address arithmetic and the fix-up are vector instructions in the MFMA stream, and
@@ -410,8 +412,17 @@ static void fill_dma(const tnx_conv2d_args* a, const Resolved& r, GemmParams* p,
 // float32 with heads and tails in blocks of 32 channels instead of three terms (the GEMM reads a third less): 256 channels of
 // 56x56, batch 32: 319 -> 301 us; 512 of 28x28: 285 -> 261; 128 of 56x56, stride 2: 53 -> 47; 512 of 7x7, batch 8: 39 -> 30.
 // ---------------------------------------------------------------------------
+// the window route (conv_halo.h), where it is taken instead: only the weight is laid out, and the workspace is the packed route's
+struct HaloPlan {
+  const HaloEntry* e;
+  HaloGeom g;
+  int lds, kt;                     // LDS of a workgroup; slabs of two k steps of a weight row
+  int64_t w_bytes;
+};
+
 struct PackedPlan {
   const GatherEntry* e;
+  HaloPlan halo;                   // halo.e null: not taken
   int split;                       // K slices per tile
   int h_out, w_out;
   int rows, cols, step_h, step_w;  // packed image; input rows / columns per packed row / column
@@ -520,8 +531,103 @@ static bool few_taps_packed(const tnx_conv2d_args* a, const PackedPlan& p, doubl
 }
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
+// ---------------------------------------------------------------------------
+// window route (conv_halo.h): 16-bit types, filters of at least two rows and columns, a column stride of at most 2
+// ---------------------------------------------------------------------------
+// Tile numbers of tnx_conv2d_packed_info / _forward: the window tiles from here on; `split` - 1 is then by how many groups of 8 pixels
+// a tile is narrower than it could be.
+static constexpr int HALO_FROM = 64;
+
+// What a window tile costs, in microseconds: `fixed` at its start and end, `step` per k step (longer where short output rows make
+// fragments straddle them), `event` per channel block in which all eight waves move rows; of up to `per_cu` that share a CU, as
+// their LDS allows, each one more adds `share` of that; `last` as in last_round.
+struct HaloCost {
+  int bm, bn, ksp, slot, per_cu;
+  double fixed, step, event, share, last;
+};
+static const HaloCost HALO_COST[] = {
+    {256, 224, 2, 96, 1, 3.48, 0.430, 1.92, 0.00, 1.14}, {128, 192, 4, 96, 1, 2.78, 0.197, 1.08, 0.00, 1.00},
+    {128, 128, 4, 96, 1, 2.37, 0.149, 0.97, 0.00, 1.02}, {64, 256, 4, 96, 1, 2.10, 0.148, 0.64, 0.00, 1.07},
+    {64, 128, 4, 96, 2, 1.74, 0.100, 0.82, 0.65, 1.01}, {64, 64, 4, 96, 2, 1.71, 0.081, 1.08, 0.43, 0.95},
+    {32, 256, 4, 96, 2, 1.99, 0.106, 0.71, 0.90, 1.05}, {32, 128, 4, 96, 2, 1.53, 0.080, 0.84, 0.47, 0.99},
+    {128, 256, 2, 64, 1, 1.99, 0.301, 1.10, 0.00, 0.99}, {128, 128, 2, 64, 1, 2.00, 0.187, 1.13, 0.00, 0.99},
+    {128, 128, 4, 64, 1, 2.30, 0.165, 0.91, 0.00, 0.98}, {64, 256, 4, 64, 1, 2.01, 0.169, 0.77, 0.00, 1.02},
+    {64, 128, 4, 64, 2, 1.59, 0.110, 0.83, 0.62, 0.93}, {64, 64, 4, 64, 2, 1.64, 0.088, 1.01, 0.44, 0.87},
+    {32, 256, 4, 64, 2, 1.65, 0.125, 0.81, 0.60, 0.92}, {32, 128, 4, 64, 2, 1.50, 0.091, 0.70, 0.44, 0.88}};
+
+static int gcd(int a, int b) { while (b) { const int t = a % b; a = b; b = t; } return a; }
+
+// The layer as tiles of `width` pixels (a multiple of 8, at most e.bn) see it, and the LDS of a workgroup; false: not with this tile.
+static bool halo_geom(const tnx_conv2d_args* a, int h_out, int w_out, const HaloEntry& e, int width, HaloGeom* g, int* lds) {
+  if (a->filter_h < 2 || a->filter_w < 2 || a->stride_w > 2 || width < 8) return false;
+  *g = HaloGeom{};
+  g->width = width;
+  g->c_in = a->c_in; g->h_in = a->h_in; g->w_in = a->w_in; g->plane = a->h_in * a->w_in;
+  g->batch = a->batch; g->x_elems = (int)((int64_t)a->batch * a->c_in * g->plane);
+  g->stride_h = a->stride_h; g->stride_w = a->stride_w; g->pad_h = a->pad_h; g->pad_w = a->pad_w;
+  g->fh = a->filter_h; g->fw = a->filter_w; g->dil_h = a->dil_h; g->dil_w = a->dil_w; g->taps = a->filter_h * a->filter_w;
+  g->blocks = (a->c_in + 31) / 32;
+  const int64_t span = (int64_t)(a->filter_h - 1) * a->dil_h + 1, rows_img = (int64_t)(h_out - 1) * a->stride_h + span;
+  const int64_t cols = (int64_t)(w_out - 1) * a->stride_w + (int64_t)(a->filter_w - 1) * a->dil_w + 1;
+  // (a window of more than 4096 slots fits no LDS; k steps as far as their offsets do)
+  if (g->x_elems < 8 || cols > 4096 || rows_img * a->batch >= (1ll << 31) || (int64_t)g->blocks * g->taps > 16384) return false;
+  g->rows_img = (int)rows_img;
+  g->cps = (int)((cols + a->stride_w - 1) / a->stride_w);
+  g->rowslots = g->cps * a->stride_w;
+  g->hw_out = h_out * w_out; g->hwp = (g->hw_out + 7) / 8 * 8; g->w_out = w_out;
+  g->cpr = (a->w_in + 7) / 8;
+  g->ksteps = g->blocks * g->taps;
+  // the next block's window has to wait for the block before the present one, and be there a period before its own first read
+  if (g->ksteps <= e.ksp || (g->blocks > 1 && g->taps < 2 * e.ksp)) return false;
+  // Rows of the largest window: from the first to the last pixel of a tile.  Inside an image the first pixel's column is a
+  // multiple of `step`; over c image ends each adds an image's rows and takes the pixels of one (hwp - hw_out of them lie in no row)
+  const int step = gcd(gcd(width, g->hwp), w_out);
+  int64_t most = (int64_t)((w_out - step + width - 1) / w_out) * a->stride_h;
+  if (most > rows_img - span) most = rows_img - span;
+  const int ends = (g->hwp - gcd(width, g->hwp) + width - 1) / g->hwp;
+  for (int c = 1; c <= ends; ++c) {
+    const int left = width - 1 - c * g->hwp;            // pixels from the first one's place in its image to the last one's
+    const int64_t down = (left >= 0 ? (left + w_out - 1) / w_out : -(-left / w_out)) + (g->hwp != g->hw_out ? 1 : 0);
+    const int64_t d = c * rows_img + (down < h_out - 1 ? down : h_out - 1) * a->stride_h;
+    if (d > most) most = d;
+  }
+  const int64_t rows = most + span, slots = rows * g->rowslots;
+  if (slots > 4096 || rows * g->cpr > 128) return false;              // eight waves of 16 row pieces
+  g->rows = (int)rows;
+  g->buf_bytes = (int)(slots * e.slot);
+  // (behind the windows: an offset per k step, of one period past the end too, and a place per lane)
+  *lds = e.ring_bytes + 2 * g->buf_bytes + ((g->ksteps + e.ksp - 1) / e.ksp + 1) * e.ksp * 4 + 1024;
+  if (*lds < e.strip_bytes) *lds = e.strip_bytes;
+  return *lds <= TNX_LDS_LIMIT_BYTES;
+}
+
+// Modelled microseconds of the route: a least-squares fit to 16,700 launches of 2,000 layers of 2x2 to 5x5 filters and 32 channels or
+// more (7 % rms).
+static double halo_time(const tnx_conv2d_args* a, const HaloCost& c, const HaloGeom& g, int64_t n_total, int lds) {
+  const int64_t tiles = ((a->c_out + c.bm - 1) / c.bm) * ((n_total + g.width - 1) / g.width);
+  const double weight = (double)a->c_out * a->c_in * g.taps * 2e-6 * (g.taps == 9 || g.taps == 25 ? 1.0 : 2.0);    // MB
+  const double out = (double)a->batch * a->c_out * g.hw_out * 2 / 5.0e6, window = (double)g.rows * a->w_in * 64.0;
+  const double body = g.ksteps * c.step * (1.0 + 1.80 / g.w_out) + g.blocks * c.event * ((g.rows * g.cpr + 15) / 16) / 8.0;
+  const int fit = TNX_LDS_LIMIT_BYTES / lds, per_cu = fit < c.per_cu ? fit : c.per_cu;
+  auto together = [&](double n) { return c.fixed + body * (1.0 + (n - 1.0) * c.share); };
+  const int64_t slots = 256 * per_cu, full = tiles / slots, rem = tiles % slots;
+  double t = (double)full * together(per_cu);
+  if (rem) t += last_round(together, rem, full > 0, c.last);
+  return 6.11 + 1.10 * weight + 0.87 * out + 0.061 * (double)tiles * window * g.blocks / 5.0e6 + t;
+}
+
+// Modelled microseconds of the packed route, its GEMM modelled at gemm_us (the same layers, 10 % rms): where a filter tap's channels are
+// not whole slabs the GEMM reads the input tap after tap, from further away the larger it is, and rows that are not whole chunks
+// cost both ends.
+static double packed_time(const tnx_conv2d_args* a, double gemm_us, double x_bytes, double w_bytes, int h_out, int w_out) {
+  const double in = (double)a->batch * a->c_in * a->h_in * a->w_in * 2 / 5.0e6, out = (double)a->batch * a->c_out * h_out * w_out * 2 / 5.0e6;
+  const double far = x_bytes < 1.5e8 ? x_bytes / 5.0e7 : 3.0;
+  return 8.38 + 1.01 * gemm_us * (a->c_in % 64 ? 1.0 + 0.142 * far : 1.0) + 1.63 * x_bytes / 5.0e6 + (a->w_in % 8 ? 0.52 * in : 0.0) +
+         1.22 * w_bytes * 1e-6 + 0.74 * out * (w_out % 8 ? 1.69 : 1.0);
+}
+
 // tile >= 0: that tile of the type's table and that many K slices, whatever the rules below would choose
-static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, int split = 1) {
+static bool make_packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile, int split) {
   if (!a || a->loader != TNX_CONV_LOADER_AUTO || a->block_cout || a->block_pixels || a->block_k) return false;
   tnx_conv2d_args t = *a;
   const bool f32 = a->dtype == TNX_F32;
@@ -562,6 +668,33 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, 
   p->x_bytes = (int64_t)a->batch * p->rows * p->cols * p->terms * p->cp8 * 16;
   p->w_bytes = (int64_t)a->c_out * kt * 128;
   const int64_t lim = (1ll << 31) - 4096;
+  int nh = 0;
+  const HaloEntry* const* he = tnx_halo_entries(&nh);
+  auto take_halo = [&](const HaloEntry* e, int width) {
+    HaloPlan h = {e};
+    if (!halo_geom(a, h_out, w_out, *e, width, &h.g, &h.lds)) return false;
+    h.g.div_img = make_fastdiv((uint32_t)h.g.rows_img);
+    h.g.div_hwp = make_fastdiv((uint32_t)h.g.hwp);
+    h.g.div_w = make_fastdiv((uint32_t)w_out);
+    h.g.div_cpr = make_fastdiv((uint32_t)h.g.cpr);
+    h.g.div_taps = make_fastdiv((uint32_t)h.g.taps);
+    h.g.div_fw = make_fastdiv((uint32_t)h.g.fw);
+    h.kt = (h.g.ksteps + e->ksp - 1) / e->ksp * e->ksp / 2;           // whole periods
+    h.w_bytes = (int64_t)a->c_out * h.kt * 128;
+    if (p->n_total >= lim || h.w_bytes >= lim || ((a->c_out + e->bm - 1) / e->bm) * ((p->n_total + width - 1) / width) >= lim) return false;
+    p->halo = h;
+    return true;
+  };
+  if (tile >= HALO_FROM) {
+    int left = tile - HALO_FROM;
+    for (int i = 0; i < nh; ++i)
+      if (!f32 && he[i]->dtype == a->dtype && left-- == 0 && take_halo(he[i], he[i]->bn - (split - 1) * 8)) {
+        p->split = p->terms = 1;
+        p->total_bytes = up256(p->halo.w_bytes);
+        return true;
+      }
+    return false;
+  }
   if (p->n_total >= lim || p->x_bytes >= lim || p->w_bytes >= lim || (int64_t)a->c_out * kt * 8 >= lim) return false;
 
   // Tile and K cut with the smallest modelled time (gather_time): constants and form are a least-squares fit to 112,000 measured
@@ -608,12 +741,69 @@ static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, 
     const double again = p->x_bytes > 200000000 ? 2.0 * ((double)p->x_bytes - 2.0e8) : 0.0;
     if (best + PASS_US + (bytes + again) / 5.0e6 > unpacked_time(&t)) return false;
   }
+  // The window route where its modelled time is 10 % less (both models are off by 7 to 10 %), 17 % where w_out is no multiple of 8,
+  // another 10 % for filters of two columns, and at least 0.88 of a channel block's 32 are channels: of the 2,000 layers 387 are
+  // taken, which gain 25 % in the mean, 11 % over all layers of 40 us and more; 4 lose 3 % or more, the worst 9 %.  At 4 % without
+  // the other lines 931 gain 16 % in the mean, 95 lose, the worst 28 % (128 images of 51 channels, 112x112, 5x5, 48 out: 359 us packed,
+  // 387 as windows).  128 of 64, 28x28, 3x3, 64 out: 28.8 and 18.6; 32 of 256, 56x56, 256 out: 114 and 99; 32 of 128, 56x56, stride 2,
+  // 128 out: 22.1 and 17.1; 32 of 512, 14x14, 512 out: 41.3 and 43.0.
+  bool halo = false;
+  if (!f32 && tile < 0 && a->c_in * 100 >= (a->c_in + 31) / 32 * 32 * 88) {
+    const double margin = 0.9 * (w_out % 8 ? 0.92 : 1.0) * (a->filter_w == 2 ? 0.9 : 1.0);
+    double best_halo = margin * packed_time(a, best, (double)p->x_bytes, (double)p->w_bytes, h_out, w_out);
+    const HaloEntry* chosen = nullptr;
+    int chosen_width = 0;
+    for (int i = 0; i < nh; ++i) {
+      const HaloEntry& e = *he[i];
+      if (e.dtype != a->dtype) continue;
+      const HaloCost* cost = nullptr;
+      for (const HaloCost& c : HALO_COST)
+        if (c.bm == e.bm && c.bn == e.bn && c.ksp == e.ksp && c.slot == e.slot) cost = &c;
+      // tiles of whole output rows need fewer window rows (where images are whole tiles' worth of chunks, and not too much is given away)
+      const int whole = e.bn / (w_out / gcd(w_out, 8) * 8) * (w_out / gcd(w_out, 8) * 8);
+      const bool rows_too = whole < e.bn && whole >= 0.7 * e.bn && h_out * w_out % 8 == 0;
+      for (int width : {e.bn, rows_too ? whole : 0}) {
+        if (!cost || !width) continue;
+        HaloGeom g;
+        int lds;
+        if (!halo_geom(a, h_out, w_out, e, width, &g, &lds)) continue;
+        const double t = halo_time(a, *cost, g, p->n_total, lds);
+        if (t < best_halo) { best_halo = t; chosen = &e; chosen_width = width; }
+      }
+    }
+    halo = chosen && take_halo(chosen, chosen_width);
+  }
   const int64_t tiles = ((a->c_out + p->e->bm - 1) / p->e->bm) * ((p->n_total + p->e->bn - 1) / p->e->bn);
   if (tiles * p->split >= lim || (p->split > 1 && tiles > WS_MAX_TILES)) return false;
   p->slices_bytes = p->split > 1 ? WS_COUNTER_BYTES + (int64_t)p->split * tiles * p->e->bm * p->e->bn * 4 : 0;
   if (p->slices_bytes >= (1ll << 32)) return false;
   p->total_bytes = up256(p->slices_bytes) + up256(p->w_bytes) + up256(p->x_bytes);
+  // (the workspace stays the packed route's: callers ask for it once, and what happens without room for it does not change)
+  if (!halo || p->halo.w_bytes > p->total_bytes) p->halo.e = nullptr;
   return true;
+}
+
+// The library's own plans of the layers a thread met last, by their sizes: pricing them takes longer than a launch.
+static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, int split = 1) {
+  if (!a || tile >= 0) return make_packed_plan(a, p, tile, split);
+  struct Known {
+    int32_t key[22];
+    bool taken;
+    PackedPlan plan;
+  };
+  static thread_local Known known[16];
+  const int32_t key[22] = {1, a->batch, a->c_in, a->h_in, a->w_in, a->c_out, a->filter_h, a->filter_w, a->stride_h, a->stride_w, a->pad_h, a->pad_w,
+                           a->dil_h, a->dil_w, a->dtype, a->out_f32 != 0, a->bias ? 1 + a->bias_dtype : 0, a->block_pixels, a->block_cout, a->block_k,
+                           a->group_pixels, a->loader};
+  uint32_t h = 0;
+  for (int32_t v : key) h = (h ^ (uint32_t)v) * 0x01000193u;
+  Known& k = known[(h >> 16 ^ h) % 16];
+  if (memcmp(k.key, key, sizeof key)) {
+    k.taken = make_packed_plan(a, &k.plan, -1, 1);
+    memcpy(k.key, key, sizeof key);
+  }
+  *p = k.plan;
+  return k.taken;
 }
 
 extern "C" size_t tnx_conv2d_workspace_bytes(const tnx_conv2d_args* a) {
@@ -621,7 +811,45 @@ extern "C" size_t tnx_conv2d_workspace_bytes(const tnx_conv2d_args* a) {
   return packed_plan(a, &p) ? (size_t)p.total_bytes : 0;
 }
 
+static int halo_forward(const tnx_conv2d_args* a, const PackedPlan& pl) {
+  const HaloEntry& e = *pl.halo.e;
+  HaloGeom h = pl.halo.g;
+  hipStream_t stream = (hipStream_t)a->stream;
+  HaloWeight k;
+  memset(&k, 0, sizeof k);
+  k.w = (const uint8_t*)a->weight; k.out = (uint8_t*)a->workspace;
+  k.c_in = a->c_in; k.c_out = a->c_out; k.groups = h.blocks * 4; k.chunks = pl.halo.kt * 8; k.taps = h.taps;
+  k.div_groups = make_fastdiv((uint32_t)k.groups);
+  const dim3 wgrid((unsigned)(((int64_t)k.c_out * k.groups + 63) / 64));
+  if (k.taps == 9) hipLaunchKernelGGL(halo_weight_kernel<9>, wgrid, dim3(64), 0, stream, k);
+  else if (k.taps == 25) hipLaunchKernelGGL(halo_weight_kernel<25>, wgrid, dim3(64), 0, stream, k);
+  else hipLaunchKernelGGL(halo_weight_kernel<0>, wgrid, dim3(64), 0, stream, k);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) { note_hip_error((int)err); return TNX_E_HIP; }
+
+  GemmParams p;
+  memset(&p, 0, sizeof p);
+  p.a = (const uint8_t*)a->workspace; p.c = (uint8_t*)a->output;
+  p.m = a->c_out; p.n = pl.n_total; p.k = (int64_t)pl.halo.kt * 64;
+  p.sam = p.k;
+  p.tiles_m = (int)((a->c_out + e.bm - 1) / e.bm); p.tiles_n = (int)((pl.n_total + h.width - 1) / h.width);
+  p.group_m = 8; p.split_k = 1;
+  p.out_dtype = a->out_f32 ? TNX_F32 : a->dtype;
+  // the output side is conv2d's epilogue on planes of one row of hwp pixels
+  ConvGeom& c = p.cv;
+  c.c_out = a->c_out; c.h_out = 1; c.w_out = h.hw_out; c.wp = pl.hwp;
+  c.n_total = (int)pl.n_total;
+  c.div_hwp = c.div_wp = make_fastdiv((uint32_t)pl.hwp);
+  c.bias = (const uint8_t*)a->bias;
+  c.bias_dtype = a->bias_dtype;
+  h.x = (const uint8_t*)a->input;
+  err = e.launch(p, h, (unsigned)((int64_t)p.tiles_m * p.tiles_n), pl.halo.lds, stream);
+  if (err != hipSuccess) { note_hip_error((int)err); return TNX_E_HIP; }
+  return TNX_OK;
+}
+
 static int packed_forward(const tnx_conv2d_args* a, const PackedPlan& pl) {
+  if (pl.halo.e) return halo_forward(a, pl);
   uint8_t* ws = (uint8_t*)a->workspace;
   uint8_t* wp = ws + up256(pl.slices_bytes);
   uint8_t* xp = wp + up256(pl.w_bytes);
@@ -707,7 +935,8 @@ extern "C" size_t tnx_conv2d_packed_info(const tnx_conv2d_args* a, int tile, int
   PackedPlan p;
   if (!packed_plan(a, &p, tile, split)) return 0;
   if (info) {
-    const int32_t v[6] = {p.e->bm, p.e->bn, p.e->nw, p.e->stages, p.split, p.terms};
+    const HaloEntry* w = tile >= 0 ? p.halo.e : nullptr;
+    const int32_t v[6] = {w ? w->bm : p.e->bm, w ? w->bn : p.e->bn, w ? 8 : p.e->nw, w ? w->ring : p.e->stages, w ? p.halo.g.rows : p.split, w ? p.halo.lds : p.terms};
     memcpy(info, v, sizeof v);
   }
   return (size_t)p.total_bytes;
@@ -725,7 +954,9 @@ static int packed_launch(const tnx_conv2d_args* a, const PackedPlan& pl) {
 
 extern "C" int tnx_conv2d_packed_forward(const tnx_conv2d_args* a, int tile, int split) {
   PackedPlan pl;
-  return packed_plan(a, &pl, tile, split) ? packed_launch(a, pl) : TNX_E_UNSUPPORTED;
+  if (!packed_plan(a, &pl, tile, split)) return TNX_E_UNSUPPORTED;
+  if (tile < 0) pl.halo.e = nullptr;           // the packed route's own choice
+  return packed_launch(a, pl);
 }
 
 extern "C" int tnx_conv2d_supported(const tnx_conv2d_args* a) {
