@@ -18,7 +18,7 @@ constexpr int SK_KSTEP = 32;   // k rows per step
 constexpr int SK_STEP_BYTES = 3072;  // B 32x32 (2 KiB) + A 16x32 (1 KiB), 16-bit elements
 
 template <class T, int RING>
-__global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(GemmParams p) {
+__global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(PlainParams p) {
   static_assert(T::ES == 2, "16-bit element types only");
   static_assert(RING >= 2 && (RING - 1) * 3 <= 63, "ring depth out of range for vmcnt");
   typedef Mma<T, 16> MMA;
@@ -37,7 +37,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(GemmParams p
 
   // ---- DMA source offsets (bytes, constant over the loop); the chunk XORs spread LDS banks
   const int drow = lane >> 2, dchunk = lane & 3;
-  const int64_t ldb = p.sbk, lda = p.sam;
+  const int64_t ldb = p.ldb, lda = p.lda;
   uint32_t b_voff[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -121,8 +121,9 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(GemmParams p
 
 template <class T, int RING>
 hipError_t launch_skinny(const GemmParams& p, unsigned grid, hipStream_t stream) {
-  hipLaunchKernelGGL((gemm_skinny_kernel<T, RING>), dim3(grid), dim3(SK_WAVES * 64), 0, stream, p);
-  return hipGetLastError();
+  PlainParams q;
+  if (!plain_params(p, false, false, T::ES, &q)) return hipErrorInvalidValue;
+  return launch_kernel((const void*)&gemm_skinny_kernel<T, RING>, grid, SK_WAVES * 64, 0, stream, &q);
 }
 
 }  // namespace tnx

@@ -68,6 +68,10 @@ inline FastDiv make_fastdiv(uint32_t d) {
   f.mul = (uint32_t)(((1ull << 32) * ((1ull << s) - d)) / d + 1);
   return f;
 }
+// the same from its multiplier: the shift follows from the divisor
+__device__ __forceinline__ FastDiv fd_of(uint32_t mul, uint32_t d) {
+  return FastDiv{mul, d <= 1 ? 0u : 32u - (uint32_t)__builtin_clz(d - 1)};
+}
 __host__ __device__ __forceinline__ uint32_t fd_div(uint32_t n, FastDiv f) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return (__umulhi(n, f.mul) + n) >> f.shift;
@@ -141,6 +145,30 @@ struct GemmParams {
   FastDiv div_group, div_rows, div_rows_last;   // by group_m * tiles_n, by the rows of a group and by those of the last, shorter one
   ConvGeom cv;            // read by the CONV kernels; cv.bias / cv.bias_dtype also by the plain epilogue (a bias per row of C)
   PackGeom pk;            // read by the GATHER kernels (with cv's output side)
+};
+
+// GemmParams as the kernels with the DMA loader and no conv2d get them (expand_params).  Up to 112 bytes of arguments a launch
+// takes the host 2.6 us, from 120 on 3.3 to 3.8, and small products wait for the host: with GemmParams itself (480 bytes)
+// 64 x 64 x 64 through tritonix.matmul 5.99 us and 3.28 from C, with these 5.55 and 2.58.  So what a workgroup can work out in a few scalar
+// instructions is left out: counts of tiles, unit strides, shifts of divisors.
+struct PlainParams {
+  const uint8_t* a;
+  const uint8_t* b;
+  uint8_t* c;
+  uint8_t* ws;            // launches of several problems, which cut nothing: the bias
+  int64_t lda, ldb;       // of A's rows (AT: of its k), of B's k rows (BT: of its n)
+  int64_t scm, scn;
+  int32_t m, n, k;
+  int32_t group_m, split_k, split_tile0, ktiles_per_split;
+  uint32_t mul_tiles;     // multipliers of div_tiles or, with a cut, div_cut;
+  uint32_t mul_group, mul_rows, mul_rows_last;
+  uint32_t flags;
+};
+static_assert(sizeof(PlainParams) == 112, "a longer argument list costs every launch 0.7 us");
+enum : uint32_t {
+  PF_EPILOGUE = 7u, PF_OUT_SHIFT = 3, PF_BIAS_SHIFT = 6,                          // three bits each
+  PF_C_VEC = 1u << 9, PF_C_ROW = 1u << 10, PF_TAIL = 1u << 11, PF_B_ONCE = 1u << 12, PF_ORDER = 1u << 13, PF_ATOMIC = 1u << 14,
+  PF_PADDED = 1u << 15, PF_MANY = 1u << 16
 };
 
 // ---------------------------------------------------------------------------
@@ -253,11 +281,72 @@ __device__ __forceinline__ void swizzle2d(int ij, const GemmParams& p, int* oi, 
   const bool last = p.tiles_m - off_i < p.group_m;
   const int g = last ? p.tiles_m - off_i : p.group_m;
   const int r = ij - group_id * p.group_m * p.tiles_n;
-  const FastDiv d = last ? p.div_rows_last : p.div_rows;
-  const int q = (int)fd_div((uint32_t)r, d);
+  const int q = (int)fd_div((uint32_t)r, fd_of(last ? p.div_rows_last.mul : p.div_rows.mul, (uint32_t)g));
   *oi = off_i + r - q * g;
   *oj = q;
 }
+
+// false: not a launch that PlainParams can describe (none that gemm_launch makes)
+inline bool plain_params(const GemmParams& p, bool bt, bool at, int es, PlainParams* q) {
+  const bool many = p.batch > 1 || p.cv.bias;
+  const int es_out = p.out_dtype == DT_F32 || p.out_dtype == DT_I32 ? 4 : 2;
+  if (p.m > 0x7fffffff || p.n > 0x7fffffff || p.k > 0x7fffffff) return false;
+  if ((at ? p.sam : p.sak) != 1 || (bt ? p.sbk : p.sbn) != 1) return false;
+  if (many && (p.split_k > 1 || bt || at)) return false;
+  if (p.batch > 1 && (p.b_batch_bytes != p.k * p.sbk * es || p.c_batch_bytes != p.m * p.scm * es_out)) return false;
+  const bool padded = p.m_load != p.m || p.n_load != p.n;
+  if (padded && (p.m_load != (p.m + 7) / 8 * 8 || p.n_load != (p.n + 7) / 8 * 8)) return false;
+  q->a = p.a; q->b = p.b; q->c = p.c;
+  q->ws = many ? (uint8_t*)p.cv.bias : p.ws;
+  q->lda = at ? p.sak : p.sam; q->ldb = bt ? p.sbn : p.sbk;
+  q->scm = p.scm; q->scn = p.scn;
+  q->m = (int32_t)p.m; q->n = (int32_t)p.n; q->k = (int32_t)p.k;
+  q->group_m = p.group_m < p.tiles_m ? p.group_m : p.tiles_m;            // a group of more rows than there are: the same order
+  q->split_k = p.split_k; q->split_tile0 = p.split_tile0; q->ktiles_per_split = p.ktiles_per_split;
+  GemmParams d;
+  d.tiles_m = p.tiles_m; d.tiles_n = p.tiles_n; d.group_m = q->group_m; d.split_tile0 = p.split_tile0;
+  set_order_divisors(&d);
+  q->mul_tiles = p.split_k > 1 ? d.div_cut.mul : d.div_tiles.mul;
+  q->mul_group = d.div_group.mul; q->mul_rows = d.div_rows.mul; q->mul_rows_last = d.div_rows_last.mul;
+  q->flags = (uint32_t)p.epilogue | (uint32_t)p.out_dtype << PF_OUT_SHIFT | (p.cv.bias ? (uint32_t)p.cv.bias_dtype << PF_BIAS_SHIFT : 0u) |
+             (p.c_vec_ok ? PF_C_VEC : 0u) | (p.c_row_ok ? PF_C_ROW : 0u) | (p.tail_slab ? PF_TAIL : 0u) | (p.b_once ? PF_B_ONCE : 0u) |
+             (p.tile_order ? PF_ORDER : 0u) | (p.atomic_reduce ? PF_ATOMIC : 0u) | (padded ? PF_PADDED : 0u) | (many ? PF_MANY : 0u);
+  return true;
+}
+template <class C, bool BT, bool AT> __device__ __forceinline__ GemmParams expand_params(const PlainParams& q) {
+  GemmParams p;
+  const bool many = (q.flags & PF_MANY) != 0, padded = (q.flags & PF_PADDED) != 0;
+  p.a = q.a; p.b = q.b; p.c = q.c; p.ws = q.ws;
+  p.m = q.m; p.n = q.n; p.k = q.k;
+  p.sam = AT ? 1 : q.lda; p.sak = AT ? q.lda : 1;
+  p.sbk = BT ? 1 : q.ldb; p.sbn = BT ? q.ldb : 1;
+  p.scm = q.scm; p.scn = q.scn;
+  p.tiles_m = (int)(((uint32_t)q.m + C::BM - 1) / C::BM); p.tiles_n = (int)(((uint32_t)q.n + C::BN - 1) / C::BN);
+  p.group_m = q.group_m; p.split_k = q.split_k; p.split_tile0 = q.split_tile0; p.ktiles_per_split = q.ktiles_per_split;
+  p.epilogue = (int)(q.flags & PF_EPILOGUE); p.out_dtype = (int)(q.flags >> PF_OUT_SHIFT & 7u);
+  p.c_vec_ok = (q.flags & PF_C_VEC) != 0; p.c_row_ok = (q.flags & PF_C_ROW) != 0;
+  p.tail_slab = (q.flags & PF_TAIL) != 0; p.b_once = (q.flags & PF_B_ONCE) != 0;
+  p.tile_order = (q.flags & PF_ORDER) != 0; p.atomic_reduce = (q.flags & PF_ATOMIC) != 0;
+  p.m_load = padded ? (p.m + 7) / 8 * 8 : p.m; p.n_load = padded ? (p.n + 7) / 8 * 8 : p.n;
+  p.batch = many ? 2 : 1;                                               // one problem or several: what the kernel asks
+  p.b_batch_bytes = p.k * p.sbk * C::ES; p.c_batch_bytes = p.m * p.scm * (p.out_dtype == DT_F32 || p.out_dtype == DT_I32 ? 4 : 2);
+  const uint32_t tiles = (uint32_t)(p.tiles_m * p.tiles_n);
+  p.div_tiles = fd_of(q.mul_tiles, tiles); p.div_cut = fd_of(q.mul_tiles, tiles - (uint32_t)q.split_tile0);
+  p.div_group = fd_of(q.mul_group, (uint32_t)(q.group_m * p.tiles_n));
+  p.div_rows.mul = q.mul_rows; p.div_rows_last.mul = q.mul_rows_last;
+  p.cv.bias = many ? q.ws : nullptr; p.cv.bias_dtype = (int)(q.flags >> PF_BIAS_SHIFT & 7u);
+  return p;
+}
+// One launch of a kernel with one argument, straight from its address: without the stub that <<< >>> calls, 2.6 us instead of 2.75.
+inline hipError_t launch_kernel(const void* kernel, unsigned grid, unsigned threads, unsigned lds, hipStream_t stream, void* arg) {
+  void* args[] = {arg};
+  const hipError_t err = hipLaunchKernel(kernel, dim3(grid), dim3(threads), args, lds, stream);
+  if (err != hipSuccess) (void)hipGetLastError();
+  return err;
+}
+
+template <bool PLAIN> struct KernelParams { typedef GemmParams type; };
+template <> struct KernelParams<true> { typedef PlainParams type; };
 
 // Chip-level tile order for grids much larger than the CU count.  The 256 workgroups that run
 // together (one per CU) take one 16x16 super-block of tiles, so one "round" touches 16 row panels
@@ -1137,7 +1226,10 @@ constexpr int GATHER_TABLE_BYTES = 8192;
 // pixel's, kept in a register, plus the chunk's (filter tap, channels), read once per slab from a table in LDS.  Chunks
 // past the end of k get an offset outside the buffer and arrive as zeros.
 template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bool CONV = false, bool GATHER = false, bool AT = false, bool PAIR = false>
-__global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void gemm_tile_kernel(GemmParams p) {
+__global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void gemm_tile_kernel(typename KernelParams<FAST && !CONV && !GATHER>::type in) {
+  GemmParams p;
+  if constexpr (FAST && !CONV && !GATHER) p = expand_params<C, BT, AT>(in);
+  else p = in;
   constexpr int ES = C::ES, BM = C::BM, BN = C::BN, BK = C::BK, NW = C::NW, STAGES = C::STAGES;
   constexpr int MI = C::MI, TM = C::TM, TN = C::TN;
   static_assert(GATHER ? C::VALID_GATHER : C::VALID, "tile configuration not supported by this kernel");

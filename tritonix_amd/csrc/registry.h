@@ -71,10 +71,15 @@ template <class T, class C, bool FAST, bool PERSIST = false, bool BT = false, bo
           bool AT = false, bool PAIR = false>
 hipError_t launch_tile(const GemmParams& p, unsigned grid, hipStream_t stream) {
   static_assert(GATHER ? C::VALID_GATHER : C::VALID, "tile configuration is not buildable");
-  GemmParams q = p;
-  set_order_divisors(&q);
-  hipLaunchKernelGGL((gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV, GATHER, AT, PAIR>), dim3(grid), dim3(C::THREADS), 0, stream, q);
-  return hipGetLastError();
+  constexpr bool PLAIN = FAST && !CONV && !GATHER;
+  typename KernelParams<PLAIN>::type q;
+  if constexpr (PLAIN) {
+    if (!plain_params(p, BT, AT, C::ES, &q)) return hipErrorInvalidValue;
+  } else {
+    q = p;
+    set_order_divisors(&q);
+  }
+  return launch_kernel((const void*)&gemm_tile_kernel<T, C, FAST, PERSIST, BT, CONV, GATHER, AT, PAIR>, grid, C::THREADS, 0, stream, &q);
 }
 
 // The persistent variant exists for the four-wave tiles from 128x128 to 256x128 / 128x256: their ring leaves
