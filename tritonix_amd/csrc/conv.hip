@@ -889,9 +889,11 @@ static int packed_forward(const tnx_conv2d_args* a, const PackedPlan& pl) {
   k.div_chunks = make_fastdiv((uint32_t)k.chunks_pad);
   const unsigned blocks = k.w_blocks + (unsigned)((waves + 3) / 4);
   hipStream_t stream = (hipStream_t)a->stream;
-  if (!f32) hipLaunchKernelGGL((conv_pack_kernel<uint16_t, 1>), dim3(blocks), dim3(256), 0, stream, k);
-  else if (pl.terms == 2) hipLaunchKernelGGL((conv_pack_kernel<float, 2>), dim3(blocks), dim3(256), 0, stream, k);
-  else hipLaunchKernelGGL((conv_pack_kernel<float, 3>), dim3(blocks), dim3(256), 0, stream, k);
+  const bool unit = pl.step_w == 1;
+  void (*pack)(PackParams) = !f32 ? (unit ? conv_pack_kernel<uint16_t, 1, true> : conv_pack_kernel<uint16_t, 1, false>)
+                             : pl.terms == 2 ? (unit ? conv_pack_kernel<float, 2, true> : conv_pack_kernel<float, 2, false>)
+                                             : (unit ? conv_pack_kernel<float, 3, true> : conv_pack_kernel<float, 3, false>);
+  hipLaunchKernelGGL(pack, dim3(blocks), dim3(256), 0, stream, k);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) { note_hip_error((int)err); return TNX_E_HIP; }
 

@@ -17,6 +17,11 @@
 // lanes 8 neighbouring column chunks, so loads and stores both move 128-byte runs.  256 channels of 56x56, batch 32, bf16:
 // 17.9 us for 51 MB in and 55 MB out, 5.9 TB/s (a plain copy of that size: 15.7 us); with the blocks dealt round-robin to
 // the XCDs 25.3 us, with non-temporal loads 31 us.
+//
+// Small inputs are bound by the latency of one wave instead, so its loads do not wait for one another and its lanes share one
+// path (see fetch): with a condition around each load, layers took, both launches in a graph, 59 -> 64 channels of 14x14, 3x3,
+// batch 4 10.6 us, now 8.5; 512 -> 512 of 7x7, one image 15.4, 13.0; with a stride of two, where half of the lanes went element by
+// element, 384 -> 256 of 28x28, 1x1, batch 8 13.8, 9.7, and 896 -> 2048, batch 128 192, 164.
 #pragma once
 #include "gemm_tile.h"
 
@@ -68,7 +73,34 @@ template <int NT> __device__ __forceinline__ int term_chunk(int z, int cg, int c
   return NT == 2 ? (cg >> 2) * 8 + z * 4 + (cg & 3) : z * cp8 + cg;
 }
 
-template <class E, int NT>
+// Eight elements from `at` on, or from the nearest place where all eight lie inside [0, elems), elems >= 8 ...
+template <class E> constexpr int RUN = 2 * sizeof(E);                     // 32-bit words of eight elements
+template <class E> __device__ __forceinline__ void load_run(uint32_t* v, const E* src, int at, int elems) {
+  struct __attribute__((packed, aligned(sizeof(E)))) Run { uint32_t v[RUN<E>]; };
+  const Run r = *(const Run*)(src + (at < 0 ? 0 : at > elems - 8 ? elems - 8 : at));
+#pragma unroll
+  for (int i = 0; i < RUN<E>; ++i) v[i] = r.v[i];
+}
+// ... and those of them that do exist back at their index.
+template <class E> __device__ __forceinline__ void turn_run(uint32_t* v, int at, int elems) {
+  constexpr int W = RUN<E>;
+  const int d = at - (at < 0 ? 0 : at > elems - 8 ? elems - 8 : at);
+  if (d == 0 || d <= -8 || d >= 8) return;                                // (wholly outside: nothing to put back)
+#pragma unroll
+  for (int by = 1; by < 8; by *= 2) {
+    uint32_t t[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      if (W == 8) t[i] = v[(i + by) & 7];
+      else t[i] = by == 1 ? v[i] >> 16 | v[(i + 1) & 3] << 16 : v[(i + by / 2) & 3];
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i) v[i] = d & by ? t[i] : v[i];
+  }
+}
+
+// UNIT: step_w is 1 (77 registers instead of 118, float32 128 instead of 158: one kernel for both lost 1 to 5 % in float32)
+template <class E, int NT, bool UNIT>
 __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
   const int tid = threadIdx.x;
   if (blockIdx.x < p.w_blocks) {
@@ -91,12 +123,17 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
       }
       const int term = NT == 1 ? 0 : NT == 2 ? (r >> 2) & 1 : (int)fd_div((uint32_t)r, p.div_cp8);
       const int cg = NT == 2 ? (r >> 3) * 4 + (r & 3) : r - term * p.cp8;
-      const E* src = (const E*)p.w + ((int64_t)co * p.c_in + cg * 8) * p.taps + tap;
+      const E* src = (const E*)p.w + (int64_t)co * p.c_in * p.taps + tap;
+      E v8[8] = {};                                   // all loads before the first wait: a channel that does not exist repeats the last one
+      if (cg * 8 < p.c_in) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v8[e] = src[(int64_t)(cg * 8 + e < p.c_in ? cg * 8 + e : p.c_in - 1) * p.taps];
+      }
       uint16_t o[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         uint16_t t[NT];
-        pack_terms<1>(cg * 8 + e < p.c_in ? src[(int64_t)e * p.taps] : (E)0, t);
+        pack_terms<1>(cg * 8 + e < p.c_in ? v8[e] : (E)0, t);
         o[e] = t[0];
         if constexpr (NT == 2) o[e] = term == 0 ? t[0] : t[1];
         if constexpr (NT == 3) o[e] = term == 0 ? t[0] : term == 1 ? t[1] : t[2];
@@ -114,52 +151,101 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
   if (j >= p.x_items || cg >= p.cp8) return;
   const int row_all = (int)fd_div((uint32_t)j, p.div_wchunks), wc = j - row_all * p.wchunks;
   const int img = (int)fd_div((uint32_t)row_all, p.div_row), row = row_all - img * p.rows;
-  const int h = row * p.step_h - p.pad_h, col0 = wc * 8 + p.lead, w0 = col0 * p.step_w - p.pad_w;
-  E in[8][8];                                       // [channel][column]
+  const int step_w = UNIT ? 1 : p.step_w, h = row * p.step_h - p.pad_h, col0 = wc * 8 + p.lead, w0 = col0 * step_w - p.pad_w;
+  constexpr int W = RUN<E>;
+  uint32_t raw[8][W];                               // [channel][column], two 16-bit columns a word
 #pragma unroll
   for (int c = 0; c < 8; ++c)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) in[c][e] = (E)0;
-  if ((uint32_t)h < (uint32_t)p.h_in && w0 < p.w_in && w0 + 7 * p.step_w >= 0) {
+    for (int i = 0; i < W; ++i) raw[c][i] = 0;
+  if ((uint32_t)h < (uint32_t)p.h_in && w0 < p.w_in && w0 + 7 * step_w >= 0 && cg * 8 < p.c_in) {
     const int plane = p.h_in * p.w_in;
     const int o0 = ((img * p.c_in + cg * 8) * p.h_in + h) * p.w_in + w0;    // element of (channel 0, column 0)
     const E* src = (const E*)p.x;
     const int nch = p.c_in - cg * 8 < 8 ? p.c_in - cg * 8 : 8;
-    const int lo = w0 < 0 ? -w0 : 0, hi = p.w_in - w0;                      // elements [lo, hi) of a unit-stride run lie in the row
-    if (p.step_w == 1 && o0 >= 0 && o0 + (nch - 1) * plane <= p.x_elems - 8) {
+    if ((UNIT || step_w == 2) && p.x_elems >= 8) {
+      // All loads are on their way before the first is waited for, and no lane takes another path at the edges: a load under a
+      // condition of its own is waited for at the condition's end, eight latencies in a row.  So for channels that do not exist
+      // and runs past the row all lanes read the input's first elements, a run that would leave the input is moved inside it and
+      // turned back, and what lies outside the row is cleared.
+      auto at = [&](int c) { return c < nch ? o0 + c * plane : 0; };
+      const bool edge = o0 < 0 || o0 + (nch - 1) * plane + 8 * (step_w - 1) > p.x_elems - 8;
+      // NC channels, every STEP-th element of RUNS runs
+      auto fetch = [&](auto nc, auto step, auto runs) {
+        constexpr int NC = nc, STEP = step, RUNS = runs, CB = RUNS == 2 && W == 8 ? 2 : NC;   // channels at a time, as the registers allow
+        auto at_run = [&](int c, int r) { return r == 0 || w0 + 8 < p.w_in ? at(c) + 8 * r : 0; };
 #pragma unroll
-      for (int c = 0; c < 8; ++c)
-        if (c < nch) {
-          struct __attribute__((packed, aligned(sizeof(E)))) Row { E v[8]; };
-          const Row v = *(const Row*)(src + o0 + c * plane);
+        for (int c0 = 0; c0 < NC; c0 += CB) {
+          uint32_t t[CB][RUNS * W];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) in[c][e] = v.v[e];
-        }
-      if (lo > 0 || hi < 8) {
+          for (int c = 0; c < CB; ++c)
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (e < lo || e >= hi) {
+            for (int r = 0; r < RUNS; ++r) load_run<E>(t[c] + r * W, src, at_run(c0 + c, r), p.x_elems);
+          if (edge) {
 #pragma unroll
-            for (int c = 0; c < 8; ++c) in[c][e] = (E)0;
+            for (int c = 0; c < CB; ++c)
+#pragma unroll
+              for (int r = 0; r < RUNS; ++r) turn_run<E>(t[c] + r * W, at_run(c0 + c, r), p.x_elems);
           }
-      }
-    } else if (p.step_w == 2 && w0 >= 0 && w0 + 16 <= p.w_in) {
 #pragma unroll
-      for (int c = 0; c < 8; ++c)
-        if (c < nch) {
-          struct __attribute__((packed, aligned(sizeof(E)))) Row { E v[16]; };
-          const Row v = *(const Row*)(src + o0 + c * plane);
+          for (int c = 0; c < CB; ++c)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) in[c][e] = v.v[2 * e];
+            for (int i = 0; i < W * RUNS / STEP; ++i)
+              raw[c0 + c][i] = STEP == 1 ? t[c][i] : W == 8 ? t[c][2 * i] : (t[c][2 * i] & 0xffffu) | t[c][2 * i + 1] << 16;
         }
+        if (w0 < 0 || w0 + 7 * step_w >= p.w_in) {
+          auto in_row = [&](int e) { return (uint32_t)(w0 + e * step_w) < (uint32_t)p.w_in; };
+#pragma unroll
+          for (int i = 0; i < W; ++i) {
+            const uint32_t keep = W == 8 ? (in_row(i) ? ~0u : 0u) : (in_row(2 * i) ? 0xffffu : 0u) | (in_row(2 * i + 1) ? 0xffff0000u : 0u);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) raw[c][i] &= keep;
+          }
+        }
+        if (nch < NC) {
+#pragma unroll
+          for (int c = 1; c < NC; ++c)
+#pragma unroll
+            for (int i = 0; i < W; ++i) raw[c][i] = c < nch ? raw[c][i] : 0u;
+        }
+      };
+      // (rows that one run covers need no second, inputs of few channels no repeats)
+      constexpr std::integral_constant<int, 1> one;
+      constexpr std::integral_constant<int, 2> two;
+      constexpr std::integral_constant<int, 4> four;
+      constexpr std::integral_constant<int, 8> eight;
+      if constexpr (UNIT) {
+        if (p.c_in <= 4) fetch(four, one, one);
+        else fetch(eight, one, one);
+      } else {
+        if (p.w_in + p.pad_w <= 8) fetch(eight, two, one);
+        else fetch(eight, two, two);
+      }
     } else {
+#pragma unroll 1
+      for (int c = 0; c < nch; ++c) {
+        uint16_t h16[8];
+        uint32_t t[W];
 #pragma unroll
-      for (int c = 0; c < 8; ++c)
+        for (int e = 0; e < 8; ++e) {
+          const E v = (uint32_t)(w0 + e * step_w) < (uint32_t)p.w_in ? src[o0 + c * plane + e * step_w] : (E)0;
+          if constexpr (W == 8) t[e] = __builtin_bit_cast(uint32_t, v);
+          else h16[e] = v;
+        }
+        if constexpr (W == 4) __builtin_memcpy(t, h16, 16);
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (c < nch && (uint32_t)(w0 + e * p.step_w) < (uint32_t)p.w_in) in[c][e] = src[o0 + c * plane + e * p.step_w];
+        for (int x = 0; x < 8; ++x)
+#pragma unroll
+          for (int i = 0; i < W; ++i) raw[x][i] = x == c ? t[i] : raw[x][i];
+      }
     }
   }
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int i = 0; i < W; ++i) asm("" : "+v"(raw[c][i]));      // words, not halves, cross the branches
+  E in[8][8];
+  __builtin_memcpy(in, raw, sizeof in);
   uint8_t* dst = p.xp + ((int64_t)row_all * p.cols + col0) * (p.cp8 * NT) * 16;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
