@@ -1597,13 +1597,106 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
 #pragma unroll
     for (int u = 0; u < GEN_NB; ++u) gen_store_b(stage_base, t0 + u * C::THREADS, rb[u]);
   };
-  // one chunk at a time: for the prologue of the kernels without the DMA loader and the one call after the K loop
-  // of a tail_slab launch, where nothing is there to overlap with and registers are better left alone
+  // one chunk at a time: for the prologue of the kernels without the DMA loader, and for operands of a tail_slab launch whose rows are
+  // shorter than a chunk
   auto load_slab_generic = [&](int kt_global, uint32_t stage_base, int t0) __attribute__((always_inline)) {
 #pragma unroll 1
     for (int idx = t0; idx < BM * C::CPR_A; idx += C::THREADS) gen_store_a(stage_base, idx, gen_fetch_a(kt_global, idx));
 #pragma unroll 1
     for (int idx = t0; idx < GEN_B_ROWS * GEN_B_CPR; idx += C::THREADS) gen_store_b(stage_base, idx, gen_fetch_b(kt_global, idx));
+  };
+
+  // The left-out slab of a tail_slab launch, with the DMA kernels' unit strides: all of a thread's chunks are on their way before the
+  // first is waited for.  One chunk after another, each under conditions of its own, as load_slab_generic does it, cost a latency
+  // apiece with nothing to hide it (447 x 14336 x 83 int8, BT: 11.7 -> 9.2 us; 256 x 872 x 904 8.2 -> 6.4; 1150 x 2300 x 1111 bf16 18.0 -> 17.1).
+  // What lies past k is cleared; a chunk that crosses n, or m of an m-contiguous A, brings what comes after it, for columns that are never
+  // stored.  Only in the matrix's last row is there nothing after it: such a chunk is fetched as the row's last 16 bytes and shifted
+  // down.  Rows and chunks that do not exist read the first one's place.
+  auto load_tail = [&](int kt_global, uint32_t stage_base, int t0) __attribute__((always_inline)) {
+    const int64_t k0 = (int64_t)kt_global * BK;
+    const int krem = (int)(p.k - k0);                               // 1 .. BK
+    struct Side {
+      const uint8_t* base;
+      int64_t ld;
+      int rows, left, odd;         // rows of the slab, elements of a row from the slab's first on, elements of a row past whole chunks
+      bool ends;                   // a chunk that crosses the end of the matrix's last row
+    };
+    auto side = [&](const uint8_t* base, int64_t ld, int rows, bool last_row, int64_t left, int64_t len, int span) __attribute__((always_inline)) {
+      const int odd = (int)(len % EPC);
+      return Side{base, ld, rows, left < span ? (int)left : span, odd, last_row && odd != 0 && left < span};
+    };
+    auto fetch = [&](const Side& d, auto ntag, int cpr, int count, i32x4* r) __attribute__((always_inline)) {
+      constexpr int N = decltype(ntag)::value;
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        int idx = t0 + u * C::THREADS;
+        if (N * C::THREADS != count) idx = idx < count ? idx : count - 1;
+        int row = idx / cpr, pos = idx % cpr * EPC;
+        const bool none = row >= d.rows || pos >= d.left;
+        row = none ? 0 : row;
+        pos = none ? 0 : pos;
+        pos = d.ends && row == d.rows - 1 && pos + EPC > d.left ? d.left - EPC : pos;
+        r[u] = *(const gen_chunk_t*)(d.base + (uint32_t)((int64_t)row * d.ld * ES) + (int64_t)(pos * ES));
+      }
+      if (d.ends) {
+        const int cut = (EPC - d.odd) * ES;                         // bytes a crossing chunk moves down
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+          const int idx = t0 + u * C::THREADS, pos = idx % cpr * EPC;
+          if (idx / cpr == d.rows - 1 && pos < d.left && pos + EPC > d.left) {
+            uint32_t w[4] = {(uint32_t)r[u].x, (uint32_t)r[u].y, (uint32_t)r[u].z, (uint32_t)r[u].w};
+#pragma unroll
+            for (int by = 8; by >= 4; by /= 2) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) w[i] = cut & by ? (i + by / 4 < 4 ? w[i + by / 4] : 0u) : w[i];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = (uint32_t)(((uint64_t)(i < 3 ? w[i + 1] : 0u) << 32 | w[i]) >> ((cut & 3) * 8));
+            r[u] = i32x4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+          }
+        }
+      }
+    };
+    // k along the row: elements past k; k rows: rows past k
+    auto clear_k = [&](const Side& d, auto ntag, int cpr, i32x4* r) __attribute__((always_inline)) {
+      constexpr int N = decltype(ntag)::value;
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const int valid = (d.left - (t0 + u * C::THREADS) % cpr * EPC) * ES;      // bytes
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int bytes = valid - 4 * i;
+          r[u][i] &= bytes >= 4 ? -1 : bytes <= 0 ? 0 : (1 << bytes * 8) - 1;
+        }
+      }
+    };
+    auto clear_rows = [&](auto ntag, int cpr, i32x4* r) __attribute__((always_inline)) {
+      constexpr int N = decltype(ntag)::value;
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+        if ((t0 + u * C::THREADS) / cpr >= krem) r[u] = i32x4{0, 0, 0, 0};
+    };
+    const int64_t len_a = AT ? p.m : p.k, len_b = BT ? p.k : p.n;
+    // (a row-major B and one chunk of k: what exists is a few rows of B and one chunk of each row of A, and the loop that skips
+    // the rest takes no longer -- 1025 x 2050 x 4100 36.1 us against 36.6, 1100 x 1100 x 1027 11.2 against 11.5)
+    if (len_a < EPC || len_b < EPC || (!BT && krem <= EPC)) {
+      load_slab_generic(kt_global, stage_base, t0);
+      return;
+    }
+    constexpr int CPR_A = AT ? AT_CPR : C::CPR_A;
+    const int64_t lda = AT ? p.sak : p.sam, ldb = BT ? p.sbn : p.sbk, mleft = p.m - m0, nleft = p.n - n0;
+    const Side da = AT ? side(p.a + (k0 * lda + m0) * ES, lda, krem, true, mleft, len_a, BM)
+                       : side(p.a + (m0 * lda + k0) * ES, lda, mleft < BM ? (int)mleft : BM, mleft <= BM, krem, len_a, BK);
+    const Side db = BT ? side(p.b + (n0 * ldb + k0) * ES, ldb, nleft < BN ? (int)nleft : BN, nleft <= BN, krem, len_b, BK)
+                       : side(p.b + (k0 * ldb + n0) * ES, ldb, krem, true, nleft, len_b, BN);
+    i32x4 ra[GEN_NA], rb[GEN_NB];
+    fetch(da, IntTag<GEN_NA>{}, CPR_A, BM * C::CPR_A, ra);
+    fetch(db, IntTag<GEN_NB>{}, GEN_B_CPR, GEN_B_ROWS * GEN_B_CPR, rb);
+    if constexpr (AT) clear_rows(IntTag<GEN_NA>{}, CPR_A, ra);
+    else clear_k(da, IntTag<GEN_NA>{}, CPR_A, ra);
+    if constexpr (BT) clear_k(db, IntTag<GEN_NB>{}, GEN_B_CPR, rb);
+    else clear_rows(IntTag<GEN_NB>{}, GEN_B_CPR, rb);
+    gen_store(stage_base, t0, ra, rb);
   };
 
   // CONV: the first 64 threads write the taps of the next slab to tabulate into the table of its parity and move
@@ -2333,11 +2426,12 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
       if (tail_here) {
         // the left-out slab: every wave is done with the ring, slot 0 takes it, one slab of MFMAs follows
         __syncthreads();
-        load_slab_generic(kt1 - 1, stage_of(0), wave * 64 + lane);
+        load_tail(kt1 - 1, stage_of(0), wave * 64 + lane);
         __syncthreads();
         const uint32_t sa = stage_of(0), sb = sa + C::A_BYTES;
 #pragma unroll
         for (int ks = 0; ks < C::KSTEPS; ++ks) {
+          if (ks > 0 && p.k - (int64_t)(kt1 - 1) * BK <= ks * (BK / C::KSTEPS)) break;      // zeros
 #pragma unroll
           for (int idx = 0; idx < NREAD; ++idx) read_one(0, idx, sa, sb, ks);
 #pragma unroll
