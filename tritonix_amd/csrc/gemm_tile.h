@@ -286,13 +286,15 @@ __device__ __forceinline__ void swizzle2d(int ij, const GemmParams& p, int* oi, 
   *oj = q;
 }
 
-// false: not a launch that PlainParams can describe (none that gemm_launch makes)
+// false: not a launch that PlainParams can describe.  gemm_launch makes none: strides of 1 along a chunk are what its layouts ask for, a
+// split excludes problems and bias there, and the one caller with several problems (conv2d's 1x1 layers) has dense operands -- which
+// for one input channel on 1x1 planes count as a k-contiguous B.
 inline bool plain_params(const GemmParams& p, bool bt, bool at, int es, PlainParams* q) {
   const bool many = p.batch > 1 || p.cv.bias;
   const int es_out = p.out_dtype == DT_F32 || p.out_dtype == DT_I32 ? 4 : 2;
   if (p.m > 0x7fffffff || p.n > 0x7fffffff || p.k > 0x7fffffff) return false;
   if ((at ? p.sam : p.sak) != 1 || (bt ? p.sbk : p.sbn) != 1) return false;
-  if (many && (p.split_k > 1 || bt || at)) return false;
+  if (many && p.split_k > 1) return false;
   if (p.batch > 1 && (p.b_batch_bytes != p.k * p.sbk * es || p.c_batch_bytes != p.m * p.scm * es_out)) return false;
   const bool padded = p.m_load != p.m || p.n_load != p.n;
   if (padded && (p.m_load != (p.m + 7) / 8 * 8 || p.n_load != (p.n + 7) / 8 * 8)) return false;
