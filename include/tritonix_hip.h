@@ -128,12 +128,12 @@ typedef struct tnx_gemm_args {
  *   - A row-major (stride_ak == 1) and B row-major (stride_bn == 1): the direct-to-LDS loader of every built tile.
  *     With K a multiple of block_k, 16-byte aligned rows and base pointers and N a multiple of 16 bytes of elements
  *     every K slab goes through it; otherwise (rows and pointers at the element's own alignment, any K and N, row
- *     pitches at least the row length) the last K slab is loaded chunk by chunk with zero fill and the slabs
+ *     pitches at least the row length) the last K slab is loaded through registers, zeros past k, and the slabs
  *     before it through the direct loader.
  *     TNX_SCHED_PERSISTENT takes the first form only.
  *   - A row-major and B k-contiguous (stride_bk == 1, the view w.t() of a row-major weight): a direct-to-LDS loader
  *     of its own, in the tiles whose K slab is 128 bytes per row, under the same two sets of conditions (K a multiple
- *     of block_k and 16-byte aligned rows and pointers, or else the last K slab loaded chunk by chunk).
+ *     of block_k and 16-byte aligned rows and pointers, or else the last K slab loaded through registers).
  *   - anything else (strided A, overlapping rows, ...): the element-wise loader, built for two tiles per type
  *     (128x128 and 64x128, four waves, two stages); other tiles return TNX_E_UNSUPPORTED. */
 int tnx_gemm(const tnx_gemm_args* args);
@@ -217,9 +217,9 @@ size_t tnx_gemm_f32_scratch_bytes(const tnx_gemm_args* args);
 int tnx_gemm_f32(const tnx_gemm_args* args, void* scratch, size_t scratch_bytes);
 int tnx_gemm_f32_config(tnx_gemm_args* args);
 
-/* How many K slabs (of block_k) at the end of k a launch of `args` loads element by element, no access outside the
- * operands: 0 where all of them go through the ring of whole 16-byte chunks, 1 where rows, base pointers or sizes are no
- * whole chunks, all of them on the element-wise loader; -1 if tnx_gemm would refuse the arguments.  For tests and
+/* How many K slabs (of block_k) at the end of k a launch of `args` loads through registers instead of the ring of whole 16-byte
+ * chunks, no access outside the operands: 0 where rows, base pointers and sizes are whole chunks, 1 where they are
+ * not, all of them on the element-wise loader; -1 if tnx_gemm would refuse the arguments.  For tests and
  * tooling: pure host arithmetic, of a and b only the alignment counts. */
 int tnx_gemm_tail_slabs(const tnx_gemm_args* args);
 

@@ -102,7 +102,8 @@ static int check_common(const tnx_gemm_args* a, GemmForm form) {
 // *tail: the operands have such a layout but not as the DMA loader likes it best -- K no multiple of block_k, rows or
 // base pointers not 16-byte aligned (the loads take any byte address: probed on the hardware), N (layout 3: or M) ending
 // inside a 16-byte chunk -- so the last K slab, the only one whose chunks can cross the end of a row of A or of the last
-// row of B, is loaded element by element instead (GemmParams::tail_slab).
+// row of B, is left out of the ring and fetched after it (GemmParams::tail_slab).  That fetch reads into what follows a row, so
+// it needs a pitch of at least the row's length.
 // *narrow: the operands have such a layout, but rows shorter than a chunk and a last slab of few rows let a chunk of the
 // slab before it end past the operand (ring_chunks_inside): the layout is not taken.
 static int dma_layout(const tnx_gemm_args* a, bool* tail = nullptr, bool* narrow = nullptr) {
@@ -480,7 +481,7 @@ extern "C" int tnx_gemm_static_workspace(const tnx_gemm_args* a) {
 //   slab       a K slab of one workgroup per CU                        shared  a slab of as many as share a CU, against one
 //   step       what part of such a round the first workgroup in it costs (the rest grows with their number)
 //   crowd      slab's growth from few workgroups to one on every CU    bt      its growth for a k-contiguous B
-//   a_off, b_off  ... for rows of A, of B that are not 16-byte aligned  tail    the last slab, where it goes chunk by chunk
+//   a_off, b_off  ... for rows of A, of B that are not 16-byte aligned  tail    the last slab, where it is left out of the ring
 //   cut, cut_slice, cut_all  K cut: fixed, per slice of 64 KiB, and per 16 MiB of slices in all
 //   store      C, in units of 0.2 us per MB
 struct TileCost {

@@ -135,7 +135,7 @@ struct GemmParams {
   bool c_vec_ok;          // C takes 16-byte stores along n (stride_cn == 1, 16-byte aligned rows)
   bool c_row_ok;          // stride_cn == 1: rows of C take 16-byte stores at the element's own alignment
   int64_t m_load, n_load; // DMA kernels: rows of an m-contiguous A and columns of B that may be loaded (>= m, n: operands padded to whole chunks)
-  int tail_slab;          // DMA kernels: the last K slab (whole or partial) goes through the element-wise loader
+  int tail_slab;          // DMA kernels: the last K slab (whole or partial) is left out of the ring and fetched after the K loop (load_tail)
   bool b_once;            // every element of B is read by exactly one workgroup (one tile row): stream it non-temporally
   int tile_order;         // 0: XCD remap + tl.swizzle2d(group_m); 1: 16x16 super-blocks in serpentine order (superblock_order)
   int atomic_reduce;      // split-K: slices are added into one fp32/int32 copy with device-scope atomics instead of being kept apart
@@ -1318,7 +1318,8 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
   // FAST kernels move their slabs with the DMA loader.  It wants chunks that lie inside their row: with a K that is
   // no multiple of BK, rows that are not 16-byte aligned or an N that ends inside a chunk, the host sets tail_slab
   // and the last slab of the K range (the only one whose chunks can cross the end of a row of A, or the end of the
-  // last row of B) is left out of the ring and loaded element by element, zero-filled, after the K loop.
+  // last row of B) is left out of the ring and fetched after the K loop (load_tail).  Past k it then holds zeros; columns past n, or
+  // rows past m of an m-contiguous A, hold whatever follows them and must never be stored.
   const bool tail_here = FAST && !PERSIST && !CONV && !GATHER && !PAIR && p.tail_slab != 0 && kt1 == kt_total && kt1 > kt0;
   const int KT = kt1 > kt0 ? kt1 - kt0 - (tail_here ? 1 : 0) : 0;          // slabs of this workgroup in the ring (per tile)
 
@@ -1494,7 +1495,7 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
   // Loader for what the DMA path does not take: any strides, any ragged edge, zero fill.  One 16-byte chunk of the
   // slab per thread and trip: a chunk that lies inside the matrix along a unit-stride dimension is one vector load
   // at the element's own alignment, any other chunk is put together element by element.  Used for every slab of the
-  // kernels built without the DMA loader and for the left-out last slab of a tail_slab launch.
+  // kernels built without the DMA loader and for the left-out last slabs that load_tail hands on.
   // (t0: the thread's index in the workgroup, handed in so that the DMA kernels need not keep threadIdx.x alive
   // across their K loop for the one call after it)
   // The loader in two halves, so that the kernels built without the DMA loader can fetch slab t + STAGES into
@@ -1599,8 +1600,8 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
 #pragma unroll
     for (int u = 0; u < GEN_NB; ++u) gen_store_b(stage_base, t0 + u * C::THREADS, rb[u]);
   };
-  // one chunk at a time: for the prologue of the kernels without the DMA loader, and for operands of a tail_slab launch whose rows are
-  // shorter than a chunk
+  // one chunk at a time: for the prologue of the kernels without the DMA loader, and for the left-out slab of operands whose rows are
+  // shorter than a chunk or, with a row-major B, of at most one chunk of k
   auto load_slab_generic = [&](int kt_global, uint32_t stage_base, int t0) __attribute__((always_inline)) {
 #pragma unroll 1
     for (int idx = t0; idx < BM * C::CPR_A; idx += C::THREADS) gen_store_a(stage_base, idx, gen_fetch_a(kt_global, idx));
@@ -1613,7 +1614,8 @@ __global__ __launch_bounds__(C::THREADS, PERSIST ? 1 : Residency<C>::WAVES) void
   // apiece with nothing to hide it (447 x 14336 x 83 int8, BT: 11.7 -> 9.2 us; 256 x 872 x 904 8.2 -> 6.4; 1150 x 2300 x 1111 bf16 18.0 -> 17.1).
   // What lies past k is cleared; a chunk that crosses n, or m of an m-contiguous A, brings what comes after it, for columns that are never
   // stored.  Only in the matrix's last row is there nothing after it: such a chunk is fetched as the row's last 16 bytes and shifted
-  // down.  Rows and chunks that do not exist read the first one's place.
+  // down.  That the other rows do have something after them is what the layouts' pitch >= length is for (dma_layout: loose_ok).  Rows
+  // and chunks that do not exist read the first one's place.
   auto load_tail = [&](int kt_global, uint32_t stage_base, int t0) __attribute__((always_inline)) {
     const int64_t k0 = (int64_t)kt_global * BK;
     const int krem = (int)(p.k - k0);                               // 1 .. BK

@@ -182,7 +182,7 @@ def dma_layout(a, b) -> int:
     """Layout class of the operands, part of every config-memo key: 1 = row-major A and B, 2 = row-major A and
     k-contiguous B (``w.t()`` of a row-major weight), both with 16-byte aligned rows and base pointers -- the two
     layouts the direct-to-LDS loaders take as they are; 3, 4 = the same two layouts as they take them with the last K
-    slab loaded chunk by chunk (ragged K, rows off 16 bytes); 0 = anything else (the two tiles built with the element-wise loader)."""
+    slab loaded through registers (ragged K, rows off 16 bytes); 0 = anything else (the two tiles built with the element-wise loader)."""
     es = a.element_size()
     if not (a.stride(1) == 1 and a.stride(0) >= a.shape[1]):
         return 0
