@@ -99,9 +99,9 @@ template <class E> __device__ __forceinline__ void turn_run(uint32_t* v, int at,
   }
 }
 
-// UNIT: step_w is 1 (77 registers instead of 118, float32 128 instead of 158: one kernel for both lost 1 to 5 % in float32)
+// UNIT: step_w is 1 (77 registers instead of 116, float32 128 instead of 162: one kernel for both lost 1 to 5 % in float32)
 template <class E, int NT, bool UNIT>
-__global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
+__global__ __launch_bounds__(256, UNIT ? 1 : 3) void conv_pack_kernel(PackParams p) {
   const int tid = threadIdx.x;
   if (blockIdx.x < p.w_blocks) {
     const int item = blockIdx.x * 256 + tid;
@@ -163,6 +163,26 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
     const int o0 = ((img * p.c_in + cg * 8) * p.h_in + h) * p.w_in + w0;    // element of (channel 0, column 0)
     const E* src = (const E*)p.x;
     const int nch = p.c_in - cg * 8 < 8 ? p.c_in - cg * 8 : 8;
+    auto in_row = [&](int e) { return (uint32_t)(w0 + e * step_w) < (uint32_t)p.w_in; };
+    // what was read in the place of columns outside the row and of channels that do not exist
+    auto clear = [&](auto nc) {
+      constexpr int NC = nc;
+      if (w0 < 0 || w0 + 7 * step_w >= p.w_in) {
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+          const uint32_t keep = W == 8 ? (in_row(i) ? ~0u : 0u) : (in_row(2 * i) ? 0xffffu : 0u) | (in_row(2 * i + 1) ? 0xffff0000u : 0u);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) raw[c][i] &= keep;
+        }
+      }
+      if (nch < NC) {
+#pragma unroll
+        for (int c = 1; c < NC; ++c)
+#pragma unroll
+          for (int i = 0; i < W; ++i) raw[c][i] = c < nch ? raw[c][i] : 0u;
+      }
+    };
+    constexpr std::integral_constant<int, 8> eight;
     if ((UNIT || step_w == 2) && p.x_elems >= 8) {
       // All loads are on their way before the first is waited for, and no lane takes another path at the edges: a load under a
       // condition of its own is waited for at the condition's end, eight latencies in a row.  So for channels that do not exist
@@ -193,27 +213,12 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
             for (int i = 0; i < W * RUNS / STEP; ++i)
               raw[c0 + c][i] = STEP == 1 ? t[c][i] : W == 8 ? t[c][2 * i] : (t[c][2 * i] & 0xffffu) | t[c][2 * i + 1] << 16;
         }
-        if (w0 < 0 || w0 + 7 * step_w >= p.w_in) {
-          auto in_row = [&](int e) { return (uint32_t)(w0 + e * step_w) < (uint32_t)p.w_in; };
-#pragma unroll
-          for (int i = 0; i < W; ++i) {
-            const uint32_t keep = W == 8 ? (in_row(i) ? ~0u : 0u) : (in_row(2 * i) ? 0xffffu : 0u) | (in_row(2 * i + 1) ? 0xffff0000u : 0u);
-#pragma unroll
-            for (int c = 0; c < NC; ++c) raw[c][i] &= keep;
-          }
-        }
-        if (nch < NC) {
-#pragma unroll
-          for (int c = 1; c < NC; ++c)
-#pragma unroll
-            for (int i = 0; i < W; ++i) raw[c][i] = c < nch ? raw[c][i] : 0u;
-        }
+        clear(nc);
       };
       // (rows that one run covers need no second, inputs of few channels no repeats)
       constexpr std::integral_constant<int, 1> one;
       constexpr std::integral_constant<int, 2> two;
       constexpr std::integral_constant<int, 4> four;
-      constexpr std::integral_constant<int, 8> eight;
       if constexpr (UNIT) {
         if (p.c_in <= 4) fetch(four, one, one);
         else fetch(eight, one, one);
@@ -222,22 +227,69 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackParams p) {
         else fetch(eight, two, two);
       }
     } else {
-#pragma unroll 1
-      for (int c = 0; c < nch; ++c) {
-        uint16_t h16[8];
-        uint32_t t[W];
+      // Wider steps, and inputs shorter than a run: element by element, columns that a lane has not in its row read at the row's ends,
+      // channels that do not exist in the first one's place.  Up to two waves of this pass on every CU (float32: one) a wave's latency
+      // counts: all loads on their way before the first is waited for, but those of columns that no lane has.  With more it is the
+      // lines that the L1 keeps until their next column is read: a channel at a time, or in float32, whose words need no packing, all
+      // channels at once without a condition.  1x1 layers at steps of 3 and 4, both launches: 300 -> 256 channels of 14x14, batch 8, bf16
+      // 8.8 us, a channel at a time 10.5; 260 -> 256 of 56x56, batch 128, f16 37.0 and 33.6; float32 384 -> 256 of 14x14, one image 10.4 and
+      // 12.2; 512 -> 256 of 33x33, batch 32 26.4 and 23.7, all channels at once 21.8.
+      int col[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const E v = (uint32_t)(w0 + e * step_w) < (uint32_t)p.w_in ? src[o0 + c * plane + e * step_w] : (E)0;
-          if constexpr (W == 8) t[e] = __builtin_bit_cast(uint32_t, v);
-          else h16[e] = v;
-        }
-        if constexpr (W == 4) __builtin_memcpy(t, h16, 16);
-#pragma unroll
-        for (int x = 0; x < 8; ++x)
-#pragma unroll
-          for (int i = 0; i < W; ++i) raw[x][i] = x == c ? t[i] : raw[x][i];
+      for (int e = 0; e < 8; ++e) {
+        const int w = w0 + e * step_w;
+        col[e] = w < 0 ? 0 : w < p.w_in ? w : p.w_in - 1;
       }
+      auto line = [&](int c) { return src + (o0 - w0 + (c < nch ? c * plane : 0)); };
+      if (!UNIT && gridDim.x - p.w_blocks <= (W == 8 ? 64u : 128u)) {
+        bool any[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) any[e] = __builtin_amdgcn_ballot_w64(in_row(e)) != 0;
+        uint32_t t[8][8];                           // (a half in a word of its own until all are there)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const E* at = line(c);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            t[c][e] = 0;
+            if (any[e]) {
+              const E v = at[col[e]];
+              t[c][e] = W == 8 ? __builtin_bit_cast(uint32_t, (float)v) : (uint32_t)v;
+            }
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) asm("" : "+v"(t[c][e]));
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+          for (int i = 0; i < W; ++i) raw[c][i] = W == 8 ? t[c][i] : t[c][2 * i & 7] | t[c][(2 * i + 1) & 7] << 16;
+      } else if constexpr (!UNIT && W == 8) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const E* at = line(c);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) raw[c][e] = __builtin_bit_cast(uint32_t, (float)at[col[e]]);
+          __builtin_amdgcn_sched_barrier(0);        // (addresses of later channels not before: 184 registers)
+        }
+      } else {
+#pragma unroll 1
+        for (int c = 0; c < nch; ++c) {
+          const E* at = line(c);
+          E t[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[e] = at[col[e]];
+          uint32_t u[W];
+          __builtin_memcpy(u, t, sizeof u);
+#pragma unroll
+          for (int x = 0; x < 8; ++x)
+#pragma unroll
+            for (int i = 0; i < W; ++i) raw[x][i] = x == c ? u[i] : raw[x][i];
+        }
+      }
+      clear(eight);
     }
   }
 #pragma unroll
