@@ -873,7 +873,8 @@ static int packed_forward(const tnx_conv2d_args* a, const PackedPlan& pl) {
   k.whole = cpt % 8 == 0;
   k.div_taps = make_fastdiv((uint32_t)(a->filter_h * a->filter_w));
   k.cgb = (pl.cp8 + 7) / 8;
-  const int64_t x_items = (int64_t)a->batch * pl.rows * k.wchunks, waves = (x_items + 7) / 8 * k.cgb;
+  const int per_wave = 64 >> pack_cg_bits(pl.cp8);
+  const int64_t x_items = (int64_t)a->batch * pl.rows * k.wchunks, waves = (x_items + per_wave - 1) / per_wave * k.cgb;
   const int64_t w_items = (int64_t)a->c_out * k.chunks_pad;
   if (x_items >= (1ll << 31) || waves >= (1ll << 31)) return TNX_E_UNSUPPORTED;
   k.x_items = (int)x_items;

@@ -14,7 +14,7 @@
 // Bound by memory traffic: each input element is read once and written once (plus the borders).  A thread moves 8
 // channels x 8 columns: eight 16-byte loads along the rows, an 8x8 transpose of 16-bit elements in registers (32 byte
 // permutes, no LDS), eight 16-byte stores along the channels; 8 lanes are 8 neighbouring channel groups, the 8 groups of
-// lanes 8 neighbouring column chunks, so loads and stores both move 128-byte runs.  256 channels of 56x56, batch 32, bf16:
+// lanes 8 neighbouring column chunks (but see pack_cg_bits), so loads and stores both move 128-byte runs.  256 channels of 56x56, batch 32, bf16:
 // 17.9 us for 51 MB in and 55 MB out, 5.9 TB/s (a plain copy of that size: 15.7 us); with the blocks dealt round-robin to
 // the XCDs 25.3 us, with non-temporal loads 31 us.
 //
@@ -42,12 +42,17 @@ struct PackParams {
   int wchunks;                 // column chunks of 8 per packed row, counted from column `lead` (the padding before it is
   int lead;                    // written with the first chunk, that after the last input column with the last)
   bool whole;                  // a tap's channels are whole K slabs
-  int cgb;                     // blocks of 8 channel groups
+  int cgb;                     // blocks of as many channel groups as a wave has side by side (pack_cg_bits)
   int x_items, w_items;        // input: (image, row, column chunk) triples; weight: (c_out, chunk) pairs
   int x_elems;                 // elements of the input
   unsigned w_blocks;           // workgroups [0, w_blocks) lay out the weight, the others the input
   FastDiv div_cgb, div_row, div_wchunks, div_cpt, div_cp8, div_chunks, div_taps;
 };
+
+// Lanes of a wave: neighbouring channel groups by neighbouring column chunks, 8 x 8 or, with a single channel group, 1 x 64.  (With 8 x 8
+// there too seven lanes of eight had nothing to do, in eight times the waves, each of which fetches the kernel's 20 KB of
+// instructions: float32, both launches, 3 -> 80 channels of 28x28, 1x1, one image 13.4 -> 8.3 us; 5 -> 16 of 56x56, 3x3, batch 128 44.0 -> 36.3.)
+__host__ __device__ constexpr int pack_cg_bits(int cp8) { return cp8 == 1 ? 0 : 3; }
 
 // one element as its bf16 (or 16-bit) terms; side 0: input order, side 1: weight order
 template <int SIDE> __device__ __forceinline__ void pack_terms(uint16_t v, uint16_t (&t)[1]) { t[0] = v; }
@@ -147,7 +152,7 @@ __global__ __launch_bounds__(256, UNIT ? 1 : 3) void conv_pack_kernel(PackParams
   // neighbour's too, and a second L2 would have to fetch them again
   const int wave = xcd_remap(blockIdx.x - p.w_blocks, gridDim.x - p.w_blocks, 8) * 4 + (tid >> 6), lane = tid & 63;
   const int jb = (int)fd_div((uint32_t)wave, p.div_cgb), cgblk = wave - jb * p.cgb;
-  const int j = jb * 8 + (lane >> 3), cg = cgblk * 8 + (lane & 7);
+  const int cg_bits = pack_cg_bits(p.cp8), j = (jb << (6 - cg_bits)) + (lane >> cg_bits), cg = (cgblk << cg_bits) + (lane & ((1 << cg_bits) - 1));
   if (j >= p.x_items || cg >= p.cp8) return;
   const int row_all = (int)fd_div((uint32_t)j, p.div_wchunks), wc = j - row_all * p.wchunks;
   const int img = (int)fd_div((uint32_t)row_all, p.div_row), row = row_all - img * p.rows;
