@@ -69,6 +69,18 @@ def test_window_rows_hold_every_tap_of_every_tile():
         assert most <= rows and lds <= 163840, (layer, tile, narrower, most, rows)
 
 
+def test_places_behind_the_table_of_taps_are_whole_chunks():
+    """The 16-byte places that end a workgroup's LDS follow windows of whole slots and a table of 4 bytes per k step."""
+    seen = set()
+    for tile in range(FIRST, FIRST + TILES):
+        for c in range(8, 400, 8):
+            need, info = _info(_args((2, c, 12, 10, 64, 3, 3, (1, 1), (1, 1), (1, 1)), torch.bfloat16), tile)
+            if need:
+                assert info[5] % 16 == 0, (tile, c, info)
+                seen.add(tile)
+    assert len(seen) == TILES
+
+
 def test_what_the_tiles_do_not_take():
     ok = LAYERS["whole_blocks"]
     assert _info(_args(ok, torch.bfloat16), FIRST)[0] > 0 and _info(_args(ok, torch.float16), FIRST + TILES - 1)[0] > 0

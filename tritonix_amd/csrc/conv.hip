@@ -595,8 +595,7 @@ static bool halo_geom(const tnx_conv2d_args* a, int h_out, int w_out, const Halo
   if (slots > 4096 || rows * g->cpr > 128) return false;              // eight waves of 16 row pieces
   g->rows = (int)rows;
   g->buf_bytes = (int)(slots * e.slot);
-  // (behind the windows: an offset per k step, of one period past the end too, and a place per lane)
-  *lds = e.ring_bytes + 2 * g->buf_bytes + ((g->ksteps + e.ksp - 1) / e.ksp + 1) * e.ksp * 4 + 1024;
+  *lds = e.ring_bytes + 2 * g->buf_bytes + halo_table_bytes(e.ksp, (g->ksteps + e.ksp - 1) / e.ksp) + HALO_SPILL_BYTES;
   if (*lds < e.strip_bytes) *lds = e.strip_bytes;
   return *lds <= TNX_LDS_LIMIT_BYTES;
 }

@@ -44,6 +44,10 @@ template <int SLOT> __device__ __forceinline__ uint32_t halo_at(uint32_t slot_by
   return SLOT == 64 ? slot_bytes + (chunk16 ^ ((slot_bytes >> 3) & 0x20u)) : slot_bytes + chunk16;
 }
 
+// Behind the windows: an offset per k step, of one period past the end too, and from the next 16-byte boundary on a place per lane.
+__host__ __device__ constexpr int halo_table_bytes(int ksp, int periods) { return (ksp * (periods + 1) * 4 + 15) / 16 * 16; }
+constexpr int HALO_SPILL_BYTES = 64 * 16;
+
 // BM output channels x BN pixels, 8 waves; the ring holds R periods of KSP k steps
 template <class T, int BM, int BN, int KSP_, int R_, int SLOT_> struct HaloCfg {
   typedef TileCfg<T, BM, BN, 64, 8, 2> C;
@@ -130,7 +134,7 @@ __global__ __launch_bounds__(512, 2) void conv_halo_kernel(GemmParams p, HaloGeo
     t_cols = !ok ? 0 : left < used ? left : used;
     t_lds = win0 + (uint32_t)(pr * h.rowslots + (h.stride_w == 2 ? pc >> 1 : pc)) * SLOT;
   }
-  const uint32_t table = win0 + 2u * (uint32_t)h.buf_bytes, spill = table + (uint32_t)(KSP * (KT + 1) * 4) + (uint32_t)lane * 16u;
+  const uint32_t table = win0 + 2u * (uint32_t)h.buf_bytes, spill = table + (uint32_t)halo_table_bytes(KSP, KT) + (uint32_t)lane * 16u;
   const bool has_rows = wave * 16 < rows * h.cpr;         // this wave moves anything at all
   i32x4 v[8];
   auto fetch_one = [&](int c, int cb) __attribute__((always_inline)) {
