@@ -44,6 +44,21 @@ template <int SLOT> __device__ __forceinline__ uint32_t halo_at(uint32_t slot_by
   return SLOT == 64 ? slot_bytes + (chunk16 ^ ((slot_bytes >> 3) & 0x20u)) : slot_bytes + chunk16;
 }
 
+// Byte of channel c of block cb where the first channel's is `src`; and the first channel's of a lane that has no row: the tensor's end,
+// so that every channel's stays past it, where the range check drops the load.  (Not the largest number: with what the channels add it
+// wraps to a place inside the tensor.  The tensor's end does where it and an image make 4 GiB; what is read then goes to the spill place.)
+__host__ __device__ constexpr uint32_t halo_channel_at(uint32_t src, int cb, int c, int plane) {
+  return src + (uint32_t)(cb * 32 + c) * 2u * (uint32_t)plane;
+}
+__host__ __device__ constexpr uint32_t halo_nowhere(uint32_t x_bytes) { return x_bytes; }
+constexpr bool halo_nowhere_holds(uint32_t x_bytes, int c_in, int plane) {
+  for (int c = 0; c < (c_in + 31) / 32 * 32; ++c)
+    if (halo_channel_at(halo_nowhere(x_bytes), c / 32, c % 32, plane) < x_bytes) return false;
+  return true;
+}
+static_assert(halo_nowhere_holds(32u * 128 * 3136 * 2, 128, 3136) && halo_nowhere_holds(17u * 3 * 5 * 2, 17, 15) &&
+              halo_nowhere_holds(2u * 900 * 1048576 * 2, 900, 131072), "lanes without a row read nothing");
+
 // Behind the windows: an offset per k step, of one period past the end too, and from the next 16-byte boundary on a place per lane.
 __host__ __device__ constexpr int halo_table_bytes(int ksp, int periods) { return (ksp * (periods + 1) * 4 + 15) / 16 * 16; }
 constexpr int HALO_SPILL_BYTES = 64 * 16;
@@ -129,7 +144,7 @@ __global__ __launch_bounds__(512, 2) void conv_halo_kernel(GemmParams p, HaloGeo
     const int c = (tid >> 4) * 4 + (tid & 3), pr = (int)fd_div((uint32_t)c, h.div_cpr), w0 = (c - pr * h.cpr) * 8;
     const int g = row0 + pr, img = (int)fd_div((uint32_t)g, h.div_img), ih = g - img * h.rows_img - h.pad_h;
     const bool ok = pr < rows && img < h.batch && (uint32_t)ih < (uint32_t)h.h_in;
-    t_src = ok ? ((uint32_t)(img * h.c_in + cg8) * (uint32_t)h.plane + (uint32_t)(ih * h.w_in + w0)) * 2u : 0xfffffff0u;
+    t_src = ok ? ((uint32_t)(img * h.c_in + cg8) * (uint32_t)h.plane + (uint32_t)(ih * h.w_in + w0)) * 2u : halo_nowhere(x_bytes);
     const int pc = w0 + h.pad_w, left = h.w_in - w0, used = h.rowslots - pc;
     t_cols = !ok ? 0 : left < used ? left : used;
     t_lds = win0 + (uint32_t)(pr * h.rowslots + (h.stride_w == 2 ? pc >> 1 : pc)) * SLOT;
@@ -139,7 +154,7 @@ __global__ __launch_bounds__(512, 2) void conv_halo_kernel(GemmParams p, HaloGeo
   i32x4 v[8];
   auto fetch_one = [&](int c, int cb) __attribute__((always_inline)) {
     // (channels past the last one: zeros past the tensor, or whatever is there before its end, cleared by `put_begin`)
-    v[c] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, t_src + (uint32_t)(cb * 32 + c) * 2u * (uint32_t)h.plane, 0, 0);
+    v[c] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, halo_channel_at(t_src, cb, c, h.plane), 0, 0);
   };
   // even and odd columns of a chunk: neighbours, or apart where the stride is 2
   const bool strided = h.stride_w == 2, odd0 = strided && (h.pad_w & 1);
@@ -150,7 +165,7 @@ __global__ __launch_bounds__(512, 2) void conv_halo_kernel(GemmParams p, HaloGeo
     if (cb != h.blocks - 1) return;
     const int nch = h.c_in - cb * 32 - cg8;               // channels of this group that exist
     // the tensor's last chunk may end past it, and the loads drop every dword that is not whole: element by element
-    const uint32_t last = t_src + (uint32_t)(cb * 32 + nch - 1) * (uint32_t)h.plane * 2u;
+    const uint32_t last = halo_channel_at(t_src, cb, nch - 1, h.plane);
     const bool over = t_cols > 0 && nch > 0 && nch <= 8 && last + 16u > x_bytes;
     if (__builtin_amdgcn_ballot_w64(over) != 0) {
       uint16_t e[8];
