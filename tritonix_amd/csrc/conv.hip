@@ -4,6 +4,9 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <new>
+#include <unordered_map>
+
 #include "../../include/tritonix_hip.h"
 #include "conv_halo.h"
 #include "conv_pack.h"
@@ -557,11 +560,10 @@ static const HaloCost HALO_COST[] = {
 
 static int gcd(int a, int b) { while (b) { const int t = a % b; a = b; b = t; } return a; }
 
-// The layer as tiles of `width` pixels (a multiple of 8, at most e.bn) see it, and the LDS of a workgroup; false: not with this tile.
-static bool halo_geom(const tnx_conv2d_args* a, int h_out, int w_out, const HaloEntry& e, int width, HaloGeom* g, int* lds) {
-  if (a->filter_h < 2 || a->filter_w < 2 || a->stride_w > 2 || width < 8) return false;
+// What of the geometry is the layer's; false: not with any tile.
+static bool halo_layer(const tnx_conv2d_args* a, int h_out, int w_out, HaloGeom* g) {
+  if (a->filter_h < 2 || a->filter_w < 2 || a->stride_w > 2) return false;
   *g = HaloGeom{};
-  g->width = width;
   g->c_in = a->c_in; g->h_in = a->h_in; g->w_in = a->w_in; g->plane = a->h_in * a->w_in;
   g->batch = a->batch; g->x_elems = (int)((int64_t)a->batch * a->c_in * g->plane);
   g->stride_h = a->stride_h; g->stride_w = a->stride_w; g->pad_h = a->pad_h; g->pad_w = a->pad_w;
@@ -577,22 +579,34 @@ static bool halo_geom(const tnx_conv2d_args* a, int h_out, int w_out, const Halo
   g->hw_out = h_out * w_out; g->hwp = (g->hw_out + 7) / 8 * 8; g->w_out = w_out;
   g->cpr = (a->w_in + 7) / 8;
   g->ksteps = g->blocks * g->taps;
-  // the next block's window has to wait for the block before the present one, and be there a period before its own first read
-  if (g->ksteps <= e.ksp || (g->blocks > 1 && g->taps < 2 * e.ksp)) return false;
-  // Rows of the largest window: from the first to the last pixel of a tile.  Inside an image the first pixel's column is a
-  // multiple of `step`; over c image ends each adds an image's rows and takes the pixels of one (hwp - hw_out of them lie in no row)
-  const int step = gcd(gcd(width, g->hwp), w_out);
-  int64_t most = (int64_t)((w_out - step + width - 1) / w_out) * a->stride_h;
+  return true;
+}
+
+// Rows of the largest window of tiles of `width` pixels: from the first to the last pixel of a tile.  Inside an image the first pixel's
+// column is a multiple of `step`; over c image ends each adds an image's rows and takes the pixels of one (hwp - hw_out of them lie in
+// no row)
+static int64_t halo_rows(const HaloGeom& g, int h_out, int width) {
+  const int64_t span = (int64_t)(g.fh - 1) * g.dil_h + 1, rows_img = g.rows_img;
+  const int w_out = g.w_out, common = gcd(width, g.hwp), step = gcd(common, w_out);
+  int64_t most = (int64_t)((w_out - step + width - 1) / w_out) * g.stride_h;
   if (most > rows_img - span) most = rows_img - span;
-  const int ends = (g->hwp - gcd(width, g->hwp) + width - 1) / g->hwp;
+  const int ends = (g.hwp - common + width - 1) / g.hwp;
   for (int c = 1; c <= ends; ++c) {
-    const int left = width - 1 - c * g->hwp;            // pixels from the first one's place in its image to the last one's
-    const int64_t down = (left >= 0 ? (left + w_out - 1) / w_out : -(-left / w_out)) + (g->hwp != g->hw_out ? 1 : 0);
-    const int64_t d = c * rows_img + (down < h_out - 1 ? down : h_out - 1) * a->stride_h;
+    const int left = width - 1 - c * g.hwp;             // pixels from the first one's place in its image to the last one's
+    const int64_t down = (left >= 0 ? (left + w_out - 1) / w_out : -(-left / w_out)) + (g.hwp != g.hw_out ? 1 : 0);
+    const int64_t d = c * rows_img + (down < h_out - 1 ? down : h_out - 1) * g.stride_h;
     if (d > most) most = d;
   }
-  const int64_t rows = most + span, slots = rows * g->rowslots;
+  return most + span;
+}
+
+// The layer as tiles of `width` pixels, whose largest window has `rows` rows, see it, and the LDS of a workgroup; false: not with this tile.
+static bool halo_tile(const HaloEntry& e, int width, int64_t rows, HaloGeom* g, int* lds) {
+  // the next block's window has to wait for the block before the present one, and be there a period before its own first read
+  if (g->ksteps <= e.ksp || (g->blocks > 1 && g->taps < 2 * e.ksp)) return false;
+  const int64_t slots = rows * g->rowslots;
   if (slots > 4096 || rows * g->cpr > 128) return false;              // eight waves of 16 row pieces
+  g->width = width;
   g->rows = (int)rows;
   g->buf_bytes = (int)(slots * e.slot);
   *lds = e.ring_bytes + 2 * g->buf_bytes + halo_table_bytes(e.ksp, (g->ksteps + e.ksp - 1) / e.ksp) + HALO_SPILL_BYTES;
@@ -669,9 +683,11 @@ static bool make_packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile, 
   const int64_t lim = (1ll << 31) - 4096;
   int nh = 0;
   const HaloEntry* const* he = tnx_halo_entries(&nh);
+  HaloGeom layer;
+  const bool windows = !f32 && (tile < 0 || tile >= HALO_FROM) && halo_layer(a, h_out, w_out, &layer);
   auto take_halo = [&](const HaloEntry* e, int width) {
-    HaloPlan h = {e};
-    if (!halo_geom(a, h_out, w_out, *e, width, &h.g, &h.lds)) return false;
+    HaloPlan h = {e, layer};
+    if (width < 8 || !halo_tile(*e, width, halo_rows(layer, h_out, width), &h.g, &h.lds)) return false;
     h.g.div_img = make_fastdiv((uint32_t)h.g.rows_img);
     h.g.div_hwp = make_fastdiv((uint32_t)h.g.hwp);
     h.g.div_w = make_fastdiv((uint32_t)w_out);
@@ -687,7 +703,7 @@ static bool make_packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile, 
   if (tile >= HALO_FROM) {
     int left = tile - HALO_FROM;
     for (int i = 0; i < nh; ++i)
-      if (!f32 && he[i]->dtype == a->dtype && left-- == 0 && take_halo(he[i], he[i]->bn - (split - 1) * 8)) {
+      if (windows && he[i]->dtype == a->dtype && left-- == 0 && take_halo(he[i], he[i]->bn - (split - 1) * 8)) {
         p->split = p->terms = 1;
         p->total_bytes = up256(p->halo.w_bytes);
         return true;
@@ -747,11 +763,12 @@ static bool make_packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile, 
   // 387 as windows).  128 of 64, 28x28, 3x3, 64 out: 28.8 and 18.6; 32 of 256, 56x56, 256 out: 114 and 99; 32 of 128, 56x56, stride 2,
   // 128 out: 22.1 and 17.1; 32 of 512, 14x14, 512 out: 41.3 and 43.0.
   bool halo = false;
-  if (!f32 && tile < 0 && a->c_in * 100 >= (a->c_in + 31) / 32 * 32 * 88) {
+  if (windows && tile < 0 && a->c_in * 100 >= (a->c_in + 31) / 32 * 32 * 88) {
     const double margin = 0.9 * (w_out % 8 ? 0.92 : 1.0) * (a->filter_w == 2 ? 0.9 : 1.0);
     double best_halo = margin * packed_time(a, best, (double)p->x_bytes, (double)p->w_bytes, h_out, w_out);
     const HaloEntry* chosen = nullptr;
     int chosen_width = 0;
+    int64_t rows_of[256 / 8 + 1] = {};           // by width / 8: most tiles share theirs
     for (int i = 0; i < nh; ++i) {
       const HaloEntry& e = *he[i];
       if (e.dtype != a->dtype) continue;
@@ -763,9 +780,10 @@ static bool make_packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile, 
       const bool rows_too = whole < e.bn && whole >= 0.7 * e.bn && h_out * w_out % 8 == 0;
       for (int width : {e.bn, rows_too ? whole : 0}) {
         if (!cost || !width) continue;
-        HaloGeom g;
+        HaloGeom g = layer;
         int lds;
-        if (!halo_geom(a, h_out, w_out, e, width, &g, &lds)) continue;
+        if (!rows_of[width / 8]) rows_of[width / 8] = halo_rows(layer, h_out, width);
+        if (!halo_tile(e, width, rows_of[width / 8], &g, &lds)) continue;
         const double t = halo_time(a, *cost, g, p->n_total, lds);
         if (t < best_halo) { best_halo = t; chosen = &e; chosen_width = width; }
       }
@@ -782,27 +800,51 @@ static bool make_packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile, 
   return true;
 }
 
-// The library's own plans of the layers a thread met last, by their sizes: pricing them takes longer than a launch.
+// The library's own plans of the layers a thread has met, by their sizes: pricing one takes 2.3 us, finding it 0.1.  512 layers, more than
+// a network has of different ones (at about 500 bytes each), and from the first again once they are full.
+namespace {
+struct LayerKey {
+  int32_t v[22];
+  bool operator==(const LayerKey& o) const { return memcmp(v, o.v, sizeof v) == 0; }
+};
+struct LayerHash {
+  size_t operator()(const LayerKey& k) const {
+    uint64_t h = 0x9e3779b97f4a7c15ull;
+    for (int i = 0; i < 22; i += 2) {
+      uint64_t w;
+      memcpy(&w, k.v + i, 8);
+      h = (h ^ w) * 0xff51afd7ed558ccdull;
+      h ^= h >> 32;
+    }
+    return (size_t)h;
+  }
+};
+struct KnownPlan {
+  bool taken;
+  PackedPlan plan;
+};
+constexpr size_t MOST_PLANS = 512;
+}  // namespace
+
 static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, int split = 1) {
   if (!a || tile >= 0) return make_packed_plan(a, p, tile, split);
-  struct Known {
-    int32_t key[22];
-    bool taken;
-    PackedPlan plan;
-  };
-  static thread_local Known known[16];
-  const int32_t key[22] = {1, a->batch, a->c_in, a->h_in, a->w_in, a->c_out, a->filter_h, a->filter_w, a->stride_h, a->stride_w, a->pad_h, a->pad_w,
-                           a->dil_h, a->dil_w, a->dtype, a->out_f32 != 0, a->bias ? 1 + a->bias_dtype : 0, a->block_pixels, a->block_cout, a->block_k,
-                           a->group_pixels, a->loader};
-  uint32_t h = 0;
-  for (int32_t v : key) h = (h ^ (uint32_t)v) * 0x01000193u;
-  Known& k = known[(h >> 16 ^ h) % 16];
-  if (memcmp(k.key, key, sizeof key)) {
-    k.taken = make_packed_plan(a, &k.plan, -1, 1);
-    memcpy(k.key, key, sizeof key);
+  static thread_local std::unordered_map<LayerKey, KnownPlan, LayerHash> known;
+  const LayerKey key = {{a->batch, a->c_in, a->h_in, a->w_in, a->c_out, a->filter_h, a->filter_w, a->stride_h, a->stride_w, a->pad_h, a->pad_w,
+                         a->dil_h, a->dil_w, a->dtype, a->out_f32 != 0, a->bias ? 1 + a->bias_dtype : 0, a->block_pixels, a->block_cout, a->block_k,
+                         a->group_pixels, a->loader, 0}};
+  const auto hit = known.find(key);
+  if (hit != known.end()) {
+    *p = hit->second.plan;
+    return hit->second.taken;
   }
-  *p = k.plan;
-  return k.taken;
+  *p = PackedPlan{};
+  const bool taken = make_packed_plan(a, p, -1, 1);
+  try {
+    if (known.size() >= MOST_PLANS) known.clear();
+    known.emplace(key, KnownPlan{taken, *p});
+  } catch (const std::bad_alloc&) {              // no room to keep it: made again by the next call
+  }
+  return taken;
 }
 
 extern "C" size_t tnx_conv2d_workspace_bytes(const tnx_conv2d_args* a) {
