@@ -82,6 +82,9 @@ def test_what_a_bias_or_a_tile_changes():
     assert taken[0] > 0
     a.bias, a.bias_dtype = 4096, 17              # never dereferenced: a type that there is not
     assert _plan(a)[0] == 0
+    for dtype in (_C.F16, _C.BF16, _C.F32):
+        a.bias_dtype = dtype
+        assert _plan(a) == taken == _in_a_new_thread(lambda: _plan(a))
     a.bias = None
     a.block_cout, a.block_pixels, a.block_k = 128, 64, 64
     assert _plan(a)[0] == 0

@@ -829,8 +829,10 @@ constexpr size_t MOST_PLANS = 512;
 static bool packed_plan(const tnx_conv2d_args* a, PackedPlan* p, int tile = -1, int split = 1) {
   if (!a || tile >= 0) return make_packed_plan(a, p, tile, split);
   static thread_local std::unordered_map<LayerKey, KnownPlan, LayerHash> known;
+  // (of a bias only whether its type is one that there is: the workspace is asked for without it)
+  const bool odd_bias = a->bias && a->bias_dtype != TNX_F16 && a->bias_dtype != TNX_BF16 && a->bias_dtype != TNX_F32;
   const LayerKey key = {{a->batch, a->c_in, a->h_in, a->w_in, a->c_out, a->filter_h, a->filter_w, a->stride_h, a->stride_w, a->pad_h, a->pad_w,
-                         a->dil_h, a->dil_w, a->dtype, a->out_f32 != 0, a->bias ? 1 + a->bias_dtype : 0, a->block_pixels, a->block_cout, a->block_k,
+                         a->dil_h, a->dil_w, a->dtype, a->out_f32 != 0, odd_bias, a->block_pixels, a->block_cout, a->block_k,
                          a->group_pixels, a->loader, 0}};
   const auto hit = known.find(key);
   if (hit != known.end()) {
