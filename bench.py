@@ -446,19 +446,14 @@ def graph_replay_ms(torch, bind, per_graph=100, replays=20):
         return None
 
 
-def default_loader(conv_args):
-    """Which of the conv2d kernels a launch with these arguments runs (tnx_conv_loader), by asking the library."""
+def conv_route(conv_args):
+    """Which of the conv2d kernels a launch with these arguments runs, by asking the library."""
     import ctypes
 
     from tritonix_amd import _C
 
-    if conv_args.workspace:
-        return 4                             # scratch was asked for: the packed kernels
-    probe = type(conv_args).from_buffer_copy(conv_args)
-    if probe.loader:
-        return probe.loader
-    probe.loader = _C.CONV_LOADER_DMA        # with a tile given, "auto" takes the direct-to-LDS kernel whenever it is allowed
-    return _C.CONV_LOADER_DMA if _C.load().tnx_conv2d_supported(ctypes.byref(probe)) == _C.OK else _C.CONV_LOADER_REGISTERS
+    return {_C.CONV_ROUTE_REGISTERS: "registers", _C.CONV_ROUTE_DMA: "dma", _C.CONV_ROUTE_GEMM: "gemm", _C.CONV_ROUTE_PACKED: "packed",
+            _C.CONV_ROUTE_WINDOW: "window"}[_C.load().tnx_conv2d_route(ctypes.byref(conv_args), None)]
 
 
 def extras(torch, dev, oracle, mm, sg, args, operands, wanted):
@@ -645,7 +640,7 @@ def extras(torch, dev, oracle, mm, sg, args, operands, wanted):
                                                     gm, gn, gk, **cfg)
             r = measure(name, lambda i: lc(), flops, bytes_, "bf16", "mfma")
             r["tile"] = cfg
-            r["loader"] = {1: "registers", 2: "dma", 3: "gemm", 4: "packed"}[default_loader(lc.args)]
+            r["loader"] = conv_route(lc.args)
             r["workload"] = (f"conv2d forward bf16: input [{n_},{c_},{hw_},{hw_}], weight [{k_},{c_},{f_},{f_}], bias, "
                              f"stride {st_}, padding {pd_}")
             ref = oracle.reference_conv2d(x_cpu[5:6], w_cpu, b_cpu, *geo)

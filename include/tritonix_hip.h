@@ -291,12 +291,24 @@ size_t tnx_conv2d_workspace_bytes(const tnx_conv2d_args* args);
 
 /* For tests and tooling: the packed route with tile number `tile` of the type's table (bfloat16's for TNX_F32; counted from
  * 0, the tiles of 32 output channels and of small rings from 32) and `split` K slices (1 to 16) instead of the library's choice, on any layer the route can lay out; tile < 0 asks for
- * that choice.  _info: its scratch bytes, or 0 where there is none, and in info[6] output channels and pixels per
+ * the tile that the library would give the layer on this route, also where tnx_conv2d_forward takes the windows instead (tnx_conv2d_route
+ * tells).  _info: its scratch bytes, or 0 where there is none, and in info[6] output channels and pixels per
  * tile, waves, ring slots, K slices, and bf16 terms per element.  _forward: launches it in args->workspace.
  * Tiles from 64 on are those that take their windows from the tensor: `split` - 1 is by how many groups of 8 pixels a tile is narrower
  * than it can be, and info[4] and info[5] are the rows of the largest window and a workgroup's LDS bytes. */
 size_t tnx_conv2d_packed_info(const tnx_conv2d_args* args, int tile, int split, int32_t* info);
 int tnx_conv2d_packed_forward(const tnx_conv2d_args* args, int tile, int split);
+
+/* For tests and tooling: which kernels tnx_conv2d_forward runs for these args (of the pointers only the alignment counts, and of the
+ * workspace whether there is one), or 0 where it would refuse them.  info (may be NULL): output channels and pixels per tile, K slices. */
+enum tnx_conv_route {
+  TNX_CONV_ROUTE_REGISTERS = 1,   /* the loaders of tnx_conv_loader ... */
+  TNX_CONV_ROUTE_DMA = 2,
+  TNX_CONV_ROUTE_GEMM = 3,
+  TNX_CONV_ROUTE_PACKED = 4,      /* ... and with a workspace: input and weight laid out and one GEMM, */
+  TNX_CONV_ROUTE_WINDOW = 5       /* or the weight laid out and the input taken from the tensor */
+};
+int tnx_conv2d_route(const tnx_conv2d_args* args, int32_t info[3]);
 
 /* TNX_OK if tnx_conv2d_forward would accept these args (pointers are not inspected, apart from their
  * alignment), otherwise the status it would return.  Pure host arithmetic. */

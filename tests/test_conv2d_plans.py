@@ -11,7 +11,7 @@ from tritonix_amd import _C
 def _layers(count, seed):
     rng, out, seen = random.Random(seed), [], set()
     while len(out) < count:
-        f, batch, c, k, hw = rng.choice([2, 3, 3, 5]), rng.choice([1, 8, 32]), rng.randrange(32, 513, 8), rng.randrange(32, 513, 8), rng.randint(7, 60)
+        f, batch, c, k, hw = rng.choice([2, 3, 3, 5]), rng.choice([1, 8, 32]), rng.randrange(32, 257, 32), rng.randrange(32, 513, 8), rng.choice([8, 14, 16, 28, 32, 48, 56])
         stride, dtype = rng.choice([1, 1, 2]), rng.choice([_C.BF16, _C.F16, _C.F32])
         if (f, batch, c, k, hw, stride, dtype) in seen:
             continue
@@ -27,9 +27,12 @@ def _layers(count, seed):
 
 
 def _plan(a):
-    info = (ctypes.c_int32 * 6)()
+    info, tile = (ctypes.c_int32 * 6)(), (ctypes.c_int32 * 3)()
     lib = _C.load()
-    return lib.tnx_conv2d_workspace_bytes(ctypes.byref(a)), lib.tnx_conv2d_packed_info(ctypes.byref(a), -1, 1, info), tuple(info)
+    need, again = lib.tnx_conv2d_workspace_bytes(ctypes.byref(a)), lib.tnx_conv2d_packed_info(ctypes.byref(a), -1, 1, info)
+    given = _C.Conv2dArgs.from_buffer_copy(a)
+    given.workspace = 4096                       # never dereferenced
+    return need, again, tuple(info), lib.tnx_conv2d_route(ctypes.byref(given), tile), tuple(tile)
 
 
 def _in_a_new_thread(fn):
@@ -58,7 +61,9 @@ def test_every_layer_of_a_network_keeps_its_plan():
 
 
 def test_kept_plans_are_the_ones_made_first():
-    layers = _layers(700, 2)                     # more than are kept
+    layers = _layers(700, 2)                     # more than are kept, on both routes
+    routes = [_plan(a)[3] for a in layers]
+    assert min(routes.count(_C.CONV_ROUTE_PACKED), routes.count(_C.CONV_ROUTE_WINDOW)) >= 50          # (66 of the drawn ones)
     rng = random.Random(3)
     for rounds in range(3):
         order = list(range(len(layers)))

@@ -81,6 +81,31 @@ def test_places_behind_the_table_of_taps_are_whole_chunks():
     assert len(seen) == TILES
 
 
+def _route(layer, dtype, workspace=True):
+    a, tile = _args(layer, dtype), (ctypes.c_int32 * 3)()
+    a.workspace = 4096 if workspace else None               # never dereferenced
+    return _C.load().tnx_conv2d_route(ctypes.byref(a), tile), tuple(tile)
+
+
+def test_which_route_a_call_takes():
+    bf16, unit = torch.bfloat16, ((1, 1), (1, 1), (1, 1))
+    # layers that the margins leave to the windows by far, and tiles that were built for them
+    for layer in ((32, 256, 56, 56, 256, 3, 3) + unit, (32, 128, 56, 56, 128, 3, 3, (2, 2), (1, 1), (1, 1)), (32, 128, 28, 28, 128, 3, 3) + unit,
+                  (128, 64, 28, 28, 64, 3, 3) + unit):
+        for dtype in (bf16, torch.float16):
+            route, (bm, width, cut) = _route(layer, dtype)
+            tiles = [info for info in (_info(_args(layer, dtype), t)[1] for t in range(FIRST, FIRST + TILES)) if info[0] == bm and info[1] >= width]
+            assert route == _C.CONV_ROUTE_WINDOW and width % 8 == 0 and tiles and cut == 1
+        assert _route(layer, torch.float32)[0] == _C.CONV_ROUTE_PACKED
+        assert _route(layer, bf16, workspace=False)[0] in (_C.CONV_ROUTE_DMA, _C.CONV_ROUTE_REGISTERS)
+    # one row or column of taps, channels that are a fifth padding, few outputs
+    for layer in ((32, 128, 28, 28, 128, 1, 3) + unit, (32, 128, 28, 28, 128, 3, 1) + unit, (32, 40, 56, 56, 128, 3, 3) + unit, (1, 512, 7, 7, 512, 3, 3) + unit,
+                  (32, 256, 56, 56, 256, 1, 1, (2, 2), (0, 0), (1, 1))):
+        assert _route(layer, bf16)[0] == _C.CONV_ROUTE_PACKED, layer
+    assert _route((32, 256, 56, 56, 256, 1, 1, (1, 1), (0, 0), (1, 1)), bf16)[0] == _C.CONV_ROUTE_GEMM
+    assert _route((1, 8, 2, 2, 8, 5, 5, (1, 1), (0, 0), (1, 1)), bf16) == (0, (0, 0, 0))
+
+
 def test_what_the_tiles_do_not_take():
     ok = LAYERS["whole_blocks"]
     assert _info(_args(ok, torch.bfloat16), FIRST)[0] > 0 and _info(_args(ok, torch.float16), FIRST + TILES - 1)[0] > 0
@@ -160,8 +185,20 @@ def test_binary32_output_and_bias(device, problems):
 
 @pytest.mark.gpu
 def test_the_route_is_taken_by_the_call_and_replays(device, monkeypatch):
-    """A layer the library's choice gives to the window tiles, through the public call, in a graph with new operands for each replay."""
+    """A layer the library's choice gives to the window tiles, through the public call, in a graph with new operands for each replay: the bits
+    are those of a window tile (any of them sums in the same order), which are not the packed route's."""
     monkeypatch.setenv("TRITONIX_AUTOTUNE", "0")
+    layer = (32, 128, 28, 28, 128, 3, 3, (1, 1), (1, 1), (1, 1))
+    route, (bm, _, _) = _route(layer, torch.bfloat16)
+    assert route == _C.CONV_ROUTE_WINDOW
+
+    def forced(tile):
+        a, out = _args(layer, torch.bfloat16), torch.empty(32, 128, 28, 28, dtype=torch.bfloat16, device=device)
+        need, info = _info(a, tile)
+        _bind(a, x, w, None, out, torch.empty(need, dtype=torch.uint8, device=device))
+        assert _C.load().tnx_conv2d_packed_forward(ctypes.byref(a), tile, 1) == _C.OK
+        return out, info
+
     x, w = torch.randn(32, 128, 28, 28, device=device).bfloat16(), (torch.randn(128, 128, 3, 3, device=device) / 34).bfloat16()
     args = (x, w, None, (1, 1), (1, 1), (1, 1))
     conv2d_forward(*args)
@@ -175,6 +212,8 @@ def test_the_route_is_taken_by_the_call_and_replays(device, monkeypatch):
         eager = conv2d_forward(*args)
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+        window, info = forced(next(t for t in range(FIRST, FIRST + TILES) if _info(_args(layer, torch.bfloat16), t)[1][0] == bm))
+        assert info[0] == bm and torch.equal(out, window) and not torch.equal(out, forced(-1)[0])
         ref = torch.nn.functional.conv2d(x[:2].cpu().double(), w.cpu().double(), None, 1, 1)
         assert ((out[:2].cpu().double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1152 * 2.0 ** -24 * 40).all()
 

@@ -29,12 +29,14 @@ OK, E_INVALID, E_UNSUPPORTED, E_LDS, E_WORKSPACE, E_HIP, E_STATIC_LIMIT = 0, 1, 
 STATIC_WORKSPACE_BYTES = 65536 + (32 << 20)
 # enum tnx_conv_loader
 CONV_LOADER_AUTO, CONV_LOADER_REGISTERS, CONV_LOADER_DMA, CONV_LOADER_GEMM = 0, 1, 2, 3
+# enum tnx_conv_route
+CONV_ROUTE_REGISTERS, CONV_ROUTE_DMA, CONV_ROUTE_GEMM, CONV_ROUTE_PACKED, CONV_ROUTE_WINDOW = 1, 2, 3, 4, 5
 
 EXPORTS = ("tnx_gemm", "tnx_gemm_static_workspace", "tnx_gemm_workspace_bytes", "tnx_gemm_lds_bytes", "tnx_gemm_supported",
            "tnx_gemm_default_config", "tnx_gemm_f32_config", "tnx_tile_coords", "tnx_split_f32", "tnx_gemm_f32_scratch_bytes",
            "tnx_gemm_f32", "tnx_gemm_tail_slabs", "tnx_kernel_count", "tnx_kernel_name", "tnx_strerror",
            "tnx_last_hip_error", "tnx_version", "tnx_conv2d_forward", "tnx_conv2d_workspace_bytes",
-           "tnx_conv2d_packed_info", "tnx_conv2d_packed_forward", "tnx_conv2d_supported",
+           "tnx_conv2d_packed_info", "tnx_conv2d_packed_forward", "tnx_conv2d_route", "tnx_conv2d_supported",
            "tnx_conv2d_output_size",
            "tnx_conv2d_default_config", "tnx_conv2d_kernel_count", "tnx_conv2d_kernel_name")
 
@@ -131,6 +133,8 @@ def load() -> ctypes.CDLL:
     lib.tnx_conv2d_packed_info.restype = ctypes.c_size_t
     lib.tnx_conv2d_packed_forward.argtypes = [cp, ctypes.c_int, ctypes.c_int]
     lib.tnx_conv2d_packed_forward.restype = ctypes.c_int
+    lib.tnx_conv2d_route.argtypes = [cp, ctypes.POINTER(ctypes.c_int32)]
+    lib.tnx_conv2d_route.restype = ctypes.c_int
     lib.tnx_conv2d_workspace_bytes.argtypes = [cp]
     lib.tnx_conv2d_workspace_bytes.restype = ctypes.c_size_t
     lib.tnx_conv2d_output_size.argtypes = [cp, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]

@@ -1001,8 +1001,27 @@ static int packed_launch(const tnx_conv2d_args* a, const PackedPlan& pl) {
 extern "C" int tnx_conv2d_packed_forward(const tnx_conv2d_args* a, int tile, int split) {
   PackedPlan pl;
   if (!packed_plan(a, &pl, tile, split)) return TNX_E_UNSUPPORTED;
-  if (tile < 0) pl.halo.e = nullptr;           // the packed route's own choice
+  if (tile < 0) pl.halo.e = nullptr;           // this route's tile, whichever the layer takes
   return packed_launch(a, pl);
+}
+
+extern "C" int tnx_conv2d_route(const tnx_conv2d_args* a, int32_t info[3]) {
+  PackedPlan pl;
+  Resolved r;
+  int route = 0, tile[3] = {0, 0, 1};
+  if (a && a->workspace && packed_plan(a, &pl)) {
+    const HaloEntry* w = pl.halo.e;
+    route = w ? TNX_CONV_ROUTE_WINDOW : TNX_CONV_ROUTE_PACKED;
+    tile[0] = w ? w->bm : pl.e->bm;
+    tile[1] = w ? pl.halo.g.width : pl.e->bn;
+    tile[2] = w ? 1 : pl.split;
+  } else if (resolve(a, &r, true) == TNX_OK) {
+    route = r.gemm ? TNX_CONV_ROUTE_GEMM : r.dma ? TNX_CONV_ROUTE_DMA : TNX_CONV_ROUTE_REGISTERS;
+    tile[0] = r.bcout;
+    tile[1] = r.bpix;
+  }
+  if (info && route) memcpy(info, tile, sizeof tile);
+  return route;
 }
 
 extern "C" int tnx_conv2d_supported(const tnx_conv2d_args* a) {
