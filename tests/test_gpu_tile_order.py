@@ -1,5 +1,6 @@
 """Every tile of the grid is computed once in whatever order a workgroup finds it: groups of rows that do not divide the tiles, of one
-row, larger than the grid, up to the largest int32; tiles cut along K, all of them and the last ones only; many problems in one grid.
+row, larger than the grid, up to the largest int32; tiles cut along K, all of them and the last ones only.  (Several problems in one
+grid: test_several_problems.py.)
 
 int8 products are exact, so every comparison is for equality with the int64 product."""
 import ctypes
