@@ -277,7 +277,8 @@ enum tnx_conv_loader {
   TNX_CONV_LOADER_GEMM = 3
 };
 
-/* Launch one conv2d forward.  Returns a tnx_status.  Asynchronous, allocates nothing. */
+/* Launch one conv2d forward.  Returns a tnx_status.  Asynchronous, allocates no device memory.  (What it decides about a layer's sizes it
+ * keeps, per thread and of up to 512 layers.) */
 int tnx_conv2d_forward(const tnx_conv2d_args* args);
 
 /* Scratch bytes of the packed route for these args (TNX_CONV_LOADER_AUTO and no tile given), or 0 where the library
